@@ -91,6 +91,42 @@ __device__ inline uint64_t wave_sum(uint64_t v) {
   for (int m = 1; m < kWave; m <<= 1) v += shfl_xor64(v, m);
   return v;
 }
+// 64 x 64 bit transpose across a wave: lane r passes row r, lane c gets column c (bit r of it =
+// bit c of row r). Block swaps of halving size, 32 to 1: for size j, lane l and l ^ j exchange the
+// half of every 2j bits that the other keeps. About 35 vector instructions, against 64 ballots.
+__device__ inline uint64_t wave_transpose(uint64_t row) {
+  const uint32_t lane = lane_id();
+  const auto halves =
+      __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(row), static_cast<uint32_t>(row >> 32), false, false);
+  uint32_t t[2] = {halves[0], halves[1]};
+  // One step on 32-bit words: keep the bits of m (upper lanes: the others), take the partner's
+  // word y rotated by j for the rest.
+  const auto step = [&](uint32_t j, uint32_t m, uint32_t v, uint32_t y) {
+    const bool up = lane & j;
+    const uint32_t keep = up ? ~m : m;
+    const uint32_t turned = __builtin_amdgcn_alignbit(y, y, up ? j : 32 - j);
+    return (v & keep) | (turned & ~keep);
+  };
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    uint32_t v = t[k];
+    const auto rows = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // [0]: even rows twice, [1]: odd rows
+    v = step(16, 0x0000FFFFu, v, (lane & 16) ? rows[0] : rows[1]);
+    const int x8 = static_cast<int>(v);
+    v = step(8, 0x00FF00FFu, v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x8, 0x128, 0xF, 0xF, true)));  // row_ror:8
+    const int x4 = static_cast<int>(v);
+    const int up4 = __builtin_amdgcn_update_dpp(0, x4, 0x104, 0xF, 0x5, false);  // row_shl:4, banks 0 and 2
+    v = step(4, 0x0F0F0F0Fu, v,
+             static_cast<uint32_t>(__builtin_amdgcn_update_dpp(up4, x4, 0x114, 0xF, 0xA, false)));  // row_shr:4
+    const int x2 = static_cast<int>(v);
+    v = step(2, 0x33333333u, v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x2, 0x4E, 0xF, 0xF, true)));  // quad 2301
+    const int x1 = static_cast<int>(v);
+    v = step(1, 0x55555555u, v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x1, 0xB1, 0xF, 0xF, true)));  // quad 1032
+    t[k] = v;
+  }
+  return (static_cast<uint64_t>(t[1]) << 32) | t[0];
+}
+
 // Orders LDS accesses of one wave across lanes (no cross-wave effect).
 __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

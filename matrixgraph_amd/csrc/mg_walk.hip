@@ -2212,24 +2212,138 @@ __global__ void __launch_bounds__(kBlock) chunk_bits_kernel(const Chunk* __restr
   if (threadIdx.x == 0) bits_out[blockIdx.x] = static_cast<uint32_t>(s_bits);
 }
 
-// Export tile (xr, y) of X_k in the reference orientation: X tile word c (source xr*64+c)
-// bit r (vertex y*64+r) = bit c of vertex-major word w0+xr of vertex y*64+r.
-__global__ void __launch_bounds__(kBlock) export_tiles_kernel(const uint32_t* __restrict__ row_idx,
-                                                              const uint32_t* __restrict__ col_idx, uint32_t n_tiles,
-                                                              const uint64_t* __restrict__ x, uint32_t W, uint32_t w0,
-                                                              const uint32_t* __restrict__ map,
-                                                              uint64_t* __restrict__ out) {
+// Export of X_k in the reference orientation: tile (xr, y) word c (source xr*64+c) bit r (vertex
+// y*64+r) = bit c of vertex-major word w0+xr of vertex y*64+r, for the structural tiles (bit
+// w0+xr of S_k of the strip). Tile rows xr < rows <= 64; groups of 64 vertex strips.
+//
+// Occupancy of each group: mask[xr*n_groups + g], bit i = strip 64g+i has a tile in row xr, and
+// its popcount.
+__global__ void __launch_bounds__(kBlock) export_mask_kernel(const uint64_t* __restrict__ s_in, uint32_t n_strips,
+                                                             const uint32_t* __restrict__ map, uint32_t w0,
+                                                             uint32_t rows, uint32_t n_groups,
+                                                             uint64_t* __restrict__ mask, uint32_t* __restrict__ count) {
   const uint32_t lane = lane_id();
-  const uint32_t n_waves = gridDim.x * kWaves;
-  for (uint32_t i = read_first_lane(blockIdx.x * kWaves + threadIdx.x / kWave); i < n_tiles; i += n_waves) {
-    const uint32_t xr = row_idx[i], y = col_idx[i];
-    const uint64_t w = x[engine_row(map, static_cast<uint64_t>(y) * 64 + lane) * W + w0 + xr];
-    uint64_t mine = 0;
-    for (int c = 0; c < 64; ++c) {
-      const uint64_t m = ballot((w >> c) & 1);
-      if (lane == static_cast<uint32_t>(c)) mine = m;
+  const uint32_t g = blockIdx.x * kWaves + threadIdx.x / kWave;
+  if (g >= n_groups) return;
+  const uint32_t y = g * 64 + lane;
+  const uint64_t s = y < n_strips ? s_in[map ? map[y] : y] : 0ull;
+  const uint64_t m = wave_transpose(s >> w0);  // lane xr: the group's strips with bit w0 + xr
+  if (lane < rows) {
+    mask[static_cast<uint64_t>(lane) * n_groups + g] = m;
+    count[static_cast<uint64_t>(lane) * n_groups + g] = static_cast<uint32_t>(__popcll(m));
+  }
+}
+
+// Exclusive scan of n counts in place, the total at [n]: one workgroup, for the few entries of an
+// export (a library scan is three launches).
+constexpr uint32_t kScanBlock = 1024;
+__global__ void __launch_bounds__(kScanBlock) scan_in_place_kernel(uint32_t* __restrict__ v, uint32_t n) {
+  __shared__ uint32_t s_sum[kScanBlock / kWave];
+  // A thread's entries in 16-byte loads, all in flight (one load at a time: 111 us for 65536 entries).
+  const uint32_t per = (n + 4 * kScanBlock - 1) / (4 * kScanBlock) * 4;
+  const uint32_t lo = min(n, threadIdx.x * per), hi = min(n, lo + per);
+  uint32_t sum = 0;
+#pragma unroll 8
+  for (uint32_t i = lo; i + 4 <= hi; i += 4) {
+    const uint4 q = *reinterpret_cast<const uint4*>(v + i);
+    sum += q.x + q.y + q.z + q.w;
+  }
+  for (uint32_t i = lo + (hi - lo) / 4 * 4; i < hi; ++i) sum += v[i];
+  uint32_t incl = sum;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d, kWave));
+    if (lane_id() >= static_cast<uint32_t>(d)) incl += o;
+  }
+  if (lane_id() == kWave - 1) s_sum[threadIdx.x / kWave] = incl;
+  __syncthreads();
+  uint32_t at = incl - sum;
+  for (uint32_t w = 0; w < threadIdx.x / kWave; ++w) at += s_sum[w];
+#pragma unroll 8
+  for (uint32_t i = lo; i + 4 <= hi; i += 4) {
+    const uint4 q = *reinterpret_cast<const uint4*>(v + i);
+    *reinterpret_cast<uint4*>(v + i) = make_uint4(at, at + q.x, at + q.x + q.y, at + q.x + q.y + q.z);
+    at += q.x + q.y + q.z + q.w;
+  }
+  for (uint32_t i = lo + (hi - lo) / 4 * 4; i < hi; ++i) {
+    const uint32_t c = v[i];
+    v[i] = at;
+    at += c;
+  }
+  if (threadIdx.x == kScanBlock - 1) v[n] = at;
+}
+
+// Row pointer and tile index of the export; base: the scanned counts. One wave per (row, group).
+__global__ void __launch_bounds__(kBlock) export_index_kernel(const uint64_t* __restrict__ mask,
+                                                              const uint32_t* __restrict__ base, uint32_t rows,
+                                                              uint32_t n_groups, uint32_t n_strips,
+                                                              uint32_t* __restrict__ offset_row,
+                                                              uint32_t* __restrict__ row_idx,
+                                                              uint32_t* __restrict__ col_idx) {
+  const uint32_t lane = lane_id();
+  const uint32_t n_items = rows * n_groups;
+  for (uint32_t x = blockIdx.x * kBlock + threadIdx.x; x <= n_strips; x += gridDim.x * kBlock)
+    offset_row[x] = base[x < rows ? x * n_groups : n_items];
+  for (uint32_t i = read_first_lane(blockIdx.x * kWaves + threadIdx.x / kWave); i < n_items; i += gridDim.x * kWaves) {
+    const uint64_t m = mask[i];
+    if (!((m >> lane) & 1)) continue;
+    const uint32_t pos = base[i] + lanes_below(m);
+    row_idx[pos] = i / n_groups;
+    col_idx[pos] = (i % n_groups) * 64 + lane;
+  }
+}
+
+// The tiles: a workgroup takes `strips` neighbouring vertex strips, reads their words
+// w0 .. w0 + rows - 1 once in whole rows into LDS (row stride `stride` words, odd) and transposes one
+// (strip, word) per wave at a time. What it moves is what bounds it: 8 bytes in and 8 out per
+// word. With a wave per tile in index order instead, every 128-byte line of X was read once per
+// word and transposed by 64 ballots: 7.0 ms for 4.2 M tiles (R-MAT 22, 4096 sources), now 1.13
+// (3.8 TB/s; eight waves share the 33 KiB of LDS, so that four workgroups fill a CU's wave slots:
+// 1.60 ms with four). pad = rows rounded up to a power of two.
+constexpr int kExportBlock = 512;
+constexpr int kExportLoads = 8;
+__global__ void __launch_bounds__(kExportBlock) export_tiles_kernel(const uint64_t* __restrict__ x, uint32_t W, uint32_t w0,
+                                                              const uint32_t* __restrict__ map, uint32_t n_strips,
+                                                              const uint64_t* __restrict__ mask,
+                                                              const uint32_t* __restrict__ base, uint32_t rows,
+                                                              uint32_t n_groups, uint32_t pad, uint32_t stride,
+                                                              uint32_t strips, uint64_t* __restrict__ out) {
+  extern __shared__ uint64_t s_words[];
+  const uint32_t lane = lane_id();
+  const uint32_t y0 = blockIdx.x * strips;
+  const uint32_t n = min(strips, n_strips - y0);
+  const uint32_t w = threadIdx.x & (pad - 1);
+  // Thread -> (row of the strips, word); kExportBlock / pad rows per step.
+  const uint32_t rows_step = kExportBlock / pad;
+  if (w < rows)
+    for (uint32_t r = threadIdx.x / pad; r < n * 64; r += rows_step * kExportLoads) {
+      uint64_t v[kExportLoads];
+#pragma unroll
+      for (int q = 0; q < kExportLoads; ++q) {
+        const uint32_t rq = r + rows_step * q;
+        v[q] = 0;
+        if (rq < n * 64) {
+          const uint32_t y = y0 + rq / 64;
+          v[q] = x[(static_cast<uint64_t>(map ? map[y] : y) * 64 + rq % 64) * W + w0 + w];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kExportLoads; ++q) {
+        const uint32_t rq = r + rows_step * q;
+        if (rq < n * 64) s_words[rq * stride + w] = v[q];
+      }
     }
-    out[static_cast<uint64_t>(i) * kTile + lane] = mine;
+  __syncthreads();
+  const uint32_t n_tiles = n * rows;
+  for (uint32_t t = read_first_lane(threadIdx.x / kWave); t < n_tiles; t += kExportBlock / kWave) {
+    const uint32_t k = t / rows, xr = t % rows;
+    const uint32_t y = y0 + k;
+    const uint64_t m = mask[static_cast<uint64_t>(xr) * n_groups + y / 64];
+    if (!((m >> (y % 64)) & 1)) continue;
+    const uint64_t pos = base[static_cast<uint64_t>(xr) * n_groups + y / 64] +
+                         static_cast<uint32_t>(__popcll(m & ((1ull << (y % 64)) - 1)));
+    const uint64_t tile = wave_transpose(s_words[(k * 64 + lane) * stride + xr]);
+    __builtin_nontemporal_store(tile, out + pos * kTile + lane);
   }
 }
 
@@ -3420,36 +3534,42 @@ uint64_t frontier_digest(mg_context* ctx, const uint64_t* x, uint64_t nv, uint32
 // g: the plan of the frontier's graph (its strip order).
 mg_tiled_matrix* export_frontier(mg_context* ctx, const uint64_t* x, const uint64_t* s_dev, uint32_t ns, uint32_t W,
                                  uint32_t w0, uint32_t rows, const GraphPlan& g) {
-  std::vector<uint64_t> s_eng(ns), s(ns);
-  MG_HIP(hipMemcpyAsync(s_eng.data(), s_dev, sizeof(uint64_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
-  MG_HIP(hipStreamSynchronize(ctx->stream));
-  for (uint32_t y = 0; y < ns; ++y) s[y] = s_eng[g.map.empty() ? y : g.map[y]];  // vertex strip order
-  // Tile index in row-major (x, y) order over the padded-square grid.
-  std::vector<uint32_t> off(ns + 1ull, 0), ri, ci;
-  for (uint32_t xr = 0; xr < rows; ++xr) {
-    for (uint32_t y = 0; y < ns; ++y)
-      if ((s[y] >> (w0 + xr)) & 1) {
-        ri.push_back(xr);
-        ci.push_back(y);
-      }
-    off[xr + 1] = static_cast<uint32_t>(ri.size());
+  hipStream_t st = ctx->stream;
+  const uint32_t* map = g.device_map();
+  const uint32_t n_groups = (ns + 63) / 64;
+  const uint32_t n_items = rows * n_groups;
+  StreamBuf<uint64_t> mask(n_items, st);
+  StreamBuf<uint32_t> base(n_items + 1ull, st);
+  uint32_t nt = 0;
+  if (n_items) {
+    export_mask_kernel<<<(n_groups + kWaves - 1) / kWaves, kBlock, 0, st>>>(s_dev, ns, map, w0, rows, n_groups,
+                                                                            mask.get(), base.get());
+    MG_LAUNCH_CHECK();
+    scan_in_place_kernel<<<1, kScanBlock, 0, st>>>(base.get(), n_items);
+    MG_LAUNCH_CHECK();
+    MG_HIP(hipMemcpyAsync(&nt, base.get() + n_items, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    MG_HIP(hipStreamSynchronize(st));
   }
-  for (uint32_t xr = rows; xr < ns; ++xr) off[xr + 1] = off[xr];
   auto m = std::make_unique<mg_tiled_matrix>();
   m->device = ctx->device;
-  const uint32_t nt = static_cast<uint32_t>(ri.size());
   alloc_tiled_matrix(m.get(), ns, nt);
-  MG_HIP(hipMemcpyAsync(m->offset_row.get(), off.data(), sizeof(uint32_t) * off.size(), hipMemcpyHostToDevice,
-                        ctx->stream));
+  if (n_items) {
+    export_index_kernel<<<grid_for(std::max<uint64_t>(n_items * 64ull, ns + 1ull), kBlock, 4096), kBlock, 0, st>>>(
+        mask.get(), base.get(), rows, n_groups, ns, m->offset_row.get(), m->row_idx.get(), m->col_idx.get());
+    MG_LAUNCH_CHECK();
+  } else {
+    MG_HIP(hipMemsetAsync(m->offset_row.get(), 0, sizeof(uint32_t) * (ns + 1ull), st));
+  }
   if (nt) {
-    MG_HIP(hipMemcpyAsync(m->row_idx.get(), ri.data(), sizeof(uint32_t) * nt, hipMemcpyHostToDevice, ctx->stream));
-    MG_HIP(hipMemcpyAsync(m->col_idx.get(), ci.data(), sizeof(uint32_t) * nt, hipMemcpyHostToDevice, ctx->stream));
-    export_tiles_kernel<<<grid_for(nt, kWaves, 65536), kBlock, 0, ctx->stream>>>(m->row_idx.get(), m->col_idx.get(),
-                                                                                 nt, x, W, w0, g.device_map(),
-                                                                                 m->data.get());
+    uint32_t pad = 1;
+    while (pad < rows) pad <<= 1;
+    const uint32_t stride = pad | 1;
+    const uint32_t strips = std::max<uint32_t>(1, 16 / pad);  // at least 16 tiles for the eight waves
+    export_tiles_kernel<<<(ns + strips - 1) / strips, kExportBlock, sizeof(uint64_t) * 64 * strips * stride, st>>>(
+        x, W, w0, map, ns, mask.get(), base.get(), rows, n_groups, pad, stride, strips, m->data.get());
     MG_LAUNCH_CHECK();
   }
-  MG_HIP(hipStreamSynchronize(ctx->stream));
+  MG_HIP(hipStreamSynchronize(st));
   return m.release();
 }
 }  // namespace

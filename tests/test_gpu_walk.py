@@ -417,3 +417,31 @@ def test_narrow_walk_matches_oracle(ctx, n_src, flags):
             keys = np.unique(s.astype(np.uint64) * n + d)
             assert st["edges_visited"] == int(v_cur[(keys // n).astype(np.int64)].sum())
             s_cur, v_cur = s_next, xs[k].any(axis=1)
+
+
+# Exports at the edges of the word padding and of the strips per workgroup, on ragged graphs.
+@pytest.mark.parametrize("n_src,n", [(1, 100), (64, 4096), (65, 5000), (200, 4100), (600, 3000), (1100, 9003), (4096, 4500)])
+def test_export_matches_frontier(ctx, n_src, n):
+    M = mg()
+    rng = np.random.default_rng(n)
+    s, d = (rng.integers(0, n, 6 * n).astype(np.uint32) for _ in range(2))
+    at = M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True)
+    ath = at.download()
+    ns = at.n_strips
+    sources = rng.choice(n, min(n_src, n), replace=False).astype(np.uint32)
+    w = M.Walk(ctx, at, n_src, 2)
+    w.run(sources, 2)
+    rows = -(-len(sources) // 64)
+    s_cur = s_masks(ns, sources)
+    for k in range(3):
+        got = w.export(k).download()
+        tiles = [(x, y) for x in range(rows) for y in range(ns) if (int(s_cur[y]) >> x) & 1]
+        assert [(int(a), int(b)) for a, b in zip(got.row_idx, got.col_idx)] == tiles
+        assert np.array_equal(got.offset_row, np.searchsorted(got.row_idx, np.arange(ns + 1)))
+        xk = w.frontier(k)
+        bits = np.unpackbits(xk.view(np.uint8).reshape(ns, 64, -1), axis=2, bitorder="little")  # strip, vertex, source
+        want = [np.packbits(np.ascontiguousarray(bits[y, :, x * 64:x * 64 + 64].T), axis=1, bitorder="little")
+                for x, y in tiles]
+        want = np.ascontiguousarray(want).view(np.uint64)
+        assert np.array_equal(got.data, want.reshape(-1, 64))
+        s_cur, _ = O.walk_symbolic(ns, ath.offset_row, ath.col_idx, s_cur)
