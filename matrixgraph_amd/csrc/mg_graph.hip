@@ -794,6 +794,7 @@ extern "C" int mg_edges_destroy(mg_edge_list* el) {
   return guarded([&] {
     if (!el) return;
     DeviceGuard g(el->device);
+    FreeScope frees;
     delete el;
   });
 }

@@ -207,6 +207,7 @@ extern "C" int mg_tiled_matrix_destroy(mg_tiled_matrix* m) {
   return guarded([&] {
     if (!m) return;
     DeviceGuard g(m->device);
+    FreeScope frees;
     delete m;
   });
 }

@@ -421,6 +421,7 @@ extern "C" int mg_mlp_destroy(mg_mlp* p) {
   return guarded([&] {
     if (!p) return;
     DeviceGuard g(p->device);
+    FreeScope frees;
     delete p;
   });
 }

@@ -3601,6 +3601,7 @@ extern "C" int mg_walk_destroy(mg_walk* w) {
   return guarded([&] {
     if (!w) return;
     DeviceGuard g(w->device);
+    FreeScope frees;
     delete w;
   });
 }
@@ -3934,6 +3935,7 @@ extern "C" int mg_walk_batch_destroy(mg_walk_batch* b) {
   return guarded([&] {
     if (!b) return;
     DeviceGuard g(b->device);
+    FreeScope frees;
     delete b;
   });
 }

@@ -1,0 +1,78 @@
+"""Device memory kept between objects: results dropped while work is still queued, threads with
+their own contexts, and blocks given back with the last context. Every result is compared with the
+oracle's, so a block handed out too early would show."""
+import threading
+
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def square(M, ctx, scale, seed):
+    el = M.EdgeList.rmat(ctx, scale, 16, 0.57, 0.19, 0.19, seed)
+    a, at = el.to_tiled_matrix(False), el.to_tiled_matrix(True)
+    el.close()
+    return a, at
+
+
+def oracle_square(scale, seed):
+    n = 1 << scale
+    s, d = O.rmat_edges(scale, 16, 0.57, 0.19, 0.19, seed)
+    ah, ath = O.edges_to_tiles(n, s, d), O.edges_to_tiles(n, s, d, transpose=True)
+    _, c_row, c_col, _ = O.tile_symbolic(ah[0], ah[1], ah[3], ath[1], ath[3])
+    return O.tile_numeric(ah[0], ah[1:], ath[1:], c_row, c_col)
+
+
+def test_dropped_results_do_not_reach_later_ones(ctx):
+    import matrixgraph_amd as M
+
+    want = {seed: oracle_square(11, seed) for seed in (1, 2)}
+    ops = {seed: square(M, ctx, 11, seed) for seed in (1, 2)}
+    for i in range(12):
+        seed = 1 + i % 2
+        c, _ = M.multiply(ctx, *ops[seed])
+        c.close()  # the numeric pass may still be running
+        c, _ = M.multiply(ctx, *ops[3 - seed])
+        assert np.array_equal(c.download().data, want[3 - seed])
+        c.close()
+
+
+def test_threads_with_their_own_contexts():
+    import matrixgraph_amd as M
+
+    want = {seed: oracle_square(10, seed) for seed in range(4)}
+    bad = []
+
+    def work(seed):
+        c = M.Context(0)
+        for _ in range(8):
+            a, at = square(M, c, 10, seed)
+            p, _ = M.multiply(c, a, at)
+            if not np.array_equal(p.download().data, want[seed]):
+                bad.append(seed)
+            for m in (p, a, at):
+                m.close()
+        c.close()
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+@pytest.mark.parametrize("size", [1, 511, 512, 513, 3 << 20, 200 << 20])
+def test_buffers_come_back_zeroed(ctx, size):
+    import matrixgraph_amd as M
+
+    for _ in range(3):
+        b = M.DeviceBuffer(ctx, size)
+        assert not b.to_array(np.uint8).any()
+        b.close()
+        b = M.DeviceBuffer.from_array(ctx, np.full(size, 7, np.uint8))
+        assert (b.to_array(np.uint8) == 7).all()
+        b.close()
