@@ -53,3 +53,34 @@ def test_mlp_training_reduces_loss(ctx):
     l0, _ = m.loss_grad(x, t)
     l1 = m.train(x, t, epochs=5, batch=512, lr=3e-3)
     assert l1 < 0.5 * l0
+
+
+# Around the 32-row tiles and the largest grid (512 workgroups of a gradient, 1024 of a forward pass).
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 97, 512 * 32 + 1, 1024 * 32 + 33])
+@pytest.mark.parametrize("n_in,n_out", [(4, 1), (4, 2), (8, 1), (8, 2), (16, 1), (16, 2)])
+def test_mlp_tiles_match_oracle(ctx, n, n_in, n_out):
+    M = mg()
+    m = M.MLP(ctx, n_in, n_out, seed=n + n_in)
+    rng = np.random.default_rng(n)
+    master = m.params()[0] + rng.normal(0, 0.05, m.n_params).astype(np.float32)  # biases too
+    m.set_params(master)
+    _, bf16 = m.params()
+    wq = (bf16.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    x, t = data(n, n_in, n_out, n)
+    w1, b1, w2, b2, w3, b3 = np.split(wq, np.cumsum([64 * n_in, 64, 4096, 64, 64 * n_out]))
+    h = np.maximum(x.astype(np.float64) @ w1.reshape(64, n_in).T + b1, 0)
+    h = np.maximum(h @ w2.reshape(64, 64).T + b2, 0)
+    want = h @ w3.reshape(n_out, 64).T + b3
+    assert np.abs(m.forward(x) - want).max() <= 1e-5 * np.abs(want).max()
+    loss_ref, grad_ref = O.mlp_loss_grad(n_in, n_out, wq, x, t)
+    loss, grad = m.loss_grad(x, t)
+    assert loss == pytest.approx(loss_ref, rel=1e-4)
+    scale = np.abs(grad_ref).max()
+    assert np.abs(grad - grad_ref).max() <= 1e-4 * scale + 1e-7
+    # One Adam step is lr * g / (|g| + eps), whatever the size of g; the loss is that of the new weights.
+    after = m.train(x, t, epochs=1, batch=n, lr=1e-3)
+    moved, bf16 = m.params()
+    big = np.abs(grad_ref) > 1e-2 * scale
+    assert np.abs(moved - (master - 1e-3 * np.sign(grad_ref)))[big].max() <= 1e-6
+    wq = (bf16.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    assert after == pytest.approx(O.mlp_loss_grad(n_in, n_out, wq, x, t)[0], rel=1e-4)
