@@ -239,14 +239,15 @@ typedef struct mg_product_stats {
  * the temporaries are stream-ordered pool allocations. stats may be NULL. */
 int mg_multiply_symbolic(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt,
                          mg_tiled_matrix** c, mg_product_stats* stats);
-/* Keeps m's per-tile payloads (16 bytes) and set-bit counts (4 bytes) with the handle, so the
- * products that take m as an operand (mg_multiply_numeric*, mg_multiply_pruned*) copy them
- * instead of reading m's tiles again: a walk by products, X_{k+1} = X_k * A, takes A^T at every
- * hop. No counterpart in the reference (its products re-read every tile). The kept copy is
- * dropped by the next library call that writes m's tiles (a numeric pass into m); after
- * writing m's arrays through the pointers of mg_tiled_matrix_device_arrays, call it again.
- * A call while the kept copy is current does nothing; otherwise it synchronises the context's
- * stream. */
+/* Keeps with the handle what the products read of m as an operand (mg_multiply_numeric*,
+ * mg_multiply_pruned*), so that they need not make it from m's tiles again: a walk by products,
+ * X_{k+1} = X_k * A, takes A^T at every hop. Per tile 16 bytes of payload, twice 16 bytes of head,
+ * 4 bytes of index and 8 bytes per column in use; up to 16384 strips a bitmap of 16 bytes per 64 tiles
+ * of the n_strips x n_strips grid. No counterpart in the reference (its products re-read every
+ * tile). The kept copy is dropped by the next library call that writes m's tiles (a numeric pass
+ * into m); after writing m's arrays through the pointers of mg_tiled_matrix_device_arrays, call it
+ * again. A call while the kept copy is current does nothing; otherwise it synchronises the
+ * context's stream. */
 int mg_tiled_matrix_prepare_operand(mg_context* ctx, mg_tiled_matrix* m);
 /* Numeric pass into a C produced by mg_multiply_symbolic (OR-accumulates).
  * Replaces PPRQuery::FillTilesUnifiedMemory (ppr_query.cu:459-780). Asynchronous on the
@@ -257,9 +258,8 @@ int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, const mg_tile
                         mg_tiled_matrix* c);
 /* The numeric pass with a per-tile-pair choice of engine: a pair whose two tiles both have
  * at least min_bits set bits is multiplied on the matrix cores; every other pair on the
- * vector ALUs. The dense tiles of each operand are expanded once to one byte per bit (4 KiB
- * per tile, at most 32 GiB per operand), the vector pass records the dense pairs of every C
- * tile, and a second kernel sums each C tile's dense pairs in int32 (int8 0/1 products) and
+ * vector ALUs. The vector pass records the dense pairs of every C tile, and a second kernel
+ * expands their tiles in registers, sums each C tile's pairs in int32 (int8 0/1 products) and
  * turns counts > 0 into bits once. min_bits = 0 sends every pair to the matrix cores,
  * min_bits > 4096 none. *dense_products (may be NULL) receives the number of matrix-core tile
  * products. Same result as mg_multiply_numeric. Synchronises.

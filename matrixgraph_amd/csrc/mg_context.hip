@@ -92,7 +92,11 @@ void cache_drop_context(int device) noexcept {
     std::lock_guard<std::mutex> lock(cache().mu);
     last = --cache().devices[device].contexts == 0;
   }
-  if (last) flush_device(device);
+  if (!last) return;
+  flush_device(device);
+  hipMemPool_t pool = nullptr;  // and the temporaries' pool (StreamBuf)
+  if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+  (void)hipGetLastError();
 }
 
 void* cached_alloc(size_t bytes) {

@@ -223,10 +223,16 @@ struct mg_tiled_matrix {
   mgamd::DevBuf<uint64_t> data;        // 64 * n_nz_tile
   // Bumped by every library call that writes this matrix's tiles (the numeric passes into C).
   uint64_t version = 0;
-  // mg_tiled_matrix_prepare_operand: the product path's per-tile payloads (16 B) and set-bit
-  // counts, valid while prep_version == version.
+  // mg_tiled_matrix_prepare_operand, valid while prep_version == version: payloads (16 B a tile, the
+  // allocation-free pass) and the inputs of mg_product.hpp: heads by tile and by position of B,
+  // column words, bitmap; ranks, row offsets and tiles by position.
   mgamd::DevBuf<uint64_t> prep_payload;
-  mgamd::DevBuf<uint32_t> prep_bits;
+  mgamd::DevBuf<uint64_t> prep_head;
+  mgamd::DevBuf<uint64_t> prep_right_head;
+  mgamd::DevBuf<uint64_t> prep_words;
+  mgamd::DevBuf<uint64_t> prep_bitmap;
+  mgamd::DevBuf<uint32_t> prep_index;
+  mgamd::DevBuf<uint32_t> prep_weight;  // per tile row: columns in use of its tiles
   uint64_t prep_version = ~0ull;
 };
 

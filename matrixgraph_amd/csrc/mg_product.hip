@@ -1,0 +1,1047 @@
+// Numeric pass of the handle-level tile products C = A * B (B supplied transposed).
+//
+// The product of two tiles is the OR over their common inner indices j of (column j of the A tile)
+// x (row j of the B tile), and column words of both operands (row j of B = column j of Bt) are all
+// it needs: 8 bytes a side for a j, dense tile or not. Most pairs of tiles that meet share few j:
+// on C = A*A of R-MAT 14 (25.8 K tiles, 16 edges a vertex) the 3.7 M structural pairs have 6.0 M
+// common j in all, and 47 % of them none.
+//
+// A workgroup takes a tile row x of A and a window of up to kWindow strips of C, whose tiles it
+// keeps in LDS. The pairs come straight from the lists, A(x, t) against the B(t, y) of the window,
+// nothing is searched, and each of three stages queues in LDS for the next so that every stage runs
+// on full waves:
+//   1. lane = A tile: the window's strips y of B row t (a few bits of its bitmap word);
+//   2. lane = pair: the two heads (16 bytes each), common j = the ANDed masks;
+//   3. lane = (pair, j): one column word of each side, then the fewer ORs of two: the column word of
+//      B into each row the A word has, or the A word into each column of the transposed C tile.
+// Stages 2 and 3 fetch a batch before they work on the one before it. Pairs with more than
+// kFewCommon common j go through stage 3 at once, lane = j, their column words being contiguous. The
+// two halves of a C tile, by rows and by columns, meet at the end (wave_transpose).
+//
+// Measured (both operands prepared), against one wave per C tile that searches the shorter tile list
+// in the longer one and multiplies payloads of 16 bytes: A*A of R-MAT 14 136 us, before 518; of
+// R-MAT 16 with 16 planted communities (191 K tiles, 70 M pairs) 1.45 ms, before 4.63; a frontier of
+// 1000 rows x R-MAT 18 (7.3 K tiles, 6.8 M pairs) 156 us, before 482. Bound by the vector ALUs: on
+// the second 0.67 G wave instructions, 75 % of the issue slots.
+#include <algorithm>
+#include <string>
+
+#include "mg_device.hpp"
+#include "mg_product.hpp"
+
+namespace mgamd {
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kWavesPerBlock = kBlock / kWave;
+
+// Lanes below this one whose bit of `mask` is set.
+__device__ inline uint32_t lanes_under(uint64_t mask) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
+}
+__device__ inline uint32_t lane_u32(uint32_t v, int src) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), src));
+}
+// Sum over the wave (DPP: within rows of 16, then across them; lane 63 has it).
+__device__ inline uint32_t wave_sum32(uint32_t v) {
+  int x = static_cast<int>(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return lane_u32(static_cast<uint32_t>(x), kWave - 1);
+}
+__device__ inline int lowest(uint64_t m) { return __ffsll(static_cast<unsigned long long>(m)) - 1; }
+
+// --- heads and column words ------------------------------------------------------------
+
+// Where a tile's head goes: its own place (bm null) or the position of B(t, y).
+struct PositionMap {
+  const uint32_t* row;  // per tile of Bt: y and t
+  const uint32_t* col;
+  const BitmapWord* bm;
+  uint32_t wpr;         // bitmap words per row
+  __device__ uint32_t operator()(uint32_t i) const {
+    if (!bm) return i;
+    const uint32_t y = row[i], t = col[i];
+    const BitmapWord w = bm[static_cast<uint64_t>(t) * wpr + (y >> 6)];
+    return w.at + static_cast<uint32_t>(__popcll(w.bits & ((1ull << (y & 63)) - 1)));
+  }
+};
+struct HeadJob {
+  const uint64_t* data;
+  uint32_t n;
+  PositionMap where;
+  TileHead* head;          // by where(i)
+  TileHead* head_by_tile;  // may be null
+  uint32_t* tile;          // inverse of where (may be null)
+  uint8_t* used;           // columns in use, by tile
+};
+
+// Heads and column words of the tiles of two operands (blockIdx.y). One pass over the tiles is
+// what bounds it: a wave has kHeadLoads of them in flight and transposes each (wave_transpose); a
+// workgroup takes the place of all its non-zero words in `words` with one atomic (12 ns each on one
+// address: one per wave and round would take longer than the reads). No room left, or none
+// asked for (cap 0): kNoWords.
+constexpr int kHeadLoads = 8;
+constexpr int kHeadWaves = 16;
+constexpr uint32_t kHeadTiles = kHeadWaves * kHeadLoads;  // of a workgroup's round
+__global__ void __launch_bounds__(kHeadWaves* kWave) tile_heads_kernel(HeadJob job0, HeadJob job1, bool want_bits,
+                                                                       uint64_t* __restrict__ words, uint64_t cap,
+                                                                       unsigned long long* __restrict__ next) {
+  __shared__ uint32_t s_count[kHeadWaves];
+  __shared__ unsigned long long s_base;
+  const HeadJob& job = blockIdx.y ? job1 : job0;
+  const uint32_t lane = lane_id(), wave = read_first_lane(threadIdx.x / kWave), n = job.n;
+  for (uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kHeadTiles; r0 < n;
+       r0 += static_cast<uint64_t>(gridDim.x) * kHeadTiles) {
+    const uint64_t i0 = r0 + wave * kHeadLoads;
+    uint64_t word[kHeadLoads];
+#pragma unroll
+    for (int q = 0; q < kHeadLoads; ++q)
+      word[q] = i0 + q < n ? __builtin_nontemporal_load(job.data + (i0 + q) * kTile + lane) : 0ull;
+    const bool writes = lane < kHeadLoads && i0 + lane < n;  // lane q: tile i0 + q
+    const uint32_t at = writes ? job.where(static_cast<uint32_t>(i0) + lane) : 0u;
+    uint64_t l_mask = 0;
+    uint32_t l_at = 0, l_bits = 0, count = 0;
+#pragma unroll
+    for (int q = 0; q < kHeadLoads; ++q) {
+      word[q] = wave_transpose(word[q]);
+      const uint64_t mask = ballot(word[q] != 0);
+      const uint32_t bits = want_bits ? wave_sum32(static_cast<uint32_t>(__popcll(word[q]))) : 0u;
+      if (lane == q) {
+        l_mask = mask;
+        l_at = count;
+        l_bits = bits;
+      }
+      count += static_cast<uint32_t>(__popcll(mask));
+    }
+    bool fits = false;
+    uint64_t base = 0;
+    if (cap) {
+      if (lane == 0) s_count[wave] = count;
+      __syncthreads();
+      uint32_t before = 0, total = 0;
+      for (uint32_t w = 0; w < kHeadWaves; ++w) {
+        const uint32_t c = s_count[w];
+        if (w < wave) before += c;
+        total += c;
+      }
+      if (threadIdx.x == 0 && total) s_base = atomicAdd(next, static_cast<unsigned long long>(total));
+      __syncthreads();
+      fits = total != 0 && s_base + total <= cap;
+      base = s_base + before;
+      __syncthreads();
+    }
+    if (fits) {
+      uint64_t to = base;
+#pragma unroll
+      for (int q = 0; q < kHeadLoads; ++q) {
+        const uint64_t mask = ballot(word[q] != 0);
+        if (word[q]) words[to + lanes_under(mask)] = word[q];
+        to += static_cast<uint32_t>(__popcll(mask));
+      }
+    }
+    if (writes) {
+      const uint64_t i = i0 + lane;
+      const TileHead h{l_mask, fits ? static_cast<uint32_t>(base) + l_at : kNoWords, l_bits};
+      job.head[at] = h;
+      if (job.head_by_tile) job.head_by_tile[i] = h;
+      if (job.tile) job.tile[at] = static_cast<uint32_t>(i);
+      job.used[i] = static_cast<uint8_t>(__popcll(l_mask));
+    }
+  }
+}
+
+// Weights of an operand's tile rows: the columns in use of their tiles, summed; then the sums of kWindow
+// rows each and of all (an estimate: it may wrap). A workgroup takes kWindow rows, a wave each.
+constexpr uint32_t kWindow = 16;  // strips of C per workgroup of the product: 16 KiB of LDS for their tiles
+struct WeightJob {
+  const uint8_t* used;
+  const uint32_t* off;
+  uint32_t* weight;  // n_strips, total (cleared), groups; null: none
+};
+__global__ void __launch_bounds__(kWindow* kWave) row_weights_kernel(WeightJob job0, WeightJob job1, uint32_t n_strips) {
+  __shared__ uint32_t s_sum[kWindow];
+  const WeightJob& job = blockIdx.y ? job1 : job0;
+  if (!job.weight) return;
+  const uint32_t lane = lane_id(), wave = read_first_lane(threadIdx.x / kWave);
+  uint32_t all = 0;
+  for (uint32_t g = blockIdx.x; g * kWindow < n_strips; g += gridDim.x) {
+    const uint32_t x = g * kWindow + wave;
+    uint32_t sum = 0;
+    if (x < n_strips) {
+      const uint32_t end = job.off[x + 1];
+      for (uint32_t i = job.off[x] + lane; i < end; i += kWave) sum += job.used[i];
+    }
+    sum = wave_sum32(sum);
+    if (lane == 0) {
+      s_sum[wave] = sum;
+      if (x < n_strips) job.weight[x] = sum;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const uint32_t group = wave_sum32(lane < kWindow ? s_sum[lane] : 0u);
+      if (lane == 0) job.weight[n_strips + 1 + g] = group;
+      all += group;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && all) atomicAdd(job.weight + n_strips, all);
+}
+
+// --- B by tile rows, windows of C ----------------------------------------------------------
+
+__global__ void __launch_bounds__(kBlock) clear_words_kernel(uint64_t* __restrict__ v, uint64_t n) {
+  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += static_cast<uint64_t>(gridDim.x) * kBlock) v[i] = 0;
+}
+
+__global__ void __launch_bounds__(kBlock) clear_u32_kernel(uint32_t* __restrict__ v, uint32_t n) {
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) v[i] = 0;
+}
+
+__global__ void __launch_bounds__(kBlock) b_bitmap_kernel(const uint32_t* __restrict__ row,
+                                                          const uint32_t* __restrict__ col, uint32_t n, uint32_t wpr,
+                                                          BitmapWord* __restrict__ bm) {
+  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    const uint32_t y = row[i];
+    atomicOr(reinterpret_cast<unsigned long long*>(&bm[static_cast<uint64_t>(col[i]) * wpr + (y >> 6)].bits),
+             1ull << (y & 63));
+  }
+}
+
+// Tiles of every row; then (off: the rows' first positions) the position of every word. One wave
+// per row.
+__global__ void __launch_bounds__(kBlock) b_rank_kernel(BitmapWord* __restrict__ bm, uint32_t n, uint32_t wpr,
+                                                        uint32_t* __restrict__ count, const uint32_t* __restrict__ off) {
+  const uint32_t lane = lane_id();
+  const uint32_t n_waves = gridDim.x * kWavesPerBlock;
+  for (uint32_t t = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); t < n; t += n_waves) {
+    uint32_t before = off ? off[t] : 0u;
+    for (uint32_t w0 = 0; w0 < wpr; w0 += kWave) {
+      BitmapWord* const word = bm + static_cast<uint64_t>(t) * wpr + w0 + lane;
+      const uint32_t c = w0 + lane < wpr ? static_cast<uint32_t>(__popcll(word->bits)) : 0u;
+      uint32_t incl = c;
+#pragma unroll
+      for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d, kWave));
+        if (lane >= static_cast<uint32_t>(d)) incl += o;
+      }
+      if (off && w0 + lane < wpr) word->at = before + incl - c;
+      before += lane_u32(incl, kWave - 1);
+    }
+    if (lane == 0 && !off) count[t] = before;
+  }
+}
+
+// off[0 .. n] = exclusive prefix sums of count[0 .. n); one workgroup (n <= kBitmapStrips).
+constexpr int kScanWaves = 16;
+__global__ void __launch_bounds__(kScanWaves* kWave) row_offsets_kernel(const uint32_t* __restrict__ count, uint32_t n,
+                                                                        uint32_t* __restrict__ off) {
+  __shared__ uint32_t s_sum[kScanWaves];
+  const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
+  uint32_t before = 0;
+  for (uint32_t i0 = 0; i0 < n; i0 += kScanWaves * kWave) {
+    const uint32_t i = i0 + threadIdx.x;
+    const uint32_t c = i < n ? count[i] : 0u;
+    uint32_t incl = c;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d, kWave));
+      if (lane >= static_cast<uint32_t>(d)) incl += o;
+    }
+    if (lane == kWave - 1) s_sum[wave] = incl;
+    __syncthreads();
+    uint32_t base = before, total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kScanWaves; ++w) {
+      if (w < wave) base += s_sum[w];
+      total += s_sum[w];
+    }
+    if (i < n) off[i] = base + incl - c;
+    before += total;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) off[n] = before;
+}
+
+// Windows of C in use: kWindow strips; kWindow / 4 or one where they would be much work. A
+// window's work is about the columns in use in A's row times those in its rows of Bt, and one
+// with more than 1 / kShares of the whole product's is cut: the hubs of a power-law graph make
+// windows that one workgroup would still be at long after the rest (A*A of R-MAT 14: 405 us without
+// the cut, 172 with; 1024 or 16384 shares: 177, 194).
+constexpr float kShares = 4096;
+__global__ void __launch_bounds__(kScanWaves* kWave) windows_kernel(ProductTiles C, uint32_t n_strips,
+                                                         const uint32_t* __restrict__ off_a,
+                                                         const uint32_t* __restrict__ weight_a,
+                                                         const uint32_t* __restrict__ weight_b,
+                                                         const uint32_t* __restrict__ group_b,
+                                                         Window* __restrict__ windows,
+                                                         uint32_t* __restrict__ n_windows) {
+  const uint32_t lane = lane_id();
+  __shared__ uint32_t s_count[kScanWaves], s_base;
+  const float total = static_cast<float>(weight_a[n_strips]) * static_cast<float>(weight_b[n_strips]);
+  const uint32_t wave = threadIdx.x / kWave;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  for (uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * blockDim.x; i0 < C.n_c; i0 += stride) {
+    const uint64_t i = i0 + threadIdx.x;
+    bool head = false;
+    uint32_t width = kWindow;
+    if (i < C.n_c) {
+      const uint32_t x = C.row[i], y = C.col[i];
+      const float share =
+          total > 0 ? static_cast<float>(weight_a[x]) * static_cast<float>(group_b[y / kWindow]) * kShares / total : 0.0f;
+      width = share <= 1.0f ? kWindow : share <= 4.0f ? kWindow / 4 : 1;
+      head = i == 0 || C.row[i - 1] != x || C.col[i - 1] / width != y / width;
+    }
+    const uint64_t m = ballot(head);
+    if (lane == 0) s_count[wave] = static_cast<uint32_t>(__popcll(m));
+    __syncthreads();
+    uint32_t before = 0, sum = 0;
+    for (uint32_t w = 0; w < kScanWaves; ++w) {
+      if (w < wave) before += s_count[w];
+      sum += s_count[w];
+    }
+    if (threadIdx.x == 0) s_base = sum ? atomicAdd(n_windows, sum) : 0u;
+    __syncthreads();
+    const uint32_t base = s_base + before;
+    __syncthreads();
+    if (head) {
+      const uint32_t x = C.row[i], y = C.col[i];
+      windows[base + lanes_under(m)] = Window{static_cast<uint32_t>(i), x, y / kWindow * kWindow,
+                                              y / width * width + width, off_a[x], off_a[x + 1], {0, 0}};
+    }
+  }
+}
+
+// Set bits of row t of B / its tiles with at least min_bits; one wave per row of a bitmap grid, else
+// per tile with atomics into a cleared out.
+__device__ inline uint64_t row_term(const TileHead& h, uint32_t min_bits, bool count) {
+  return count ? (h.bits >= min_bits ? 1u : 0u) : h.bits;
+}
+__global__ void __launch_bounds__(kBlock) row_sum_kernel(RightOperand B, uint32_t n, uint32_t min_bits, bool count,
+                                                         unsigned long long* __restrict__ out) {
+  const uint32_t n_waves = gridDim.x * kWavesPerBlock;
+  for (uint32_t t = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); t < n; t += n_waves) {
+    uint64_t sum = 0;
+    const uint32_t end = B.off[t + 1];
+    for (uint32_t p = B.off[t] + lane_id(); p < end; p += kWave) sum += row_term(B.head[p], min_bits, count);
+    sum = wave_sum(sum);
+    if (lane_id() == 0) out[t] = sum;
+  }
+}
+__global__ void __launch_bounds__(kBlock) tile_sum_kernel(RightOperand B, uint32_t n_b, uint32_t min_bits, bool count,
+                                                          unsigned long long* __restrict__ out) {
+  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n_b; i += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    const uint64_t v = row_term(B.head[i], min_bits, count);
+    if (v) atomicAdd(out + B.bt_col[i], static_cast<unsigned long long>(v));
+  }
+}
+// Pairs of tiles that both have at least min_bits set bits (count: B's per row).
+__global__ void __launch_bounds__(kBlock) heavy_pairs_kernel(LeftOperand A, uint32_t n_a, uint32_t min_bits,
+                                                             const unsigned long long* __restrict__ count,
+                                                             unsigned long long* __restrict__ out) {
+  uint64_t local = 0;
+  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n_a; i += static_cast<uint64_t>(gridDim.x) * kBlock)
+    if (A.head[i].bits >= min_bits) local += count[A.col[i]];
+  local = wave_sum(local);
+  if (lane_id() == 0 && local) atomicAdd(out, static_cast<unsigned long long>(local));
+}
+
+// --- the product ------------------------------------------------------------------------
+
+constexpr uint32_t kQueue = 128;     // entries of a wave's queues (two full waves)
+// Common inner indices up to which a pair is queued per index: 1.45 ms on the communities above
+// at 16, 1.56 at 8, 1.54 at 64 (always).
+constexpr int kFewCommon = 16;
+constexpr int kPairBatch = 4;        // pairs with more whose loads are in flight together (8: 7 % slower)
+// Waves of a workgroup. More do not shorten a window's chain of loads, they only halve its batches:
+// 1.45 ms with 4, 2.14 with 8, 3.21 with 16 (communities).
+constexpr uint32_t kProductWaves = 4;
+
+struct WaveQueues {
+  uint32_t pair_a[kQueue], pair_b[kQueue];  // tile of A, position of B
+  uint32_t item_a[kQueue], item_b[kQueue];  // column words
+  uint8_t pair_s[kQueue], item_s[kQueue];   // strip of the window
+};
+
+// A dense pair of C tile `c`, to be multiplied on the matrix cores.
+struct HeavyPair {
+  uint32_t c, a, b;
+};
+struct HeavyRecord {
+  HeavyPair* pairs;
+  uint32_t* count;               // per C tile
+  unsigned long long* counter;   // pairs recorded
+  uint64_t cap;
+  uint32_t min_bits;
+};
+
+// First index of a[lo, hi) (ascending) not below key.
+__device__ inline uint32_t lower_bound(const uint32_t* __restrict__ a, uint32_t lo, uint32_t hi, uint32_t key) {
+  while (lo < hi) {
+    const uint32_t mid = lo + ((hi - lo) >> 1);
+    if (a[mid] < key) lo = mid + 1; else hi = mid;
+  }
+  return lo;
+}
+
+// The outer product rows x cols into the C tile at `by_row` / `by_col`. Each lane starts at another
+// bit: neighbours' words are often alike, and equal addresses would queue up.
+__device__ inline void or_outer(unsigned long long* by_row, unsigned long long* by_col, uint64_t rows, uint64_t cols,
+                                uint32_t lane) {
+  const bool r = __popcll(rows) <= __popcll(cols);
+  unsigned long long* const acc = r ? by_row : by_col;
+  const uint64_t word = r ? rows : cols;
+  const unsigned long long val = r ? cols : rows;
+  uint64_t each = (word >> lane) | (word << ((64 - lane) & 63));
+  if (val)
+    for (; each; each &= each - 1) atomicOr(acc + ((lowest(each) + lane) & 63), val);
+}
+
+template <bool kHeavy, int kOut, bool kBitmap>
+__global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTiles C, const Window* __restrict__ windows,
+                                                                   const uint32_t* __restrict__ n_windows, uint32_t wpr,
+                                                                   LeftOperand A, RightOperand B, ProductOut out,
+                                                                   HeavyRecord heavy) {
+  __shared__ unsigned long long by_row[kWindow * kTile], by_col[kWindow * kTile];
+  __shared__ WaveQueues s_queues[kProductWaves];
+  __shared__ uint32_t s_used;
+  __shared__ unsigned long long s_slot;
+  const uint32_t lane = lane_id();
+  const uint32_t wave = read_first_lane(threadIdx.x / kWave);
+  constexpr uint32_t n_waves = kProductWaves;
+  WaveQueues& q = s_queues[wave];
+  const uint32_t n_items = *n_windows;
+  for (uint32_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const Window win = windows[item];
+    const uint32_t y0 = win.y0, a0 = win.a0, a1 = win.a1;
+    const uint32_t mine = win.first + lane;
+    const bool in_row = lane < kWindow && lane < C.n_c - win.first && C.row[mine] == win.x;
+    const uint32_t col = in_row ? C.col[mine] : win.end;
+    uint32_t present = col < win.end ? 1u << (col - y0) : 0u;  // strips with a tile of C
+#pragma unroll
+    for (uint32_t d = 1; d < kWindow; d <<= 1) present |= shfl_xor32(present, static_cast<int>(d));
+    present = read_first_lane(present);
+    const auto c_tile = [&](uint32_t s) { return win.first + static_cast<uint32_t>(__popc(present & ((1u << s) - 1))); };
+    for (uint32_t i = threadIdx.x; i < kWindow * kTile; i += kProductWaves * kWave) by_row[i] = by_col[i] = 0;
+    __syncthreads();
+
+    uint32_t n_pairs = 0, n_queued = 0;  // queued (wave-uniform)
+    // Stages 2 and 3 issue the loads of one batch before they work on the one before it.
+    uint64_t item_r = 0, item_c = 0;
+    uint32_t item_s = 0;
+    // Stage 3: fetches the last n <= 64 queued (pair, j).
+    const auto multiply = [&](uint32_t n) {
+      n_queued -= n;
+      wave_lds_sync();
+      uint64_t r = 0, c = 0;
+      uint32_t s = 0;
+      if (lane < n) {
+        const uint32_t at = n_queued + lane;
+        r = A.words[q.item_a[at]];
+        c = B.words[q.item_b[at]];
+        s = q.item_s[at] * kTile;
+      }
+      or_outer(by_row + item_s, by_col + item_s, item_r, item_c, lane);
+      item_r = r;
+      item_c = c;
+      item_s = s;
+      wave_lds_sync();
+    };
+    uint32_t next_a = 0, next_b = 0, next_s = 0;
+    TileHead next_ha{0, 0, 0}, next_hb{0, 0, 0};
+    uint32_t fetched = 0;  // pairs (wave-uniform)
+    // Stage 2: fetches the heads of the last n <= 64 queued pairs.
+    const auto filter = [&](uint32_t n) {
+      const uint32_t ia = next_a, pb = next_b, s = next_s;
+      const TileHead ha = next_ha, hb = next_hb;
+      n_pairs -= n;
+      wave_lds_sync();
+      next_ha.mask = next_hb.mask = 0;
+      if constexpr (kHeavy) next_ha.bits = next_hb.bits = 0;
+      if (lane < n) {
+        const uint32_t at = n_pairs + lane;
+        next_a = q.pair_a[at];
+        next_b = q.pair_b[at];
+        next_s = q.pair_s[at];
+        next_ha = A.head[next_a];
+        next_hb = B.head[next_b];
+      }
+      wave_lds_sync();
+      const bool has = lane < fetched;
+      fetched = n;
+      uint64_t common = ha.mask & hb.mask;
+      if constexpr (kHeavy) {
+        const bool h = has && ha.bits >= heavy.min_bits && hb.bits >= heavy.min_bits;
+        const uint64_t hm = ballot(h);
+        if (hm) {
+          unsigned long long base = 0;
+          if (lane == 0) base = atomicAdd(heavy.counter, static_cast<unsigned long long>(__popcll(hm)));
+          base = read_first_lane64(base) + lanes_under(hm);
+          if (h && base < heavy.cap) {
+            const uint32_t c = c_tile(s);
+            heavy.pairs[base] = HeavyPair{c, ia, B.tile ? B.tile[pb] : pb};
+            atomicAdd(heavy.count + c, 1u);
+          }
+          if (h) common = 0;
+        }
+      }
+      const int n_common = __popcll(common);
+      const bool whole = n_common > kFewCommon || (common && (ha.off == kNoWords || hb.off == kNoWords));
+      // Pairs with many common indices (or words that are not stored): lane = j.
+      for (uint64_t wm = ballot(whole); wm;) {
+        uint64_t r[kPairBatch], c[kPairBatch];
+        uint32_t sp[kPairBatch];
+#pragma unroll
+        for (int k = 0; k < kPairBatch; ++k) {
+          r[k] = 0;
+          c[k] = 0;
+          sp[k] = 0;
+          if (wm) {
+            const int src = lowest(wm);
+            wm &= wm - 1;
+            const uint64_t ma = read_lane(ha.mask, src), mb = read_lane(hb.mask, src);
+            const uint32_t oa = lane_u32(ha.off, src), ob = lane_u32(hb.off, src);
+            sp[k] = lane_u32(s, src) * kTile;
+            const bool use = ((ma & mb) >> lane) & 1;
+            if (oa != kNoWords) {
+              if (use) r[k] = A.words[oa + lanes_under(ma)];
+            } else {
+              const uint64_t t = wave_transpose(A.data[static_cast<uint64_t>(lane_u32(ia, src)) * kTile + lane]);
+              if (use) r[k] = t;
+            }
+            if (ob != kNoWords) {
+              if (use) c[k] = B.words[ob + lanes_under(mb)];
+            } else {
+              const uint32_t p = lane_u32(pb, src);
+              const uint64_t t = wave_transpose(B.data[static_cast<uint64_t>(B.tile ? B.tile[p] : p) * kTile + lane]);
+              if (use) c[k] = t;
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kPairBatch; ++k) or_outer(by_row + sp[k], by_col + sp[k], r[k], c[k], lane);
+      }
+      if (whole) common = 0;
+      for (uint64_t m = ballot(common != 0); m; m = ballot(common != 0)) {
+        if (common) {
+          const uint64_t below = (common & (0 - common)) - 1;
+          const uint32_t to = n_queued + lanes_under(m);
+          q.item_a[to] = ha.off + static_cast<uint32_t>(__popcll(ha.mask & below));
+          q.item_b[to] = hb.off + static_cast<uint32_t>(__popcll(hb.mask & below));
+          q.item_s[to] = static_cast<uint8_t>(s);
+          common &= common - 1;
+        }
+        n_queued += static_cast<uint32_t>(__popcll(m));
+        if (n_queued >= kWave) multiply(kWave);
+      }
+    };
+
+    // Stage 1: the row's tiles, dealt one by one to the waves, so that short rows use them all.
+    if constexpr (kBitmap) {
+      for (uint32_t k0 = a0; k0 < a1; k0 += kWave * n_waves) {
+        const uint32_t ia = k0 + lane * n_waves + wave;
+        uint32_t bits = 0, pb = 0;  // strips of the window, and the position of the lowest
+        if (ia < a1) {
+          const uint32_t t = A.col[ia];
+          const BitmapWord w = B.bm[static_cast<uint64_t>(t) * wpr + (y0 >> 6)];
+          bits = static_cast<uint32_t>(w.bits >> (y0 & 63)) & ((1u << kWindow) - 1);
+          pb = w.at + static_cast<uint32_t>(__popcll(w.bits & ((1ull << (y0 & 63)) - 1)));
+        }
+        const uint32_t all = bits;
+        bits &= present;
+        for (uint64_t m = ballot(bits != 0); m; m = ballot(bits != 0)) {
+          if (bits) {
+            const uint32_t s = static_cast<uint32_t>(__ffs(static_cast<int>(bits)) - 1);
+            const uint32_t to = n_pairs + lanes_under(m);
+            q.pair_a[to] = ia;
+            q.pair_b[to] = pb + static_cast<uint32_t>(__popc(all & ((1u << s) - 1)));
+            q.pair_s[to] = static_cast<uint8_t>(s);
+            bits &= bits - 1;
+          }
+          n_pairs += static_cast<uint32_t>(__popcll(m));
+          if (n_pairs >= kWave) filter(kWave);
+        }
+      }
+    } else {
+      // Wide grid: every strip's Bt row against A's, the shorter searched in the longer.
+      for (uint32_t left = present; left; left &= left - 1) {
+        const uint32_t s = static_cast<uint32_t>(__ffs(static_cast<int>(left)) - 1);
+        const uint32_t b0 = B.bt_off[y0 + s], b1 = B.bt_off[y0 + s + 1];
+        const bool a_short = a1 - a0 <= b1 - b0;
+        const uint32_t s0 = a_short ? a0 : b0, s1 = a_short ? a1 : b1, l0 = a_short ? b0 : a0, l1 = a_short ? b1 : a1;
+        const uint32_t* const s_col = a_short ? A.col : B.bt_col;
+        const uint32_t* const l_col = a_short ? B.bt_col : A.col;
+        for (uint32_t k0 = s0; k0 < s1; k0 += kWave * n_waves) {
+          const uint32_t k = k0 + lane * n_waves + wave;
+          uint32_t at = l1;
+          bool has = k < s1;
+          if (has) {
+            const uint32_t key = s_col[k];
+            at = lower_bound(l_col, l0, l1, key);
+            has = at < l1 && l_col[at] == key;
+          }
+          const uint64_t m = ballot(has);
+          if (has) {
+            const uint32_t to = n_pairs + lanes_under(m);
+            q.pair_a[to] = a_short ? k : at;
+            q.pair_b[to] = a_short ? at : k;
+            q.pair_s[to] = static_cast<uint8_t>(s);
+          }
+          n_pairs += static_cast<uint32_t>(__popcll(m));
+          if (n_pairs >= kWave) filter(kWave);
+        }
+      }
+    }
+    while (n_pairs || fetched) filter(n_pairs);
+    multiply(n_queued);
+    multiply(0);
+    __syncthreads();
+    // Write-out: one C tile per wave at a time.
+    if constexpr (kOut == kOutAppend) {
+      // The window's non-empty tiles take their slots together: one counter for all of C.
+      if (threadIdx.x == 0) s_used = 0;
+      __syncthreads();
+      for (uint32_t s = wave; s < kWindow; s += n_waves) {
+        if (!((present >> s) & 1)) continue;
+        const uint64_t val = by_row[s * kTile + lane] | wave_transpose(by_col[s * kTile + lane]);
+        by_row[s * kTile + lane] = val;
+        if (ballot(val != 0) && lane == 0) atomicOr(&s_used, 1u << s);
+      }
+      __syncthreads();
+      const uint32_t used = s_used;
+      if (threadIdx.x == 0) s_slot = used ? atomicAdd(out.counter, static_cast<unsigned long long>(__popc(used))) : 0ull;
+      __syncthreads();
+      for (uint32_t s = wave; s < kWindow; s += n_waves) {
+        const uint64_t slot = s_slot + static_cast<uint32_t>(__popc(used & ((1u << s) - 1)));
+        if (!((used >> s) & 1) || slot >= out.capacity) continue;
+        out.data[slot * kTile + lane] = by_row[s * kTile + lane];
+        if (lane == 0) out.key[slot] = c_tile(s);
+      }
+      __syncthreads();
+      continue;
+    }
+    for (uint32_t s = wave; s < kWindow; s += n_waves) {
+      if (!((present >> s) & 1)) continue;
+      const uint64_t val = by_row[s * kTile + lane] | wave_transpose(by_col[s * kTile + lane]);
+      const uint32_t i = c_tile(s);
+      if constexpr (kOut == kOutStruct) {
+        // Only this wave has the tile; an atomic needs no answer, a load would be waited for.
+        if (val) atomicOr(reinterpret_cast<unsigned long long*>(out.data) + static_cast<uint64_t>(i) * kTile + lane,
+                          static_cast<unsigned long long>(val));
+      } else {
+        const bool nz = ballot(val != 0) != 0;
+        if constexpr (kOut == kOutFlag) {
+          if (lane == 0) out.flag[i] = nz ? 1u : 0u;
+        } else if (nz) {
+          out.data[static_cast<uint64_t>(out.pos[i]) * kTile + lane] = val;
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Heavy pairs to their C tile's place, and the C tiles' tasks of up to kTaskPairs pairs.
+constexpr uint32_t kTaskPairs = 64;
+__global__ void __launch_bounds__(kBlock) heavy_scatter_kernel(const HeavyPair* __restrict__ in, uint32_t n,
+                                                               const uint32_t* __restrict__ base,
+                                                               uint32_t* __restrict__ cursor,
+                                                               uint2* __restrict__ pairs) {
+  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    const HeavyPair p = in[i];
+    pairs[base[p.c] + atomicAdd(cursor + p.c, 1u)] = uint2{p.a, p.b};
+  }
+}
+
+// Dense tile pairs on the matrix cores, as one contraction per C tile: for every pair
+// (A(x,k), Bt(y,k)) whose two tiles both hold at least min_bits set bits, the vector kernel
+// records the pair (its two tile indices) instead of multiplying it; then
+// dense_contract_kernel sums, per C tile, the int8 0/1 products of all its recorded pairs in
+// int32 (v_mfma_i32_32x32x32_i8, four 32 x 32 output blocks, two K-steps of 32 per pair) and
+// turns counts > 0 into bit rows once, ORed into C. Operands are expanded from the bit tiles
+// in registers: a lane loads one 64-bit row of each tile (A row r, Bt row c = B column c) and
+// turns 4 bits at a time into 4 bytes of 0/1 with a 24-bit multiply.
+// Lane layout (32x32x32 i8): lane l holds 16 bytes of A row l % 32 and of B column l % 32,
+// at k = 16 * (l / 32) .. +15 of the K-step (any k order works if both operands use it);
+// result register v of lane l is C[8 * (v / 4) + 4 * (l / 32) + v % 4][l % 32].
+typedef int mg_v16i __attribute__((ext_vector_type(16)));
+typedef int mg_v4i __attribute__((ext_vector_type(4)));
+
+// Bits 0..15 of x as 16 bytes of value 0 or 1 (byte j = bit j): nibble * 0x204081 puts bit
+// i of the nibble at bit 8i (the four shifted copies do not overlap), the mask keeps those.
+__device__ inline mg_v4i bits16_to_bytes(uint32_t x) {
+  mg_v4i out;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    out[q] = static_cast<int>(__umul24((x >> (4 * q)) & 0xFu, 0x204081u) & 0x01010101u);
+  return out;
+}
+
+// Up to kTaskPairs of a C tile's dense pairs.
+struct DenseTask {
+  uint32_t tile, base, n;
+};
+// One wave per recorded task: int32 counts of the 64 x 64 output over all the task's pairs
+// on the matrix cores, then one threshold; the rows are ORed into C atomically (several
+// tasks may share a C tile).
+__global__ void __launch_bounds__(kBlock) dense_contract_kernel(const DenseTask* __restrict__ tasks,
+                                                                const uint32_t* __restrict__ n_tasks_ptr,
+                                                                const uint2* __restrict__ pairs,
+                                                                const uint64_t* __restrict__ data_a,
+                                                                const uint64_t* __restrict__ data_bt,
+                                                                uint64_t* __restrict__ data_c) {
+  const uint32_t lane = lane_id();
+  const uint32_t lo = lane & 31, hi = lane >> 5;
+  const uint32_t n_tasks = *n_tasks_ptr;
+  const uint32_t n_waves = gridDim.x * kWavesPerBlock;
+  for (uint32_t t = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); t < n_tasks; t += n_waves) {
+    const DenseTask T = tasks[t];
+    mg_v16i acc00 = {}, acc01 = {}, acc10 = {}, acc11 = {};
+    const uint32_t p_end = T.base + T.n;
+    for (uint32_t p = T.base; p < p_end; ++p) {
+      const uint2 pr = pairs[p];
+      const uint64_t* A = data_a + static_cast<uint64_t>(pr.x) * kTile;
+      const uint64_t* B = data_bt + static_cast<uint64_t>(pr.y) * kTile;
+      const uint64_t ra0 = A[lo], ra1 = A[32 + lo], rb0 = B[lo], rb1 = B[32 + lo];
+#pragma unroll
+      for (uint32_t st = 0; st < 2; ++st) {
+        const uint32_t k = 32 * st + 16 * hi;
+        const mg_v4i a0 = bits16_to_bytes(static_cast<uint32_t>(ra0 >> k));
+        const mg_v4i a1 = bits16_to_bytes(static_cast<uint32_t>(ra1 >> k));
+        const mg_v4i b0 = bits16_to_bytes(static_cast<uint32_t>(rb0 >> k));
+        const mg_v4i b1 = bits16_to_bytes(static_cast<uint32_t>(rb1 >> k));
+        acc00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, acc00, 0, 0, 0);
+        acc01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b1, acc01, 0, 0, 0);
+        acc10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b0, acc10, 0, 0, 0);
+        acc11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, acc11, 0, 0, 0);
+      }
+    }
+    uint64_t out = 0;  // output row `lane`
+#pragma unroll
+    for (uint32_t v = 0; v < 16; ++v) {
+      const uint32_t i0 = 8 * (v / 4) + (v % 4);
+      const uint64_t b00 = ballot(acc00[v] > 0), b01 = ballot(acc01[v] > 0);
+      const uint64_t b10 = ballot(acc10[v] > 0), b11 = ballot(acc11[v] > 0);
+      if (lane == i0) out |= (b00 & 0xFFFFFFFFull) | ((b01 & 0xFFFFFFFFull) << 32);
+      if (lane == i0 + 4) out |= (b00 >> 32) | ((b01 >> 32) << 32);
+      if (lane == 32 + i0) out |= (b10 & 0xFFFFFFFFull) | ((b11 & 0xFFFFFFFFull) << 32);
+      if (lane == 32 + i0 + 4) out |= (b10 >> 32) | ((b11 >> 32) << 32);
+    }
+    if (out) atomicOr(reinterpret_cast<unsigned long long*>(data_c) + static_cast<uint64_t>(T.tile) * kTile + lane,
+                      static_cast<unsigned long long>(out));
+  }
+}
+
+
+__global__ void __launch_bounds__(kBlock) heavy_tasks_kernel(const uint32_t* __restrict__ base, uint32_t n_c,
+                                                             DenseTask* __restrict__ tasks,
+                                                             uint32_t* __restrict__ n_tasks) {
+  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n_c; i += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    const uint32_t p0 = base[i], p1 = base[i + 1];
+    if (p0 == p1) continue;
+    uint32_t to = atomicAdd(n_tasks, (p1 - p0 + kTaskPairs - 1) / kTaskPairs);
+    for (uint32_t p = p0; p < p1; p += kTaskPairs)
+      tasks[to++] = DenseTask{static_cast<uint32_t>(i), p, min(kTaskPairs, p1 - p)};
+  }
+}
+
+template <bool kHeavy, int kOut>
+void launch_product(mg_context* ctx, const ProductInputs& P, const ProductOut& out, const HeavyRecord& heavy) {
+  const ProductTiles& C = P.c;
+  if (!C.n_c) return;
+  const uint32_t grid = std::min(65536u, C.n_c), wpr = (P.n_strips + 63) / 64;
+  if (P.b.bm)
+    product_kernel<kHeavy, kOut, true><<<grid, kProductWaves * kWave, 0, ctx->stream>>>(C, P.windows, P.n_windows, wpr, P.a, P.b, out,
+                                                                                    heavy);
+  else
+    product_kernel<kHeavy, kOut, false><<<grid, kProductWaves * kWave, 0, ctx->stream>>>(C, P.windows, P.n_windows, wpr, P.a, P.b, out,
+                                                                                     heavy);
+  MG_LAUNCH_CHECK();
+}
+
+void clear_u32(hipStream_t st, uint32_t* v, uint32_t n) {
+  if (!n) return;
+  clear_u32_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, st>>>(v, n);
+  MG_LAUNCH_CHECK();
+}
+
+// Bitmap, ranks and row offsets of B; grids up to kBitmapStrips.
+struct RightIndex {
+  BitmapWord* bm;
+  uint32_t* off;    // n_strips + 1
+  uint32_t* count;  // n_strips, scratch
+};
+// bm cleared, its bits set.
+void launch_ranks(hipStream_t st, uint32_t ns, uint32_t wpr, const RightIndex& R) {
+  b_rank_kernel<<<grid_for(ns, kWavesPerBlock, 4096), kBlock, 0, st>>>(R.bm, ns, wpr, R.count, nullptr);
+  MG_LAUNCH_CHECK();
+  row_offsets_kernel<<<1, kScanWaves * kWave, 0, st>>>(R.count, ns, R.off);
+  MG_LAUNCH_CHECK();
+  b_rank_kernel<<<grid_for(ns, kWavesPerBlock, 4096), kBlock, 0, st>>>(R.bm, ns, wpr, R.count, R.off);
+  MG_LAUNCH_CHECK();
+}
+
+void launch_heads(hipStream_t st, const HeadJob& a, const HeadJob& b, bool want_bits, uint64_t* words, uint64_t cap,
+                  unsigned long long* next) {
+  const uint32_t most = std::max(a.n, b.n);
+  if (!most) return;
+  tile_heads_kernel<<<dim3(grid_for(most, kHeadTiles, 4096), 2), kHeadWaves * kWave, 0, st>>>(a, b, want_bits, words, cap,
+                                                                                             next);
+  MG_LAUNCH_CHECK();
+}
+
+void launch_weights(hipStream_t st, const WeightJob& a, const WeightJob& b, uint32_t ns) {
+  if ((!a.weight && !b.weight) || !ns) return;
+  row_weights_kernel<<<dim3(grid_for(ns, kWindow, 512), 2), kWindow * kWave, 0, st>>>(a, b, ns);
+  MG_LAUNCH_CHECK();
+}
+
+// Words of an operand's row weights: the rows', their total, and those of kWindow rows each.
+uint32_t weight_words(uint32_t ns) { return ns + 1 + (ns + kWindow - 1) / kWindow; }
+
+// Room for column words: every one of up to 2^20 tiles, 16 a tile beyond (and no less than that).
+uint64_t word_room(uint64_t n) {
+  return std::min<uint64_t>(kNoWords - 1ull, std::min<uint64_t>(n * kTile, std::max<uint64_t>(1ull << 26, 16 * n)));
+}
+
+}  // namespace
+
+bool prepared(const mg_tiled_matrix* m) { return m->prep_version == m->version && m->prep_head.get(); }
+
+void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
+  hipStream_t st = ctx->stream;
+  const uint32_t n = m->n_nz_tile, ns = m->n_strips;
+  const bool bitmap = ns <= kBitmapStrips;
+  const uint32_t wpr = (ns + 63) / 64;
+  const uint64_t bm = bitmap ? 2ull * ns * wpr : 0;  // u64 words
+  m->prep_head.alloc(2ull * std::max<uint32_t>(1, n));
+  m->prep_words.alloc(1);
+  StreamBuf<unsigned long long> next(1, st);
+  clear_words_kernel<<<1, kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(next.get()), 1);
+  MG_LAUNCH_CHECK();
+  StreamBuf<uint8_t> used(n, st);
+  m->prep_weight.alloc(weight_words(ns));
+  clear_u32(st, m->prep_weight.get(), weight_words(ns));
+  HeadJob as_a{m->data.get(), n, {}, reinterpret_cast<TileHead*>(m->prep_head.get()), nullptr, nullptr,
+               used.get()};
+  HeadJob as_b{};
+  if (bitmap) {
+    m->prep_right_head.alloc(2ull * std::max<uint32_t>(1, n));
+    m->prep_bitmap.alloc(std::max<uint64_t>(1, bm));
+    m->prep_index.alloc(ns + 1ull + n);
+    StreamBuf<uint32_t> count(ns, st);
+    const RightIndex R{reinterpret_cast<BitmapWord*>(m->prep_bitmap.get()), m->prep_index.get(), count.get()};
+    clear_words_kernel<<<grid_for(bm, kBlock, 8192), kBlock, 0, st>>>(m->prep_bitmap.get(), bm);
+    MG_LAUNCH_CHECK();
+    b_bitmap_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, st>>>(m->row_idx.get(), m->col_idx.get(), n, wpr,
+                                                                  R.bm);
+    MG_LAUNCH_CHECK();
+    launch_ranks(st, ns, wpr, R);
+    as_b = as_a;
+    as_b.where = PositionMap{m->row_idx.get(), m->col_idx.get(), R.bm, wpr};
+    as_b.head_by_tile = as_a.head;
+    as_b.head = reinterpret_cast<TileHead*>(m->prep_right_head.get());
+    as_b.tile = R.off + ns + 1;
+    as_a.n = 0;
+  }
+  const uint64_t room = word_room(n);
+  StreamBuf<uint64_t> words(room, st);
+  launch_heads(st, as_a, as_b, true, words.get(), room, next.get());
+  launch_weights(st, WeightJob{used.get(), m->offset_row.get(), m->prep_weight.get()}, WeightJob{}, ns);
+  unsigned long long taken = 0;
+  MG_HIP(hipMemcpyAsync(&taken, next.get(), sizeof(taken), hipMemcpyDeviceToHost, st));
+  MG_HIP(hipStreamSynchronize(st));
+  taken = std::min<unsigned long long>(taken, room);
+  if (taken) {
+    m->prep_words.alloc(taken);
+    MG_HIP(hipMemcpyAsync(m->prep_words.get(), words.get(), taken * sizeof(uint64_t), hipMemcpyDeviceToDevice, st));
+  }
+}
+
+void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const ProductTiles& c,
+                    bool want_bits, bool want_words, ProductInputs& P) {
+  hipStream_t st = ctx->stream;
+  const uint32_t ns = a->n_strips, wpr = (ns + 63) / 64;
+  const bool bitmap = ns <= kBitmapStrips;
+  const bool pa = prepared(a), pb = prepared(bt), same = a == bt && bitmap;
+  const uint64_t na = pa ? 0 : a->n_nz_tile, nb = pb ? 0 : bt->n_nz_tile;
+  const uint64_t bm = bitmap && !pb ? 2ull * ns * wpr : 0;  // u64 words
+  // Cleared: counters (column words taken; windows), the bitmap and the weights.
+  const uint64_t weights = pa && pb ? 0 : 2ull * weight_words(ns);
+  const uint64_t clear = (2 + bm + (weights + 1) / 2 + 1) & ~1ull;
+  const uint64_t windows_at = clear + 2 * (na + nb), words_at = windows_at + 4ull * c.n_c;
+  const uint64_t u32s = (bm ? 2ull * ns + 1 + nb : 0) + (na + nb + 3) / 4;  // then the tiles' columns in use (u8)
+  uint64_t room = want_words ? word_room(same && !pa ? nb : na + nb) : 0;
+  uint64_t* base = nullptr;
+  try {
+    base = ctx_scratch(ctx, words_at + room + (u32s + 1) / 2);
+  } catch (const std::exception&) {
+    // No memory for the column words: the product makes them from the tiles (wave_transpose).
+    if (!room) throw;
+    room = 0;
+    base = ctx_scratch(ctx, words_at + (u32s + 1) / 2);
+  }
+  unsigned long long* const next = reinterpret_cast<unsigned long long*>(base);
+  BitmapWord* const bitmap_words = reinterpret_cast<BitmapWord*>(base + 2);
+  uint32_t* const weight = reinterpret_cast<uint32_t*>(base + 2 + bm);
+  uint32_t* const weight2 = weight + weight_words(ns);
+  TileHead* const head_a = reinterpret_cast<TileHead*>(base + clear);
+  TileHead* const head_b = head_a + na;
+  P.n_strips = ns;
+  P.c = c;
+  P.n_windows = reinterpret_cast<uint32_t*>(next + 1);
+  P.windows = reinterpret_cast<Window*>(base + windows_at);
+  uint64_t* const words = base + words_at;
+  uint32_t* const at32 = reinterpret_cast<uint32_t*>(words + room);
+  clear_words_kernel<<<grid_for(clear, kBlock, 4096), kBlock, 0, st>>>(base, clear);
+  MG_LAUNCH_CHECK();
+  if (bm && bt->n_nz_tile) {
+    b_bitmap_kernel<<<grid_for(bt->n_nz_tile, kBlock, 4096), kBlock, 0, st>>>(
+        bt->row_idx.get(), bt->col_idx.get(), bt->n_nz_tile, wpr, bitmap_words);
+    MG_LAUNCH_CHECK();
+  }
+  uint8_t* const used = reinterpret_cast<uint8_t*>(at32 + (bm ? 2ull * ns + 1 + nb : 0));
+  HeadJob job_a{a->data.get(), static_cast<uint32_t>(na), {}, head_a, nullptr, nullptr, used};
+  HeadJob job_b{bt->data.get(), static_cast<uint32_t>(nb), {}, head_b, nullptr, nullptr, used + na};
+  if (bm) {
+    const RightIndex R{bitmap_words, at32, at32 + ns + 1};
+    launch_ranks(st, ns, wpr, R);
+    job_b.where = PositionMap{bt->row_idx.get(), bt->col_idx.get(), R.bm, wpr};
+    job_b.tile = R.count + ns;
+    P.b.bm = R.bm;
+    P.b.off = R.off;
+    P.b.tile = job_b.tile;
+  }
+  if (same && !pa) {  // one pass makes both operands' heads
+    job_b.head_by_tile = head_a;
+    job_a.n = 0;
+  }
+  launch_heads(st, job_a, job_b, want_bits, words, room, next);
+  if (c.n_c) {
+    launch_weights(st, pa || same ? WeightJob{} : WeightJob{used, a->offset_row.get(), weight},
+                   pb ? WeightJob{} : WeightJob{used + na, bt->offset_row.get(), weight2}, ns);
+    const uint32_t* const weight_b = pb ? bt->prep_weight.get() : weight2;
+    const uint32_t* const weight_a = pa ? a->prep_weight.get() : same ? weight_b : weight;
+    windows_kernel<<<grid_for(c.n_c, kScanWaves * kWave, 1024), kScanWaves * kWave, 0, st>>>(c, ns, a->offset_row.get(), weight_a, weight_b,
+                                                                      weight_b + ns + 1, P.windows, P.n_windows);
+    MG_LAUNCH_CHECK();
+  }
+  P.a = {head_a, words, a->data.get(), a->offset_row.get(), a->col_idx.get()};
+  if (pa) {
+    P.a.head = reinterpret_cast<const TileHead*>(a->prep_head.get());
+    P.a.words = a->prep_words.get();
+  }
+  P.b.head = head_b;
+  P.b.words = words;
+  P.b.data = bt->data.get();
+  P.b.bt_off = bt->offset_row.get();
+  P.b.bt_col = bt->col_idx.get();
+  if (pb) {
+    P.b.words = bt->prep_words.get();
+    P.b.head = reinterpret_cast<const TileHead*>(bt->prep_head.get());
+    if (bitmap) {
+      P.b.head = reinterpret_cast<const TileHead*>(bt->prep_right_head.get());
+      P.b.bm = reinterpret_cast<const BitmapWord*>(bt->prep_bitmap.get());
+      P.b.off = bt->prep_index.get();
+      P.b.tile = P.b.off + ns + 1;
+    }
+  }
+}
+
+void run_product(mg_context* ctx, const ProductInputs& P, int out_mode, const ProductOut& out) {
+  switch (out_mode) {
+    case kOutStruct: launch_product<false, kOutStruct>(ctx, P, out, HeavyRecord{}); break;
+    case kOutAppend: launch_product<false, kOutAppend>(ctx, P, out, HeavyRecord{}); break;
+    case kOutFlag: launch_product<false, kOutFlag>(ctx, P, out, HeavyRecord{}); break;
+    case kOutPos: launch_product<false, kOutPos>(ctx, P, out, HeavyRecord{}); break;
+    default: fail(MG_ERR_INTERNAL, "run_product: output mode");
+  }
+}
+
+namespace {
+void right_row_sums(mg_context* ctx, const mg_tiled_matrix* bt, const ProductInputs& P, uint32_t min_bits, bool count,
+                    unsigned long long* out) {
+  hipStream_t st = ctx->stream;
+  if (!P.n_strips) return;
+  if (P.b.bm) {
+    row_sum_kernel<<<grid_for(P.n_strips, kWavesPerBlock, 4096), kBlock, 0, st>>>(P.b, P.n_strips, min_bits, count, out);
+    MG_LAUNCH_CHECK();
+    return;
+  }
+  clear_words_kernel<<<grid_for(P.n_strips, kBlock, 4096), kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(out), P.n_strips);
+  MG_LAUNCH_CHECK();
+  tile_sum_kernel<<<grid_for(bt->n_nz_tile, kBlock, 4096), kBlock, 0, st>>>(P.b, bt->n_nz_tile, min_bits, count, out);
+  MG_LAUNCH_CHECK();
+}
+}  // namespace
+
+void right_row_bits(mg_context* ctx, const mg_tiled_matrix* bt, const ProductInputs& P, unsigned long long* out) {
+  right_row_sums(ctx, bt, P, 0, false, out);
+}
+
+uint64_t run_product_dense(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt,
+                           const ProductInputs& P, uint32_t min_bits, uint64_t* data_c) {
+  hipStream_t st = ctx->stream;
+  ProductOut out{};
+  out.data = data_c;
+  // The structural pairs of two heavy tiles: what the record may hold at most.
+  uint64_t most = 0;
+  if (a->n_nz_tile && bt->n_nz_tile) {
+    StreamBuf<unsigned long long> count(P.n_strips + 1ull, st);
+    unsigned long long* const total = count.get() + P.n_strips;
+    right_row_sums(ctx, bt, P, min_bits, true, count.get());
+    clear_words_kernel<<<1, kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(total), 1);
+    MG_LAUNCH_CHECK();
+    heavy_pairs_kernel<<<grid_for(a->n_nz_tile, kBlock, 1024), kBlock, 0, st>>>(P.a, a->n_nz_tile, min_bits, count.get(),
+                                                                               total);
+    MG_LAUNCH_CHECK();
+    unsigned long long h = 0;
+    MG_HIP(hipMemcpyAsync(&h, total, sizeof(h), hipMemcpyDeviceToHost, st));
+    MG_HIP(hipStreamSynchronize(st));
+    most = h;
+  }
+  MG_REQUIRE(most < (1ull << 31), "mg_multiply_numeric_dense: more than 2^31 dense tile pairs");
+  if (!P.c.n_c) return 0;
+  if (!most) {
+    launch_product<false, kOutStruct>(ctx, P, out, HeavyRecord{});
+    MG_HIP(hipStreamSynchronize(st));
+    return 0;
+  }
+  StreamBuf<HeavyPair> found(most, st);
+  StreamBuf<unsigned long long> n_found(1 + P.c.n_c, st);  // then the C tiles' counts and cursors (u32)
+  uint32_t* const count = reinterpret_cast<uint32_t*>(n_found.get() + 1);
+  uint32_t* const cursor = count + P.c.n_c;
+  clear_words_kernel<<<grid_for(n_found.size(), kBlock, 4096), kBlock, 0, st>>>(
+      reinterpret_cast<uint64_t*>(n_found.get()), n_found.size());
+  MG_LAUNCH_CHECK();
+  launch_product<true, kOutStruct>(ctx, P, out, HeavyRecord{found.get(), count, n_found.get(), most, min_bits});
+  StreamBuf<uint32_t> base(P.c.n_c + 1ull, st);
+  exclusive_scan_u32(ctx, count, base.get(), P.c.n_c);
+  unsigned long long n = 0;
+  MG_HIP(hipMemcpyAsync(&n, n_found.get(), sizeof(n), hipMemcpyDeviceToHost, st));
+  MG_HIP(hipStreamSynchronize(st));
+  MG_REQUIRE(n <= most, "mg_multiply_numeric_dense: more dense pairs recorded than counted");
+  if (!n) return 0;
+  StreamBuf<uint2> pairs(n, st);
+  const uint64_t max_tasks = std::min<uint64_t>(n, P.c.n_c + n / kTaskPairs);
+  StreamBuf<DenseTask> tasks(max_tasks, st);
+  StreamBuf<uint32_t> n_tasks(2, st);
+  clear_words_kernel<<<1, kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(n_tasks.get()), 1);
+  MG_LAUNCH_CHECK();
+  heavy_scatter_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, st>>>(found.get(), static_cast<uint32_t>(n), base.get(),
+                                                                    cursor, pairs.get());
+  MG_LAUNCH_CHECK();
+  heavy_tasks_kernel<<<grid_for(P.c.n_c, kBlock, 4096), kBlock, 0, st>>>(base.get(), P.c.n_c, tasks.get(), n_tasks.get());
+  MG_LAUNCH_CHECK();
+  dense_contract_kernel<<<grid_for(max_tasks, kWavesPerBlock, 16384), kBlock, 0, st>>>(
+      tasks.get(), n_tasks.get(), pairs.get(), a->data.get(), bt->data.get(), data_c);
+  MG_LAUNCH_CHECK();
+  return n;
+}
+
+}  // namespace mgamd

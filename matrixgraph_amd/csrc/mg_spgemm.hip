@@ -7,8 +7,9 @@
 // Rt[c] (row c of the transposed right tile); output row r bit c = (L[r] & Rt[c]) != 0.
 // The loop runs only over non-zero Rt rows (wave ballot), so sparse tiles cost a few
 // instructions; dense tiles (64 non-zero rows) take 64 iterations. The handle-based numeric
-// pass multiplies pairs of tiles with at most 10 bits from their entry lists instead, one
-// pair per lane (fill_tiles_payload_kernel), and keeps the wave product for denser tiles.
+// passes are in mg_product.hip, except the allocation-free one: it multiplies pairs of tiles with at
+// most 10 bits from their entry lists, one pair per lane (fill_tiles_payload_kernel), and keeps
+// the wave product for denser tiles.
 #include <mutex>
 #include <string>
 
@@ -16,6 +17,7 @@
 
 #include "mg_device.hpp"
 #include "mg_internal.hpp"
+#include "mg_product.hpp"
 
 namespace mgamd {
 namespace {
@@ -39,125 +41,6 @@ __device__ inline uint64_t tile_product(uint64_t l_row, uint64_t rt_row) {
     out |= static_cast<uint64_t>((l_row & w) != 0) << c;
   }
   return out;
-}
-
-// Dense tile pairs on the matrix cores, as one contraction per C tile: for every pair
-// (A(x,k), Bt(y,k)) whose two tiles both hold at least min_bits set bits, the vector kernel
-// records the pair (its two tile indices) instead of multiplying it; then
-// dense_contract_kernel sums, per C tile, the int8 0/1 products of all its recorded pairs in
-// int32 (v_mfma_i32_32x32x32_i8, four 32 x 32 output blocks, two K-steps of 32 per pair) and
-// turns counts > 0 into bit rows once, ORed into C. Operands are expanded from the bit tiles
-// in registers: a lane loads one 64-bit row of each tile (A row r, Bt row c = B column c) and
-// turns 4 bits at a time into 4 bytes of 0/1 with a 24-bit multiply.
-// Lane layout (32x32x32 i8): lane l holds 16 bytes of A row l % 32 and of B column l % 32,
-// at k = 16 * (l / 32) .. +15 of the K-step (any k order works if both operands use it);
-// result register v of lane l is C[8 * (v / 4) + 4 * (l / 32) + v % 4][l % 32].
-typedef int mg_v16i __attribute__((ext_vector_type(16)));
-typedef int mg_v4i __attribute__((ext_vector_type(4)));
-
-// Bits 0..15 of x as 16 bytes of value 0 or 1 (byte j = bit j): nibble * 0x204081 puts bit
-// i of the nibble at bit 8i (the four shifted copies do not overlap), the mask keeps those.
-__device__ inline mg_v4i bits16_to_bytes(uint32_t x) {
-  mg_v4i out;
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    out[q] = static_cast<int>(__umul24((x >> (4 * q)) & 0xFu, 0x204081u) & 0x01010101u);
-  return out;
-}
-
-// Recorded dense pairs of one C tile (from one 64-tile step of its index intersection).
-struct DenseTask {
-  uint32_t tile, base, n;
-};
-struct DenseRecord {
-  uint2* pairs;  // (A tile, Bt tile)
-  DenseTask* tasks;
-  unsigned long long* counter;  // pairs recorded (low 32 bits) and tasks (high 32 bits)
-  uint32_t cap;            // capacity of pairs and of tasks (the exact dense pair count)
-  const uint32_t* bits_a;  // set bits per tile
-  const uint32_t* bits_bt;
-  uint32_t min_bits;
-};
-
-// One wave per recorded task: int32 counts of the 64 x 64 output over all the task's pairs
-// on the matrix cores, then one threshold; the rows are ORed into C atomically (several
-// tasks may share a C tile).
-__global__ void __launch_bounds__(kBlock) dense_contract_kernel(const DenseTask* __restrict__ tasks,
-                                                                const unsigned long long* __restrict__ counter,
-                                                                uint32_t cap, const uint2* __restrict__ pairs,
-                                                                const uint64_t* __restrict__ data_a,
-                                                                const uint64_t* __restrict__ data_bt,
-                                                                uint64_t* __restrict__ data_c) {
-  const uint32_t lane = lane_id();
-  const uint32_t lo = lane & 31, hi = lane >> 5;
-  const uint32_t n_tasks = min(static_cast<uint32_t>(*counter >> 32), cap);
-  const uint32_t n_waves = gridDim.x * kWavesPerBlock;
-  for (uint32_t t = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); t < n_tasks; t += n_waves) {
-    const DenseTask T = tasks[t];
-    mg_v16i acc00 = {}, acc01 = {}, acc10 = {}, acc11 = {};
-    const uint32_t p_end = min(T.base + T.n, cap);
-    for (uint32_t p = T.base; p < p_end; ++p) {
-      const uint2 pr = pairs[p];
-      const uint64_t* A = data_a + static_cast<uint64_t>(pr.x) * kTile;
-      const uint64_t* B = data_bt + static_cast<uint64_t>(pr.y) * kTile;
-      const uint64_t ra0 = A[lo], ra1 = A[32 + lo], rb0 = B[lo], rb1 = B[32 + lo];
-#pragma unroll
-      for (uint32_t st = 0; st < 2; ++st) {
-        const uint32_t k = 32 * st + 16 * hi;
-        const mg_v4i a0 = bits16_to_bytes(static_cast<uint32_t>(ra0 >> k));
-        const mg_v4i a1 = bits16_to_bytes(static_cast<uint32_t>(ra1 >> k));
-        const mg_v4i b0 = bits16_to_bytes(static_cast<uint32_t>(rb0 >> k));
-        const mg_v4i b1 = bits16_to_bytes(static_cast<uint32_t>(rb1 >> k));
-        acc00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, acc00, 0, 0, 0);
-        acc01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b1, acc01, 0, 0, 0);
-        acc10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b0, acc10, 0, 0, 0);
-        acc11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, acc11, 0, 0, 0);
-      }
-    }
-    uint64_t out = 0;  // output row `lane`
-#pragma unroll
-    for (uint32_t v = 0; v < 16; ++v) {
-      const uint32_t i0 = 8 * (v / 4) + (v % 4);
-      const uint64_t b00 = ballot(acc00[v] > 0), b01 = ballot(acc01[v] > 0);
-      const uint64_t b10 = ballot(acc10[v] > 0), b11 = ballot(acc11[v] > 0);
-      if (lane == i0) out |= (b00 & 0xFFFFFFFFull) | ((b01 & 0xFFFFFFFFull) << 32);
-      if (lane == i0 + 4) out |= (b00 >> 32) | ((b01 >> 32) << 32);
-      if (lane == 32 + i0) out |= (b10 & 0xFFFFFFFFull) | ((b11 & 0xFFFFFFFFull) << 32);
-      if (lane == 32 + i0 + 4) out |= (b10 >> 32) | ((b11 >> 32) << 32);
-    }
-    if (out) atomicOr(reinterpret_cast<unsigned long long*>(data_c) + static_cast<uint64_t>(T.tile) * kTile + lane,
-                      static_cast<unsigned long long>(out));
-  }
-}
-
-// Per Bt column k: the dense Bt tiles in it; then the dense pairs of the product: sum over
-// dense A tiles (x, k) of that count (the structural pair count restricted to dense tiles).
-__global__ void __launch_bounds__(kBlock) dense_col_count_kernel(const uint32_t* __restrict__ col, uint32_t n,
-                                                                 const uint32_t* __restrict__ bits,
-                                                                 uint32_t min_bits, uint32_t* __restrict__ count) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    if (bits[i] >= min_bits) atomicAdd(count + col[i], 1u);
-}
-__global__ void __launch_bounds__(kBlock) dense_pair_count_kernel(const uint32_t* __restrict__ col, uint32_t n,
-                                                                  const uint32_t* __restrict__ bits,
-                                                                  uint32_t min_bits,
-                                                                  const uint32_t* __restrict__ count,
-                                                                  unsigned long long* __restrict__ out) {
-  uint64_t local = 0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    if (bits[i] >= min_bits) local += count[col[i]];
-  local = wave_sum(local);
-  if (lane_id() == 0 && local) atomicAdd(out, static_cast<unsigned long long>(local));
-}
-
-// Set bits of every tile (for the dense-pair dispatch).
-__global__ void __launch_bounds__(kBlock) tile_bits_kernel(const uint64_t* __restrict__ data, uint32_t n_tiles,
-                                                           uint32_t* __restrict__ bits) {
-  const uint32_t n_waves = gridDim.x * kWavesPerBlock;
-  for (uint32_t i = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); i < n_tiles; i += n_waves) {
-    const uint64_t c = wave_sum(__popcll(data[static_cast<uint64_t>(i) * kTile + lane_id()]));
-    if (lane_id() == 0) bits[i] = static_cast<uint32_t>(c);
-  }
 }
 
 // Index of key in sorted a[lo, hi), or -1.
@@ -246,8 +129,8 @@ __device__ inline uint64_t tile_product_common(uint64_t l_row, uint64_t rt_row, 
 
 // 16-byte compact payload of a tile with at most kWideMax set bits: entry i = (row << 6) |
 // column in bits 12(i % 5).. of word i / 5, the entry count in bits 60..63 of word 1; count
-// kWideDense marks a denser tile, whose word 0 then holds the OR of its rows (the columns in
-// use: the inner indices j through which it meets the other operand's tiles).
+// kWideDense marks a denser tile, whose word 0 then holds the OR of its rows (the columns in use:
+// the inner indices j through which it meets the other operand's tiles).
 typedef uint64_t WidePayload __attribute__((ext_vector_type(2)));
 constexpr uint32_t kWideMax = 10;
 constexpr uint32_t kWideDense = 15;
@@ -258,12 +141,10 @@ __device__ inline uint32_t wide_entry(WidePayload p, uint32_t i) {
 }
 
 // Wide payload of every tile of both operands, one wave per tile (lane r holds row r): tiles
-// [0, n_a) of data_a, then the n_bt tiles of data_bt, at the same positions of `payload`; with
-// `bits`, also each tile's set-bit count at the same position.
+// [0, n_a) of data_a, then the n_bt tiles of data_bt, at the same positions of `payload`.
 __global__ void __launch_bounds__(kBlock) payload_kernel(const uint64_t* __restrict__ data_a, uint32_t n_a,
                                                          const uint64_t* __restrict__ data_bt, uint32_t n_bt,
-                                                         WidePayload* __restrict__ payload,
-                                                         uint32_t* __restrict__ bits = nullptr) {
+                                                         WidePayload* __restrict__ payload) {
   const uint32_t n_waves = gridDim.x * kWavesPerBlock;
   const uint64_t n_tiles = static_cast<uint64_t>(n_a) + n_bt;
   for (uint64_t i = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); i < n_tiles; i += n_waves) {
@@ -286,43 +167,21 @@ __global__ void __launch_bounds__(kBlock) payload_kernel(const uint64_t* __restr
       pl.x = w[0];
       pl.y = w[1] | (static_cast<uint64_t>(n) << 60);
     }
-    if (lane_id() == 0) {
-      payload[i] = pl;
-      if (bits) bits[i] = static_cast<uint32_t>(total);
-    }
+    if (lane_id() == 0) payload[i] = pl;
   }
 }
 
-bool prepared(const mg_tiled_matrix* m) { return m->prep_version == m->version && m->prep_payload.get(); }
-
-// Payloads of A's tiles at pl[0, n_a) and of Bt's at pl[n_a, n_a + n_bt), one launch (with
-// `bits`, the tiles' set-bit counts at the same positions). An operand prepared by
-// mg_tiled_matrix_prepare_operand is copied from its kept payloads instead (16 + 4 bytes per
-// tile rather than a read of its 512-byte tiles).
-void launch_payloads(hipStream_t st, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, WidePayload* pl,
-                     uint32_t* bits = nullptr) {
-  const bool pa = prepared(a) && a->n_nz_tile, pb = prepared(bt) && bt->n_nz_tile;
+// Payloads alone of A's tiles at pl[0, n_a) and of Bt's at pl[n_a, n_a + n_bt) (the allocation-free
+// pass); those of a prepared operand are copied.
+void launch_payloads(hipStream_t st, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, WidePayload* pl) {
   const uint32_t na = a->n_nz_tile, nb = bt->n_nz_tile;
-  if (pa) {
-    MG_HIP(hipMemcpyAsync(pl, a->prep_payload.get(), sizeof(WidePayload) * na, hipMemcpyDeviceToDevice, st));
-    if (bits) MG_HIP(hipMemcpyAsync(bits, a->prep_bits.get(), sizeof(uint32_t) * na, hipMemcpyDeviceToDevice, st));
-  }
-  if (pb) {
-    MG_HIP(hipMemcpyAsync(pl + na, bt->prep_payload.get(), sizeof(WidePayload) * nb, hipMemcpyDeviceToDevice, st));
-    if (bits)
-      MG_HIP(hipMemcpyAsync(bits + na, bt->prep_bits.get(), sizeof(uint32_t) * nb, hipMemcpyDeviceToDevice, st));
-  }
-  // The rest in one launch: both operands, or the one that is not prepared.
-  const uint64_t n = (pa ? 0ull : na) + (pb ? 0ull : nb);
-  if (!n) return;
-  if (!pa && !pb)
-    payload_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, st>>>(a->data.get(), na, bt->data.get(), nb, pl,
-                                                                          bits);
-  else if (!pa)
-    payload_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, st>>>(a->data.get(), na, nullptr, 0, pl, bits);
-  else
-    payload_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, st>>>(bt->data.get(), nb, nullptr, 0, pl + na,
-                                                                          bits ? bits + na : nullptr);
+  const bool pa = prepared(a) && na, pb = prepared(bt) && nb;
+  if (pa) MG_HIP(hipMemcpyAsync(pl, a->prep_payload.get(), sizeof(WidePayload) * na, hipMemcpyDeviceToDevice, st));
+  if (pb) MG_HIP(hipMemcpyAsync(pl + na, bt->prep_payload.get(), sizeof(WidePayload) * nb, hipMemcpyDeviceToDevice, st));
+  const uint32_t ma = pa ? 0 : na, mb = pb ? 0 : nb;
+  if (ma + mb == 0) return;
+  payload_kernel<<<grid_for(static_cast<uint64_t>(ma) + mb, kWavesPerBlock, 65536), kBlock, 0, st>>>(
+      a->data.get(), ma, bt->data.get(), mb, pa ? pl + na : pl);
   MG_LAUNCH_CHECK();
 }
 
@@ -331,29 +190,13 @@ void launch_payloads(hipStream_t st, const mg_tiled_matrix* a, const mg_tiled_ma
 // tiles is multiplied by that lane alone: every entry (r, j) of the A tile meets every entry
 // (c, j) of the Bt tile with the same j and sets bit c of row r in the wave's LDS
 // accumulator. Pairs with a denser tile take the full-tile wave product, kPairBatch at a time.
-// kMfma: a pair whose two tiles both hold at least rec.min_bits set bits is recorded for
-// dense_contract_kernel instead.
-// kOut: where a finished C tile goes (PrunedOut): ORed into data_c at its structural index
-// (kOutStruct), or, for a pruned product, only if it is non-zero: appended at the next slot
-// of out.data with its structural index in out.key (kOutAppend, slots past out.capacity are
-// counted but not written), flagged in out.flag (kOutFlag, no data written), or written at
-// out.pos[i] (kOutPos).
-enum : int { kOutStruct = 0, kOutAppend = 1, kOutFlag = 2, kOutPos = 3 };
-struct PrunedOut {
-  uint64_t* data;
-  uint32_t* key;
-  uint32_t* flag;
-  const uint32_t* pos;
-  unsigned long long* counter;
-  uint64_t capacity;
-};
-template <bool kMfma, int kOut = kOutStruct>
+// Only the allocation-free pass runs it: its 16 bytes of scratch per tile hold neither heads nor column
+// words (product_kernel takes 136 us where this one takes 518: C = A*A, R-MAT 14).
 __global__ void __launch_bounds__(kBlock) fill_tiles_payload_kernel(
     uint32_t n_c, const uint32_t* __restrict__ off_a, const uint32_t* __restrict__ off_bt,
     const uint32_t* __restrict__ row_c, const uint32_t* __restrict__ col_c, const uint32_t* __restrict__ col_a,
     const uint32_t* __restrict__ col_bt, const uint64_t* __restrict__ data_a, const uint64_t* __restrict__ data_bt,
-    const WidePayload* __restrict__ pl_a, const WidePayload* __restrict__ pl_bt, uint64_t* __restrict__ data_c,
-    DenseRecord rec, PrunedOut out = PrunedOut{}) {
+    const WidePayload* __restrict__ pl_a, const WidePayload* __restrict__ pl_bt, uint64_t* __restrict__ data_c) {
   __shared__ unsigned long long s_acc[kWavesPerBlock][kTile];
   const uint32_t lane = lane_id();
   unsigned long long* const acc_l = s_acc[threadIdx.x / kWave];
@@ -378,17 +221,14 @@ __global__ void __launch_bounds__(kBlock) fill_tiles_payload_kernel(
       const bool has = pos >= 0;
       const uint32_t ia = has ? (a_short ? j : static_cast<uint32_t>(pos)) : 0u;
       const uint32_t ib = has ? (a_short ? static_cast<uint32_t>(pos) : j) : 0u;
-      bool mfma = false;
-      if constexpr (kMfma) mfma = has && rec.bits_a[ia] >= rec.min_bits && rec.bits_bt[ib] >= rec.min_bits;
-      // Payloads only for the pairs the vector ALUs multiply.
       WidePayload pa = {0, 0}, pb = {0, 0};
-      if (has && !mfma) {
+      if (has) {
         pa = pl_a[ia];
         pb = pl_bt[ib];
       }
       const uint32_t na = wide_count(pa), nb = wide_count(pb);
-      const bool dense = has && !mfma && (na == kWideDense || nb == kWideDense);
-      if (has && !mfma && !dense) {
+      const bool dense = has && (na == kWideDense || nb == kWideDense);
+      if (has && !dense) {
         // Only the inner indices j present in both tiles give bits: per common j, the Bt
         // entries' columns are collected into one mask and ORed into the row of every A
         // entry with that j (na + nb steps per common j instead of na * nb comparisons).
@@ -406,24 +246,6 @@ __global__ void __launch_bounds__(kBlock) fill_tiles_payload_kernel(
             const uint32_t ea = wide_entry(pa, u);
             if ((ea & 63u) == jj) atomicOr(acc_l + (ea >> 6), cols);
           }
-        }
-      }
-      if constexpr (kMfma) {
-        // Record this step's dense pairs as one task of C tile i (dense_contract_kernel).
-        const uint64_t mm = ballot(mfma);
-        if (mm) {
-          const uint32_t n = static_cast<uint32_t>(__popcll(mm));
-          // One atomic reserves both the pair positions and the task slot.
-          unsigned long long both = 0;
-          if (lane == 0) both = atomicAdd(rec.counter, (1ull << 32) | n);
-          both = read_first_lane64(both);
-          const uint32_t base = static_cast<uint32_t>(both);
-          const uint32_t task = static_cast<uint32_t>(both >> 32);
-          if (mfma) {
-            const uint32_t at = base + static_cast<uint32_t>(__popcll(mm & ((1ull << lane) - 1)));
-            if (at < rec.cap) rec.pairs[at] = make_uint2(ia, ib);
-          }
-          if (lane == 0 && task < rec.cap) rec.tasks[task] = DenseTask{i, base, n};
         }
       }
       // Pairs with one dense tile: the dense tile's rows (lane = row) against the other tile's
@@ -523,28 +345,33 @@ __global__ void __launch_bounds__(kBlock) fill_tiles_payload_kernel(
     acc |= acc_l[lane];
     acc_l[lane] = 0;
     wave_lds_sync();
-    if constexpr (kOut == kOutStruct) {
-      uint64_t* dst = data_c + static_cast<uint64_t>(i) * kTile + lane;
-      if (acc) *dst |= acc;
-    } else {
-      const bool nz = ballot(acc != 0) != 0;  // wave-uniform
-      if constexpr (kOut == kOutFlag) {
-        if (lane == 0) out.flag[i] = nz ? 1u : 0u;
-      } else if constexpr (kOut == kOutPos) {
-        if (nz) out.data[static_cast<uint64_t>(out.pos[i]) * kTile + lane] = acc;
-      } else {
-        if (nz) {
-          unsigned long long slot = 0;
-          if (lane == 0) slot = atomicAdd(out.counter, 1ull);
-          slot = read_first_lane64(slot);
-          if (slot < out.capacity) {
-            out.data[slot * kTile + lane] = acc;
-            if (lane == 0) out.key[slot] = i;
-          }
-        }
-      }
-    }
+    uint64_t* dst = data_c + static_cast<uint64_t>(i) * kTile + lane;
+    if (acc) *dst |= acc;
   }
+}
+
+// Block-wide exclusive scan of one u32 per thread (kWaves waves).
+template <int kWaves>
+__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_tmp, uint32_t* total) {
+  const uint32_t lane = lane_id();
+  const uint32_t wave = threadIdx.x / kWave;
+  uint32_t incl = v;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d, kWave));
+    if (lane >= static_cast<uint32_t>(d)) incl += o;
+  }
+  if (lane == kWave - 1) s_tmp[wave] = incl;
+  __syncthreads();
+  uint32_t base = 0, tot = 0;
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t t = s_tmp[w];
+    if (w < static_cast<int>(wave)) base += t;
+    tot += t;
+  }
+  __syncthreads();
+  *total = tot;
+  return base + incl - v;
 }
 
 // len (<= 64) bits of a bit-packed array starting at bit `start`.
@@ -659,30 +486,6 @@ __global__ void col_scatter_kernel(const uint32_t* __restrict__ row, const uint3
   }
 }
 
-// Block-wide exclusive scan of one u32 per thread (kWaves waves).
-template <int kWaves>
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_tmp, uint32_t* total) {
-  const uint32_t lane = lane_id();
-  const uint32_t wave = threadIdx.x / kWave;
-  uint32_t incl = v;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d, kWave));
-    if (lane >= static_cast<uint32_t>(d)) incl += o;
-  }
-  if (lane == kWave - 1) s_tmp[wave] = incl;
-  __syncthreads();
-  uint32_t base = 0, tot = 0;
-  for (int w = 0; w < kWaves; ++w) {
-    const uint32_t t = s_tmp[w];
-    if (w < static_cast<int>(wave)) base += t;
-    tot += t;
-  }
-  __syncthreads();
-  *total = tot;
-  return base + incl - v;
-}
-
 // Per output row x: union over t in A.row(x) of B.row(t) in an LDS bitmap.
 // EMIT = false: count[x] = |union|, tp[x] = sum |B.row(t)|; with `sums`, the block's totals are
 // added to sums[0] (tile products), sums[1] (tiles of the B rows that A references, ref[x]:
@@ -775,34 +578,10 @@ void launch_fill_tiles(hipStream_t s, uint32_t n_c, const uint32_t* off_a, const
   MG_LAUNCH_CHECK();
 }
 
-// Numeric pass of the handle-level product: payloads of both operands (stream-ordered in the
-// context's scratch), then fill_tiles_payload_kernel; with a dense record (rec.pairs set), the
-// pairs of dense tiles are recorded there and dense_contract_kernel multiplies them after.
-// `pl` holds payload_words(a, bt) words of device scratch (the context's, or the static array
-// of the allocation-free entry point).
+// Words of payload scratch of the allocation-free pass.
 size_t payload_words(const mg_tiled_matrix* a, const mg_tiled_matrix* bt) {
   return 2 * (static_cast<size_t>(a->n_nz_tile) + bt->n_nz_tile + 1);
 }
-
-void launch_payload_product(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt,
-                            mg_tiled_matrix* c, WidePayload* pl, const DenseRecord& rec) {
-  if (c->n_nz_tile == 0) return;
-  hipStream_t st = ctx->stream;
-  WidePayload* pl_a = pl;
-  WidePayload* pl_bt = pl + a->n_nz_tile;
-  launch_payloads(st, a, bt, pl);
-  const uint32_t grid = grid_for(c->n_nz_tile, kWavesPerBlock, 65536);
-  if (rec.pairs)
-    fill_tiles_payload_kernel<true><<<grid, kBlock, 0, st>>>(
-        c->n_nz_tile, a->offset_row.get(), bt->offset_row.get(), c->row_idx.get(), c->col_idx.get(),
-        a->col_idx.get(), bt->col_idx.get(), a->data.get(), bt->data.get(), pl_a, pl_bt, c->data.get(), rec);
-  else
-    fill_tiles_payload_kernel<false><<<grid, kBlock, 0, st>>>(
-        c->n_nz_tile, a->offset_row.get(), bt->offset_row.get(), c->row_idx.get(), c->col_idx.get(),
-        a->col_idx.get(), bt->col_idx.get(), a->data.get(), bt->data.get(), pl_a, pl_bt, c->data.get(), rec);
-  MG_LAUNCH_CHECK();
-}
-
 
 // --- structural pass shared by the handle-level products ----------------------
 // Row form of B (B.row(t) = { y : Bt(y,t) present }), per-row structural counts and tile
@@ -927,27 +706,10 @@ __global__ void __launch_bounds__(kBlock) row_hist_kernel(const uint32_t* __rest
     atomicAdd(hist + row[i], 1u);
 }
 
-template <int kOut>
-void launch_pruned(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, uint32_t n_s,
-                   const uint32_t* row_s, const uint32_t* col_s, WidePayload* pl, const PrunedOut& out) {
-  if (!n_s) return;
-  fill_tiles_payload_kernel<false, kOut><<<grid_for(n_s, kWavesPerBlock, 65536), kBlock, 0, ctx->stream>>>(
-      n_s, a->offset_row.get(), bt->offset_row.get(), row_s, col_s, a->col_idx.get(), bt->col_idx.get(),
-      a->data.get(), bt->data.get(), pl, pl + a->n_nz_tile, nullptr, DenseRecord{}, out);
-  MG_LAUNCH_CHECK();
-}
-
 // Per C row: features of the cost model (see mg_multiply_row_features).
-__global__ void __launch_bounds__(kBlock) brow_bits_kernel(const uint32_t* __restrict__ col, uint32_t n,
-                                                           const uint32_t* __restrict__ bits,
-                                                           unsigned long long* __restrict__ out) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    atomicAdd(out + col[i], static_cast<unsigned long long>(bits[i]));
-}
-
 __global__ void __launch_bounds__(kBlock) row_features_kernel(uint32_t n, const uint32_t* __restrict__ off_a,
                                                               const uint32_t* __restrict__ col_a,
-                                                              const uint32_t* __restrict__ bits_a,
+                                                              const TileHead* __restrict__ head_a,
                                                               const unsigned long long* __restrict__ brow_bits,
                                                               const uint32_t* __restrict__ cnt,
                                                               const unsigned long long* __restrict__ tp,
@@ -958,7 +720,7 @@ __global__ void __launch_bounds__(kBlock) row_features_kernel(uint32_t n, const 
     const uint32_t a0 = off_a[x], a1 = off_a[x + 1];
     uint64_t abits = 0, bbits = 0, amax = 0;
     for (uint32_t k = a0 + lane; k < a1; k += kWave) {
-      const uint64_t ab = bits_a[k];
+      const uint64_t ab = head_a[k].bits;
       abits += ab;
       amax = ab > amax ? ab : amax;
       bbits += brow_bits[col_a[k]];
@@ -1118,12 +880,12 @@ extern "C" int mg_tiled_matrix_prepare_operand(mg_context* ctx, mg_tiled_matrix*
     hipStream_t st = ctx->stream;
     const uint32_t n = m->n_nz_tile;
     m->prep_payload.alloc(2ull * std::max<uint32_t>(1, n));
-    m->prep_bits.alloc(std::max<uint32_t>(1, n));
     if (n) {
       payload_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, st>>>(
-          m->data.get(), n, nullptr, 0, reinterpret_cast<WidePayload*>(m->prep_payload.get()), m->prep_bits.get());
+          m->data.get(), n, nullptr, 0, reinterpret_cast<WidePayload*>(m->prep_payload.get()));
       MG_LAUNCH_CHECK();
     }
+    prepare_operand(ctx, m);
     MG_HIP(hipStreamSynchronize(st));
     m->prep_version = m->version;
   });
@@ -1138,70 +900,47 @@ extern "C" int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, co
     DeviceGuard g(ctx->device);
     ++c->version;
     if (c->n_nz_tile == 0) return;
-    WidePayload* pl = reinterpret_cast<WidePayload*>(ctx_scratch(ctx, payload_words(a, bt)));
-    launch_payload_product(ctx, a, bt, c, pl, DenseRecord{});
+    ProductInputs in;
+    product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, false, true, in);
+    ProductOut out{};
+    out.data = c->data.get();
+    run_product(ctx, in, kOutStruct, out);
   });
 }
 
 namespace mgamd {
 namespace {
 
-// Structural index, operand payloads and features of a pruned product.
+// Structural index and operand inputs of a pruned product.
 struct PrunedPlan {
   Structural S;
   StreamBuf<uint32_t> row_s, col_s;
-  WidePayload* pl = nullptr;
-  StreamBuf<uint32_t> bits;  // set bits per tile of A, then of Bt (from the payload pass)
+  ProductInputs in;
 };
 
 void pruned_prepare(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, PrunedPlan& P,
-                    const char* who) {
+                    bool want_bits, const char* who) {
   hipStream_t s = ctx->stream;
   structural_pass(ctx, a, bt, P.S, who);
   const uint32_t n_s = static_cast<uint32_t>(P.S.n_c);
   P.row_s.alloc(n_s, s);
   P.col_s.alloc(n_s, s);
   structural_emit(ctx, a, P.S, P.row_s.get(), P.col_s.get());
-  P.pl = reinterpret_cast<WidePayload*>(ctx_scratch(ctx, payload_words(a, bt)));
-  P.bits.alloc(static_cast<size_t>(a->n_nz_tile) + bt->n_nz_tile + 1, s);
-  launch_payloads(s, a, bt, P.pl, P.bits.get());
+  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s.get(), P.col_s.get()}, want_bits, true, P.in);
 }
 
 // Features of every C row into feat (device, n_strips x kRowFeatures).
-// known_bits: the tiles' set-bit counts of A then Bt when a payload pass already made them
-// (else they are counted here).
+// in: the product's inputs, with set-bit counts.
 void row_features_into(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const Structural& S,
-                       float* feat, const uint32_t* known_bits = nullptr) {
+                       const ProductInputs& in, float* feat) {
   hipStream_t s = ctx->stream;
   const uint32_t n = S.n;
-  StreamBuf<uint32_t> counted(known_bits ? 0 : static_cast<size_t>(a->n_nz_tile) + bt->n_nz_tile + 1, s);
+  if (!n) return;
   StreamBuf<unsigned long long> brow(n, s);
-  MG_HIP(hipMemsetAsync(brow.get(), 0, sizeof(unsigned long long) * std::max<uint32_t>(1, n), s));
-  if (!known_bits) {
-    if (a->n_nz_tile) {
-      tile_bits_kernel<<<grid_for(a->n_nz_tile, kWavesPerBlock, 65536), kBlock, 0, s>>>(a->data.get(),
-                                                                                         a->n_nz_tile, counted.get());
-      MG_LAUNCH_CHECK();
-    }
-    if (bt->n_nz_tile) {
-      tile_bits_kernel<<<grid_for(bt->n_nz_tile, kWavesPerBlock, 65536), kBlock, 0, s>>>(
-          bt->data.get(), bt->n_nz_tile, counted.get() + a->n_nz_tile);
-      MG_LAUNCH_CHECK();
-    }
-  }
-  const uint32_t* bits_a = known_bits ? known_bits : counted.get();
-  const uint32_t* bits_b = bits_a + a->n_nz_tile;
-  if (bt->n_nz_tile) {
-    // Set bits of each row t of B = of the Bt tiles in column t.
-    brow_bits_kernel<<<grid_for(bt->n_nz_tile, kBlock), kBlock, 0, s>>>(bt->col_idx.get(), bt->n_nz_tile, bits_b,
-                                                                       brow.get());
-    MG_LAUNCH_CHECK();
-  }
-  if (n) {
-    row_features_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, s>>>(
-        n, a->offset_row.get(), a->col_idx.get(), bits_a, brow.get(), S.cnt.get(), S.tp.get(), feat);
-    MG_LAUNCH_CHECK();
-  }
+  right_row_bits(ctx, bt, in, brow.get());
+  row_features_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, s>>>(
+      n, a->offset_row.get(), a->col_idx.get(), in.a.head, brow.get(), S.cnt.get(), S.tp.get(), feat);
+  MG_LAUNCH_CHECK();
 }
 
 // Output slots from a prediction: per row min(structural, ceil(structural * clamp(y) *
@@ -1238,9 +977,9 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   if (capacity == MG_PRUNED_EXACT || n_s == 0) {
     // Exact: flag pass, scan, then each non-empty tile written at its final position.
     StreamBuf<uint32_t> flag(n_s, s), pos(n_s + 1ull, s);
-    PrunedOut fo{};
+    ProductOut fo{};
     fo.flag = flag.get();
-    launch_pruned<kOutFlag>(ctx, a, bt, n_s, row_s, col_s, P.pl, fo);
+    run_product(ctx, P.in, kOutFlag, fo);
     exclusive_scan_u32(ctx, flag.get(), pos.get(), n_s);
     uint32_t n32 = 0;
     MG_HIP(hipMemcpyAsync(&n32, pos.get() + n_s, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -1248,10 +987,10 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
     n_num = n32;
     alloc_tiled_matrix(c, S.n, n32);
     if (n32) {
-      PrunedOut po{};
+      ProductOut po{};
       po.data = c->data.get();
       po.pos = pos.get();
-      launch_pruned<kOutPos>(ctx, a, bt, n_s, row_s, col_s, P.pl, po);
+      run_product(ctx, P.in, kOutPos, po);
       place_pruned_index_kernel<<<grid_for(n_s, kBlock), kBlock, 0, s>>>(n_s, flag.get(), pos.get(), row_s, col_s,
                                                                         c->row_idx.get(), c->col_idx.get());
       MG_LAUNCH_CHECK();
@@ -1269,12 +1008,12 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
       StreamBuf<uint64_t> scratch(slots * kTile, s);
       StreamBuf<uint32_t> keys(slots, s);
       MG_HIP(hipMemsetAsync(counter.get(), 0, sizeof(unsigned long long), s));
-      PrunedOut ao{};
+      ProductOut ao{};
       ao.data = scratch.get();
       ao.key = keys.get();
       ao.counter = counter.get();
       ao.capacity = cap;
-      launch_pruned<kOutAppend>(ctx, a, bt, n_s, row_s, col_s, P.pl, ao);
+      run_product(ctx, P.in, kOutAppend, ao);
       unsigned long long got = 0;
       MG_HIP(hipMemcpyAsync(&got, counter.get(), sizeof(got), hipMemcpyDeviceToHost, s));
       MG_HIP(hipStreamSynchronize(s));
@@ -1334,7 +1073,7 @@ extern "C" int mg_multiply_pruned(mg_context* ctx, const mg_tiled_matrix* a, con
     *c_out = nullptr;
     DeviceGuard g(ctx->device);
     PrunedPlan P;
-    pruned_prepare(ctx, a, bt, P, "mg_multiply_pruned");
+    pruned_prepare(ctx, a, bt, P, false, "mg_multiply_pruned");
     auto c = std::make_unique<mg_tiled_matrix>();
     c->device = ctx->device;
     mg_pruned_stats st{};
@@ -1358,14 +1097,14 @@ extern "C" int mg_multiply_pruned_model(mg_context* ctx, const mg_tiled_matrix* 
     DeviceGuard g(ctx->device);
     hipStream_t s = ctx->stream;
     PrunedPlan P;
-    pruned_prepare(ctx, a, bt, P, "mg_multiply_pruned_model");
+    pruned_prepare(ctx, a, bt, P, true, "mg_multiply_pruned_model");
     const uint32_t n = P.S.n;
     uint64_t capacity = MG_PRUNED_EXACT;
     if (P.S.n_c) {
       StreamBuf<float> feat(static_cast<uint64_t>(n) * kRowFeatures, s), y(static_cast<uint64_t>(n) * n_out, s),
           pred(n, s);
       StreamBuf<unsigned long long> total(1, s);
-      row_features_into(ctx, a, bt, P.S, feat.get(), P.bits.get());
+      row_features_into(ctx, a, bt, P.S, P.in, feat.get());
       if (mg_mlp_forward(ctx, model, feat.get(), n, y.get()) != MG_OK)
         fail(MG_ERR_INTERNAL, std::string("mg_multiply_pruned_model: ") + mg_last_error());
       MG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), s));
@@ -1399,7 +1138,9 @@ extern "C" int mg_multiply_row_features(mg_context* ctx, const mg_tiled_matrix* 
     structural_pass(ctx, a, bt, S, "mg_multiply_row_features");
     const uint32_t n = S.n;
     StreamBuf<float> feat(static_cast<uint64_t>(n) * kRowFeatures, s);
-    row_features_into(ctx, a, bt, S, feat.get());
+    ProductInputs in;
+    product_inputs(ctx, a, bt, ProductTiles{}, true, false, in);
+    row_features_into(ctx, a, bt, S, in, feat.get());
     if (n) {
       MG_HIP(hipMemcpyAsync(features, feat.get(), sizeof(float) * n * kRowFeatures, hipMemcpyDeviceToHost, s));
       if (structural)
@@ -1428,7 +1169,11 @@ extern "C" int mg_multiply_numeric_noalloc(mg_context* ctx, const mg_tiled_matri
     // The device address of this device's copy of `scratch`, looked up when the context was
     // created; the kernels write every payload word they read, so nothing is cleared.
     WidePayload* pl = reinterpret_cast<WidePayload*>(noalloc_scratch(ctx->device));
-    launch_payload_product(ctx, a, bt, c, pl, DenseRecord{});
+    launch_payloads(ctx->stream, a, bt, pl);
+    fill_tiles_payload_kernel<<<grid_for(c->n_nz_tile, kWavesPerBlock, 65536), kBlock, 0, ctx->stream>>>(
+        c->n_nz_tile, a->offset_row.get(), bt->offset_row.get(), c->row_idx.get(), c->col_idx.get(), a->col_idx.get(),
+        bt->col_idx.get(), a->data.get(), bt->data.get(), pl, pl + a->n_nz_tile, c->data.get());
+    MG_LAUNCH_CHECK();
   });
 }
 
@@ -1440,55 +1185,9 @@ extern "C" int mg_multiply_numeric_dense(mg_context* ctx, const mg_tiled_matrix*
                "mg_multiply_numeric_dense: operands differ in n_strips");
     DeviceGuard g(ctx->device);
     ++c->version;
-    hipStream_t st = ctx->stream;
-    StreamBuf<uint32_t> ba(a->n_nz_tile, st), bb(bt->n_nz_tile, st);
-    if (a->n_nz_tile) {
-      tile_bits_kernel<<<grid_for(a->n_nz_tile, kWavesPerBlock, 65536), kBlock, 0, st>>>(a->data.get(), a->n_nz_tile,
-                                                                                         ba.get());
-      MG_LAUNCH_CHECK();
-    }
-    if (bt->n_nz_tile) {
-      tile_bits_kernel<<<grid_for(bt->n_nz_tile, kWavesPerBlock, 65536), kBlock, 0, st>>>(bt->data.get(),
-                                                                                          bt->n_nz_tile, bb.get());
-      MG_LAUNCH_CHECK();
-    }
-    // Exact number of dense pairs: the capacity of the pair and task lists.
-    uint64_t n_pairs = 0;
-    if (a->n_nz_tile && bt->n_nz_tile) {
-      StreamBuf<uint32_t> colcount(a->n_strips, st);
-      StreamBuf<unsigned long long> total(1, st);
-      MG_HIP(hipMemsetAsync(colcount.get(), 0, sizeof(uint32_t) * a->n_strips, st));
-      MG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), st));
-      dense_col_count_kernel<<<grid_for(bt->n_nz_tile, kBlock), kBlock, 0, st>>>(bt->col_idx.get(), bt->n_nz_tile,
-                                                                                bb.get(), min_bits, colcount.get());
-      MG_LAUNCH_CHECK();
-      dense_pair_count_kernel<<<grid_for(a->n_nz_tile, kBlock, 4096), kBlock, 0, st>>>(
-          a->col_idx.get(), a->n_nz_tile, ba.get(), min_bits, colcount.get(), total.get());
-      MG_LAUNCH_CHECK();
-      unsigned long long h = 0;
-      MG_HIP(hipMemcpyAsync(&h, total.get(), sizeof(h), hipMemcpyDeviceToHost, st));
-      MG_HIP(hipStreamSynchronize(st));
-      n_pairs = h;
-    }
-    MG_REQUIRE(n_pairs < (1ull << 31), "mg_multiply_numeric_dense: more than 2^31 dense tile pairs");
-    const uint32_t cap = static_cast<uint32_t>(n_pairs);
-    StreamBuf<uint2> pairs(cap, st);
-    StreamBuf<DenseTask> tasks(cap, st);
-    StreamBuf<unsigned long long> counter(1, st);
-    MG_HIP(hipMemsetAsync(counter.get(), 0, sizeof(unsigned long long), st));
-    DenseRecord rec{pairs.get(), tasks.get(), counter.get(), cap, ba.get(), bb.get(), min_bits};
-    WidePayload* pl = reinterpret_cast<WidePayload*>(ctx_scratch(ctx, payload_words(a, bt)));
-    launch_payload_product(ctx, a, bt, c, pl, rec);
-    if (cap && c->n_nz_tile) {
-      dense_contract_kernel<<<grid_for(cap, kWavesPerBlock, 16384), kBlock, 0, st>>>(
-          tasks.get(), counter.get(), cap, pairs.get(), a->data.get(), bt->data.get(), c->data.get());
-      MG_LAUNCH_CHECK();
-    }
-    unsigned long long h = 0;
-    MG_HIP(hipMemcpyAsync(&h, counter.get(), sizeof(h), hipMemcpyDeviceToHost, st));
-    MG_HIP(hipStreamSynchronize(st));
-    const uint64_t recorded = h & 0xFFFFFFFFull;
-    MG_REQUIRE(recorded <= n_pairs, "mg_multiply_numeric_dense: more dense pairs recorded than counted");
+    ProductInputs in;
+    product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, true, true, in);
+    const uint64_t recorded = run_product_dense(ctx, a, bt, in, min_bits, c->data.get());
     if (dense_products) *dense_products = recorded;
   });
 }

@@ -259,3 +259,115 @@ def test_layer1_fill_tiles_and_count(ctx):
     assert lib.mg_count(_stream(), 64, ns, len(c_row), dc.ptr, cnt.ptr) == 0
     assert int(_host(cnt, np.uint64)[0]) == int(np.unpackbits((c_data | prior).view(np.uint8)).sum())
     assert lib.mg_fill_tiles(_stream(), 32, ns, 0, 0, 1, None, *([None] * 12)) == 4
+
+
+# --- forms of the numeric pass ---------------------------------------------------
+def mixed_blocks(ns, rng):
+    """ns x ns tiles of mixed density (empty to full) around the 10-bit limit of compact tiles."""
+    out = np.zeros((ns * 64, ns * 64), np.uint8)
+    for i in range(ns):
+        for j in range(ns):
+            kind = rng.integers(6)
+            block = out[i * 64:i * 64 + 64, j * 64:j * 64 + 64]
+            if kind == 1:
+                block[rng.integers(0, 64, 3), rng.integers(0, 64, 3)] = 1
+            elif kind == 2:
+                block[rng.integers(0, 64, 10), rng.integers(0, 64, 10)] = 1  # at most the limit
+            elif kind == 3:
+                block.flat[rng.choice(4096, 11, replace=False)] = 1  # just above
+            elif kind == 4:
+                block[:] = rng.random((64, 64)) < 0.02
+            elif kind == 5 and rng.integers(8) == 0:
+                block[:] = 1
+    return out
+
+
+@pytest.mark.parametrize("ns", [1, 2, 17, 65])
+@pytest.mark.parametrize("prepare", ["", "a", "b", "ab"])
+def test_numeric_forms_match_oracle(ctx, ns, prepare):
+    M = mg()
+    rng = np.random.default_rng(ns)
+    if ns <= 17:
+        a_h, b_h = (M.HostTiledMatrix.from_dense(mixed_blocks(ns, rng)) for _ in range(2))
+    else:  # two words of tile columns
+        a_h, b_h = (M.HostTiledMatrix.from_dense((rng.random((ns * 64, ns * 64)) < p).astype(np.uint8))
+                    for p in (0.0008, 0.004))
+    a, b = M.TiledMatrix.upload(ctx, a_h), M.TiledMatrix.upload(ctx, b_h)
+    for m, name in ((a, "a"), (b, "b")):
+        if name in prepare:
+            m.prepare_operand()
+    for left, right, lh, rh in ((a, b, a_h, b_h), (a, a, a_h, a_h)):
+        c, _ = M.multiply(ctx, left, right)
+        tup = [(h.offset_row, h.row_idx, h.col_idx, h.data) for h in (lh, rh)]
+        got = c.download()
+        want = O.tile_numeric(ns, tup[0], tup[1], got.row_idx, got.col_idx)
+        assert np.array_equal(got.data, want)
+        c2, _ = M.multiply_symbolic(ctx, left, right)
+        for min_bits in (0, 11, 100):
+            M.multiply_numeric_dense(ctx, left, right, c2, min_bits)  # ORs the same tiles
+            assert np.array_equal(c2.download().data, want), min_bits
+        for cap in (M.PRUNED_EXACT, M.PRUNED_STRUCTURAL, 1):
+            p, _ = M.multiply_pruned(ctx, left, right, cap)
+            ph, full = p.download(), want.any(axis=1)
+            assert np.array_equal(ph.data, want[full])
+            assert np.array_equal(ph.row_idx, got.row_idx[full]) and np.array_equal(ph.col_idx, got.col_idx[full])
+
+
+@pytest.mark.parametrize("ns", [16384, 16385])  # the widest grid with row bitmaps, the first without
+def test_numeric_wide_grid(ctx, ns):
+    M = mg()
+    rng = np.random.default_rng(ns)
+    n, hub = ns * 64, 700
+    s = np.concatenate([rng.integers(0, n, 20000), np.full(9000, hub), rng.integers(0, n, 9000)]).astype(np.uint32)
+    d = np.concatenate([rng.integers(0, n, 20000), rng.integers(0, n, 9000), np.full(9000, hub)]).astype(np.uint32)
+    el = M.EdgeList.upload(ctx, n, s, d)
+    a, at = el.to_tiled_matrix(False), el.to_tiled_matrix(True)
+    firsts = s[::13]
+    x = M.EdgeList.upload(ctx, n, np.arange(len(firsts), dtype=np.uint32), firsts).to_tiled_matrix(False)
+    want = set()
+    succ = {}
+    for u, v in zip(s.tolist(), d.tolist()):
+        succ.setdefault(u, set()).add(v)
+    for r, u in enumerate(firsts.tolist()):
+        want.update((r, v) for v in succ.get(u, ()))
+    for min_bits in (None, 0, 3):
+        c, _ = M.multiply_symbolic(ctx, x, at)
+        if min_bits is None:
+            M.multiply_numeric(ctx, x, at, c)
+        else:
+            M.multiply_numeric_dense(ctx, x, at, c, min_bits)
+        e = c.to_edges()
+        got = set(zip(*(v.tolist() for v in e.download())))
+        assert got == want, min_bits
+        for m in (c, e):
+            m.close()
+    for m in (a, at, x, el):
+        m.close()
+
+
+def test_numeric_more_columns_than_words(ctx):
+    """4.2 M tiles with about 20 columns in use: more than the right operand has room for (2^26), so that
+    some tiles' column words are made on the way."""
+    M = mg()
+    el = M.EdgeList.er(ctx, 17, 3, 9, 3)
+    at = el.to_tiled_matrix(transpose=True)
+    el.close()
+    n = at.n_strips * 64
+    sources = O.sample_sources(n, 64, 5)
+    w = M.Walk(ctx, at, 64, 1)
+    w.run(sources, 1)
+    ref = w.export(1)
+    w.close()
+    x = M.EdgeList.upload(ctx, n, np.arange(64, dtype=np.uint32), sources).to_tiled_matrix(False)
+    c, _ = M.multiply(ctx, x, at)
+    assert c.digest() == ref.digest()
+    # A row strip whose own tiles are dense; then against the prepared operand.
+    deg = np.repeat(np.arange(64, dtype=np.uint32), 40)
+    x2 = M.EdgeList.upload(ctx, n, deg, np.random.default_rng(1).integers(0, 4096, len(deg)).astype(np.uint32))
+    x2 = x2.to_tiled_matrix(False)
+    c1, _ = M.multiply(ctx, x2, at)
+    at.prepare_operand()
+    c2, _ = M.multiply(ctx, x2, at)
+    assert c1.digest() == c2.digest() and c1.popcount() > 0
+    for m in (c, c1, c2, x, x2, at, ref):
+        m.close()
