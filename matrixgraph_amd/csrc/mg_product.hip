@@ -617,10 +617,15 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
       if (threadIdx.x == 0) s_slot = used ? atomicAdd(out.counter, static_cast<unsigned long long>(__popc(used))) : 0ull;
       __syncthreads();
       for (uint32_t s = wave; s < kWindow; s += n_waves) {
+        if (!((present >> s) & 1)) continue;
+        const bool nz = (used >> s) & 1;
         const uint64_t slot = s_slot + static_cast<uint32_t>(__popc(used & ((1u << s) - 1)));
-        if (!((used >> s) & 1) || slot >= out.capacity) continue;
-        out.data[slot * kTile + lane] = by_row[s * kTile + lane];
-        if (lane == 0) out.key[slot] = c_tile(s);
+        const uint32_t i = c_tile(s);
+        if (lane == 0) {
+          out.flag[i] = nz ? 1u : 0u;
+          if (nz) out.slot[i] = static_cast<uint32_t>(slot);
+        }
+        if (nz && slot < out.capacity) out.data[slot * kTile + lane] = by_row[s * kTile + lane];
       }
       __syncthreads();
       continue;

@@ -80,14 +80,14 @@ bool prepared(const mg_tiled_matrix* m);
 void prepare_operand(mg_context* ctx, mg_tiled_matrix* m);
 
 // Where a finished C tile goes: ORed into data at its index (kOutStruct), or, for a pruned product,
-// only if it is non-zero: appended at the next slot of data with its index in key (kOutAppend;
-// slots past capacity are counted but not written), flagged in flag (kOutFlag, no data
+// only if it is non-zero: into the next slot of data, whether and which in flag and slot
+// (kOutAppend; slots past capacity are counted but not written), flagged in flag (kOutFlag, no data
 // written), or written at pos[i] (kOutPos).
 enum : int { kOutStruct = 0, kOutAppend = 1, kOutFlag = 2, kOutPos = 3 };
 struct ProductOut {
   uint64_t* data = nullptr;
-  uint32_t* key = nullptr;
-  uint32_t* flag = nullptr;
+  uint32_t* flag = nullptr;  // per structural tile
+  uint32_t* slot = nullptr;
   const uint32_t* pos = nullptr;
   unsigned long long* counter = nullptr;
   uint64_t capacity = 0;

@@ -13,8 +13,6 @@
 #include <mutex>
 #include <string>
 
-#include <hipcub/hipcub.hpp>
-
 #include "mg_device.hpp"
 #include "mg_internal.hpp"
 #include "mg_product.hpp"
@@ -659,54 +657,59 @@ void structural_emit(mg_context* ctx, const mg_tiled_matrix* a, const Structural
 }
 
 // --- pruned product: only the numerically non-empty tiles of C ------------------
-// Final index of the appended tiles: sorted keys (structural indices) give each output
-// tile its row and column; data moves from its slot. One wave per tile.
-__global__ void __launch_bounds__(kBlock) gather_pruned_kernel(uint32_t n, const uint32_t* __restrict__ keys,
-                                                               const uint32_t* __restrict__ slots,
-                                                               const uint32_t* __restrict__ row_s,
-                                                               const uint32_t* __restrict__ col_s,
-                                                               const uint64_t* __restrict__ scratch,
-                                                               uint32_t* __restrict__ row_c,
-                                                               uint32_t* __restrict__ col_c,
-                                                               uint64_t* __restrict__ data_c) {
+// The pruned C from the flags of its structural tiles and their exclusive scan `pos` (n_s + 1): row and
+// column of every flagged tile, the row pointer (pos at the structural rows' starts), and, for tiles
+// that were appended, their data from their slots. A wave takes kPlaceTiles structural tiles and has
+// up to four in flight.
+constexpr uint32_t kPlaceTiles = 16;
+struct PrunedTiles {
+  uint32_t n_s, n_strips;
+  const uint32_t *flag, *pos, *row, *col, *off;
+  const uint32_t* slot;    // null: the data is in place
+  const uint64_t* scratch;
+};
+__global__ void __launch_bounds__(kBlock) place_pruned_kernel(PrunedTiles S, uint32_t* __restrict__ row_c,
+                                                              uint32_t* __restrict__ col_c,
+                                                              uint32_t* __restrict__ off_c,
+                                                              uint64_t* __restrict__ data_c) {
   const uint32_t lane = lane_id();
-  const uint32_t n_waves = gridDim.x * kWavesPerBlock;
-  for (uint32_t j = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); j < n; j += n_waves) {
-    const uint32_t k = keys[j];
-    data_c[static_cast<uint64_t>(j) * kTile + lane] = scratch[static_cast<uint64_t>(slots[j]) * kTile + lane];
-    if (lane == 0) {
-      row_c[j] = row_s[k];
-      col_c[j] = col_s[k];
+  for (uint64_t x = blockIdx.x * kBlock + threadIdx.x; x <= S.n_strips; x += static_cast<uint64_t>(gridDim.x) * kBlock)
+    off_c[x] = S.pos[S.off[x]];
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kWavesPerBlock * kPlaceTiles;
+  for (uint64_t i0 = static_cast<uint64_t>(read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave)) * kPlaceTiles;
+       i0 < S.n_s; i0 += stride) {
+    const uint64_t i = i0 + lane;
+    const bool has = lane < kPlaceTiles && i < S.n_s && S.flag[i] != 0;
+    const uint32_t to = has ? S.pos[i] : 0u, from = has && S.slot ? S.slot[i] : 0u;
+    if (has) {
+      row_c[to] = S.row[i];
+      col_c[to] = S.col[i];
+    }
+    if (!S.slot) continue;
+    for (uint64_t m = ballot(has); m;) {
+      uint64_t word[4];
+      uint32_t at[4];
+      uint32_t n = 0;  // wave-uniform
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        word[q] = 0;
+        at[q] = 0;
+        if (m) {
+          const int k = __ffsll(static_cast<unsigned long long>(m)) - 1;
+          m &= m - 1;
+          at[q] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(to), k));
+          const uint64_t src = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), k));
+          word[q] = S.scratch[src * kTile + lane];
+          ++n;
+        }
+      }
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q)
+        if (q < n) data_c[static_cast<uint64_t>(at[q]) * kTile + lane] = word[q];
     }
   }
 }
 
-// Index of the flagged tiles at their exact positions (kOutPos pass): pos = exclusive scan
-// of the flags.
-__global__ void __launch_bounds__(kBlock) place_pruned_index_kernel(uint32_t n_s, const uint32_t* __restrict__ flag,
-                                                                    const uint32_t* __restrict__ pos,
-                                                                    const uint32_t* __restrict__ row_s,
-                                                                    const uint32_t* __restrict__ col_s,
-                                                                    uint32_t* __restrict__ row_c,
-                                                                    uint32_t* __restrict__ col_c) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_s; i += gridDim.x * blockDim.x)
-    if (flag[i]) {
-      row_c[pos[i]] = row_s[i];
-      col_c[pos[i]] = col_s[i];
-    }
-}
-
-__global__ void __launch_bounds__(kBlock) iota_u32_kernel(uint32_t* __restrict__ out, uint32_t n) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = i;
-}
-
-__global__ void __launch_bounds__(kBlock) row_hist_kernel(const uint32_t* __restrict__ row, uint32_t n,
-                                                          uint32_t* __restrict__ hist) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    atomicAdd(hist + row[i], 1u);
-}
-
-// Per C row: features of the cost model (see mg_multiply_row_features).
 __global__ void __launch_bounds__(kBlock) row_features_kernel(uint32_t n, const uint32_t* __restrict__ off_a,
                                                               const uint32_t* __restrict__ col_a,
                                                               const TileHead* __restrict__ head_a,
@@ -974,9 +977,15 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   st.tile_products = S.tile_products;
   uint64_t n_num = 0;
   uint64_t cap = capacity == MG_PRUNED_STRUCTURAL ? n_s : std::min<uint64_t>(capacity, n_s);
+  StreamBuf<uint32_t> flag(n_s, s), pos(n_s + 1ull, s);
+  PrunedTiles tiles{n_s, S.n, flag.get(), pos.get(), row_s, col_s, S.off_c.get(), nullptr, nullptr};
+  const auto place = [&] {
+    place_pruned_kernel<<<grid_for(std::max<uint64_t>(n_s, S.n + 1ull), kWavesPerBlock * kPlaceTiles, 16384), kBlock, 0, s>>>(
+        tiles, c->row_idx.get(), c->col_idx.get(), c->offset_row.get(), c->data.get());
+    MG_LAUNCH_CHECK();
+  };
   if (capacity == MG_PRUNED_EXACT || n_s == 0) {
     // Exact: flag pass, scan, then each non-empty tile written at its final position.
-    StreamBuf<uint32_t> flag(n_s, s), pos(n_s + 1ull, s);
     ProductOut fo{};
     fo.flag = flag.get();
     run_product(ctx, P.in, kOutFlag, fo);
@@ -991,10 +1000,8 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
       po.data = c->data.get();
       po.pos = pos.get();
       run_product(ctx, P.in, kOutPos, po);
-      place_pruned_index_kernel<<<grid_for(n_s, kBlock), kBlock, 0, s>>>(n_s, flag.get(), pos.get(), row_s, col_s,
-                                                                        c->row_idx.get(), c->col_idx.get());
-      MG_LAUNCH_CHECK();
     }
+    place();
     st.passes = 2;
     st.capacity = n32;
     st.scratch_bytes = 0;
@@ -1002,15 +1009,16 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
     // One pass into `cap` slots; a capacity below the non-empty count is found by the
     // counter, which keeps counting past it, and the pass is run again with the exact count.
     StreamBuf<unsigned long long> counter(1, s);
+    StreamBuf<uint32_t> slot(n_s, s);
     st.capacity = cap;
     for (int attempt = 0;; ++attempt) {
       const uint64_t slots = std::max<uint64_t>(1, cap);
       StreamBuf<uint64_t> scratch(slots * kTile, s);
-      StreamBuf<uint32_t> keys(slots, s);
       MG_HIP(hipMemsetAsync(counter.get(), 0, sizeof(unsigned long long), s));
       ProductOut ao{};
       ao.data = scratch.get();
-      ao.key = keys.get();
+      ao.flag = flag.get();
+      ao.slot = slot.get();
       ao.counter = counter.get();
       ao.capacity = cap;
       run_product(ctx, P.in, kOutAppend, ao);
@@ -1026,38 +1034,15 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
         continue;
       }
       n_num = got;
-      const uint32_t n32 = static_cast<uint32_t>(got);
-      alloc_tiled_matrix(c, S.n, n32);
-      if (n32) {
-        // Row-major order: sort the slots by structural index, then move the tiles.
-        StreamBuf<uint32_t> slot_in(n32, s), keys_out(n32, s), slot_out(n32, s);
-        iota_u32_kernel<<<grid_for(n32, kBlock), kBlock, 0, s>>>(slot_in.get(), n32);
-        MG_LAUNCH_CHECK();
-        int bits = 1;
-        while ((1ull << bits) < n_s) ++bits;
-        size_t temp_bytes = 0;
-        MG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, temp_bytes, keys.get(), keys_out.get(), slot_in.get(),
-                                                  slot_out.get(), static_cast<int>(n32), 0, bits, s));
-        StreamBuf<uint8_t> temp(temp_bytes, s);
-        MG_HIP(hipcub::DeviceRadixSort::SortPairs(temp.get(), temp_bytes, keys.get(), keys_out.get(), slot_in.get(),
-                                                  slot_out.get(), static_cast<int>(n32), 0, bits, s));
-        gather_pruned_kernel<<<grid_for(n32, kWavesPerBlock, 65536), kBlock, 0, s>>>(
-            n32, keys_out.get(), slot_out.get(), row_s, col_s, scratch.get(), c->row_idx.get(), c->col_idx.get(),
-            c->data.get());
-        MG_LAUNCH_CHECK();
-      }
+      alloc_tiled_matrix(c, S.n, static_cast<uint32_t>(got));
+      // Row-major order: the tiles' places are the scan of their flags.
+      exclusive_scan_u32(ctx, flag.get(), pos.get(), n_s);
+      tiles.slot = slot.get();
+      tiles.scratch = scratch.get();
+      place();
       break;
     }
   }
-  // Row pointer of the pruned C from its row index.
-  StreamBuf<uint32_t> hist(S.n, s);
-  MG_HIP(hipMemsetAsync(hist.get(), 0, sizeof(uint32_t) * S.n, s));
-  if (n_num) {
-    row_hist_kernel<<<grid_for(n_num, kBlock), kBlock, 0, s>>>(c->row_idx.get(), static_cast<uint32_t>(n_num),
-                                                               hist.get());
-    MG_LAUNCH_CHECK();
-  }
-  exclusive_scan_u32(ctx, hist.get(), c->offset_row.get(), S.n);
   MG_HIP(hipStreamSynchronize(s));
   st.numeric_tiles = n_num;
   st.output_bytes = n_num * kTile * sizeof(uint64_t);
