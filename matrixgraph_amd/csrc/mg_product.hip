@@ -237,10 +237,9 @@ __global__ void __launch_bounds__(kBlock) b_rank_kernel(BitmapWord* __restrict__
   }
 }
 
-// off[0 .. n] = exclusive prefix sums of count[0 .. n); one workgroup (n <= kBitmapStrips).
+// off[0 .. n] = exclusive prefix sums of count[0 .. n), returned: their sum. One workgroup.
 constexpr int kScanWaves = 16;
-__global__ void __launch_bounds__(kScanWaves* kWave) row_offsets_kernel(const uint32_t* __restrict__ count, uint32_t n,
-                                                                        uint32_t* __restrict__ off) {
+__device__ inline uint32_t row_offsets(const uint32_t* __restrict__ count, uint32_t n, uint32_t* __restrict__ off) {
   __shared__ uint32_t s_sum[kScanWaves];
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
   uint32_t before = 0;
@@ -266,6 +265,11 @@ __global__ void __launch_bounds__(kScanWaves* kWave) row_offsets_kernel(const ui
     __syncthreads();
   }
   if (threadIdx.x == 0) off[n] = before;
+  return before;
+}
+__global__ void __launch_bounds__(kScanWaves* kWave) row_offsets_kernel(const uint32_t* __restrict__ count, uint32_t n,
+                                                                        uint32_t* __restrict__ off) {
+  row_offsets(count, n, off);
 }
 
 // Windows of C in use: kWindow strips; kWindow / 4 or one where they would be much work. A
@@ -313,6 +317,123 @@ __global__ void __launch_bounds__(kScanWaves* kWave) windows_kernel(ProductTiles
       const uint32_t x = C.row[i], y = C.col[i];
       windows[base + lanes_under(m)] = Window{static_cast<uint32_t>(i), x, y / kWindow * kWindow,
                                               y / width * width + width, off_a[x], off_a[x + 1], {0, 0}};
+    }
+  }
+}
+
+// Structural pass. Workgroup = tile row x: lane = word of B's bitmap rows, ORed over A's tiles in
+// registers, kUnionLoads rows in flight per wave; the waves meet in LDS. A frontier has few rows and
+// many tiles in each, so a row has 16 waves.
+constexpr int kUnionWaves = 16;
+constexpr int kUnionLoads = 8;
+__global__ void __launch_bounds__(kUnionWaves* kWave) union_rows_kernel(const uint32_t* __restrict__ off_a,
+                                                                        const uint32_t* __restrict__ col_a,
+                                                                        const BitmapWord* __restrict__ bm,
+                                                                        const uint32_t* __restrict__ off_b, uint32_t n,
+                                                                        uint32_t wpr, SymbolicRows S) {
+  __shared__ unsigned long long s_or[kWave], s_tp;
+  const uint32_t lane = lane_id(), wave = read_first_lane(threadIdx.x / kWave);
+  for (uint32_t x = blockIdx.x; x < n; x += gridDim.x) {
+    const uint32_t a0 = off_a[x], a1 = off_a[x + 1];
+    if (a0 == a1) {  // uniform
+      if (threadIdx.x == 0) {
+        S.cnt[x] = 0;
+        S.tp[x] = 0;
+      }
+      continue;
+    }
+    if (threadIdx.x == 0) s_tp = 0;
+    __syncthreads();
+    uint64_t tp = 0;
+    for (uint32_t k = a0 + threadIdx.x; k < a1; k += kUnionWaves * kWave) {
+      const uint32_t t = col_a[k];
+      tp += off_b[t + 1] - off_b[t];
+      S.ref[t] = 1;
+    }
+    tp = wave_sum(tp);
+    if (lane == 0 && tp) atomicAdd(&s_tp, static_cast<unsigned long long>(tp));
+    uint32_t count = 0;
+    for (uint32_t w0 = 0; w0 < wpr; w0 += kWave) {
+      if (wave == 0) s_or[lane] = 0;
+      __syncthreads();
+      const bool has = w0 + lane < wpr;
+      uint64_t acc = 0;
+      for (uint32_t k0 = a0 + wave * kUnionLoads; k0 < a1; k0 += kUnionWaves * kUnionLoads) {
+        uint64_t word[kUnionLoads];
+#pragma unroll
+        for (int q = 0; q < kUnionLoads; ++q) {
+          word[q] = 0;
+          if (k0 + q < a1 && has) word[q] = bm[static_cast<uint64_t>(col_a[k0 + q]) * wpr + w0 + lane].bits;
+        }
+#pragma unroll
+        for (int q = 0; q < kUnionLoads; ++q) acc |= word[q];
+      }
+      if (acc) atomicOr(&s_or[lane], static_cast<unsigned long long>(acc));
+      __syncthreads();
+      if (wave == 0) {
+        const uint64_t bits = s_or[lane];
+        if (has) S.c_bits[static_cast<uint64_t>(x) * wpr + w0 + lane] = bits;
+        count += wave_sum32(static_cast<uint32_t>(__popcll(bits)));
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      S.cnt[x] = count;
+      S.tp[x] = s_tp;
+    }
+    __syncthreads();
+  }
+}
+
+// C's row pointer and the totals; one workgroup.
+__global__ void __launch_bounds__(kScanWaves* kWave) symbolic_totals_kernel(SymbolicRows S,
+                                                                            const uint32_t* __restrict__ off_b,
+                                                                            uint32_t n) {
+  __shared__ unsigned long long s_tp, s_used;
+  if (threadIdx.x == 0) s_tp = s_used = 0;
+  __syncthreads();
+  uint64_t tp = 0, used = 0;
+  for (uint32_t x = threadIdx.x; x < n; x += kScanWaves * kWave) {
+    tp += S.tp[x];
+    if (S.ref[x]) used += off_b[x + 1] - off_b[x];
+  }
+  tp = wave_sum(tp);
+  used = wave_sum(used);
+  if (lane_id() == 0) {
+    atomicAdd(&s_tp, static_cast<unsigned long long>(tp));
+    atomicAdd(&s_used, static_cast<unsigned long long>(used));
+  }
+  const uint32_t n_c = row_offsets(S.cnt, n, S.off_c);
+  if (threadIdx.x == 0) {
+    S.sums[0] = s_tp;
+    S.sums[1] = s_used;
+    S.sums[2] = n_c;  // fits: kBitmapStrips rows of as many strips
+  }
+}
+
+// One wave per row: each word's tiles, lane = strip.
+__global__ void __launch_bounds__(kBlock) symbolic_emit_kernel(SymbolicRows S, uint32_t n, uint32_t wpr,
+                                                               uint32_t* __restrict__ row_c,
+                                                               uint32_t* __restrict__ col_c) {
+  const uint32_t lane = lane_id();
+  const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * kWavesPerBlock, per_row = (wpr + kWave - 1) / kWave;
+  for (uint64_t i = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); i < n * per_row; i += n_waves) {
+    const uint32_t x = static_cast<uint32_t>(i / per_row), w0 = static_cast<uint32_t>(i % per_row) * kWave;
+    uint32_t at = S.off_c[x];
+    if (at == S.off_c[x + 1]) continue;
+    const uint64_t* const row = S.c_bits + static_cast<uint64_t>(x) * wpr;
+    for (uint32_t w = lane; w < w0; w += kWave) at += static_cast<uint32_t>(__popcll(row[w]));
+    at = wave_sum32(at) - (kWave - 1) * S.off_c[x];
+    const uint64_t bits = w0 + lane < wpr ? row[w0 + lane] : 0ull;
+    for (uint64_t m = ballot(bits != 0); m; m &= m - 1) {
+      const int w = lowest(m);
+      const uint64_t word = read_lane(bits, w);
+      if ((word >> lane) & 1) {
+        const uint32_t to = at + lanes_under(word);
+        row_c[to] = x;
+        col_c[to] = (w0 + static_cast<uint32_t>(w)) * 64 + lane;
+      }
+      at += static_cast<uint32_t>(__popcll(word));
     }
   }
 }
@@ -775,19 +896,22 @@ void clear_u32(hipStream_t st, uint32_t* v, uint32_t n) {
   MG_LAUNCH_CHECK();
 }
 
-// Bitmap, ranks and row offsets of B; grids up to kBitmapStrips.
-struct RightIndex {
-  BitmapWord* bm;
-  uint32_t* off;    // n_strips + 1
-  uint32_t* count;  // n_strips, scratch
-};
-// bm cleared, its bits set.
-void launch_ranks(hipStream_t st, uint32_t ns, uint32_t wpr, const RightIndex& R) {
-  b_rank_kernel<<<grid_for(ns, kWavesPerBlock, 4096), kBlock, 0, st>>>(R.bm, ns, wpr, R.count, nullptr);
+// B's index: the words of bm cleared, then its bits, its rows' tiles and the words' positions.
+// count: n_strips of scratch.
+void launch_right_index(hipStream_t st, const mg_tiled_matrix* bt, BitmapWord* bm, uint32_t* off, uint32_t* count) {
+  const uint32_t ns = bt->n_strips, wpr = (ns + 63) / 64, n = bt->n_nz_tile;
+  const uint64_t words = 2ull * ns * wpr;
+  clear_words_kernel<<<grid_for(words, kBlock, 8192), kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(bm), words);
   MG_LAUNCH_CHECK();
-  row_offsets_kernel<<<1, kScanWaves * kWave, 0, st>>>(R.count, ns, R.off);
+  if (n) {
+    b_bitmap_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, st>>>(bt->row_idx.get(), bt->col_idx.get(), n, wpr, bm);
+    MG_LAUNCH_CHECK();
+  }
+  b_rank_kernel<<<grid_for(ns, kWavesPerBlock, 4096), kBlock, 0, st>>>(bm, ns, wpr, count, nullptr);
   MG_LAUNCH_CHECK();
-  b_rank_kernel<<<grid_for(ns, kWavesPerBlock, 4096), kBlock, 0, st>>>(R.bm, ns, wpr, R.count, R.off);
+  row_offsets_kernel<<<1, kScanWaves * kWave, 0, st>>>(count, ns, off);
+  MG_LAUNCH_CHECK();
+  b_rank_kernel<<<grid_for(ns, kWavesPerBlock, 4096), kBlock, 0, st>>>(bm, ns, wpr, count, off);
   MG_LAUNCH_CHECK();
 }
 
@@ -840,18 +964,13 @@ void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
     m->prep_bitmap.alloc(std::max<uint64_t>(1, bm));
     m->prep_index.alloc(ns + 1ull + n);
     StreamBuf<uint32_t> count(ns, st);
-    const RightIndex R{reinterpret_cast<BitmapWord*>(m->prep_bitmap.get()), m->prep_index.get(), count.get()};
-    clear_words_kernel<<<grid_for(bm, kBlock, 8192), kBlock, 0, st>>>(m->prep_bitmap.get(), bm);
-    MG_LAUNCH_CHECK();
-    b_bitmap_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, st>>>(m->row_idx.get(), m->col_idx.get(), n, wpr,
-                                                                  R.bm);
-    MG_LAUNCH_CHECK();
-    launch_ranks(st, ns, wpr, R);
+    BitmapWord* const words = reinterpret_cast<BitmapWord*>(m->prep_bitmap.get());
+    launch_right_index(st, m, words, m->prep_index.get(), count.get());
     as_b = as_a;
-    as_b.where = PositionMap{m->row_idx.get(), m->col_idx.get(), R.bm, wpr};
+    as_b.where = PositionMap{m->row_idx.get(), m->col_idx.get(), words, wpr};
     as_b.head_by_tile = as_a.head;
     as_b.head = reinterpret_cast<TileHead*>(m->prep_right_head.get());
-    as_b.tile = R.off + ns + 1;
+    as_b.tile = m->prep_index.get() + ns + 1;
     as_a.n = 0;
   }
   const uint64_t room = word_room(n);
@@ -869,18 +988,20 @@ void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
 }
 
 void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const ProductTiles& c,
-                    bool want_bits, bool want_words, ProductInputs& P) {
+                    bool want_bits, bool want_words, ProductInputs& P, const RightIndex& known) {
   hipStream_t st = ctx->stream;
   const uint32_t ns = a->n_strips, wpr = (ns + 63) / 64;
   const bool bitmap = ns <= kBitmapStrips;
   const bool pa = prepared(a), pb = prepared(bt), same = a == bt && bitmap;
   const uint64_t na = pa ? 0 : a->n_nz_tile, nb = pb ? 0 : bt->n_nz_tile;
-  const uint64_t bm = bitmap && !pb ? 2ull * ns * wpr : 0;  // u64 words
-  // Cleared: counters (column words taken; windows), the bitmap and the weights.
+  const bool index_b = bitmap && !pb;
+  const uint64_t bm = index_b && !known.bm ? 2ull * ns * wpr : 0;  // u64 words
+  // Cleared: counters (column words taken; windows) and the weights.
   const uint64_t weights = pa && pb ? 0 : 2ull * weight_words(ns);
-  const uint64_t clear = (2 + bm + (weights + 1) / 2 + 1) & ~1ull;
-  const uint64_t windows_at = clear + 2 * (na + nb), words_at = windows_at + 4ull * c.n_c;
-  const uint64_t u32s = (bm ? 2ull * ns + 1 + nb : 0) + (na + nb + 3) / 4;  // then the tiles' columns in use (u8)
+  const uint64_t clear = (2 + (weights + 1) / 2 + 1) & ~1ull;
+  const uint64_t heads_at = clear + bm, windows_at = heads_at + 2 * (na + nb), words_at = windows_at + 4ull * c.n_c;
+  const uint64_t index32 = index_b ? 2ull * ns + 1 + nb : 0;  // row pointer, scratch, tiles by position
+  const uint64_t u32s = index32 + (na + nb + 3) / 4;          // then the tiles' columns in use (u8)
   uint64_t room = want_words ? word_room(same && !pa ? nb : na + nb) : 0;
   uint64_t* base = nullptr;
   try {
@@ -892,10 +1013,9 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
     base = ctx_scratch(ctx, words_at + (u32s + 1) / 2);
   }
   unsigned long long* const next = reinterpret_cast<unsigned long long*>(base);
-  BitmapWord* const bitmap_words = reinterpret_cast<BitmapWord*>(base + 2);
-  uint32_t* const weight = reinterpret_cast<uint32_t*>(base + 2 + bm);
+  uint32_t* const weight = reinterpret_cast<uint32_t*>(base + 2);
   uint32_t* const weight2 = weight + weight_words(ns);
-  TileHead* const head_a = reinterpret_cast<TileHead*>(base + clear);
+  TileHead* const head_a = reinterpret_cast<TileHead*>(base + heads_at);
   TileHead* const head_b = head_a + na;
   P.n_strips = ns;
   P.c = c;
@@ -905,21 +1025,20 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   uint32_t* const at32 = reinterpret_cast<uint32_t*>(words + room);
   clear_words_kernel<<<grid_for(clear, kBlock, 4096), kBlock, 0, st>>>(base, clear);
   MG_LAUNCH_CHECK();
-  if (bm && bt->n_nz_tile) {
-    b_bitmap_kernel<<<grid_for(bt->n_nz_tile, kBlock, 4096), kBlock, 0, st>>>(
-        bt->row_idx.get(), bt->col_idx.get(), bt->n_nz_tile, wpr, bitmap_words);
-    MG_LAUNCH_CHECK();
-  }
-  uint8_t* const used = reinterpret_cast<uint8_t*>(at32 + (bm ? 2ull * ns + 1 + nb : 0));
+  uint8_t* const used = reinterpret_cast<uint8_t*>(at32 + index32);
   HeadJob job_a{a->data.get(), static_cast<uint32_t>(na), {}, head_a, nullptr, nullptr, used};
   HeadJob job_b{bt->data.get(), static_cast<uint32_t>(nb), {}, head_b, nullptr, nullptr, used + na};
-  if (bm) {
-    const RightIndex R{bitmap_words, at32, at32 + ns + 1};
-    launch_ranks(st, ns, wpr, R);
-    job_b.where = PositionMap{bt->row_idx.get(), bt->col_idx.get(), R.bm, wpr};
-    job_b.tile = R.count + ns;
-    P.b.bm = R.bm;
-    P.b.off = R.off;
+  if (index_b) {
+    P.b.bm = known.bm;
+    P.b.off = known.off;
+    if (!known.bm) {
+      BitmapWord* const words_b = reinterpret_cast<BitmapWord*>(base + clear);
+      launch_right_index(st, bt, words_b, at32, at32 + ns + 1);
+      P.b.bm = words_b;
+      P.b.off = at32;
+    }
+    job_b.where = PositionMap{bt->row_idx.get(), bt->col_idx.get(), P.b.bm, wpr};
+    job_b.tile = at32 + 2ull * ns + 1;
     P.b.tile = job_b.tile;
   }
   if (same && !pa) {  // one pass makes both operands' heads
@@ -956,6 +1075,37 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
       P.b.tile = P.b.off + ns + 1;
     }
   }
+}
+
+RightIndex right_index(mg_context* ctx, const mg_tiled_matrix* bt, StreamBuf<uint64_t>& mem) {
+  if (prepared(bt)) return {reinterpret_cast<const BitmapWord*>(bt->prep_bitmap.get()), bt->prep_index.get()};
+  const uint32_t ns = bt->n_strips;
+  const uint64_t words = 2ull * ns * ((ns + 63) / 64);
+  mem.alloc(words + ns + 1, ctx->stream);  // then the row pointer and scratch
+  BitmapWord* const bm = reinterpret_cast<BitmapWord*>(mem.get());
+  uint32_t* const off = reinterpret_cast<uint32_t*>(mem.get() + words);
+  launch_right_index(ctx->stream, bt, bm, off, off + ns + 1);
+  return {bm, off};
+}
+
+void symbolic_rows(mg_context* ctx, const mg_tiled_matrix* a, const RightIndex& b, const SymbolicRows& S) {
+  hipStream_t st = ctx->stream;
+  const uint32_t ns = a->n_strips, wpr = (ns + 63) / 64;
+  clear_u32(st, S.ref, ns);
+  if (ns) {
+    union_rows_kernel<<<grid_for(ns, 1, 16384), kUnionWaves * kWave, 0, st>>>(a->offset_row.get(), a->col_idx.get(), b.bm,
+                                                                             b.off, ns, wpr, S);
+    MG_LAUNCH_CHECK();
+  }
+  symbolic_totals_kernel<<<1, kScanWaves * kWave, 0, st>>>(S, b.off, ns);
+  MG_LAUNCH_CHECK();
+}
+
+void symbolic_emit(mg_context* ctx, uint32_t n_strips, const SymbolicRows& S, uint32_t* row_c, uint32_t* col_c) {
+  const uint32_t wpr = (n_strips + 63) / 64;
+  const uint64_t waves = static_cast<uint64_t>(n_strips) * ((wpr + kWave - 1) / kWave);
+  symbolic_emit_kernel<<<grid_for(waves, kWavesPerBlock, 16384), kBlock, 0, ctx->stream>>>(S, n_strips, wpr, row_c, col_c);
+  MG_LAUNCH_CHECK();
 }
 
 void run_product(mg_context* ctx, const ProductInputs& P, int out_mode, const ProductOut& out) {

@@ -46,6 +46,29 @@ struct RightOperand {
 };
 constexpr uint32_t kBitmapStrips = 16384;
 
+// The bitmap of B and its row pointer (grids up to kBitmapStrips).
+struct RightIndex {
+  const BitmapWord* bm = nullptr;
+  const uint32_t* off = nullptr;
+};
+// Of a prepared operand from its handle, else made in mem.
+RightIndex right_index(mg_context* ctx, const mg_tiled_matrix* bt, StreamBuf<uint64_t>& mem);
+
+// Structural pass of C = A * B over bitmaps: per tile row x of C its strips in c_bits (n_strips rows of
+// 64-bit words; rows without tiles of A are not written), their count cnt, and the tile products tp; then
+// C's row pointer and the totals (tile products, tiles of the B rows that A refers to, C tiles).
+struct SymbolicRows {
+  uint64_t* c_bits;
+  uint32_t* cnt;
+  unsigned long long* tp;
+  uint32_t* off_c;            // n_strips + 1
+  uint32_t* ref;              // n_strips, scratch
+  unsigned long long* sums;   // 3
+};
+void symbolic_rows(mg_context* ctx, const mg_tiled_matrix* a, const RightIndex& b, const SymbolicRows& S);
+// Row and column of every tile of C, row-major.
+void symbolic_emit(mg_context* ctx, uint32_t n_strips, const SymbolicRows& S, uint32_t* row_c, uint32_t* col_c);
+
 // The n_c tiles of C, row-major.
 struct ProductTiles {
   uint32_t n_c;
@@ -72,9 +95,10 @@ struct ProductInputs {
 };
 
 // Stream-ordered, no synchronisation; no allocation if the context's scratch is large enough.
-// want_bits: TileHead::bits; want_words: false leaves the column words out (heads only).
+// want_bits: TileHead::bits; want_words: false leaves the column words out (heads only). known: B's
+// index if it is made already.
 void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const ProductTiles& c,
-                    bool want_bits, bool want_words, ProductInputs& P);
+                    bool want_bits, bool want_words, ProductInputs& P, const RightIndex& known = {});
 // Operand kept with its handle (mg_tiled_matrix_prepare_operand): all but the payloads.
 bool prepared(const mg_tiled_matrix* m);
 void prepare_operand(mg_context* ctx, mg_tiled_matrix* m);

@@ -586,8 +586,11 @@ size_t payload_words(const mg_tiled_matrix* a, const mg_tiled_matrix* bt) {
 // products of C = A*B, C's row pointer, and the totals.
 struct Structural {
   uint32_t n = 0;  // n_strips
-  StreamBuf<uint32_t> off_b, col_b, cnt, off_c;
-  StreamBuf<unsigned long long> tp;
+  StreamBuf<uint64_t> mem;      // rows: counts, tile products, row pointer, totals
+  SymbolicRows rows{};
+  StreamBuf<uint64_t> index;    // by bitmaps: B's
+  RightIndex b{};
+  StreamBuf<uint32_t> off_b, col_b;  // by lists: B's rows
   uint64_t n_c = 0, tile_products = 0, right_used = 0;
 };
 
@@ -599,43 +602,54 @@ void structural_pass(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_m
   if (n_words > kMaxLdsBitmapWords) fail(MG_ERR_UNSUPPORTED, std::string(who) + ": n_strips > 524288 not supported");
   hipStream_t s = ctx->stream;
   S.n = n;
-  // One zeroed block: the totals (tile products, right tiles used, C tiles; u64), then the
-  // histogram, the scatter cursors and the referenced-row flags of the strips (u32 each).
-  StreamBuf<unsigned long long> zero(3 + (3ull * n + 1) / 2, s);
-  unsigned long long* const sums = zero.get();
-  uint32_t* const hist = reinterpret_cast<uint32_t*>(sums + 3);
-  uint32_t* const cursor = hist + n;
-  uint32_t* const ref = cursor + n;
-  MG_HIP(hipMemsetAsync(zero.get(), 0, zero.bytes(), s));
-  S.off_b.alloc(n + 1ull, s);
-  S.col_b.alloc(bt->n_nz_tile, s);
-  if (bt->n_nz_tile || a->n_nz_tile) {
-    col_hist_mark_kernel<<<grid_for(static_cast<uint64_t>(bt->n_nz_tile) + a->n_nz_tile, 256), 256, 0, s>>>(
-        bt->col_idx.get(), bt->n_nz_tile, a->col_idx.get(), a->n_nz_tile, hist, ref);
+  // Bitmaps wherever a grid has them: faster than the lists from 16 tiles to 2 M, on 64 to 16384 strips,
+  // also where a row of B has one tile per 32 words (7.9 K tiles on 4096 strips: 163 us, by lists
+  // 243; 1.0 M: 2.1 ms, 2.9, most of it the clearing of C).
+  const bool bitmaps = n <= kBitmapStrips;
+  // u64: totals (tile products, right tiles used, C tiles), tile products of the rows, C's bitmap;
+  // u32: referenced-row flags, counts, row pointer; by lists also histogram and scatter cursors.
+  const uint64_t c_bits = bitmaps ? static_cast<uint64_t>(n) * n_words : 0;
+  S.mem.alloc(3 + n + c_bits + (5ull * n + 2) / 2, s);
+  S.rows.sums = reinterpret_cast<unsigned long long*>(S.mem.get());
+  S.rows.tp = S.rows.sums + 3;
+  S.rows.c_bits = S.mem.get() + 3 + n;
+  S.rows.ref = reinterpret_cast<uint32_t*>(S.rows.c_bits + c_bits);
+  S.rows.cnt = S.rows.ref + n;
+  S.rows.off_c = S.rows.cnt + n;
+  if (bitmaps) {
+    S.b = right_index(ctx, bt, S.index);
+    symbolic_rows(ctx, a, S.b, S.rows);
+  } else {
+    uint32_t* const hist = S.rows.off_c + n + 1;
+    uint32_t* const cursor = hist + n;
+    MG_HIP(hipMemsetAsync(S.mem.get(), 0, S.mem.bytes(), s));
+    S.off_b.alloc(n + 1ull, s);
+    S.col_b.alloc(bt->n_nz_tile, s);
+    if (bt->n_nz_tile || a->n_nz_tile) {
+      col_hist_mark_kernel<<<grid_for(static_cast<uint64_t>(bt->n_nz_tile) + a->n_nz_tile, 256), 256, 0, s>>>(
+          bt->col_idx.get(), bt->n_nz_tile, a->col_idx.get(), a->n_nz_tile, hist, S.rows.ref);
+      MG_LAUNCH_CHECK();
+    }
+    exclusive_scan_u32(ctx, hist, S.off_b.get(), n);
+    if (bt->n_nz_tile) {
+      col_scatter_kernel<<<grid_for(bt->n_nz_tile, 256), 256, 0, s>>>(bt->row_idx.get(), bt->col_idx.get(),
+                                                                      bt->n_nz_tile, S.off_b.get(), cursor,
+                                                                      S.col_b.get());
+      MG_LAUNCH_CHECK();
+    }
+    const size_t lds = sizeof(uint64_t) * n_words;
+    const unsigned grid = grid_for(n, 1, 16384);
+    // The row kernel also adds up the totals. C's tile index is 32-bit (the reference's
+    // n_nz_tile is u32): the 64-bit C tile total is read with the other sums and checked before
+    // anything uses the 32-bit scan.
+    symbolic_row_kernel<false><<<grid, kRowBlock, lds, s>>>(n, a->offset_row.get(), a->col_idx.get(), S.off_b.get(),
+                                                            S.col_b.get(), S.rows.cnt, S.rows.tp, nullptr, nullptr,
+                                                            nullptr, S.rows.ref, S.rows.sums);
     MG_LAUNCH_CHECK();
+    exclusive_scan_u32(ctx, S.rows.cnt, S.rows.off_c, n);
   }
-  exclusive_scan_u32(ctx, hist, S.off_b.get(), n);
-  if (bt->n_nz_tile) {
-    col_scatter_kernel<<<grid_for(bt->n_nz_tile, 256), 256, 0, s>>>(bt->row_idx.get(), bt->col_idx.get(),
-                                                                    bt->n_nz_tile, S.off_b.get(), cursor,
-                                                                    S.col_b.get());
-    MG_LAUNCH_CHECK();
-  }
-  S.cnt.alloc(n, s);
-  S.off_c.alloc(n + 1ull, s);
-  S.tp.alloc(n, s);
-  const size_t lds = sizeof(uint64_t) * n_words;
-  const unsigned grid = grid_for(n, 1, 16384);
-  // The row kernel also adds up the totals. C's tile index is 32-bit (the reference's
-  // n_nz_tile is u32): the 64-bit C tile total is read with the other sums and checked before
-  // anything uses the 32-bit scan.
-  symbolic_row_kernel<false><<<grid, kRowBlock, lds, s>>>(n, a->offset_row.get(), a->col_idx.get(),
-                                                          S.off_b.get(), S.col_b.get(), S.cnt.get(), S.tp.get(),
-                                                          nullptr, nullptr, nullptr, ref, sums);
-  MG_LAUNCH_CHECK();
-  exclusive_scan_u32(ctx, S.cnt.get(), S.off_c.get(), n);
   unsigned long long h_sums[3] = {0, 0, 0};
-  MG_HIP(hipMemcpyAsync(h_sums, sums, sizeof(h_sums), hipMemcpyDeviceToHost, s));
+  MG_HIP(hipMemcpyAsync(h_sums, S.rows.sums, sizeof(h_sums), hipMemcpyDeviceToHost, s));
   MG_HIP(hipStreamSynchronize(s));  // the one synchronisation of the pass: the totals
   const uint64_t n_c64 = h_sums[2];
   MG_REQUIRE(n_c64 <= 0xFFFFFFFFull, std::string(who) + ": " + std::to_string(n_c64) +
@@ -649,9 +663,10 @@ void structural_pass(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_m
 void structural_emit(mg_context* ctx, const mg_tiled_matrix* a, const Structural& S, uint32_t* row_c,
                      uint32_t* col_c) {
   if (!S.n_c) return;
+  if (S.b.bm) return symbolic_emit(ctx, S.n, S.rows, row_c, col_c);
   const size_t lds = sizeof(uint64_t) * ((S.n + 63) / 64);
   symbolic_row_kernel<true><<<grid_for(S.n, 1, 16384), kRowBlock, lds, ctx->stream>>>(
-      S.n, a->offset_row.get(), a->col_idx.get(), S.off_b.get(), S.col_b.get(), nullptr, nullptr, S.off_c.get(),
+      S.n, a->offset_row.get(), a->col_idx.get(), S.off_b.get(), S.col_b.get(), nullptr, nullptr, S.rows.off_c,
       row_c, col_c);
   MG_LAUNCH_CHECK();
 }
@@ -858,7 +873,7 @@ extern "C" int mg_multiply_symbolic(mg_context* ctx, const mg_tiled_matrix* a, c
     auto c = std::make_unique<mg_tiled_matrix>();
     c->device = ctx->device;
     alloc_tiled_matrix(c.get(), S.n, static_cast<uint32_t>(S.n_c));
-    MG_HIP(hipMemcpyAsync(c->offset_row.get(), S.off_c.get(), sizeof(uint32_t) * (S.n + 1ull),
+    MG_HIP(hipMemcpyAsync(c->offset_row.get(), S.rows.off_c, sizeof(uint32_t) * (S.n + 1ull),
                           hipMemcpyDeviceToDevice, s));
     if (S.n_c) {
       MG_HIP(hipMemsetAsync(c->data.get(), 0, c->data.bytes(), s));
@@ -929,7 +944,7 @@ void pruned_prepare(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   P.row_s.alloc(n_s, s);
   P.col_s.alloc(n_s, s);
   structural_emit(ctx, a, P.S, P.row_s.get(), P.col_s.get());
-  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s.get(), P.col_s.get()}, want_bits, true, P.in);
+  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s.get(), P.col_s.get()}, want_bits, true, P.in, P.S.b);
 }
 
 // Features of every C row into feat (device, n_strips x kRowFeatures).
@@ -942,7 +957,7 @@ void row_features_into(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled
   StreamBuf<unsigned long long> brow(n, s);
   right_row_bits(ctx, bt, in, brow.get());
   row_features_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, s>>>(
-      n, a->offset_row.get(), a->col_idx.get(), in.a.head, brow.get(), S.cnt.get(), S.tp.get(), feat);
+      n, a->offset_row.get(), a->col_idx.get(), in.a.head, brow.get(), S.rows.cnt, S.rows.tp, feat);
   MG_LAUNCH_CHECK();
 }
 
@@ -978,7 +993,7 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   uint64_t n_num = 0;
   uint64_t cap = capacity == MG_PRUNED_STRUCTURAL ? n_s : std::min<uint64_t>(capacity, n_s);
   StreamBuf<uint32_t> flag(n_s, s), pos(n_s + 1ull, s);
-  PrunedTiles tiles{n_s, S.n, flag.get(), pos.get(), row_s, col_s, S.off_c.get(), nullptr, nullptr};
+  PrunedTiles tiles{n_s, S.n, flag.get(), pos.get(), row_s, col_s, S.rows.off_c, nullptr, nullptr};
   const auto place = [&] {
     place_pruned_kernel<<<grid_for(std::max<uint64_t>(n_s, S.n + 1ull), kWavesPerBlock * kPlaceTiles, 16384), kBlock, 0, s>>>(
         tiles, c->row_idx.get(), c->col_idx.get(), c->offset_row.get(), c->data.get());
@@ -1093,7 +1108,7 @@ extern "C" int mg_multiply_pruned_model(mg_context* ctx, const mg_tiled_matrix* 
       if (mg_mlp_forward(ctx, model, feat.get(), n, y.get()) != MG_OK)
         fail(MG_ERR_INTERNAL, std::string("mg_multiply_pruned_model: ") + mg_last_error());
       MG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), s));
-      capacity_kernel<<<grid_for(n, kBlock, 1024), kBlock, 0, s>>>(n, P.S.cnt.get(), y.get(), n_out, margin,
+      capacity_kernel<<<grid_for(n, kBlock, 1024), kBlock, 0, s>>>(n, P.S.rows.cnt, y.get(), n_out, margin,
                                                                   pred.get(), total.get());
       MG_LAUNCH_CHECK();
       unsigned long long h = 0;
@@ -1124,12 +1139,12 @@ extern "C" int mg_multiply_row_features(mg_context* ctx, const mg_tiled_matrix* 
     const uint32_t n = S.n;
     StreamBuf<float> feat(static_cast<uint64_t>(n) * kRowFeatures, s);
     ProductInputs in;
-    product_inputs(ctx, a, bt, ProductTiles{}, true, false, in);
+    product_inputs(ctx, a, bt, ProductTiles{}, true, false, in, S.b);
     row_features_into(ctx, a, bt, S, in, feat.get());
     if (n) {
       MG_HIP(hipMemcpyAsync(features, feat.get(), sizeof(float) * n * kRowFeatures, hipMemcpyDeviceToHost, s));
       if (structural)
-        MG_HIP(hipMemcpyAsync(structural, S.cnt.get(), sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
+        MG_HIP(hipMemcpyAsync(structural, S.rows.cnt, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
     }
     MG_HIP(hipStreamSynchronize(s));
     if (tile_products) *tile_products = S.tile_products;

@@ -345,6 +345,28 @@ def test_numeric_wide_grid(ctx, ns):
         m.close()
 
 
+@pytest.mark.parametrize("prepare", [False, True])
+@pytest.mark.parametrize("ns,edges", [(1, 9), (64, 400), (65, 5000), (1023, 3000), (4097, 9000), (16385, 9000)])
+def test_symbolic_matches_oracle(ctx, ns, edges, prepare):
+    """C's tile set, its row pointer and the totals; one or several words of strips, by bitmaps and (the last) not."""
+    M = mg()
+    rng = np.random.default_rng(ns)
+    s, d = (rng.integers(0, ns * 64, edges).astype(np.uint32) for _ in range(2))
+    s[: edges // 4] = s[0]
+    a, at = O.edges_to_tiles(ns * 64, s, d), O.edges_to_tiles(ns * 64, s, d, transpose=True)
+    ga, gat = (M.TiledMatrix.upload(ctx, host(*t)) for t in (a, at))
+    if prepare:
+        gat.prepare_operand()
+    c, st = M.multiply_symbolic(ctx, ga, gat)
+    off, row, col, tp = O.tile_symbolic(ns, a[1], a[3], at[1], at[3])
+    h = c.download()
+    assert np.array_equal(h.offset_row, off) and np.array_equal(h.row_idx, row) and np.array_equal(h.col_idx, col)
+    used = int(np.isin(at[3], np.unique(a[3])).sum())
+    assert (st["tile_products"], st["out_tiles"], st["right_tiles_used"]) == (tp, len(row), used)
+    for m in (c, ga, gat):
+        m.close()
+
+
 def test_numeric_more_columns_than_words(ctx):
     """4.2 M tiles with about 20 columns in use: more than the right operand has room for (2^26), so that
     some tiles' column words are made on the way."""
