@@ -274,8 +274,13 @@ uint64_t device_sum_u32(mg_context* ctx, const uint32_t* data, uint64_t n);
 // Exclusive scan of n u32 counts into out[0..n] (out[n] = total), on ctx->stream.
 void exclusive_scan_u32(mg_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n);
 void exclusive_scan_u32_on(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n);
-// Sort u64 keys ascending and drop duplicates; returns the unique count.
-uint64_t sort_unique_u64(mg_context* ctx, DevBuf<uint64_t>& keys, uint64_t n, int end_bit);
+// Sorts n < 2^31 keys by their bits [begin_bit, end_bit), stable; returns where they are, keys or alt. temp:
+// sort_u64_bytes of scratch.
+size_t sort_u64_bytes(uint64_t n, int begin_bit, int end_bit);
+uint64_t* sort_u64(hipStream_t st, uint64_t* keys, uint64_t* alt, uint64_t n, int begin_bit, int end_bit, void* temp,
+                   size_t temp_bytes);
+// v[0 .. n] = exclusive scan of v[0 .. n) (v[n]: total), 16-byte aligned; one workgroup: for a few thousand.
+void scan_in_place(hipStream_t st, uint32_t* v, uint32_t n);
 
 inline unsigned grid_for(uint64_t work, unsigned per_block, unsigned cap = 1u << 20) {
   uint64_t g = (work + per_block - 1) / per_block;

@@ -2234,45 +2234,6 @@ __global__ void __launch_bounds__(kBlock) export_mask_kernel(const uint64_t* __r
   }
 }
 
-// Exclusive scan of n counts in place, the total at [n]: one workgroup, for the few entries of an
-// export (a library scan is three launches).
-constexpr uint32_t kScanBlock = 1024;
-__global__ void __launch_bounds__(kScanBlock) scan_in_place_kernel(uint32_t* __restrict__ v, uint32_t n) {
-  __shared__ uint32_t s_sum[kScanBlock / kWave];
-  // A thread's entries in 16-byte loads, all in flight (one load at a time: 111 us for 65536 entries).
-  const uint32_t per = (n + 4 * kScanBlock - 1) / (4 * kScanBlock) * 4;
-  const uint32_t lo = min(n, threadIdx.x * per), hi = min(n, lo + per);
-  uint32_t sum = 0;
-#pragma unroll 8
-  for (uint32_t i = lo; i + 4 <= hi; i += 4) {
-    const uint4 q = *reinterpret_cast<const uint4*>(v + i);
-    sum += q.x + q.y + q.z + q.w;
-  }
-  for (uint32_t i = lo + (hi - lo) / 4 * 4; i < hi; ++i) sum += v[i];
-  uint32_t incl = sum;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d, kWave));
-    if (lane_id() >= static_cast<uint32_t>(d)) incl += o;
-  }
-  if (lane_id() == kWave - 1) s_sum[threadIdx.x / kWave] = incl;
-  __syncthreads();
-  uint32_t at = incl - sum;
-  for (uint32_t w = 0; w < threadIdx.x / kWave; ++w) at += s_sum[w];
-#pragma unroll 8
-  for (uint32_t i = lo; i + 4 <= hi; i += 4) {
-    const uint4 q = *reinterpret_cast<const uint4*>(v + i);
-    *reinterpret_cast<uint4*>(v + i) = make_uint4(at, at + q.x, at + q.x + q.y, at + q.x + q.y + q.z);
-    at += q.x + q.y + q.z + q.w;
-  }
-  for (uint32_t i = lo + (hi - lo) / 4 * 4; i < hi; ++i) {
-    const uint32_t c = v[i];
-    v[i] = at;
-    at += c;
-  }
-  if (threadIdx.x == kScanBlock - 1) v[n] = at;
-}
-
 // Row pointer and tile index of the export; base: the scanned counts. One wave per (row, group).
 __global__ void __launch_bounds__(kBlock) export_index_kernel(const uint64_t* __restrict__ mask,
                                                               const uint32_t* __restrict__ base, uint32_t rows,
@@ -3545,8 +3506,7 @@ mg_tiled_matrix* export_frontier(mg_context* ctx, const uint64_t* x, const uint6
     export_mask_kernel<<<(n_groups + kWaves - 1) / kWaves, kBlock, 0, st>>>(s_dev, ns, map, w0, rows, n_groups,
                                                                             mask.get(), base.get());
     MG_LAUNCH_CHECK();
-    scan_in_place_kernel<<<1, kScanBlock, 0, st>>>(base.get(), n_items);
-    MG_LAUNCH_CHECK();
+    scan_in_place(st, base.get(), n_items);
     MG_HIP(hipMemcpyAsync(&nt, base.get() + n_items, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     MG_HIP(hipStreamSynchronize(st));
   }

@@ -247,3 +247,35 @@ def test_symbolic_pass_rejects_more_than_u32_output_tiles(ctx):
         M.multiply_pruned(ctx, a, bt, M.PRUNED_EXACT)
     a.close()
     bt.close()
+
+
+@pytest.mark.parametrize("n,edges", [(1, 1), (2, 5), (65, 4095), (128, 4096), (1000, 4097), (300001, 12289), (1 << 31, 5000)])
+def test_upload_sorts_and_tiles_any_list(ctx, n, edges):
+    """Duplicates, self-loops, the largest ids, tiles of few and of many edges, ends of the passes' blocks of 4096."""
+    M = mg()
+    rng = np.random.default_rng(edges)
+    s, d = (rng.integers(0, n, edges) for _ in range(2))
+    s[0] = d[0] = n - 1
+    s[: edges // 3], d[: edges // 4] = n // 2, rng.integers(max(0, n - 200), n, edges // 4)
+    s, d = s.astype(np.uint32), d.astype(np.uint32)
+    key = np.unique((s.astype(np.uint64) << np.uint64(32)) | d)
+    el = M.EdgeList.upload(ctx, n, s, d)
+    got = el.download()
+    assert np.array_equal(got[0], key >> np.uint64(32)) and np.array_equal(got[1], key & np.uint64(0xFFFFFFFF))
+    un = el.union(M.EdgeList.upload(ctx, n, d, s))
+    key2 = np.unique(np.concatenate([key, (d.astype(np.uint64) << np.uint64(32)) | s]))
+    assert un.digest() == O.edges_digest((key2 >> np.uint64(32)).astype(np.uint32), key2.astype(np.uint32))
+    if n <= 300001:
+        for transpose in (False, True):
+            t = el.to_tiled_matrix(transpose)
+            h, want = t.download(), O.edges_to_tiles(n, s, d, transpose)
+            for x, y in zip((h.offset_row, h.row_idx, h.col_idx, h.data), want[1:]):
+                assert np.array_equal(x, y)
+            t.close()
+    bad = s.copy()
+    if n < 1 << 31 and edges > 7:
+        bad[[7, edges - 1]] = n
+        with pytest.raises(M.MGError, match="edge 7 has a vertex id"):
+            M.EdgeList.upload(ctx, n, bad, d)
+    for m in (el, un):
+        m.close()
