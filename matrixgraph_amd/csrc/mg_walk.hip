@@ -1842,9 +1842,8 @@ __global__ void __launch_bounds__(kBlock) finalize_strips_kernel(const StripItem
 struct PushItem {
   uint32_t strip, begin, end, panel;
 };
-constexpr uint32_t kPushItemTiles = 512;   // column positions per item
-constexpr int kPushCap = 128;              // jobs per wave list
-constexpr int kPushUnroll = 8;             // source rows loaded per step
+constexpr uint32_t kPushItemTiles = 256;   // column positions per item (512: 45 and 222 us, 128: as 256)
+constexpr int kPushRows = 4;               // source rows loaded per step
 
 // One wave per strip of panel panels[blockIdx.y]: zero X_1 words inside the previous Z x N
 // masks, reset X_1's masks.
@@ -1940,45 +1939,22 @@ __global__ void __launch_bounds__(kBlock) push_structural_kernel(const Chunk* __
   flush_block_counters(cnt, s_cnt, as_global(L.counters), nullptr);
 }
 
-// Pushes the first n jobs of a wave list; a job is (target vertex << 32) | source vertex.
-// Each source row is loaded whole (lane = word) and its non-zero words are OR-ed into the
-// target row; the target row is marked in Z.
-template <int W>
-__device__ inline void push_drain(unsigned long long* __restrict__ jobs, uint32_t n, gptr<const uint64_t> x_in,
-                                  gptr<uint64_t> x_out, gptr<uint64_t> z_out, uint32_t lane,
-                                  unsigned long long pad_job) {
-  const uint32_t padded = (n + kPushUnroll - 1) / kPushUnroll * kPushUnroll;
-  if (lane < padded - n) jobs[n + lane] = pad_job;
-  wave_lds_sync();
-  for (uint32_t j = 0; j < padded; j += kPushUnroll) {
-    unsigned long long e[kPushUnroll];
-    uint64_t val[kPushUnroll];
-#pragma unroll
-    for (int k = 0; k < kPushUnroll; ++k) {
-      e[k] = jobs[j + k];
-      val[k] = lane < W ? x_in[(e[k] & 0xFFFFFFFFull) * W + lane] : 0ull;
-    }
-#pragma unroll
-    for (int k = 0; k < kPushUnroll; ++k) {
-      const uint64_t v = e[k] >> 32;
-      if (val[k]) atomicOr((unsigned long long*)(x_out + v * W + lane), static_cast<unsigned long long>(val[k]));
-      const uint64_t any = ballot(val[k] != 0);
-      if (lane == 0 && any != 0) atomicOr((unsigned long long*)(z_out + (v >> 6)), 1ull << (v & 63));
-    }
-  }
-  wave_lds_sync();
-}
-
 // One workgroup per item; its waves take the item's column positions in groups of 64
-// (lane = tile). Per set bit of a tile whose source vertex is non-empty in X_0: one job. With
-// s_from_columns, every tile (y, t) of the column also ORs S_0[t] & alive into S_1[y]
+// (lane = tile). X_0 is one-hot, so a source vertex's row is one word (two sources on one vertex may
+// make it more): the strip's 64 rows are read once into an LDS table of (word, value), and every set
+// bit of a tile whose source vertex is in the table costs its lane one 8-byte atomic: 38 us for 300
+// sources on 200 K vertices, 191 for 4096 on 4 M, where a wave per set bit that loads and ORs the
+// whole row took 51 and 284. Rows with several words go that way still. Z is marked once per tile.
+// What is left is the S_1 atomics (half of it at 4096 sources) and the dense tiles' loads. With s_from_columns, every tile (y, t) of the column also ORs S_0[t] & alive into S_1[y]
 // (structural X_1; tiles of other columns add nothing): a hub strip y is reached from most
 // source columns, so S_1[y] is read first and only a missing bit costs an atomic.
 template <int W>
 __global__ void __launch_bounds__(kBlock) push_first_hop_kernel(const PushItem* __restrict__ items,
                                                                 const PanelLevel* __restrict__ lv,
                                                                 bool s_from_columns) {
-  __shared__ unsigned long long jobs_all[kWaves][kPushCap];
+  __shared__ uint64_t s_val[kTile];
+  __shared__ uint32_t s_word[kTile];
+  __shared__ unsigned long long s_several;  // rows with more than one word
   __shared__ unsigned long long s_cnt[kBlockCounters];
   const uint32_t lane = lane_id();
   const uint32_t wave = threadIdx.x / kWave;
@@ -1995,14 +1971,57 @@ __global__ void __launch_bounds__(kBlock) push_first_hop_kernel(const PushItem* 
   const uint32_t t = it.strip;
   const uint64_t vm = as_global(L.v_in)[t];
   const uint64_t sm = s_from_columns ? (as_global(L.s_in)[t] & L.alive_in) : 0ull;
-  const unsigned long long pad_job = static_cast<unsigned long long>(L.n_strips) * 64;  // zero source row
-  unsigned long long* const jobs = jobs_all[wave];
   uint32_t cnt[kBlockCounters];
 #pragma unroll
   for (int i = 0; i < kBlockCounters; ++i) cnt[i] = 0;
   if (threadIdx.x < kBlockCounters) s_cnt[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_several = 0;
   __syncthreads();
-  uint32_t len = 0;
+  {
+    // Row kWaves * i + wave of the strip's set rows, kPushRows at a time.
+    uint64_t mine = vm;
+    for (uint32_t i = 0; i < wave; ++i) mine &= mine - 1;
+    while (mine) {
+      uint64_t val[kPushRows];
+      uint32_t row[kPushRows];
+#pragma unroll
+      for (int q = 0; q < kPushRows; ++q) {
+        const bool any = mine != 0;
+        row[q] = any ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(mine)) - 1) : 0u;
+        val[q] = any && lane < W ? x_in[(static_cast<uint64_t>(t) * 64 + row[q]) * W + lane] : 0ull;
+        for (int i = 0; i < kWaves; ++i) mine &= mine - 1;
+      }
+#pragma unroll
+      for (int q = 0; q < kPushRows; ++q) {
+        const uint64_t words = ballot(val[q] != 0);
+        if (!words) continue;
+        const int w = __ffsll(static_cast<unsigned long long>(words)) - 1;
+        const uint64_t v = read_lane(val[q], w);
+        if (lane == 0) {
+          s_val[row[q]] = v;
+          s_word[row[q]] = static_cast<uint32_t>(w);
+          if (words & (words - 1)) atomicOr(&s_several, 1ull << row[q]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const uint64_t several = s_several;
+  // Set bit (target row r of strip y, source row c of strip t) of the lanes that have one; a row of
+  // several words is pushed by the whole wave.
+  const auto push = [&](bool has, uint32_t y, uint32_t r, uint32_t c) {
+    const bool whole = has && ((several >> c) & 1);
+    if (has && !whole)
+      atomicOr((unsigned long long*)(x_out + (static_cast<uint64_t>(y) * 64 + r) * W + s_word[c]),
+               static_cast<unsigned long long>(s_val[c]));
+    for (uint64_t m = several ? ballot(whole) : 0ull; m; m &= m - 1) {
+      const int k = __ffsll(static_cast<unsigned long long>(m)) - 1;
+      const uint64_t to = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(y * 64 + r), k)));
+      const uint64_t from = static_cast<uint64_t>(t) * 64 + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c), k));
+      const uint64_t val = lane < W ? x_in[from * W + lane] : 0ull;
+      if (val) atomicOr((unsigned long long*)(x_out + to * W + lane), static_cast<unsigned long long>(val));
+    }
+  };
   for (uint32_t g = it.begin + 64 * wave; g < it.end; g += 64 * kWaves) {
     const uint32_t p = g + lane;
     const bool valid = p < it.end;
@@ -2019,22 +2038,16 @@ __global__ void __launch_bounds__(kBlock) push_first_hop_kernel(const PushItem* 
     const bool dense = act && (pl & kPayloadDense) != 0;
     const uint64_t ent = (act && !dense) ? pl : 0ull;
     const uint32_t n_ent = static_cast<uint32_t>(ent >> 48) & 7u;
+    uint64_t z = 0;
 #pragma unroll
     for (uint32_t k = 0; k < kPayloadMax; ++k) {
       const uint32_t e = static_cast<uint32_t>(ent >> (12 * k)) & 0xFFFu;
-      const bool ok = k < n_ent && ((vm >> (e & 63u)) & 1);
-      const uint64_t has = ballot(ok);
-      if (has) {
-        if (len + 64 > kPushCap) {
-          push_drain<W>(jobs, len, x_in, x_out, z_out, lane, pad_job);
-          len = 0;
-        }
-        if (ok)
-          jobs[len + lanes_below(has)] = (static_cast<unsigned long long>(y * 64 + (e >> 6)) << 32) | (t * 64 + (e & 63u));
-        len += __popcll(has);
-        if (lane == 0) cnt[bEdges] += __popcll(has);
-      }
+      const bool has = k < n_ent && ((vm >> (e & 63u)) & 1);
+      push(has, y, e >> 6, e & 63u);
+      z |= has ? 1ull << (e >> 6) : 0ull;
+      cnt[bEdges] += has;
     }
+    if (z) atomicOr((unsigned long long*)(z_out + y), static_cast<unsigned long long>(z));
     // Dense tiles: the whole wave loads them (lane = row), kDenseBatch at a time, with the
     // row masks loaded per lane beside the payloads.
     for (uint64_t dm = ballot(dense); dm;) {
@@ -2045,30 +2058,23 @@ __global__ void __launch_bounds__(kBlock) push_first_hop_kernel(const PushItem* 
         const bool any = dm != 0;
         const int k = any ? __ffsll(static_cast<unsigned long long>(dm)) - 1 : 0;
         dm &= dm - 1;
-          const uint64_t slot = (read_lane(pl, k) >> 13) & 0xFFFFFFFFull;
+        const uint64_t slot = (read_lane(pl, k) >> 13) & 0xFFFFFFFFull;
         yb[q] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(y), k));
         const uint64_t rm = any ? read_lane(rm_l, k) : 0ull;
         bits[q] = ((rm >> lane) & 1) ? (dense_rows[slot * kTile + lane] & vm) : 0ull;
       }
 #pragma unroll
       for (int q = 0; q < kDenseBatch; ++q) {
-        for (uint64_t has = ballot(bits[q] != 0); has; has = ballot(bits[q] != 0)) {
-          if (len + 64 > kPushCap) {
-            push_drain<W>(jobs, len, x_in, x_out, z_out, lane, pad_job);
-            len = 0;
-          }
-          if (bits[q]) {
-            const uint32_t c = static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(bits[q])) - 1);
-            jobs[len + lanes_below(has)] = (static_cast<unsigned long long>(yb[q] * 64 + lane) << 32) | (t * 64 + c);
-            bits[q] &= bits[q] - 1;
-          }
-          len += __popcll(has);
-          if (lane == 0) cnt[bEdges] += __popcll(has);
-        }
+        const uint64_t rows = ballot(bits[q] != 0);
+        if (!rows) continue;
+        if (lane == 0) atomicOr((unsigned long long*)(z_out + yb[q]), static_cast<unsigned long long>(rows));
+        cnt[bEdges] += static_cast<uint32_t>(__popcll(bits[q]));
+        for (; ballot(bits[q] != 0); bits[q] &= bits[q] - 1)
+          push(bits[q] != 0, yb[q], lane,
+               bits[q] ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(bits[q])) - 1) : 0u);
       }
     }
   }
-  if (len) push_drain<W>(jobs, len, x_in, x_out, z_out, lane, pad_job);
   flush_block_counters(cnt, s_cnt, as_global(L.counters), nullptr);
 }
 

@@ -445,3 +445,47 @@ def test_export_matches_frontier(ctx, n_src, n):
         want = np.ascontiguousarray(want).view(np.uint64)
         assert np.array_equal(got.data, want.reshape(-1, 64))
         s_cur, _ = O.walk_symbolic(ns, ath.offset_row, ath.col_idx, s_cur)
+
+
+@pytest.mark.parametrize("n_sources", [1, 65, 130, 300, 700, 1500, 4096])
+def test_first_hop_of_sources_that_share_strips(ctx, n_sources):
+    """Sources from whole strips, with hubs among sources and targets, in each width of X."""
+    M = mg()
+    rng = np.random.default_rng(n_sources)
+    n = 4500
+    s, d = (rng.integers(0, n, 20000) for _ in range(2))
+    s[:6000], d[3000:9000] = 77, rng.integers(64, 128, 6000)
+    s, d = s.astype(np.uint32), d.astype(np.uint32)
+    at = M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True)
+    adj = np.zeros((n, n), bool)
+    adj[s, d] = True
+    for sources in ((np.arange(n_sources) + 77) % n, rng.permutation(n)[:n_sources]):
+        sources = sources.astype(np.uint32)
+        w = M.Walk(ctx, at, n_sources, 1)
+        w.run(sources, 1)
+        words = (n_sources + 63) // 64
+        bits = np.zeros((n, words * 64), np.uint8)
+        bits[:, :n_sources] = adj[sources].T
+        got = np.ascontiguousarray(w.frontier(1)[:n, :words])
+        assert np.array_equal(got, np.packbits(bits, axis=1, bitorder="little").view(np.uint64))
+        w.close()
+
+
+@pytest.mark.parametrize("sizes", [(1, 1), (3, 70, 3, 200), (64, 64, 64), (500, 900, 1400)])
+def test_batch_of_queries_with_common_sources(ctx, sizes):
+    """Rows of X_0 with several words: one vertex is a source of several queries of a panel."""
+    M = mg()
+    n = 4500
+    rng = np.random.default_rng(sum(sizes))
+    s, d = (rng.integers(0, n, 30000).astype(np.uint32) for _ in range(2))
+    s[:5000] = 77
+    at = M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True)
+    queries = [M.workloads.QuerySpec(0, (np.arange(k) + 70).astype(np.uint32), 1 + i % 3) for i, k in enumerate(sizes)]
+    b = M.WalkBatch(ctx, [at], queries)
+    b.run()
+    for i, q in enumerate(queries):
+        w = M.Walk(ctx, at, len(q.sources), q.hops)
+        w.run(q.sources, q.hops)
+        assert b.query_digest(i) == w.frontier_digest(q.hops), i
+        w.close()
+    b.close()
