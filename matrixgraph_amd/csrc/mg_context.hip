@@ -233,6 +233,7 @@ extern "C" int mg_context_create(int device, mg_context** out) {
     cache_add_context(device, prop.totalGlobalMem);
     try {
       ctx->counters.alloc(64);
+      ctx->mail.alloc(kMailWords);
     } catch (...) {
       cache_drop_context(device);
       (void)hipStreamDestroy(ctx->own_stream);

@@ -402,9 +402,7 @@ std::unique_ptr<mg_edge_list> finish_packed(mg_context* ctx, const SortScratch& 
   MG_LAUNCH_CHECK();
   uint32_t u = 0;
   unsigned long long first_bad = ~0ull;
-  MG_HIP(hipMemcpyAsync(&u, w.count + w.blocks, sizeof(u), hipMemcpyDeviceToHost, st));
-  if (bad) MG_HIP(hipMemcpyAsync(&first_bad, bad, sizeof(first_bad), hipMemcpyDeviceToHost, st));
-  MG_HIP(hipStreamSynchronize(st));
+  read_words(ctx, {w.count + w.blocks, &u, sizeof(u)}, {bad, &first_bad, bad ? uint32_t{sizeof(first_bad)} : 0u});
   MG_REQUIRE(first_bad == ~0ull, "mg_edges_upload: edge " + std::to_string(first_bad) + " has a vertex id >= n_vertices");
   el->n_edges = u;
   return el;
@@ -721,8 +719,7 @@ std::unique_ptr<mg_edge_list> without_self_loops(mg_context* ctx, const mg_edge_
     off_diagonal_flag_kernel<<<grid_for(n, 256), 256, 0, st>>>(el->keys.get(), n, flag.get());
     MG_LAUNCH_CHECK();
     exclusive_scan_u32(ctx, flag.get(), pos.get(), static_cast<uint32_t>(n));
-    MG_HIP(hipMemcpyAsync(&count, pos.get() + n, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    MG_HIP(hipStreamSynchronize(st));
+    read_words(ctx, {pos.get() + n, &count, sizeof(count)});
   }
   auto out = std::make_unique<mg_edge_list>();
   out->device = ctx->device;
@@ -811,8 +808,7 @@ std::unique_ptr<mg_edge_list> tiles_to_edges(mg_context* ctx, const mg_tiled_mat
                                          " edges, more than 2^31 - 1");
   exclusive_scan_u32(ctx, count.get(), start.get(), n_slots);
   uint32_t total = 0;
-  MG_HIP(hipMemcpyAsync(&total, start.get() + n_slots, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  MG_HIP(hipStreamSynchronize(st));
+  read_words(ctx, {start.get() + n_slots, &total, sizeof(uint32_t)});
   el->n_edges = total;
   el->keys.alloc(total ? total : 1);
   if (total) {
@@ -855,8 +851,7 @@ extern "C" int mg_edges_grid_block(mg_context* ctx, const mg_edge_list* el, uint
       grid_block_flag_kernel<<<grid_for(n, 256), 256, 0, st>>>(el->keys.get(), n, scope, bx, by, flag.get());
       MG_LAUNCH_CHECK();
       exclusive_scan_u32(ctx, flag.get(), pos.get(), static_cast<uint32_t>(n));
-      MG_HIP(hipMemcpyAsync(&count, pos.get() + n, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-      MG_HIP(hipStreamSynchronize(st));
+      read_words(ctx, {pos.get() + n, &count, sizeof(count)});
     }
     auto b = std::make_unique<mg_edge_list>();
     b->device = ctx->device;
@@ -977,8 +972,7 @@ extern "C" int mg_edges_to_tiled_matrix(mg_context* ctx, const mg_edge_list* el,
     MG_LAUNCH_CHECK();
     scan_in_place(st, w.count, w.blocks);
     uint32_t n_tiles = 0;
-    MG_HIP(hipMemcpyAsync(&n_tiles, w.count + w.blocks, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    MG_HIP(hipStreamSynchronize(st));
+    read_words(ctx, {w.count + w.blocks, &n_tiles, sizeof(n_tiles)});
     alloc_tiled_matrix(m.get(), n_strips, n_tiles);
     f.row = m->row_idx.get();
     f.col = m->col_idx.get();

@@ -210,6 +210,7 @@ struct mg_context {
   // Per-call device temporaries of asynchronous calls on `stream` (calls on one context run
   // in stream order, so the next call may reuse them); grown by ctx_scratch, stream-ordered.
   mgamd::StreamBuf<uint64_t> scratch;
+  mgamd::PinnedBuf<uint32_t> mail;  // read_words
 };
 
 struct mg_tiled_matrix {
@@ -271,6 +272,15 @@ void alloc_tiled_matrix(mg_tiled_matrix* m, uint32_t n_strips, uint32_t n_nz_til
 uint64_t device_popcount(mg_context* ctx, const uint64_t* data, uint64_t n_words);
 // Sum of n u32 values, in 64 bits (for totals that a u32 scan would wrap).
 uint64_t device_sum_u32(mg_context* ctx, const uint32_t* data, uint64_t n);
+// Reads a few words of device memory (4-byte aligned, kMailWords together) into host memory once the
+// stream gets there; waits for it. A kernel writes them to pinned memory: half the time of a copy.
+struct DeviceWords {
+  const void* from;
+  void* to;
+  uint32_t bytes;
+};
+constexpr uint32_t kMailWords = 64;
+void read_words(mg_context* ctx, DeviceWords a, DeviceWords b = {nullptr, nullptr, 0});
 // Exclusive scan of n u32 counts into out[0..n] (out[n] = total), on ctx->stream.
 void exclusive_scan_u32(mg_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n);
 void exclusive_scan_u32_on(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n);

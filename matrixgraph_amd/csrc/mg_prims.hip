@@ -1,5 +1,7 @@
 // Setup-path primitives: scans and sorts (hipCUB), popcount reduction.
 // None of these run inside a walk hop; they build indices and inputs.
+#include <cstring>
+
 #include <hipcub/hipcub.hpp>
 
 #include "mg_device.hpp"
@@ -28,7 +30,25 @@ __global__ void __launch_bounds__(256) sum_u32_kernel(const uint32_t* __restrict
   if (lane_id() == 0 && local) atomicAdd(out, static_cast<unsigned long long>(local));
 }
 
+__global__ void __launch_bounds__(kWave) read_words_kernel(const uint32_t* a, uint32_t n_a, const uint32_t* b,
+                                                           uint32_t n_b, uint32_t* __restrict__ mail) {
+  const uint32_t i = threadIdx.x;
+  if (i < n_a) mail[i] = a[i];
+  if (i >= n_a && i < n_a + n_b) mail[i] = b[i - n_a];
+}
+
 }  // namespace
+
+void read_words(mg_context* ctx, DeviceWords a, DeviceWords b) {
+  const uint32_t n_a = a.bytes / 4, n_b = b.bytes / 4;
+  if (a.bytes % 4 || b.bytes % 4 || n_a + n_b > kMailWords) fail(MG_ERR_INTERNAL, "read_words: size");
+  read_words_kernel<<<1, kWave, 0, ctx->stream>>>(static_cast<const uint32_t*>(a.from), n_a,
+                                                  static_cast<const uint32_t*>(b.from), n_b, ctx->mail.get());
+  MG_LAUNCH_CHECK();
+  MG_HIP(hipStreamSynchronize(ctx->stream));
+  std::memcpy(a.to, ctx->mail.get(), a.bytes);
+  if (b.bytes) std::memcpy(b.to, ctx->mail.get() + n_a, b.bytes);
+}
 
 uint64_t device_popcount(mg_context* ctx, const uint64_t* data, uint64_t n_words) {
   unsigned long long* d = ctx->counters.get();
@@ -38,8 +58,7 @@ uint64_t device_popcount(mg_context* ctx, const uint64_t* data, uint64_t n_words
     MG_LAUNCH_CHECK();
   }
   unsigned long long h = 0;
-  MG_HIP(hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-  MG_HIP(hipStreamSynchronize(ctx->stream));
+  read_words(ctx, {d, &h, sizeof(h)});
   return h;
 }
 
@@ -51,8 +70,7 @@ uint64_t device_sum_u32(mg_context* ctx, const uint32_t* data, uint64_t n) {
     MG_LAUNCH_CHECK();
   }
   unsigned long long h = 0;
-  MG_HIP(hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-  MG_HIP(hipStreamSynchronize(ctx->stream));
+  read_words(ctx, {d, &h, sizeof(h)});
   return h;
 }
 

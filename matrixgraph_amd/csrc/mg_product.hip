@@ -1156,8 +1156,7 @@ uint64_t run_product_dense(mg_context* ctx, const mg_tiled_matrix* a, const mg_t
                                                                                total);
     MG_LAUNCH_CHECK();
     unsigned long long h = 0;
-    MG_HIP(hipMemcpyAsync(&h, total, sizeof(h), hipMemcpyDeviceToHost, st));
-    MG_HIP(hipStreamSynchronize(st));
+    read_words(ctx, {total, &h, sizeof(h)});
     most = h;
   }
   MG_REQUIRE(most < (1ull << 31), "mg_multiply_numeric_dense: more than 2^31 dense tile pairs");
@@ -1178,8 +1177,7 @@ uint64_t run_product_dense(mg_context* ctx, const mg_tiled_matrix* a, const mg_t
   StreamBuf<uint32_t> base(P.c.n_c + 1ull, st);
   exclusive_scan_u32(ctx, count, base.get(), P.c.n_c);
   unsigned long long n = 0;
-  MG_HIP(hipMemcpyAsync(&n, n_found.get(), sizeof(n), hipMemcpyDeviceToHost, st));
-  MG_HIP(hipStreamSynchronize(st));
+  read_words(ctx, {n_found.get(), &n, sizeof(n)});
   MG_REQUIRE(n <= most, "mg_multiply_numeric_dense: more dense pairs recorded than counted");
   if (!n) return 0;
   StreamBuf<uint2> pairs(n, st);

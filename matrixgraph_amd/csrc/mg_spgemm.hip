@@ -649,8 +649,7 @@ void structural_pass(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_m
     exclusive_scan_u32(ctx, S.rows.cnt, S.rows.off_c, n);
   }
   unsigned long long h_sums[3] = {0, 0, 0};
-  MG_HIP(hipMemcpyAsync(h_sums, S.rows.sums, sizeof(h_sums), hipMemcpyDeviceToHost, s));
-  MG_HIP(hipStreamSynchronize(s));  // the one synchronisation of the pass: the totals
+  read_words(ctx, {S.rows.sums, h_sums, sizeof(h_sums)});  // the one synchronisation of the pass: the totals
   const uint64_t n_c64 = h_sums[2];
   MG_REQUIRE(n_c64 <= 0xFFFFFFFFull, std::string(who) + ": " + std::to_string(n_c64) +
                                          " output tiles, more than a u32 tile index holds");
@@ -1006,8 +1005,7 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
     run_product(ctx, P.in, kOutFlag, fo);
     exclusive_scan_u32(ctx, flag.get(), pos.get(), n_s);
     uint32_t n32 = 0;
-    MG_HIP(hipMemcpyAsync(&n32, pos.get() + n_s, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    MG_HIP(hipStreamSynchronize(s));
+    read_words(ctx, {pos.get() + n_s, &n32, sizeof(n32)});
     n_num = n32;
     alloc_tiled_matrix(c, S.n, n32);
     if (n32) {
@@ -1038,8 +1036,7 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
       ao.capacity = cap;
       run_product(ctx, P.in, kOutAppend, ao);
       unsigned long long got = 0;
-      MG_HIP(hipMemcpyAsync(&got, counter.get(), sizeof(got), hipMemcpyDeviceToHost, s));
-      MG_HIP(hipStreamSynchronize(s));
+      read_words(ctx, {counter.get(), &got, sizeof(got)});
       st.passes += 1;
       st.scratch_bytes = std::max<uint64_t>(st.scratch_bytes, slots * kTile * sizeof(uint64_t));
       if (got > cap) {
@@ -1112,9 +1109,8 @@ extern "C" int mg_multiply_pruned_model(mg_context* ctx, const mg_tiled_matrix* 
                                                                   pred.get(), total.get());
       MG_LAUNCH_CHECK();
       unsigned long long h = 0;
-      MG_HIP(hipMemcpyAsync(&h, total.get(), sizeof(h), hipMemcpyDeviceToHost, s));
       if (row_predicted) MG_HIP(hipMemcpyAsync(row_predicted, pred.get(), sizeof(float) * n, hipMemcpyDeviceToHost, s));
-      MG_HIP(hipStreamSynchronize(s));
+      read_words(ctx, {total.get(), &h, sizeof(h)});
       capacity = std::max<unsigned long long>(1, h);
     } else if (row_predicted && n) {
       std::fill(row_predicted, row_predicted + n, 0.0f);

@@ -147,17 +147,16 @@ struct ChunkLog {
 static_assert(sizeof(ChunkLog) == 8, "written as one 8-byte word");
 
 // --- fills and X_0 ------------------------------------------------------------
-// Zero-fill of a list of ranges (a kernel, so it can sit inside a captured graph).
-__global__ void __launch_bounds__(kBlock) fill_zero_kernel(const FillRange* __restrict__ ranges, uint32_t n_ranges) {
+// Zero-fill of a list of ranges.
+__device__ inline void fill_zero(const FillRange* __restrict__ ranges, uint32_t n_ranges, uint32_t block, uint32_t n_blocks) {
   for (uint32_t r = 0; r < n_ranges; ++r) {
     uint64_t* p = ranges[r].ptr;
     const uint64_t n = ranges[r].n;
     const uint64_t n2 = n / 2;
     ulonglong2* p2 = reinterpret_cast<ulonglong2*>(p);
-    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n2;
-         i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
+    for (uint64_t i = static_cast<uint64_t>(block) * kBlock + threadIdx.x; i < n2; i += static_cast<uint64_t>(n_blocks) * kBlock)
       p2[i] = make_ulonglong2(0, 0);
-    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) p[n - 1] = 0;
+    if ((n & 1) && block == 0 && threadIdx.x == 0) p[n - 1] = 0;
   }
 }
 
@@ -166,12 +165,10 @@ __global__ void __launch_bounds__(kBlock) fill_zero_kernel(const FillRange* __re
 // buffers start zeroed at allocation. One wave per strip, over the strips of all panels in
 // turn: every lane reads the strip's masks before lane 0 resets them, so no barrier is needed.
 template <int W>
-__global__ void __launch_bounds__(kBlock) clear_x0_kernel(const PanelInit* __restrict__ panels,
-                                                          const uint32_t* __restrict__ n_strips, uint32_t n_panels) {
+__device__ inline void clear_x0(const PanelInit* __restrict__ panels, const uint32_t* __restrict__ n_strips,
+                                uint32_t n_panels, uint32_t first, uint32_t n_waves) {
   constexpr int kWords = 64 * W;
   const uint32_t lane = lane_id();
-  const uint32_t n_waves = gridDim.x * kWaves;
-  const uint32_t first = read_first_lane(blockIdx.x * kWaves + threadIdx.x / kWave);
   for (uint32_t p = 0; p < n_panels; ++p) {
     const PanelInit P = panels[p];
     const uint32_t ns = n_strips[p];
@@ -1774,9 +1771,8 @@ __global__ void __launch_bounds__(kBlock) seg_combine_kernel(const PanelLevel* _
 // structural masks, for every level at once, at the start of a run (nothing reads or writes a
 // level's output before its own launch).
 template <int W>
-__global__ void __launch_bounds__(kBlock) zero_split_kernel(const ZeroItem* __restrict__ items) {
+__device__ inline void zero_split(const ZeroItem& it) {
   constexpr int kWords = 64 * W;
-  const ZeroItem it = items[blockIdx.x];
   for (int i = threadIdx.x; i < kWords; i += kBlock) it.x[i] = 0;
   if (threadIdx.x == 0) *it.s = 0;
 }
@@ -1831,9 +1827,9 @@ __global__ void __launch_bounds__(kBlock) finalize_strips_kernel(const StripItem
 // X_0 is one-hot: only the A^T tile columns of the strips that hold sources carry numeric
 // work into X_1. The first hop of a walk can therefore read just those columns (through a
 // column index of A^T) and OR each source row into its target rows with global atomics,
-// instead of sweeping all strips with the LDS accumulator. Three or four launches produce the
-// same X_1, masks and counters as the sweep: push_reset (clear the previous run's words of
-// X_1, reset its masks), S_1 and the tile counts (either push_structural over the row-major
+// instead of sweeping all strips with the LDS accumulator. After reset_kernel (push_reset: clear
+// the previous run's words of X_1, reset its masks) two or three launches produce the same X_1,
+// masks and counters as the sweep: S_1 and the tile counts (either push_structural over the row-major
 // index, or push_first_hop from the source columns plus per-column counts in push_finalize),
 // push_first_hop (the jobs) and push_finalize (N, V masks, popcount and strip counts, read
 // back from the rows the pushes marked in Z).
@@ -1845,16 +1841,13 @@ struct PushItem {
 constexpr uint32_t kPushItemTiles = 256;   // column positions per item (512: 45 and 222 us, 128: as 256)
 constexpr int kPushRows = 4;               // source rows loaded per step
 
-// One wave per strip of panel panels[blockIdx.y]: zero X_1 words inside the previous Z x N
-// masks, reset X_1's masks.
+// One wave per strip of a pushed panel: zero X_1 words inside the previous Z x N masks, reset
+// X_1's masks.
 template <int W>
-__global__ void __launch_bounds__(kBlock) push_reset_kernel(const PanelLevel* __restrict__ lv,
-                                                            const uint32_t* __restrict__ panels) {
-  const PanelLevel& L = lv[panels[blockIdx.y]];
+__device__ inline void push_reset(const PanelLevel& L, uint32_t first, uint32_t n_waves) {
   const uint32_t lane = lane_id();
   const gptr<uint64_t> x = as_global(L.x_out);
-  const uint32_t n_waves = gridDim.x * kWaves;
-  for (uint32_t y = read_first_lane(blockIdx.x * kWaves + threadIdx.x / kWave); y < L.n_strips; y += n_waves) {
+  for (uint32_t y = first; y < L.n_strips; y += n_waves) {
     const uint64_t z = as_global(L.z_out)[y];
     const uint64_t n = as_global(L.n_out)[y];
     if (z != 0 && n != 0) {
@@ -1871,6 +1864,32 @@ __global__ void __launch_bounds__(kBlock) push_reset_kernel(const PanelLevel* __
       as_global(L.s_out)[y] = 0;
     }
   }
+}
+
+// Everything a run clears before its sources are set, in one launch (four took 15 us of a small
+// walk's 164): the counters, X_0 and its masks, the strips that pieces of chunks OR into (a workgroup
+// each, the first n_zero), and X_1 of the panels whose first hop is pushed. None reads what another
+// clears: X_0's rows are found in its own masks, X_1's in its own.
+struct ResetWork {
+  const FillRange* fills;
+  const PanelInit* inits;
+  const uint32_t* n_strips;   // per panel
+  const ZeroItem* zero_items;
+  const PanelLevel* lv0;
+  const uint32_t* push_panels;
+  uint32_t n_fills, n_panels, n_zero, n_push_panels;
+};
+template <int W>
+__global__ void __launch_bounds__(kBlock) reset_kernel(ResetWork R) {
+  if (blockIdx.x < R.n_zero) {
+    zero_split<W>(R.zero_items[blockIdx.x]);
+    return;
+  }
+  const uint32_t block = blockIdx.x - R.n_zero, n_blocks = gridDim.x - R.n_zero;
+  fill_zero(R.fills, R.n_fills, block, n_blocks);
+  const uint32_t first = read_first_lane(block * kWaves + threadIdx.x / kWave);
+  clear_x0<W>(R.inits, R.n_strips, R.n_panels, first, n_blocks * kWaves);
+  for (uint32_t i = 0; i < R.n_push_panels; ++i) push_reset<W>(R.lv0[R.push_panels[i]], first, n_blocks * kWaves);
 }
 
 // S_1 and the tile-product counts of the first hop when the pushed columns hold many of the
@@ -3077,11 +3096,6 @@ void launch_push_first_hop_w(hipStream_t st, Engine* e, const PushLaunch& pl, hi
     MG_HIP(hipEventRecord(ev[1], st));
     MG_HIP(hipEventRecord(ev[2], st));
   }
-  if (pl.n_panels) {
-    push_reset_kernel<W><<<dim3(grid_for(pl.max_strips, kWaves, 4096), pl.n_panels), kBlock, 0, st>>>(e->lv[0].get(),
-                                                                                                    pl.panels);
-    MG_LAUNCH_CHECK();
-  }
   if (!pl.s_from_columns && pl.n_chunks) {
     push_structural_kernel<<<pl.n_chunks, kBlock, 0, st>>>(pl.chunks, e->lv[0].get());
     MG_LAUNCH_CHECK();
@@ -3126,33 +3140,32 @@ uint64_t push_items_for(const GraphPlan& g, uint32_t panel, const std::vector<ui
   return tiles;
 }
 
-// X_0 fills + source bits (sources already on the device).
+// Clears (reset_kernel; push_panels: n_push_panels panels whose first hop is pushed), then X_0 from
+// `sources` (device or pinned memory).
 template <int W>
-void launch_clear_x0(hipStream_t st, Engine* e) {
-  clear_x0_kernel<W><<<2048, kBlock, 0, st>>>(e->inits.get(), e->panel_strips.get(),
-                                              static_cast<uint32_t>(e->panels.size()));
+void launch_reset(hipStream_t st, Engine* e, const uint32_t* push_panels, uint32_t n_push_panels) {
+  uint32_t max_strips = 1;
+  for (const auto& p : e->panels) max_strips = std::max(max_strips, p.n_strips);
+  const ResetWork r{e->fills.get(), e->inits.get(), e->panel_strips.get(), e->zero_items.get(), e->lv[0].get(), push_panels,
+                    e->n_fills, static_cast<uint32_t>(e->panels.size()), e->n_zero_items, n_push_panels};
+  reset_kernel<W><<<e->n_zero_items + grid_for(max_strips, kWaves, 2048), kBlock, 0, st>>>(r);
   MG_LAUNCH_CHECK();
-  if (e->n_zero_items) {
-    zero_split_kernel<W><<<e->n_zero_items, kBlock, 0, st>>>(e->zero_items.get());
-    MG_LAUNCH_CHECK();
-  }
 }
 
-void launch_init(hipStream_t st, Engine* e, uint32_t n_sources) {
-  fill_zero_kernel<<<64, kBlock, 0, st>>>(e->fills.get(), e->n_fills);
-  MG_LAUNCH_CHECK();
+void launch_init(hipStream_t st, Engine* e, const SourceItem* sources, uint32_t n_sources, const uint32_t* push_panels,
+                 uint32_t n_push_panels) {
   switch (e->W) {
-    case 1: launch_clear_x0<1>(st, e); break;
-    case 2: launch_clear_x0<2>(st, e); break;
-    case 4: launch_clear_x0<4>(st, e); break;
-    case 8: launch_clear_x0<8>(st, e); break;
-    case 16: launch_clear_x0<16>(st, e); break;
-    case 32: launch_clear_x0<32>(st, e); break;
-    case 64: launch_clear_x0<64>(st, e); break;
+    case 1: launch_reset<1>(st, e, push_panels, n_push_panels); break;
+    case 2: launch_reset<2>(st, e, push_panels, n_push_panels); break;
+    case 4: launch_reset<4>(st, e, push_panels, n_push_panels); break;
+    case 8: launch_reset<8>(st, e, push_panels, n_push_panels); break;
+    case 16: launch_reset<16>(st, e, push_panels, n_push_panels); break;
+    case 32: launch_reset<32>(st, e, push_panels, n_push_panels); break;
+    case 64: launch_reset<64>(st, e, push_panels, n_push_panels); break;
     default: fail(MG_ERR_INTERNAL, "walk: unsupported words per vertex");
   }
   if (n_sources) {
-    init_sources_kernel<<<grid_for(n_sources, 256), 256, 0, st>>>(e->sources.get(), n_sources, e->inits.get(), e->W);
+    init_sources_kernel<<<grid_for(n_sources, 256), 256, 0, st>>>(sources, n_sources, e->inits.get(), e->W);
     MG_LAUNCH_CHECK();
   }
 }
@@ -3203,10 +3216,9 @@ struct mg_walk {
   PinnedBuf<SourceItem> staging;
   // First hop by push: per-run items (source strips' column ranges) and their staging.
   PinnedBuf<PushItem> push_staging;
-  DevBuf<PushItem> push_items;
   uint32_t max_push_items = 0;
   bool last_push = false;              // the last run's first hop was pushed
-  hipEvent_t staging_read = nullptr;   // the last run's uploads have left the staging buffers
+  hipEvent_t staging_read = nullptr;   // the last run's kernels have read the staging buffers
   // Timing log: per timed run, 4 events per hop (symbolic start/end, numeric kernel
   // start/end), kept for every run since timing was enabled.
   std::vector<std::vector<hipEvent_t>> run_events;
@@ -3268,12 +3280,10 @@ extern "C" int mg_walk_create(mg_context* ctx, const mg_tiled_matrix* at, uint32
     }
     build_engine(&e, ctx->stream);
     apply_seg(&e, default_segments(), ctx->stream);
-    e.sources.alloc(max_sources);
     w->staging.alloc(max_sources);
     if (!(flags & MG_WALK_SWEEP_FIRST_HOP)) {
       // Each source strip's column is cut into pieces of kPushItemTiles positions.
       w->max_push_items = max_sources + at->n_nz_tile / kPushItemTiles + 1;
-      w->push_items.alloc(w->max_push_items);
       w->push_staging.alloc(w->max_push_items);
       const uint32_t zero = 0;
       e.push_panels.alloc(1);
@@ -3331,12 +3341,11 @@ extern "C" int mg_walk_run(mg_context* ctx, mg_walk* w, uint32_t n_sources, cons
     w->n_sources = n_sources;
     w->hops = hops;
     w->e.used_words = (n_sources + 63) / 64;
-    // The previous run's uploads read the staging buffers asynchronously.
+    // The previous run's kernels read the staging buffers asynchronously.
     MG_HIP(hipEventSynchronize(w->staging_read));
     SourceItem* stg = w->staging.get();
     const GraphPlan& gp = w->e.graphs[0];
     for (uint32_t i = 0; i < n_sources; ++i) stg[i] = {0, i, gp.engine_vertex(sources[i])};
-    MG_HIP(hipMemcpyAsync(w->e.sources.get(), stg, sizeof(SourceItem) * n_sources, hipMemcpyHostToDevice, st));
     // First hop: push from the source strips when their A^T columns hold at most half of the
     // tiles (the sweep reads every tile once; the push reads the source columns).
     uint32_t n_items = 0;
@@ -3356,13 +3365,11 @@ extern "C" int mg_walk_run(mg_context* ctx, mg_walk* w, uint32_t n_sources, cons
         n_items = static_cast<uint32_t>(items.size());
         MG_REQUIRE(n_items <= w->max_push_items, "mg_walk_run: internal push item overflow");
         std::copy(items.begin(), items.end(), w->push_staging.get());
-        if (n_items)
-          MG_HIP(hipMemcpyAsync(w->push_items.get(), w->push_staging.get(), sizeof(PushItem) * n_items,
-                                hipMemcpyHostToDevice, st));
       }
     }
-    MG_HIP(hipEventRecord(w->staging_read, st));
-    launch_init(st, &w->e, n_sources);
+    // The kernels read sources and items from the pinned staging buffers: a few KB over the host link
+    // cost less than a copy before them (two took 12 us of a small walk).
+    launch_init(st, &w->e, stg, n_sources, w->e.push_panels.get(), push ? 1u : 0u);
     std::vector<hipEvent_t> ev;
     if (w->timing) {
       ev.resize(4 * static_cast<size_t>(hops));
@@ -3372,11 +3379,12 @@ extern "C" int mg_walk_run(mg_context* ctx, mg_walk* w, uint32_t n_sources, cons
       hipEvent_t* const evk = w->timing ? &ev[4 * k] : nullptr;
       if (k == 0 && push)
         launch_push_first_hop(st, &w->e,
-                              PushLaunch{w->push_items.get(), n_items, w->e.chunks[0].get(), w->e.n_chunks[0],
+                              PushLaunch{w->push_staging.get(), n_items, w->e.chunks[0].get(), w->e.n_chunks[0],
                                          w->e.push_panels.get(), 1u, w->e.panels[0].n_strips, s_cols},
                               evk);
       else
         launch_level(st, &w->e, k, evk);
+      if (k == 0) MG_HIP(hipEventRecord(w->staging_read, st));
     }
     w->last_push = push;
     if (w->timing) w->run_events.push_back(std::move(ev));
@@ -3472,11 +3480,11 @@ extern "C" int mg_walk_frontier_download(mg_context* ctx, const mg_walk* w, uint
     if (!map) {
       MG_HIP(hipMemcpyAsync(xt, x.get(), words * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     } else {
-      DevBuf<uint64_t> tmp(words);  // X_hop in vertex order
+      uint64_t* const tmp = ctx_scratch(ctx, words);  // X_hop in vertex order
       frontier_slice_kernel<<<grid_for(words, kBlock * 8, 16384), kBlock, 0, ctx->stream>>>(x.get(), nv, w->e.W, 0,
-                                                                                           w->e.W, map, tmp.get());
+                                                                                           w->e.W, map, tmp);
       MG_LAUNCH_CHECK();
-      MG_HIP(hipMemcpyAsync(xt, tmp.get(), words * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+      MG_HIP(hipMemcpyAsync(xt, tmp, words * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     }
     MG_HIP(hipStreamSynchronize(ctx->stream));
   });
@@ -3505,23 +3513,22 @@ mg_tiled_matrix* export_frontier(mg_context* ctx, const uint64_t* x, const uint6
   const uint32_t* map = g.device_map();
   const uint32_t n_groups = (ns + 63) / 64;
   const uint32_t n_items = rows * n_groups;
-  StreamBuf<uint64_t> mask(n_items, st);
-  StreamBuf<uint32_t> base(n_items + 1ull, st);
+  uint64_t* const mask = ctx_scratch(ctx, n_items + (n_items + 6ull) / 2);
+  uint32_t* const base = reinterpret_cast<uint32_t*>(mask + n_items + (n_items & 1));  // 16-byte aligned
   uint32_t nt = 0;
   if (n_items) {
     export_mask_kernel<<<(n_groups + kWaves - 1) / kWaves, kBlock, 0, st>>>(s_dev, ns, map, w0, rows, n_groups,
-                                                                            mask.get(), base.get());
+                                                                            mask, base);
     MG_LAUNCH_CHECK();
-    scan_in_place(st, base.get(), n_items);
-    MG_HIP(hipMemcpyAsync(&nt, base.get() + n_items, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    MG_HIP(hipStreamSynchronize(st));
+    scan_in_place(st, base, n_items);
+    read_words(ctx, {base + n_items, &nt, sizeof(nt)});
   }
   auto m = std::make_unique<mg_tiled_matrix>();
   m->device = ctx->device;
   alloc_tiled_matrix(m.get(), ns, nt);
   if (n_items) {
     export_index_kernel<<<grid_for(std::max<uint64_t>(n_items * 64ull, ns + 1ull), kBlock, 4096), kBlock, 0, st>>>(
-        mask.get(), base.get(), rows, n_groups, ns, m->offset_row.get(), m->row_idx.get(), m->col_idx.get());
+        mask, base, rows, n_groups, ns, m->offset_row.get(), m->row_idx.get(), m->col_idx.get());
     MG_LAUNCH_CHECK();
   } else {
     MG_HIP(hipMemsetAsync(m->offset_row.get(), 0, sizeof(uint32_t) * (ns + 1ull), st));
@@ -3532,7 +3539,7 @@ mg_tiled_matrix* export_frontier(mg_context* ctx, const uint64_t* x, const uint6
     const uint32_t stride = pad | 1;
     const uint32_t strips = std::max<uint32_t>(1, 16 / pad);  // at least 16 tiles for the eight waves
     export_tiles_kernel<<<(ns + strips - 1) / strips, kExportBlock, sizeof(uint64_t) * 64 * strips * stride, st>>>(
-        x, W, w0, map, ns, mask.get(), base.get(), rows, n_groups, pad, stride, strips, m->data.get());
+        x, W, w0, map, ns, mask, base, rows, n_groups, pad, stride, strips, m->data.get());
     MG_LAUNCH_CHECK();
   }
   MG_HIP(hipStreamSynchronize(st));
@@ -3598,7 +3605,7 @@ namespace {
 
 void record_batch(hipStream_t st, mg_walk_batch* b) {
   Engine& e = b->e;
-  launch_init(st, &e, e.n_sources);
+  launch_init(st, &e, e.sources.get(), e.n_sources, e.push_panels.get(), e.n_push_panels);
   for (uint32_t k = 0; k < e.max_hops; ++k) {
     if (k == 0 && e.n_push_panels)
       launch_push_first_hop(st, &e,
