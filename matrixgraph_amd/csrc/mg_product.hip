@@ -19,10 +19,11 @@
 // two halves of a C tile, by rows and by columns, meet at the end (wave_transpose).
 //
 // Measured (both operands prepared), against one wave per C tile that searches the shorter tile list
-// in the longer one and multiplies payloads of 16 bytes: A*A of R-MAT 14 136 us, before 518; of
-// R-MAT 16 with 16 planted communities (191 K tiles, 70 M pairs) 1.45 ms, before 4.63; a frontier of
-// 1000 rows x R-MAT 18 (7.3 K tiles, 6.8 M pairs) 156 us, before 482. Bound by the vector ALUs: on
-// the second 0.67 G wave instructions, 75 % of the issue slots.
+// in the longer one and multiplies payloads of 16 bytes: A*A of R-MAT 14 119 us, before 518; of
+// R-MAT 16 with 16 planted communities (191 K tiles, 70 M pairs) 1.28 ms, before 4.63; a frontier of
+// 1000 rows x R-MAT 18 (7.3 K tiles, 6.8 M pairs) 140 us, before 482. Bound by the vector ALUs (75 %
+// of the issue slots on the second) and by the chains of ballots and LDS writes in between: filling the
+// queue of stage 3 is half of the time, the ORs themselves nothing.
 #include <algorithm>
 #include <string>
 
@@ -474,13 +475,13 @@ __global__ void __launch_bounds__(kBlock) heavy_pairs_kernel(LeftOperand A, uint
 
 // --- the product ------------------------------------------------------------------------
 
-constexpr uint32_t kQueue = 128;     // entries of a wave's queues (two full waves)
-// Common inner indices up to which a pair is queued per index: 1.45 ms on the communities above
-// at 16, 1.56 at 8, 1.54 at 64 (always).
+constexpr uint32_t kQueue = 192;     // entries of a wave's queues: less than a wave's, and two from each lane
+// Common inner indices up to which a pair is queued per index (8 or 64: 7 and 6 % slower on the
+// communities above).
 constexpr int kFewCommon = 16;
 constexpr int kPairBatch = 4;        // pairs with more whose loads are in flight together (8: 7 % slower)
 // Waves of a workgroup. More do not shorten a window's chain of loads, they only halve its batches:
-// 1.45 ms with 4, 2.14 with 8, 3.21 with 16 (communities).
+// 1.45 ms with 4, 2.14 with 8, 3.21 with 16 (communities, before the queues took two entries a step).
 constexpr uint32_t kProductWaves = 4;
 
 struct WaveQueues {
@@ -648,18 +649,33 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
         for (int k = 0; k < kPairBatch; ++k) or_outer(by_row + sp[k], by_col + sp[k], r[k], c[k], lane);
       }
       if (whole) common = 0;
-      for (uint64_t m = ballot(common != 0); m; m = ballot(common != 0)) {
-        if (common) {
-          const uint64_t below = (common & (0 - common)) - 1;
-          const uint32_t to = n_queued + lanes_under(m);
-          q.item_a[to] = ha.off + static_cast<uint32_t>(__popcll(ha.mask & below));
-          q.item_b[to] = hb.off + static_cast<uint32_t>(__popcll(hb.mask & below));
-          q.item_s[to] = static_cast<uint8_t>(s);
-          common &= common - 1;
+      // The rest, two j per lane at a time (1.32 ms instead of 1.43: a step's ballots, branch and LDS
+      // writes are one dependent chain), a 32-bit half of the masks after the other: bits of the half
+      // below j, counted onto the words before it, give the two column words.
+      const auto queue = [&](uint32_t left, uint32_t in_a, uint32_t in_b, uint32_t first_a, uint32_t first_b) {
+        const auto put = [&](uint32_t bits, uint64_t m) {
+          if (bits) {
+            const uint32_t below = (bits - 1) & ~bits;
+            const uint32_t to = n_queued + lanes_under(m);
+            q.item_a[to] = first_a + static_cast<uint32_t>(__popc(in_a & below));
+            q.item_b[to] = first_b + static_cast<uint32_t>(__popc(in_b & below));
+            q.item_s[to] = static_cast<uint8_t>(s);
+          }
+          n_queued += static_cast<uint32_t>(__popcll(m));
+        };
+        for (uint64_t m = ballot(left != 0); m; m = ballot(left != 0)) {
+          const uint32_t next = left & (left - 1);
+          const uint64_t m_next = ballot(next != 0);
+          put(left, m);
+          put(next, m_next);
+          left = next & (next - 1);
+          while (n_queued >= kWave) multiply(kWave);
         }
-        n_queued += static_cast<uint32_t>(__popcll(m));
-        if (n_queued >= kWave) multiply(kWave);
-      }
+      };
+      const uint32_t lo_a = static_cast<uint32_t>(ha.mask), lo_b = static_cast<uint32_t>(hb.mask);
+      queue(static_cast<uint32_t>(common), lo_a, lo_b, ha.off, hb.off);
+      queue(static_cast<uint32_t>(common >> 32), static_cast<uint32_t>(ha.mask >> 32), static_cast<uint32_t>(hb.mask >> 32),
+            ha.off + static_cast<uint32_t>(__popc(lo_a)), hb.off + static_cast<uint32_t>(__popc(lo_b)));
     };
 
     // Stage 1: the row's tiles, dealt one by one to the waves, so that short rows use them all.
@@ -675,17 +691,23 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
         }
         const uint32_t all = bits;
         bits &= present;
-        for (uint64_t m = ballot(bits != 0); m; m = ballot(bits != 0)) {
-          if (bits) {
-            const uint32_t s = static_cast<uint32_t>(__ffs(static_cast<int>(bits)) - 1);
+        const auto put = [&](uint32_t left, uint64_t m) {
+          if (left) {
+            const uint32_t below = (left - 1) & ~left;
             const uint32_t to = n_pairs + lanes_under(m);
             q.pair_a[to] = ia;
-            q.pair_b[to] = pb + static_cast<uint32_t>(__popc(all & ((1u << s) - 1)));
-            q.pair_s[to] = static_cast<uint8_t>(s);
-            bits &= bits - 1;
+            q.pair_b[to] = pb + static_cast<uint32_t>(__popc(all & below));
+            q.pair_s[to] = static_cast<uint8_t>(__popc(below));
           }
           n_pairs += static_cast<uint32_t>(__popcll(m));
-          if (n_pairs >= kWave) filter(kWave);
+        };
+        for (uint64_t m = ballot(bits != 0); m; m = ballot(bits != 0)) {
+          const uint32_t next = bits & (bits - 1);
+          const uint64_t m_next = ballot(next != 0);
+          put(bits, m);
+          put(next, m_next);
+          bits = next & (next - 1);
+          while (n_pairs >= kWave) filter(kWave);
         }
       }
     } else {

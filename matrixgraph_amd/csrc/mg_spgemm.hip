@@ -189,7 +189,7 @@ void launch_payloads(hipStream_t st, const mg_tiled_matrix* a, const mg_tiled_ma
 // (c, j) of the Bt tile with the same j and sets bit c of row r in the wave's LDS
 // accumulator. Pairs with a denser tile take the full-tile wave product, kPairBatch at a time.
 // Only the allocation-free pass runs it: its 16 bytes of scratch per tile hold neither heads nor column
-// words (product_kernel takes 136 us where this one takes 518: C = A*A, R-MAT 14).
+// words (product_kernel takes 119 us where this one takes 518: C = A*A, R-MAT 14).
 __global__ void __launch_bounds__(kBlock) fill_tiles_payload_kernel(
     uint32_t n_c, const uint32_t* __restrict__ off_a, const uint32_t* __restrict__ off_bt,
     const uint32_t* __restrict__ row_c, const uint32_t* __restrict__ col_c, const uint32_t* __restrict__ col_a,
