@@ -548,6 +548,9 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
 #pragma unroll
     for (uint32_t d = 1; d < kWindow; d <<= 1) present |= shfl_xor32(present, static_cast<int>(d));
     present = read_first_lane(present);
+    if constexpr (kOut == kOutRest) {  // windows without a tile to write: uniform over the workgroup
+      if (!ballot(col < win.end && out.flag[mine] && out.slot[mine] >= out.capacity)) continue;
+    }
     const auto c_tile = [&](uint32_t s) { return win.first + static_cast<uint32_t>(__popc(present & ((1u << s) - 1))); };
     for (uint32_t i = threadIdx.x; i < kWindow * kTile; i += kProductWaves * kWave) by_row[i] = by_col[i] = 0;
     __syncthreads();
@@ -781,6 +784,9 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
         // Only this wave has the tile; an atomic needs no answer, a load would be waited for.
         if (val) atomicOr(reinterpret_cast<unsigned long long*>(out.data) + static_cast<uint64_t>(i) * kTile + lane,
                           static_cast<unsigned long long>(val));
+      } else if constexpr (kOut == kOutRest) {
+        const uint64_t slot = out.flag[i] ? out.slot[i] : 0u;
+        if (slot >= out.capacity) out.data[(slot - out.capacity) * kTile + lane] = val;
       } else {
         const bool nz = ballot(val != 0) != 0;
         if constexpr (kOut == kOutFlag) {
@@ -1136,6 +1142,7 @@ void run_product(mg_context* ctx, const ProductInputs& P, int out_mode, const Pr
     case kOutAppend: launch_product<false, kOutAppend>(ctx, P, out, HeavyRecord{}); break;
     case kOutFlag: launch_product<false, kOutFlag>(ctx, P, out, HeavyRecord{}); break;
     case kOutPos: launch_product<false, kOutPos>(ctx, P, out, HeavyRecord{}); break;
+    case kOutRest: launch_product<false, kOutRest>(ctx, P, out, HeavyRecord{}); break;
     default: fail(MG_ERR_INTERNAL, "run_product: output mode");
   }
 }

@@ -105,9 +105,10 @@ void prepare_operand(mg_context* ctx, mg_tiled_matrix* m);
 
 // Where a finished C tile goes: ORed into data at its index (kOutStruct), or, for a pruned product,
 // only if it is non-zero: into the next slot of data, whether and which in flag and slot
-// (kOutAppend; slots past capacity are counted but not written), flagged in flag (kOutFlag, no data
-// written), or written at pos[i] (kOutPos).
-enum : int { kOutStruct = 0, kOutAppend = 1, kOutFlag = 2, kOutPos = 3 };
+// (kOutAppend; slots past capacity are counted but not written), the same tiles whose slots of an
+// earlier kOutAppend were past capacity (kOutRest, slot - capacity), flagged in flag (kOutFlag, no
+// data written), or written at pos[i] (kOutPos).
+enum : int { kOutStruct = 0, kOutAppend = 1, kOutFlag = 2, kOutPos = 3, kOutRest = 4 };
 struct ProductOut {
   uint64_t* data = nullptr;
   uint32_t* flag = nullptr;  // per structural tile

@@ -680,7 +680,9 @@ struct PrunedTiles {
   uint32_t n_s, n_strips;
   const uint32_t *flag, *pos, *row, *col, *off;
   const uint32_t* slot;    // null: the data is in place
-  const uint64_t* scratch;
+  const uint64_t* scratch; // slots below `capacity`; the others in `rest`
+  const uint64_t* rest;
+  uint64_t capacity;
 };
 __global__ void __launch_bounds__(kBlock) place_pruned_kernel(PrunedTiles S, uint32_t* __restrict__ row_c,
                                                               uint32_t* __restrict__ col_c,
@@ -713,7 +715,7 @@ __global__ void __launch_bounds__(kBlock) place_pruned_kernel(PrunedTiles S, uin
           m &= m - 1;
           at[q] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(to), k));
           const uint64_t src = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), k));
-          word[q] = S.scratch[src * kTile + lane];
+          word[q] = (src < S.capacity ? S.scratch + src * kTile : S.rest + (src - S.capacity) * kTile)[lane];
           ++n;
         }
       }
@@ -931,7 +933,9 @@ namespace {
 // Structural index and operand inputs of a pruned product.
 struct PrunedPlan {
   Structural S;
-  StreamBuf<uint32_t> row_s, col_s;
+  StreamBuf<uint32_t> mem;  // the structural tiles: rows, columns, flags, slots, the flags' scan
+  uint32_t *row_s, *col_s, *flag, *slot, *pos;
+  unsigned long long* counter;
   ProductInputs in;
 };
 
@@ -940,23 +944,27 @@ void pruned_prepare(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   hipStream_t s = ctx->stream;
   structural_pass(ctx, a, bt, P.S, who);
   const uint32_t n_s = static_cast<uint32_t>(P.S.n_c);
-  P.row_s.alloc(n_s, s);
-  P.col_s.alloc(n_s, s);
-  structural_emit(ctx, a, P.S, P.row_s.get(), P.col_s.get());
-  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s.get(), P.col_s.get()}, want_bits, true, P.in, P.S.b);
+  P.mem.alloc(5ull * n_s + 4, s);
+  P.counter = reinterpret_cast<unsigned long long*>(P.mem.get());
+  P.row_s = P.mem.get() + 2;
+  P.col_s = P.row_s + n_s;
+  P.flag = P.col_s + n_s;
+  P.slot = P.flag + n_s;
+  P.pos = P.slot + n_s;
+  structural_emit(ctx, a, P.S, P.row_s, P.col_s);
+  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s, P.col_s}, want_bits, true, P.in, P.S.b);
 }
 
 // Features of every C row into feat (device, n_strips x kRowFeatures).
-// in: the product's inputs, with set-bit counts.
+// in: the product's inputs, with set-bit counts. brow: n_strips of scratch.
 void row_features_into(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const Structural& S,
-                       const ProductInputs& in, float* feat) {
+                       const ProductInputs& in, unsigned long long* brow, float* feat) {
   hipStream_t s = ctx->stream;
   const uint32_t n = S.n;
   if (!n) return;
-  StreamBuf<unsigned long long> brow(n, s);
-  right_row_bits(ctx, bt, in, brow.get());
+  right_row_bits(ctx, bt, in, brow);
   row_features_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, s>>>(
-      n, a->offset_row.get(), a->col_idx.get(), in.a.head, brow.get(), S.rows.cnt, S.rows.tp, feat);
+      n, a->offset_row.get(), a->col_idx.get(), in.a.head, brow, S.rows.cnt, S.rows.tp, feat);
   MG_LAUNCH_CHECK();
 }
 
@@ -985,14 +993,11 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   hipStream_t s = ctx->stream;
   const Structural& S = P.S;
   const uint32_t n_s = static_cast<uint32_t>(S.n_c);
-  const uint32_t* row_s = P.row_s.get();
-  const uint32_t* col_s = P.col_s.get();
   st.structural_tiles = n_s;
   st.tile_products = S.tile_products;
   uint64_t n_num = 0;
   uint64_t cap = capacity == MG_PRUNED_STRUCTURAL ? n_s : std::min<uint64_t>(capacity, n_s);
-  StreamBuf<uint32_t> flag(n_s, s), pos(n_s + 1ull, s);
-  PrunedTiles tiles{n_s, S.n, flag.get(), pos.get(), row_s, col_s, S.rows.off_c, nullptr, nullptr};
+  PrunedTiles tiles{n_s, S.n, P.flag, P.pos, P.row_s, P.col_s, S.rows.off_c, nullptr, nullptr, nullptr, 0};
   const auto place = [&] {
     place_pruned_kernel<<<grid_for(std::max<uint64_t>(n_s, S.n + 1ull), kWavesPerBlock * kPlaceTiles, 16384), kBlock, 0, s>>>(
         tiles, c->row_idx.get(), c->col_idx.get(), c->offset_row.get(), c->data.get());
@@ -1001,17 +1006,17 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   if (capacity == MG_PRUNED_EXACT || n_s == 0) {
     // Exact: flag pass, scan, then each non-empty tile written at its final position.
     ProductOut fo{};
-    fo.flag = flag.get();
+    fo.flag = P.flag;
     run_product(ctx, P.in, kOutFlag, fo);
-    exclusive_scan_u32(ctx, flag.get(), pos.get(), n_s);
+    exclusive_scan_u32(ctx, P.flag, P.pos, n_s);
     uint32_t n32 = 0;
-    read_words(ctx, {pos.get() + n_s, &n32, sizeof(n32)});
+    read_words(ctx, {P.pos + n_s, &n32, sizeof(n32)});
     n_num = n32;
     alloc_tiled_matrix(c, S.n, n32);
     if (n32) {
       ProductOut po{};
       po.data = c->data.get();
-      po.pos = pos.get();
+      po.pos = P.pos;
       run_product(ctx, P.in, kOutPos, po);
     }
     place();
@@ -1019,41 +1024,37 @@ void pruned_execute(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
     st.capacity = n32;
     st.scratch_bytes = 0;
   } else {
-    // One pass into `cap` slots; a capacity below the non-empty count is found by the
-    // counter, which keeps counting past it, and the pass is run again with the exact count.
-    StreamBuf<unsigned long long> counter(1, s);
-    StreamBuf<uint32_t> slot(n_s, s);
+    // One pass into `cap` slots; the counter keeps counting past them, and the tiles that found none are
+    // made in a second pass over their windows.
     st.capacity = cap;
-    for (int attempt = 0;; ++attempt) {
-      const uint64_t slots = std::max<uint64_t>(1, cap);
-      StreamBuf<uint64_t> scratch(slots * kTile, s);
-      MG_HIP(hipMemsetAsync(counter.get(), 0, sizeof(unsigned long long), s));
-      ProductOut ao{};
-      ao.data = scratch.get();
-      ao.flag = flag.get();
-      ao.slot = slot.get();
-      ao.counter = counter.get();
-      ao.capacity = cap;
-      run_product(ctx, P.in, kOutAppend, ao);
-      unsigned long long got = 0;
-      read_words(ctx, {counter.get(), &got, sizeof(got)});
-      st.passes += 1;
-      st.scratch_bytes = std::max<uint64_t>(st.scratch_bytes, slots * kTile * sizeof(uint64_t));
-      if (got > cap) {
-        MG_REQUIRE(attempt == 0, "mg_multiply_pruned: internal capacity overflow after the exact retry");
-        st.fallback = 1;
-        cap = got;
-        continue;
-      }
-      n_num = got;
-      alloc_tiled_matrix(c, S.n, static_cast<uint32_t>(got));
-      // Row-major order: the tiles' places are the scan of their flags.
-      exclusive_scan_u32(ctx, flag.get(), pos.get(), n_s);
-      tiles.slot = slot.get();
-      tiles.scratch = scratch.get();
-      place();
-      break;
+    StreamBuf<uint64_t> scratch(cap * kTile, s), rest;
+    MG_HIP(hipMemsetAsync(P.counter, 0, sizeof(unsigned long long), s));
+    ProductOut ao{};
+    ao.data = scratch.get();
+    ao.flag = P.flag;
+    ao.slot = P.slot;
+    ao.counter = P.counter;
+    ao.capacity = cap;
+    run_product(ctx, P.in, kOutAppend, ao);
+    // Row-major order: the tiles' places are the scan of their flags.
+    exclusive_scan_u32(ctx, P.flag, P.pos, n_s);
+    unsigned long long got = 0;
+    read_words(ctx, {P.counter, &got, sizeof(got)});
+    n_num = got;
+    st.passes = got > cap ? 2 : 1;
+    st.fallback = got > cap ? 1 : 0;
+    st.scratch_bytes = std::max<uint64_t>(got, cap) * kTile * sizeof(uint64_t);
+    if (got > cap) {
+      rest.alloc((got - cap) * kTile, s);
+      ao.data = rest.get();
+      run_product(ctx, P.in, kOutRest, ao);
     }
+    alloc_tiled_matrix(c, S.n, static_cast<uint32_t>(got));
+    tiles.slot = P.slot;
+    tiles.scratch = scratch.get();
+    tiles.rest = rest.get();
+    tiles.capacity = cap;
+    place();
   }
   MG_HIP(hipStreamSynchronize(s));
   st.numeric_tiles = n_num;
@@ -1098,19 +1099,22 @@ extern "C" int mg_multiply_pruned_model(mg_context* ctx, const mg_tiled_matrix* 
     const uint32_t n = P.S.n;
     uint64_t capacity = MG_PRUNED_EXACT;
     if (P.S.n_c) {
-      StreamBuf<float> feat(static_cast<uint64_t>(n) * kRowFeatures, s), y(static_cast<uint64_t>(n) * n_out, s),
-          pred(n, s);
-      StreamBuf<unsigned long long> total(1, s);
-      row_features_into(ctx, a, bt, P.S, P.in, feat.get());
-      if (mg_mlp_forward(ctx, model, feat.get(), n, y.get()) != MG_OK)
+      // u64: total, B's row bits; then the features, the model's outputs and the rows' predictions.
+      const uint64_t feat_at = (1ull + n + 31) / 32 * 32;  // the model loads rows of 32 bytes
+      StreamBuf<unsigned long long> mem(feat_at + (static_cast<uint64_t>(n) * (kRowFeatures + n_out + 1) + 1) / 2, s);
+      unsigned long long* const total = mem.get();
+      float* const feat = reinterpret_cast<float*>(total + feat_at);
+      float* const y = feat + static_cast<uint64_t>(n) * kRowFeatures;
+      float* const pred = y + static_cast<uint64_t>(n) * n_out;
+      row_features_into(ctx, a, bt, P.S, P.in, total + 1, feat);
+      if (mg_mlp_forward(ctx, model, feat, n, y) != MG_OK)
         fail(MG_ERR_INTERNAL, std::string("mg_multiply_pruned_model: ") + mg_last_error());
-      MG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), s));
-      capacity_kernel<<<grid_for(n, kBlock, 1024), kBlock, 0, s>>>(n, P.S.rows.cnt, y.get(), n_out, margin,
-                                                                  pred.get(), total.get());
+      MG_HIP(hipMemsetAsync(total, 0, sizeof(unsigned long long), s));
+      capacity_kernel<<<grid_for(n, kBlock, 1024), kBlock, 0, s>>>(n, P.S.rows.cnt, y, n_out, margin, pred, total);
       MG_LAUNCH_CHECK();
       unsigned long long h = 0;
-      if (row_predicted) MG_HIP(hipMemcpyAsync(row_predicted, pred.get(), sizeof(float) * n, hipMemcpyDeviceToHost, s));
-      read_words(ctx, {total.get(), &h, sizeof(h)});
+      if (row_predicted) MG_HIP(hipMemcpyAsync(row_predicted, pred, sizeof(float) * n, hipMemcpyDeviceToHost, s));
+      read_words(ctx, {total, &h, sizeof(h)});
       capacity = std::max<unsigned long long>(1, h);
     } else if (row_predicted && n) {
       std::fill(row_predicted, row_predicted + n, 0.0f);
@@ -1136,7 +1140,8 @@ extern "C" int mg_multiply_row_features(mg_context* ctx, const mg_tiled_matrix* 
     StreamBuf<float> feat(static_cast<uint64_t>(n) * kRowFeatures, s);
     ProductInputs in;
     product_inputs(ctx, a, bt, ProductTiles{}, true, false, in, S.b);
-    row_features_into(ctx, a, bt, S, in, feat.get());
+    StreamBuf<unsigned long long> brow(n, s);
+    row_features_into(ctx, a, bt, S, in, brow.get(), feat.get());
     if (n) {
       MG_HIP(hipMemcpyAsync(features, feat.get(), sizeof(float) * n * kRowFeatures, hipMemcpyDeviceToHost, s));
       if (structural)
