@@ -810,30 +810,41 @@ class MLP:
 
     def forward(self, x: np.ndarray) -> np.ndarray:
         x = np.ascontiguousarray(x, np.float32)
-        dx = DeviceBuffer.from_array(self.ctx, x)
-        dy = DeviceBuffer(self.ctx, x.shape[0] * self.n_out * 4)
-        _check(lib().mg_mlp_forward(self.ctx.h, self.h, C.c_void_p(dx.ptr), x.shape[0], C.c_void_p(dy.ptr)),
-               "mg_mlp_forward")
-        self.ctx.synchronize()
-        return dy.to_array(np.float32).reshape(x.shape[0], self.n_out)
+        y = np.empty((x.shape[0], self.n_out), np.float32)
+        buf, (dx, dy) = self._on_device(x, None, y.nbytes)
+        _check(lib().mg_mlp_forward(self.ctx.h, self.h, C.c_void_p(dx), x.shape[0], C.c_void_p(dy)), "mg_mlp_forward")
+        _check(lib().mg_buffer_download(self.ctx.h, _ptr(y), C.c_void_p(dy), y.nbytes), "mg_buffer_download")
+        buf.close()
+        return y
+
+    def _on_device(self, x, t, extra=0):
+        """x, t (may be None) and `extra` bytes in one device buffer: (buffer, [addresses])."""
+        first = -(-x.nbytes // 256) * 256
+        buf = DeviceBuffer(self.ctx, first + (extra if t is None else t.nbytes))
+        for a, at in ((x, 0), (t, first)):
+            if a is not None:
+                _check(lib().mg_buffer_upload(self.ctx.h, C.c_void_p(buf.ptr + at), _ptr(a), a.nbytes), "mg_buffer_upload")
+        return buf, (buf.ptr, buf.ptr + first)
 
     def loss_grad(self, x, t):
         x = np.ascontiguousarray(x, np.float32)
         t = np.ascontiguousarray(t, np.float32)
-        dx, dt = DeviceBuffer.from_array(self.ctx, x), DeviceBuffer.from_array(self.ctx, t)
+        buf, (dx, dt) = self._on_device(x, t)
         loss = C.c_float()
         grad = np.empty(self.n_params, np.float32)
-        _check(lib().mg_mlp_loss_grad(self.ctx.h, self.h, C.c_void_p(dx.ptr), C.c_void_p(dt.ptr), x.shape[0],
+        _check(lib().mg_mlp_loss_grad(self.ctx.h, self.h, C.c_void_p(dx), C.c_void_p(dt), x.shape[0],
                                       C.byref(loss), _ptr(grad)), "mg_mlp_loss_grad")
+        buf.close()
         return loss.value, grad
 
     def train(self, x, t, epochs=10, batch=1024, lr=1e-3) -> float:
         x = np.ascontiguousarray(x, np.float32)
         t = np.ascontiguousarray(t, np.float32)
-        dx, dt = DeviceBuffer.from_array(self.ctx, x), DeviceBuffer.from_array(self.ctx, t)
+        buf, (dx, dt) = self._on_device(x, t)
         loss = C.c_float()
-        _check(lib().mg_mlp_train(self.ctx.h, self.h, C.c_void_p(dx.ptr), C.c_void_p(dt.ptr), x.shape[0], epochs,
+        _check(lib().mg_mlp_train(self.ctx.h, self.h, C.c_void_p(dx), C.c_void_p(dt), x.shape[0], epochs,
                                   batch, lr, C.byref(loss)), "mg_mlp_train")
+        buf.close()
         return loss.value
 
     def close(self):

@@ -627,9 +627,8 @@ extern "C" int mg_mlp_loss_grad(mg_context* ctx, mg_mlp* p, const float* x, cons
     DeviceGuard g(ctx->device);
     compute_grad(ctx, p, x, t, n);
     float l = 0.f;
-    MG_HIP(hipMemcpyAsync(&l, p->loss.get(), sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     if (grad) MG_HIP(hipMemcpyAsync(grad, p->grad.get(), sizeof(float) * p->d.n_params, hipMemcpyDeviceToHost, ctx->stream));
-    MG_HIP(hipStreamSynchronize(ctx->stream));
+    read_words(ctx, {p->loss.get(), &l, sizeof(l)});
     if (loss) *loss = l / (static_cast<float>(n) * p->d.n_out);
   });
 }
@@ -659,8 +658,7 @@ extern "C" int mg_mlp_train(mg_context* ctx, mg_mlp* p, const float* x, const fl
           p->partial.get(), p->loss_part.get(), blocks, 0, p->grad.get(), p->loss.get(), AdamStep{});
       MG_LAUNCH_CHECK();
       float l = 0.f;
-      MG_HIP(hipMemcpyAsync(&l, p->loss.get(), sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-      MG_HIP(hipStreamSynchronize(ctx->stream));
+      read_words(ctx, {p->loss.get(), &l, sizeof(l)});
       *final_loss = l / (static_cast<float>(n) * p->d.n_out);
     }
   });
