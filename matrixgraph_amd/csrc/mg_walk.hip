@@ -2417,6 +2417,14 @@ struct GraphPlan {
   DevBuf<NarrowChunk> narrow_chunks;
   uint32_t n_narrow_chunks = 0;
   DevBuf<uint32_t> strip_job;
+  // Pieces of the chunks for walk_lean_kernel (build_pieces): those of chunk i are piece_off[i] ..;
+  // piece_split: the strips that they split.
+  std::vector<uint32_t> host_off;    // row pointer in engine order
+  std::vector<uint32_t> chunk_bits;  // set bits of each chunk
+  std::vector<Chunk> pieces;
+  std::vector<uint32_t> piece_off;
+  std::vector<uint64_t> piece_cost;
+  std::vector<uint32_t> piece_split;
 };
 
 // Launch-order key of each chunk, in hundredths: its set bits + 0.35 per tile + 24 per
@@ -2425,10 +2433,14 @@ struct GraphPlan {
 // Within one allocation this order beat ordering by tiles alone by 2-4 % on hops 2-4 of the
 // 4096-source walk on R-MAT 22 (tiles alone beat strip order by 4 % and reversed by 35 %).
 // *total_bits receives the set bits of all chunks (every tile once).
-std::vector<uint64_t> chunk_costs(const GraphPlan& g, hipStream_t st, uint64_t* total_bits) {
+uint64_t chunk_cost(const Chunk& c, uint64_t bits) {
+  return 100ull * bits + 35ull * (c.tile_end - c.tile_begin) + 2400ull * (c.strip_end - c.strip_begin);
+}
+std::vector<uint64_t> chunk_costs(GraphPlan& g, hipStream_t st, uint64_t* total_bits) {
   *total_bits = 0;
   const size_t n = g.chunks.size();
   std::vector<uint64_t> cost(n, 0);
+  g.chunk_bits.assign(n, 0);
   if (!n || !g.at->n_nz_tile) return cost;
   DevBuf<Chunk> dch(n);
   DevBuf<uint32_t> bits(n);
@@ -2439,10 +2451,10 @@ std::vector<uint64_t> chunk_costs(const GraphPlan& g, hipStream_t st, uint64_t* 
   MG_HIP(hipMemcpyAsync(hb.data(), bits.get(), sizeof(uint32_t) * n, hipMemcpyDeviceToHost, st));
   MG_HIP(hipStreamSynchronize(st));
   for (size_t i = 0; i < n; ++i) {
-    const Chunk& c = g.chunks[i];
-    cost[i] = 100ull * hb[i] + 35ull * (c.tile_end - c.tile_begin) + 2400ull * (c.strip_end - c.strip_begin);
+    cost[i] = chunk_cost(g.chunks[i], hb[i]);
     *total_bits += hb[i];
   }
+  g.chunk_bits.swap(hb);
   return cost;
 }
 
@@ -2492,6 +2504,84 @@ void build_job_list(GraphPlan& g, hipStream_t st) {
   }
   MG_HIP(hipStreamSynchronize(st));  // bits is freed on return
   g.has_jobs = true;
+}
+
+// Where a chunk with many jobs is cut: tile `at` such that the tiles before it hold about j / m of the
+// chunk's jobs.
+struct PieceCut {
+  uint32_t tile_begin, tile_end, j, m;
+};
+__global__ void __launch_bounds__(kBlock) piece_cut_kernel(const PieceCut* __restrict__ cuts, uint32_t n,
+                                                           const uint32_t* __restrict__ job_off,
+                                                           uint32_t* __restrict__ at) {
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    const PieceCut c = cuts[i];
+    const uint64_t first = job_off[c.tile_begin], jobs = job_off[c.tile_end] - first;
+    const uint64_t want = first + jobs * c.j / c.m;
+    uint32_t lo = c.tile_begin, hi = c.tile_end;
+    while (lo < hi) {
+      const uint32_t mid = lo + ((hi - lo) >> 1);
+      if (job_off[mid] < want) lo = mid + 1; else hi = mid;
+    }
+    at[i] = lo;
+  }
+}
+
+// Pieces of at most about `limit` jobs of every chunk (the scheduler's chunks hold kDefaultChunkTiles
+// tiles, and a hub strip's tiles have hundreds of bits). A cut inside a strip makes it a split strip.
+void build_pieces(GraphPlan& g, uint64_t limit, hipStream_t st) {
+  std::vector<PieceCut> cuts;
+  for (size_t i = 0; i < g.chunks.size(); ++i) {
+    const Chunk& c = g.chunks[i];
+    const uint64_t m = std::min<uint64_t>((g.chunk_bits[i] + limit - 1) / limit, c.tile_end - c.tile_begin);
+    for (uint32_t j = 1; j < m; ++j) cuts.push_back({c.tile_begin, c.tile_end, j, static_cast<uint32_t>(m)});
+  }
+  std::vector<uint32_t> at(cuts.size());
+  if (!cuts.empty()) {
+    DevBuf<PieceCut> d_cuts(cuts.size());
+    DevBuf<uint32_t> d_at(cuts.size());
+    MG_HIP(hipMemcpyAsync(d_cuts.get(), cuts.data(), sizeof(PieceCut) * cuts.size(), hipMemcpyHostToDevice, st));
+    piece_cut_kernel<<<grid_for(cuts.size(), kBlock, 1024), kBlock, 0, st>>>(
+        d_cuts.get(), static_cast<uint32_t>(cuts.size()), g.job_off.get(), d_at.get());
+    MG_LAUNCH_CHECK();
+    MG_HIP(hipMemcpyAsync(at.data(), d_at.get(), sizeof(uint32_t) * at.size(), hipMemcpyDeviceToHost, st));
+    MG_HIP(hipStreamSynchronize(st));
+  }
+  g.pieces.clear();
+  g.piece_off.assign(1, 0);
+  g.piece_cost.clear();
+  g.piece_split = g.split;
+  size_t next = 0;
+  for (size_t i = 0; i < g.chunks.size(); ++i) {
+    const Chunk& c = g.chunks[i];
+    Chunk p = c;
+    std::vector<uint32_t> ends;
+    for (; next < cuts.size() && cuts[next].tile_begin == c.tile_begin && cuts[next].tile_end == c.tile_end; ++next)
+      if (at[next] > c.tile_begin && at[next] < c.tile_end && (ends.empty() || at[next] > ends.back()))
+        ends.push_back(at[next]);
+    const uint64_t bits = g.chunk_bits[i] / (ends.size() + 1);
+    for (uint32_t t : ends) {
+      // The strip with tile t, last of those that start there (the others are empty).
+      const auto it = std::upper_bound(g.host_off.begin() + c.strip_begin, g.host_off.begin() + c.strip_end + 1, t) - 1;
+      const uint32_t y = static_cast<uint32_t>(it - g.host_off.begin());
+      const bool inside = *it < t;
+      p.strip_end = inside ? y + 1 : y;
+      p.tile_end = t;
+      g.pieces.push_back(p);
+      g.piece_cost.push_back(chunk_cost(p, bits));
+      if (inside) g.piece_split.push_back(y);
+      p.strip_begin = y;
+      p.tile_begin = t;
+      p.col_begin = p.col_end = 0;  // the first piece counts the chunk's columns
+    }
+    p.strip_end = c.strip_end;
+    p.tile_end = c.tile_end;
+    g.pieces.push_back(p);
+    g.piece_cost.push_back(chunk_cost(p, bits));
+    g.piece_off.push_back(static_cast<uint32_t>(g.pieces.size()));
+  }
+  std::sort(g.piece_split.begin(), g.piece_split.end());
+  g.piece_split.erase(std::unique(g.piece_split.begin(), g.piece_split.end()), g.piece_split.end());
 }
 
 // strip_job[y] = first job of strip y (y = n_strips: the job count).
@@ -2673,6 +2763,7 @@ GraphPlan plan_graph(const mg_tiled_matrix* at, uint32_t chunk_tiles, hipStream_
     MG_HIP(hipStreamSynchronize(st));
   }
   g.chunk_cost = chunk_costs(g, st, &g.total_bits);
+  g.host_off.swap(off);
   return g;
 }
 
@@ -2750,6 +2841,7 @@ struct Engine {
   uint32_t W = 64;
   // Hop kernel of the 64-word levels from level seg_from on: 0 = tile-decoding sweep
   // (walk_numeric64_kernel), G = 1, 2, 4 or 8 = job-list kernel with G row segments.
+  // G = 1 also takes the first hop where it is swept (4096 sources on R-MAT 14: 694 us a walk before, 278).
   uint32_t seg = 0;
   uint32_t seg_from = 1;
   // One-graph walks of fewer than 64 words: the hops run walk_narrow_kernel; used_words: words of
@@ -2771,6 +2863,11 @@ struct Engine {
   std::vector<uint32_t> n_chunks;
   std::vector<DevBuf<StripItem>> split;
   std::vector<uint32_t> n_split;
+  // walk_lean_kernel's launches: the chunks' pieces and the strips that they split (build_lean).
+  std::vector<DevBuf<Chunk>> lean;
+  std::vector<uint32_t> n_lean;
+  std::vector<DevBuf<StripItem>> lean_split;
+  std::vector<uint32_t> n_lean_split;
   DevBuf<ZeroItem> zero_items;  // the split strips of every level
   uint32_t n_zero_items = 0;
   // X_0 setup
@@ -2799,6 +2896,96 @@ struct Engine {
 };
 
 namespace {
+
+// Heaviest chunks first (chunk_costs) so the tail of the launch is made of light ones.
+// Among equal costs, the same chunk of every panel of one graph is adjacent, so the
+// panels' reads of those A^T tiles follow each other closely and the repeats are served
+// from cache.
+void sort_by_cost(const Engine& e, std::vector<Chunk>& ch, const std::vector<uint64_t>& cost) {
+  std::vector<uint32_t> idx(ch.size());
+  std::iota(idx.begin(), idx.end(), 0u);
+  std::sort(idx.begin(), idx.end(), [&](uint32_t i, uint32_t j) {
+    const Chunk &a = ch[i], &b = ch[j];
+    if (cost[i] != cost[j]) return cost[i] > cost[j];
+    const uint32_t ga = e.panels[a.panel].graph, gb = e.panels[b.panel].graph;
+    if (ga != gb) return ga < gb;
+    if (a.strip_begin != b.strip_begin) return a.strip_begin < b.strip_begin;
+    if (a.tile_begin != b.tile_begin) return a.tile_begin < b.tile_begin;
+    return a.panel < b.panel;
+  });
+  std::vector<Chunk> sorted(ch.size());
+  for (size_t i = 0; i < idx.size(); ++i) sorted[i] = ch[idx[i]];
+  ch.swap(sorted);
+}
+
+// The pieces of a level's chunks: heaviest first, or in the chunks' launch order (one that the caller
+// has set).
+std::vector<Chunk> level_pieces(const Engine& e, uint32_t k, bool by_cost) {
+  std::vector<Chunk> out;
+  std::vector<uint64_t> cost;
+  for (const Chunk& c : e.host_chunks[k]) {
+    const GraphPlan& g = e.graphs[e.panels[c.panel].graph];
+    const auto it = std::lower_bound(g.chunks.begin(), g.chunks.end(), c, [](const Chunk& a, const Chunk& b) {
+      return a.strip_begin != b.strip_begin ? a.strip_begin < b.strip_begin : a.tile_begin < b.tile_begin;
+    });
+    const size_t i = static_cast<size_t>(it - g.chunks.begin());
+    for (uint32_t p = g.piece_off[i]; p < g.piece_off[i + 1]; ++p) {
+      out.push_back(g.pieces[p]);
+      out.back().panel = c.panel;
+      cost.push_back(g.piece_cost[p]);
+    }
+  }
+  if (by_cost) sort_by_cost(e, out, cost);
+  return out;
+}
+
+void upload_zero_items(Engine* e, const std::vector<ZeroItem>& items, hipStream_t st) {
+  e->n_zero_items = static_cast<uint32_t>(items.size());
+  e->zero_items.alloc(std::max<size_t>(1, items.size()));
+  if (!items.empty())
+    MG_HIP(hipMemcpyAsync(e->zero_items.get(), items.data(), sizeof(ZeroItem) * items.size(), hipMemcpyHostToDevice, st));
+  MG_HIP(hipStreamSynchronize(st));
+}
+
+// Pieces of the chunks of every level for walk_lean_kernel, and the strips to clear for them and for the
+// chunks (which logged levels launch). A piece has at most 1 / kLeanShares of the jobs of all panels, and
+// kLeanMinJobs or more: the chunks alone leave a hop waiting for the hub strip's (a steady hop of 4096
+// sources on R-MAT 14, 16, 18, 20, 22: 522, 693, 902, 875, 3806 us with whole chunks, 11, 45, 233, 775,
+// 3688 in pieces). 1024 shares: 14, 68, 262, 773, 3695; 4096: 55, 91, 251, 802, 3675 (1024 jobs at least);
+// 16384: 32, 59, 279, 932, 3745; at least 256 or 128 jobs: as 512.
+constexpr uint64_t kLeanShares = 2048;
+constexpr uint64_t kLeanMinJobs = 512;
+void build_lean(Engine* e, hipStream_t st) {
+  uint64_t jobs = 0;
+  for (const Panel& p : e->panels) jobs += e->graphs[p.graph].total_bits;
+  for (GraphPlan& g : e->graphs) build_pieces(g, std::max(kLeanMinJobs, jobs / kLeanShares), st);
+  e->lean.resize(e->max_hops);
+  e->n_lean.assign(e->max_hops, 0);
+  e->lean_split.resize(e->max_hops);
+  e->n_lean_split.assign(e->max_hops, 0);
+  std::vector<ZeroItem> zero;
+  for (uint32_t k = 0; k < e->max_hops; ++k) {
+    const std::vector<Chunk> ch = level_pieces(*e, k, true);
+    std::vector<StripItem> sp;
+    for (uint32_t pi = 0; pi < e->panels.size(); ++pi) {
+      Panel& p = e->panels[pi];
+      if (k >= p.hops || (k == 0 && pi < e->push0.size() && e->push0[pi])) continue;
+      for (uint32_t y : e->graphs[p.graph].piece_split) {
+        sp.push_back({pi, y});
+        zero.push_back({p.x[k + 1].get() + static_cast<uint64_t>(y) * 64 * e->W, p.s[k + 1].get() + y});
+      }
+    }
+    e->n_lean[k] = static_cast<uint32_t>(ch.size());
+    e->lean[k].alloc(std::max<size_t>(1, ch.size()));
+    if (!ch.empty()) MG_HIP(hipMemcpyAsync(e->lean[k].get(), ch.data(), sizeof(Chunk) * ch.size(), hipMemcpyHostToDevice, st));
+    e->n_lean_split[k] = static_cast<uint32_t>(sp.size());
+    e->lean_split[k].alloc(std::max<size_t>(1, sp.size()));
+    if (!sp.empty())
+      MG_HIP(hipMemcpyAsync(e->lean_split[k].get(), sp.data(), sizeof(StripItem) * sp.size(), hipMemcpyHostToDevice, st));
+    MG_HIP(hipStreamSynchronize(st));  // ch and sp are about to go out of scope
+  }
+  upload_zero_items(e, zero, st);
+}
 
 // Allocate frontiers, build the per-level descriptor tables, chunk lists and items.
 // All copies and fills are ordered on `st` (the context stream); host sources stay alive
@@ -2890,26 +3077,7 @@ void build_engine(Engine* e, hipStream_t st) {
           zero_items.push_back({p.x[k + 1].get() + static_cast<uint64_t>(y) * 64 * e->W, p.s[k + 1].get() + y});
         }
     }
-    // Heaviest chunks first (chunk_costs) so the tail of the launch is made of light ones.
-    // Among equal costs, the same chunk of every panel of one graph is adjacent, so the
-    // panels' reads of those A^T tiles follow each other closely and the repeats are served
-    // from cache.
-    {
-      std::vector<uint32_t> idx(ch.size());
-      std::iota(idx.begin(), idx.end(), 0u);
-      std::sort(idx.begin(), idx.end(), [&](uint32_t i, uint32_t j) {
-        const Chunk &a = ch[i], &b = ch[j];
-        if (cost[i] != cost[j]) return cost[i] > cost[j];
-        const uint32_t ga = e->panels[a.panel].graph, gb = e->panels[b.panel].graph;
-        if (ga != gb) return ga < gb;
-        if (a.strip_begin != b.strip_begin) return a.strip_begin < b.strip_begin;
-        if (a.tile_begin != b.tile_begin) return a.tile_begin < b.tile_begin;
-        return a.panel < b.panel;
-      });
-      std::vector<Chunk> sorted(ch.size());
-      for (size_t i = 0; i < idx.size(); ++i) sorted[i] = ch[idx[i]];
-      ch.swap(sorted);
-    }
+    sort_by_cost(*e, ch, cost);
     e->lv[k].alloc(P);
     MG_HIP(hipMemcpyAsync(e->lv[k].get(), lv.data(), sizeof(PanelLevel) * P, hipMemcpyHostToDevice, st));
     e->host_lv.push_back(lv);
@@ -2931,11 +3099,7 @@ void build_engine(Engine* e, hipStream_t st) {
     if (!sp.empty()) MG_HIP(hipMemcpyAsync(e->split[k].get(), sp.data(), sizeof(StripItem) * sp.size(), hipMemcpyHostToDevice, st));
     MG_HIP(hipStreamSynchronize(st));  // lv, ch, pch and sp are about to go out of scope
   }
-  e->n_zero_items = static_cast<uint32_t>(zero_items.size());
-  e->zero_items.alloc(std::max<size_t>(1, zero_items.size()));
-  if (!zero_items.empty())
-    MG_HIP(hipMemcpyAsync(e->zero_items.get(), zero_items.data(), sizeof(ZeroItem) * zero_items.size(),
-                          hipMemcpyHostToDevice, st));
+  upload_zero_items(e, zero_items, st);
   // X_0 fills: frontier and masks of every panel, plus all counters.
   std::vector<PanelInit> inits(P);
   std::vector<uint32_t> strips(P);
@@ -2967,6 +3131,7 @@ void apply_seg(Engine* e, uint32_t G, hipStream_t st) {
       if (!job_list_fits(g)) G = 0;
   if (G) {
     for (auto& g : e->graphs) build_job_list(g, st);
+    if (G == 1 && e->lean.empty()) build_lean(e, st);
     for (auto& p : e->panels) {
       if (G == 1) break;  // the one-segment kernel writes the masks itself
       const uint64_t need = static_cast<uint64_t>(G) * 3 * std::max<uint32_t>(1, p.n_strips);
@@ -3017,7 +3182,7 @@ void launch_level_w(hipStream_t st, Engine* e, uint32_t k, hipEvent_t ev[4]) {
   if (ev) MG_HIP(hipEventRecord(ev[0], st));
   if (ev) MG_HIP(hipEventRecord(ev[1], st));
   if (ev) MG_HIP(hipEventRecord(ev[2], st));
-  const uint32_t G = (W == 64 && e->seg && !e->logging && k >= e->seg_from) ? e->seg : 0;
+  const uint32_t G = (W == 64 && e->seg && !e->logging && (k >= e->seg_from || e->seg == 1)) ? e->seg : 0;
   if (e->n_chunks[k]) {
     ChunkLog* const log = e->logging ? e->logs[k].get() : nullptr;
     if constexpr (W == 64) {
@@ -3026,9 +3191,9 @@ void launch_level_w(hipStream_t st, Engine* e, uint32_t k, hipEvent_t ev[4]) {
         case 0: walk_numeric64_kernel<<<nb, kNumBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get(), log); break;
         case 1:
           if (e->partial[k])
-            walk_lean_kernel<true><<<nb, kLeanBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get());
+            walk_lean_kernel<true><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get());
           else
-            walk_lean_kernel<false><<<nb, kLeanBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get());
+            walk_lean_kernel<false><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get());
           break;
         case 2: walk_seg_kernel<2><<<nb * 2, kSegBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get()); break;
         case 4: walk_seg_kernel<4><<<nb * 4, kSegBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get()); break;
@@ -3052,8 +3217,10 @@ void launch_level_w(hipStream_t st, Engine* e, uint32_t k, hipEvent_t ev[4]) {
     seg_combine_kernel<<<dim3(grid_for(max_strips, kBlock, 1024), n_panels), kBlock, 0, st>>>(e->lv[k].get(), G);
     MG_LAUNCH_CHECK();
   }
-  if (e->n_split[k]) {
-    finalize_strips_kernel<W><<<e->n_split[k], kBlock, 0, st>>>(e->split[k].get(), e->lv[k].get());
+  const uint32_t n_split = G == 1 ? e->n_lean_split[k] : e->n_split[k];
+  if (n_split) {
+    finalize_strips_kernel<W><<<n_split, kBlock, 0, st>>>(G == 1 ? e->lean_split[k].get() : e->split[k].get(),
+                                                          e->lv[k].get());
     MG_LAUNCH_CHECK();
   }
 }
@@ -4016,6 +4183,11 @@ extern "C" int mg_walk_batch_set_level_order(mg_walk_batch* b, uint32_t level, c
     ch.swap(next);
     if (!ch.empty())
       MG_HIP(hipMemcpy(e.chunks[level].get(), ch.data(), sizeof(Chunk) * ch.size(), hipMemcpyHostToDevice));
+    if (!e.lean.empty()) {
+      const std::vector<Chunk> pieces = level_pieces(e, level, false);
+      if (!pieces.empty())
+        MG_HIP(hipMemcpy(e.lean[level].get(), pieces.data(), sizeof(Chunk) * pieces.size(), hipMemcpyHostToDevice));
+    }
     if (!e.logs.empty()) MG_HIP(hipMemset(e.logs[level].get(), 0, e.logs[level].bytes()));
     MG_HIP(hipDeviceSynchronize());  // null-stream fill; runs use the context's stream
   });

@@ -489,3 +489,28 @@ def test_batch_of_queries_with_common_sources(ctx, sizes):
         assert b.query_digest(i) == w.frontier_digest(q.hops), i
         w.close()
     b.close()
+
+
+@pytest.mark.parametrize("sweep", [False, True])
+@pytest.mark.parametrize("n_sources", [2100, 4096])
+def test_pieces_of_heavy_strips(ctx, n_sources, sweep):
+    """64 words per vertex where one strip of A^T holds most edges and others none: its chunk runs in pieces."""
+    M = mg()
+    rng = np.random.default_rng(n_sources)
+    n = 9000
+    s, d = (rng.integers(0, n, 40000) for _ in range(2))
+    d[:25000] = rng.integers(640, 704, 25000)
+    d[25000:32000] = rng.integers(700, 710, 7000)
+    keep = (d // 64) % 7 != 3
+    s, d = s[keep].astype(np.uint32), d[keep].astype(np.uint32)
+    at = M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True)
+    sources = O.sample_sources(n, n_sources, 3)
+    w = M.Walk(ctx, at, n_sources, 3, M.WALK_SWEEP_FIRST_HOP if sweep else 0)
+    xs = O.walk_frontiers(n, s, d, sources, 3, W=64)
+    for _ in range(2):
+        w.run(sources, 3)
+        for k in (1, 2, 3):
+            got = w.frontier(k)
+            assert np.array_equal(got[:n], xs[k]) and not got[n:].any(), k
+            assert w.hop_stats(k)["popcount"] == np.bitwise_count(xs[k]).sum()
+    w.close()
