@@ -1511,14 +1511,45 @@ __device__ inline void lean_commit(const LeanSet& s, char* __restrict__ acc_lane
   }
 }
 
-// kPartial: some panel of the level has dead words (its gathers then read only the cache lines of
-// live words); false keeps the plain lane-per-word loads and their registers.
-template <bool kPartial>
+// A batch of a panel with at most 16 live words: each row of 16 lanes takes its own 16 jobs one after the
+// other, lane = live word (job broadcast in the row by DPP), so a load instruction gathers four rows, and
+// kFewLoads of them are in flight. What a gather costs is its instructions: one row at a time, a hop
+// takes as long with one live word as with 48. `job`: kNoJob where nothing is gathered; `edges` counts,
+// per lane, the jobs whose row has a live word.
+constexpr int kFewWords = 16;
+constexpr int kFewLoads = 4;
+template <int K0, int... K>
+__device__ inline void few_gather(std::integer_sequence<int, K...>, uint32_t job, gptr<const uint64_t> x_word,
+                                  unsigned long long* acc_word, bool live, bool count_rows, uint32_t lane,
+                                  uint32_t& edges) {
+  constexpr int N = sizeof...(K);
+  const uint32_t jb[N] = {group_lane<16, K0 + K>(job)...};
+  uint64_t v[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = live && jb[k] != kNoJob ? x_word[static_cast<uint64_t>(jb[k] >> 6) * 64] : 0ull;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    if (count_rows) edges += ((ballot(v[k] != 0) >> (lane & 48u)) & 0xFFFFu) != 0 && (lane & 15u) == 0;
+    if (v[k]) atomicOr(acc_word + (jb[k] & 63u) * 64u, static_cast<unsigned long long>(v[k]));
+  }
+}
+
+// kLeanWhole: lane = word. kLeanPartial: some panel of the launch has dead words (its gathers then read
+// only the cache lines of live words). kLeanFew: every panel has at most kFewWords live words
+// (few_gather). kLeanMixed: some have. Kernels of their own because the others fit in 64 VGPRs only
+// without few_gather: kLeanMixed spills ten more, which costs its wider panels 3-6 %, but two launches
+// one after the other cost more (a batch of 16 queries on three graphs: 2.04 ms mixed, 2.35 in two
+// launches, 2.67 without few_gather).
+enum : int { kLeanWhole = 0, kLeanPartial = 1, kLeanFew = 2, kLeanMixed = 3 };
+template <int kMode>
 __global__ void __launch_bounds__(kLeanBlock) __attribute__((amdgpu_waves_per_eu(kLeanWaves, kLeanWaves)))
     walk_lean_kernel(const Chunk* __restrict__ chunks, const PanelLevel* __restrict__ lv) {
+  constexpr bool kPartial = kMode == kLeanPartial || kMode == kLeanMixed;
+  constexpr bool kFew = kMode == kLeanFew || kMode == kLeanMixed;
   constexpr int kWords = 64 * 64;
   constexpr uint32_t kNoTile = 0xFFFFFFFFu;
   __shared__ unsigned long long acc[kWords];
+  __shared__ uint32_t s_few[kFew ? kFewWords : 1];
   // Per strip parity: N, V, Z and S masks being reduced (thread 0 stores and clears a slot
   // after the strip's second barrier; the other slot is in use by then).
   __shared__ unsigned long long s_mask[2][4];
@@ -1544,6 +1575,10 @@ __global__ void __launch_bounds__(kLeanBlock) __attribute__((amdgpu_waves_per_eu
       (!kPartial || keep) ? lane
                           : (alive_in ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(alive_in)) - 1) : 0u);
   const bool lane_next = (alive_next >> lane) & 1;  // this lane's word propagates further
+  const bool few = kMode == kLeanFew || (kMode == kLeanMixed && __popcll(alive_in) <= kFewWords);
+  if constexpr (kFew) {  // s_few[k]: the k-th live word; read after the first barrier
+    if (few && threadIdx.x < 64 && keep) s_few[__popcll(alive_in & ((1ull << lane) - 1))] = lane;
+  }
   // Per-strip values of the chunk, one strip per lane: row pointers and the job offsets of
   // the strip boundaries (clamped to the chunk's tile range).
   const uint32_t n_cs = ch.strip_end - ch.strip_begin;
@@ -1647,6 +1682,26 @@ __global__ void __launch_bounds__(kLeanBlock) __attribute__((amdgpu_waves_per_eu
       const uint64_t okm = ballot(ok);
       if (check_v) edges += static_cast<uint32_t>(__popcll(okm));
       const bool count_rows = !check_v;
+      if (kFew && few) {
+        const uint64_t vw_n = (check_v && job_n != kNoJob) ? v_in[job_n >> 12] : 0ull;
+        const uint32_t jb = ok ? job : kNoJob;
+        using Steps = std::make_integer_sequence<int, kFewLoads>;
+        const bool few_live = (lane & (kFewWords - 1)) < static_cast<uint32_t>(__popcll(alive_in));
+        const uint32_t few_word = few_live ? s_few[lane & (kFewWords - 1)] : 0u;
+        const gptr<const uint64_t> xw = x_in + few_word;
+        unsigned long long* const aw = acc + few_word;
+        if (okm) {
+          few_gather<0>(Steps{}, jb, xw, aw, few_live, count_rows, lane, cnt[bEdges]);
+          few_gather<4>(Steps{}, jb, xw, aw, few_live, count_rows, lane, cnt[bEdges]);
+          few_gather<8>(Steps{}, jb, xw, aw, few_live, count_rows, lane, cnt[bEdges]);
+          few_gather<12>(Steps{}, jb, xw, aw, few_live, count_rows, lane, cnt[bEdges]);
+        }
+        job = job_n;
+        vw = vw_n;
+        p_strip = n_strip;
+        p_base = n_base;
+        continue;
+      }
       uint64_t rows;
       uint64_t m = lean_groups(job, okm, lane, rows);
       const uint64_t row_addr = reinterpret_cast<uint64_t>(x_in) + static_cast<uint64_t>(job >> 6) * 512u;
@@ -2858,7 +2913,7 @@ struct Engine {
   bool logging = false;
   std::vector<DevBuf<PanelLevel>> lv;
   std::vector<std::vector<PanelLevel>> host_lv;  // host copies of lv
-  std::vector<uint8_t> partial;  // per level: some active panel has dead words (alive_in != all)
+  std::vector<uint8_t> partial;  // per level: walk_lean_kernel's mode, from the active panels' live words
   std::vector<DevBuf<Chunk>> chunks;
   std::vector<uint32_t> n_chunks;
   std::vector<DevBuf<StripItem>> split;
@@ -3081,9 +3136,15 @@ void build_engine(Engine* e, hipStream_t st) {
     e->lv[k].alloc(P);
     MG_HIP(hipMemcpyAsync(e->lv[k].get(), lv.data(), sizeof(PanelLevel) * P, hipMemcpyHostToDevice, st));
     e->host_lv.push_back(lv);
-    bool partial = false;
-    for (const auto& L : lv) partial |= L.x_in && L.alive_in != ~0ull;
-    e->partial.push_back(partial ? 1 : 0);
+    bool some_dead = false, some_few = false, some_many = false;
+    for (const auto& L : lv) {
+      if (!L.x_in) continue;
+      const bool is_few = __builtin_popcountll(L.alive_in) <= kFewWords;
+      some_dead |= L.alive_in != ~0ull;
+      some_few |= is_few;
+      some_many |= !is_few;
+    }
+    e->partial.push_back(some_few ? (some_many ? kLeanMixed : kLeanFew) : some_dead ? kLeanPartial : kLeanWhole);
     e->n_chunks[k] = static_cast<uint32_t>(ch.size());
     e->host_chunks[k] = ch;
     e->chunks[k].alloc(std::max<size_t>(1, ch.size()));
@@ -3190,10 +3251,12 @@ void launch_level_w(hipStream_t st, Engine* e, uint32_t k, hipEvent_t ev[4]) {
       switch (G) {
         case 0: walk_numeric64_kernel<<<nb, kNumBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get(), log); break;
         case 1:
-          if (e->partial[k])
-            walk_lean_kernel<true><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get());
-          else
-            walk_lean_kernel<false><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get());
+          switch (e->partial[k]) {
+            case kLeanWhole: walk_lean_kernel<kLeanWhole><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get()); break;
+            case kLeanPartial: walk_lean_kernel<kLeanPartial><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get()); break;
+            case kLeanFew: walk_lean_kernel<kLeanFew><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get()); break;
+            default: walk_lean_kernel<kLeanMixed><<<e->n_lean[k], kLeanBlock, 0, st>>>(e->lean[k].get(), e->lv[k].get()); break;
+          }
           break;
         case 2: walk_seg_kernel<2><<<nb * 2, kSegBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get()); break;
         case 4: walk_seg_kernel<4><<<nb * 4, kSegBlock, 0, st>>>(e->chunks[k].get(), e->lv[k].get()); break;

@@ -127,3 +127,27 @@ def test_batch_job_list_kernel_equals_sweep(ctx, segments):
     assert bj.totals() == bs.totals()
     for i in range(0, len(qs), 3):
         assert bj.query_digest(i) == bs.query_digest(i), i
+
+
+@pytest.mark.parametrize("sizes", [(5, 900), (64, 64, 64), (1000, 24), (1030,), (300, 2000, 5), (1024,)])
+def test_batch_of_few_live_words(ctx, sizes):
+    """Panels with at most 16 live words (from the start, or once longer queries are left), alone and with wider ones."""
+    M = mg()
+    rng = np.random.default_rng(sum(sizes))
+    graphs, queries = [], []
+    for g, n in enumerate((3000, 20000)):
+        s, d = (rng.integers(0, n, 12 * n).astype(np.uint32) for _ in range(2))
+        d[: 3 * n] = 70
+        graphs.append(M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True))
+        for i, k in enumerate(sizes):
+            sources = rng.permutation(n)[:k].astype(np.uint32)
+            queries.append(M.workloads.QuerySpec(g, sources, 5 - 2 * (k > 1000) - i % 2))
+    b = M.WalkBatch(ctx, graphs, queries)
+    for _ in range(2):
+        b.run()
+        for i, q in enumerate(queries):
+            w = M.Walk(ctx, graphs[q.graph], len(q.sources), q.hops)
+            w.run(q.sources, q.hops)
+            assert b.query_digest(i) == w.frontier_digest(q.hops), i
+            w.close()
+    b.close()
