@@ -251,9 +251,11 @@ int mg_multiply_symbolic(mg_context* ctx, const mg_tiled_matrix* a, const mg_til
 int mg_tiled_matrix_prepare_operand(mg_context* ctx, mg_tiled_matrix* m);
 /* Numeric pass into a C produced by mg_multiply_symbolic (OR-accumulates).
  * Replaces PPRQuery::FillTilesUnifiedMemory (ppr_query.cu:459-780). Asynchronous on the
- * context's stream; keeps 16 bytes per operand tile in the context's scratch, which grows in
- * stream order (hipMallocAsync/hipFreeAsync on that stream: queued work that reads the old
- * buffer finishes before its memory is reused). */
+ * context's stream; keeps 32 bytes per C tile and, of operands that are not prepared, 16 bytes of
+ * head per tile, 8 per column in use of a tile and B's index in the context's scratch, which grows
+ * in stream order (hipMallocAsync/hipFreeAsync on that stream: queued work that reads the old
+ * buffer finishes before its memory is reused). Without memory for the column words it makes them
+ * from the tiles. */
 int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt,
                         mg_tiled_matrix* c);
 /* The numeric pass with a per-tile-pair choice of engine: a pair whose two tiles both have
@@ -273,9 +275,10 @@ int mg_multiply_numeric_dense(mg_context* ctx, const mg_tiled_matrix* a, const m
  * (ppr_query.cu:288-314). capacity chooses how the output is sized:
  *   MG_PRUNED_EXACT (0): a flag pass finds the non-empty tiles, a second pass writes each at
  *     its final position (two numeric passes, memory = the output);
- *   MG_PRUNED_STRUCTURAL: one pass into scratch for every structural tile, then sorted;
+ *   MG_PRUNED_STRUCTURAL: one pass into scratch for every structural tile, then put in order;
  *   any other value (e.g. a cost model's prediction): one pass into that many slots, then
- *     sorted; if more tiles are non-empty the pass is run again with the exact count (fallback).
+ *     put in order; if more tiles are non-empty, the part of the pass that found no slot is run
+ *     again with the exact count (fallback).
  * Synchronises. stats may be NULL. */
 #define MG_PRUNED_EXACT 0ull
 #define MG_PRUNED_STRUCTURAL (~0ull)
@@ -385,7 +388,8 @@ enum {
                                    (results, digests, downloads and exports are the same) */
 };
 enum {
-  MG_HOP_SWEEP = 0u, /* the hop swept every strip of A^T (walk_numeric kernels) */
+  MG_HOP_SWEEP = 0u, /* the hop took every strip of A^T in vertex-row words: by its tiles, or by its
+                        job list (walks of at most 2048 sources; a first hop that is not pushed) */
   MG_HOP_PUSH = 1u,  /* first hop pushed from the source strips' A^T columns */
   MG_HOP_JOBS = 2u   /* the hop read A^T's job list by row segments (mg_walk_set_hop_kernel) */
 };
@@ -413,7 +417,8 @@ typedef struct mg_hop_stats {
 
 /* Allocates X_0..X_max_hops (W = ceil(max_sources/64) rounded up to a power of two,
  * max_sources <= 4096) plus the strip scheduler, the per-tile row-occupancy masks of at
- * and (unless MG_WALK_SWEEP_FIRST_HOP) a column index of at (16 bytes per tile). at must
+ * a job list of at (4 bytes per set bit, tile and strip) and (unless MG_WALK_SWEEP_FIRST_HOP) a
+ * column index of it (16 bytes per tile). at must
  * outlive w and keep its contents (the masks are taken here).
  * The first hop of a run is pushed from the source strips when their columns of at hold at
  * most half of its tiles; results and statistics are the same either way. */

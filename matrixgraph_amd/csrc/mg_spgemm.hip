@@ -489,6 +489,7 @@ __global__ void col_scatter_kernel(const uint32_t* __restrict__ row, const uint3
 // added to sums[0] (tile products), sums[1] (tiles of the B rows that A references, ref[x]:
 // row x of B, as x runs over the strips) and sums[2] (C tiles).
 // EMIT = true : write the union as ascending col_idx at off_c[x], row_idx = x.
+// Grids wider than kBitmapStrips only (structural_pass), where no bitmap of B is kept.
 // BLOCK threads per row (kRowBlock = 1024: a heavy row, such as a dense frontier's tile row
 // against thousands of B rows, is the whole pass when few rows carry the work; 1024 threads
 // took the 3-hop density-mixed product walk's symbolic passes from 39 to 16 ms and C = A*A of

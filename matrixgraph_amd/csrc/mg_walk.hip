@@ -3186,7 +3186,7 @@ void build_engine(Engine* e, hipStream_t st) {
 // them. G = 0 keeps the tile-decoding sweep. Not called while a run may be in flight.
 void apply_seg(Engine* e, uint32_t G, hipStream_t st) {
   MG_REQUIRE(G == 0 || G == 1 || G == 2 || G == 4 || G == 8, "walk: row segments must be 0, 1, 2, 4 or 8");
-  if (G && e->W != 64) G = 0;  // narrower panels keep walk_numeric_kernel<W>
+  if (G && e->W != 64) G = 0;  // narrower panels have a kernel of their own
   if (G)
     for (auto& g : e->graphs)
       if (!job_list_fits(g)) G = 0;
