@@ -471,7 +471,7 @@ def mfma_section(M, ctx, densities=(0.01, 0.03, 0.1, 0.3), reps=3):
             row[key + "_products"] = dense
             row["tile_products"] = st["tile_products"]
         row["matrix_cores_vs_vector"] = round(row["vector_ms"] / row["matrix_cores_ms"], 3)
-        row["int8_ops_per_s_matrix_cores"] = round(row["matrix_cores_products"] * 2 * 64**3
+        row["ops_per_s_matrix_cores"] = round(row["matrix_cores_products"] * 2 * 64**3
                                                    / (row["matrix_cores_ms"] * 1e-3), 1)
         row["bit_exact"] = digests[4097] == digests[0]
         if not row["bit_exact"]:
@@ -487,7 +487,7 @@ def mfma_section(M, ctx, densities=(0.01, 0.03, 0.1, 0.3), reps=3):
                     "probability p, seed 3; numeric pass only (HIP events), symbolic pass excluded",
         "per_density": out,
         "matrix_cores_win_from_p": min(wins) if wins else None,
-        "int8_peak_ops_per_s": 5.0e15,
+        "fp4_peak_ops_per_s": 1.0e16,
     }
 
 

@@ -261,8 +261,8 @@ int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, const mg_tile
 /* The numeric pass with a per-tile-pair choice of engine: a pair whose two tiles both have
  * at least min_bits set bits is multiplied on the matrix cores; every other pair on the
  * vector ALUs. The vector pass records the dense pairs of every C tile, and a second kernel
- * expands their tiles in registers, sums each C tile's pairs in int32 (int8 0/1 products) and
- * turns counts > 0 into bits once. min_bits = 0 sends every pair to the matrix cores,
+ * expands their tiles in registers, sums each C tile's pairs in FP32 (exact: products of bits) and
+ * turns sums > 0 into bits once. min_bits = 0 sends every pair to the matrix cores,
  * min_bits > 4096 none. *dense_products (may be NULL) receives the number of matrix-core tile
  * products. Same result as mg_multiply_numeric. Synchronises.
  * No counterpart in the reference (its product is VALU only). */

@@ -815,35 +815,48 @@ __global__ void __launch_bounds__(kBlock) heavy_scatter_kernel(const HeavyPair* 
 // Dense tile pairs on the matrix cores, as one contraction per C tile: for every pair
 // (A(x,k), Bt(y,k)) whose two tiles both hold at least min_bits set bits, the vector kernel
 // records the pair (its two tile indices) instead of multiplying it; then
-// dense_contract_kernel sums, per C tile, the int8 0/1 products of all its recorded pairs in
-// int32 (v_mfma_i32_32x32x32_i8, four 32 x 32 output blocks, two K-steps of 32 per pair) and
-// turns counts > 0 into bit rows once, ORed into C. Operands are expanded from the bit tiles
-// in registers: a lane loads one 64-bit row of each tile (A row r, Bt row c = B column c) and
-// turns 4 bits at a time into 4 bytes of 0/1 with a 24-bit multiply.
-// Lane layout (32x32x32 i8): lane l holds 16 bytes of A row l % 32 and of B column l % 32,
-// at k = 16 * (l / 32) .. +15 of the K-step (any k order works if both operands use it);
-// result register v of lane l is C[8 * (v / 4) + 4 * (l / 32) + v % 4][l % 32].
-typedef int mg_v16i __attribute__((ext_vector_type(16)));
-typedef int mg_v4i __attribute__((ext_vector_type(4)));
+// dense_contract_kernel sums, per C tile, the products of all its recorded pairs in FP32
+// (v_mfma_f32_32x32x64, operands in 4 bits, four 32 x 32 output blocks, the 64 inner indices of a
+// pair in one step) and turns sums > 0 into bit rows once, ORed into C. Operands are expanded from
+// the bit tiles in registers: a bit becomes 1.0 or 2.0 or 0, the same power for an inner index on
+// both sides, so that a product is 1, 4 or 0 and the sums (at most 2^14) are exact.
+// Lane layout: lane l holds 32 values of A row l % 32 and of B column l % 32, half l / 32 of the
+// inner indices (any order works if both operands use it); result register v of lane l is
+// C[8 * (v / 4) + 4 * (l / 32) + v % 4][l % 32].
+typedef int mg_v8i __attribute__((ext_vector_type(8)));
+typedef float mg_v16f __attribute__((ext_vector_type(16)));
+constexpr int kFp4 = 4;            // operand format of the instruction: e2m1
+constexpr int kOne = 0x7F7F7F7F;   // block scales of 1
 
-// Bits 0..15 of x as 16 bytes of value 0 or 1 (byte j = bit j): nibble * 0x204081 puts bit
-// i of the nibble at bit 8i (the four shifted copies do not overlap), the mask keeps those.
-__device__ inline mg_v4i bits16_to_bytes(uint32_t x) {
-  mg_v4i out;
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    out[q] = static_cast<int>(__umul24((x >> (4 * q)) & 0xFu, 0x204081u) & 0x01010101u);
+// The bits of x as 32 values of four bits, bit 4 i + q in nibble i of register q: nibble 2 is 1.0,
+// nibble 4 is 2.0.
+__device__ inline mg_v8i bits_to_fp4(uint32_t x) {
+  mg_v8i out = {};
+  out[0] = static_cast<int>((x << 1) & 0x22222222u);
+  out[1] = static_cast<int>(x & 0x22222222u);
+  out[2] = static_cast<int>(x & 0x44444444u);
+  out[3] = static_cast<int>((x >> 1) & 0x44444444u);
   return out;
+}
+__device__ inline mg_v16f mfma_fp4(mg_v8i a, mg_v8i b, mg_v16f c) {
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, kFp4, kFp4, 0, kOne, 0, kOne);
 }
 
 // Up to kTaskPairs of a C tile's dense pairs.
 struct DenseTask {
   uint32_t tile, base, n;
 };
-// One wave per recorded task: int32 counts of the 64 x 64 output over all the task's pairs
-// on the matrix cores, then one threshold; the rows are ORed into C atomically (several
-// tasks may share a C tile).
-__global__ void __launch_bounds__(kBlock) dense_contract_kernel(const DenseTask* __restrict__ tasks,
+// One wave per recorded task: the sums of the 64 x 64 output over all the task's pairs on the
+// matrix cores, then one threshold; the rows are ORed into C atomically (several tasks may share a
+// C tile). The pairs are read once, one per lane, and kStep pairs' operands are loaded before the
+// step in front of them is multiplied; a last step that is not full takes the last pair twice.
+// 16.8 M pairs, 64 to a C tile: 2.4 ms (3.6e15 operations a second), 5.9 with operands in bytes,
+// whose expansion alone was 124 vector instructions a pair; now 24, and the matrix instructions
+// (0.9 ms) wait for the tiles, 1 KiB a pair from L2. Four waves a SIMD: left to itself the compiler
+// takes 204 registers, enough for two.
+constexpr uint32_t kStep = 2;
+static_assert(kTaskPairs <= kWave);
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) dense_contract_kernel(const DenseTask* __restrict__ tasks,
                                                                 const uint32_t* __restrict__ n_tasks_ptr,
                                                                 const uint2* __restrict__ pairs,
                                                                 const uint64_t* __restrict__ data_a,
@@ -851,28 +864,45 @@ __global__ void __launch_bounds__(kBlock) dense_contract_kernel(const DenseTask*
                                                                 uint64_t* __restrict__ data_c) {
   const uint32_t lane = lane_id();
   const uint32_t lo = lane & 31, hi = lane >> 5;
+  const uint32_t* const half_a = reinterpret_cast<const uint32_t*>(data_a) + 2 * lo + hi;
+  const uint32_t* const half_b = reinterpret_cast<const uint32_t*>(data_bt) + 2 * lo + hi;
   const uint32_t n_tasks = *n_tasks_ptr;
   const uint32_t n_waves = gridDim.x * kWavesPerBlock;
   for (uint32_t t = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); t < n_tasks; t += n_waves) {
     const DenseTask T = tasks[t];
-    mg_v16i acc00 = {}, acc01 = {}, acc10 = {}, acc11 = {};
-    const uint32_t p_end = T.base + T.n;
-    for (uint32_t p = T.base; p < p_end; ++p) {
-      const uint2 pr = pairs[p];
-      const uint64_t* A = data_a + static_cast<uint64_t>(pr.x) * kTile;
-      const uint64_t* B = data_bt + static_cast<uint64_t>(pr.y) * kTile;
-      const uint64_t ra0 = A[lo], ra1 = A[32 + lo], rb0 = B[lo], rb1 = B[32 + lo];
+    const uint32_t last = T.n - 1;
+    const uint2 mine = pairs[T.base + min(lane, last)];
+    mg_v16f acc00 = {}, acc01 = {}, acc10 = {}, acc11 = {};
+    uint32_t a0[kStep], a1[kStep], b0[kStep], b1[kStep];
+    const auto fetch = [&](uint32_t first) {
 #pragma unroll
-      for (uint32_t st = 0; st < 2; ++st) {
-        const uint32_t k = 32 * st + 16 * hi;
-        const mg_v4i a0 = bits16_to_bytes(static_cast<uint32_t>(ra0 >> k));
-        const mg_v4i a1 = bits16_to_bytes(static_cast<uint32_t>(ra1 >> k));
-        const mg_v4i b0 = bits16_to_bytes(static_cast<uint32_t>(rb0 >> k));
-        const mg_v4i b1 = bits16_to_bytes(static_cast<uint32_t>(rb1 >> k));
-        acc00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, acc00, 0, 0, 0);
-        acc01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b1, acc01, 0, 0, 0);
-        acc10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b0, acc10, 0, 0, 0);
-        acc11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, acc11, 0, 0, 0);
+      for (uint32_t i = 0; i < kStep; ++i) {
+        const int at = static_cast<int>(min(first + i, last));
+        const uint32_t* const A = half_a + static_cast<uint64_t>(lane_u32(mine.x, at)) * (2 * kTile);
+        const uint32_t* const B = half_b + static_cast<uint64_t>(lane_u32(mine.y, at)) * (2 * kTile);
+        a0[i] = A[0];
+        a1[i] = A[kTile];
+        b0[i] = B[0];
+        b1[i] = B[kTile];
+      }
+    };
+    fetch(0);
+    for (uint32_t p = 0; p < T.n; p += kStep) {
+      mg_v8i fa0[kStep], fa1[kStep], fb0[kStep], fb1[kStep];
+#pragma unroll
+      for (uint32_t i = 0; i < kStep; ++i) {
+        fa0[i] = bits_to_fp4(a0[i]);
+        fa1[i] = bits_to_fp4(a1[i]);
+        fb0[i] = bits_to_fp4(b0[i]);
+        fb1[i] = bits_to_fp4(b1[i]);
+      }
+      if (p + kStep < T.n) fetch(p + kStep);
+#pragma unroll
+      for (uint32_t i = 0; i < kStep; ++i) {
+        acc00 = mfma_fp4(fa0[i], fb0[i], acc00);
+        acc01 = mfma_fp4(fa0[i], fb1[i], acc01);
+        acc10 = mfma_fp4(fa1[i], fb0[i], acc10);
+        acc11 = mfma_fp4(fa1[i], fb1[i], acc11);
       }
     }
     uint64_t out = 0;  // output row `lane`

@@ -147,3 +147,26 @@ def test_community_square_on_matrix_cores_matches_oracle(ctx, min_bits):
         assert 0 < dense < st["tile_products"]
     else:
         assert dense == 0
+
+
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("pairs", [1, 2, 3, 63, 64, 65, 129])
+def test_contraction_of_any_number_of_pairs(ctx, pairs, full):
+    """C tiles with one, a few, a whole task's and more dense pairs: sparse tiles, whose every bit
+    decides a bit of C, and full ones, which give the largest sums."""
+    M = mg()
+    rng = np.random.default_rng(pairs)
+    n = 64 * max(2, pairs)
+    A = np.zeros((n, n), np.uint8)
+    B = np.zeros((n, n), np.uint8)
+    k = 64 * pairs
+    A[:64, :k] = 1 if full else rng.random((64, k)) < 0.01 + 0.2 / k
+    B[:k, :128] = 1 if full else rng.random((k, 128)) < 0.01 + 0.2 / k
+    a = M.TiledMatrix.upload(ctx, M.HostTiledMatrix.from_dense(A))
+    bt = M.TiledMatrix.upload(ctx, M.HostTiledMatrix.from_dense(B.T.copy()))
+    c, st = M.multiply_symbolic(ctx, a, bt)
+    assert M.multiply_numeric_dense(ctx, a, bt, c, 0) == st["tile_products"]
+    want = (A[:64].astype(np.int32) @ B[:, :128].astype(np.int32)) > 0
+    got = c.download().to_dense(n)
+    assert np.array_equal(got[:64, :128].astype(bool), want)
+    assert not got[64:].any() and not got[:, 128:].any()
