@@ -490,15 +490,22 @@ struct WaveQueues {
   uint8_t pair_s[kQueue], item_s[kQueue];   // strip of the window
 };
 
-// A dense pair of C tile `c`, to be multiplied on the matrix cores.
+// A dense pair of C tile `c`, to be multiplied on the matrix cores: the rank-th that was found there.
 struct HeavyPair {
-  uint32_t c, a, b;
+  uint32_t c, rank, a, b;
 };
+// The record has kHeavyParts parts of `part` places, each with a counter on a cache line of its own:
+// additions to one address come 12 ns apart, and recording 16.8 M pairs took 3.3 ms on one counter, now
+// 0.18. A wave that finds its part full goes on with the next; the parts together have room for all.
+// The rank, taken in LDS, gives heavy_scatter_kernel the pair's place (0.10 ms; 1.15 with a cursor
+// in memory for each C tile).
+constexpr uint32_t kHeavyParts = 64;
+constexpr uint32_t kPartStride = 16;  // u64 counters
 struct HeavyRecord {
   HeavyPair* pairs;
-  uint32_t* count;               // per C tile
-  unsigned long long* counter;   // pairs recorded
-  uint64_t cap;
+  uint32_t* count;              // per C tile
+  unsigned long long* counter;  // places taken of each part, or more
+  uint32_t part;
   uint32_t min_bits;
 };
 
@@ -532,11 +539,13 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
   __shared__ unsigned long long by_row[kWindow * kTile], by_col[kWindow * kTile];
   __shared__ WaveQueues s_queues[kProductWaves];
   __shared__ uint32_t s_used;
+  __shared__ uint32_t s_heavy[kHeavy ? kWindow : 1];  // dense pairs of each strip's tile
   __shared__ unsigned long long s_slot;
   const uint32_t lane = lane_id();
   const uint32_t wave = read_first_lane(threadIdx.x / kWave);
   constexpr uint32_t n_waves = kProductWaves;
   WaveQueues& q = s_queues[wave];
+  uint32_t heavy_part = (blockIdx.x * kProductWaves + wave) % kHeavyParts;
   const uint32_t n_items = *n_windows;
   for (uint32_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const Window win = windows[item];
@@ -553,6 +562,9 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
     }
     const auto c_tile = [&](uint32_t s) { return win.first + static_cast<uint32_t>(__popc(present & ((1u << s) - 1))); };
     for (uint32_t i = threadIdx.x; i < kWindow * kTile; i += kProductWaves * kWave) by_row[i] = by_col[i] = 0;
+    if constexpr (kHeavy) {
+      if (threadIdx.x < kWindow) s_heavy[threadIdx.x] = 0;
+    }
     __syncthreads();
 
     uint32_t n_pairs = 0, n_queued = 0;  // queued (wave-uniform)
@@ -604,13 +616,19 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
         const bool h = has && ha.bits >= heavy.min_bits && hb.bits >= heavy.min_bits;
         const uint64_t hm = ballot(h);
         if (hm) {
-          unsigned long long base = 0;
-          if (lane == 0) base = atomicAdd(heavy.counter, static_cast<unsigned long long>(__popcll(hm)));
-          base = read_first_lane64(base) + lanes_under(hm);
-          if (h && base < heavy.cap) {
-            const uint32_t c = c_tile(s);
-            heavy.pairs[base] = HeavyPair{c, ia, B.tile ? B.tile[pb] : pb};
-            atomicAdd(heavy.count + c, 1u);
+          const uint32_t rank = h ? atomicAdd(&s_heavy[s], 1u) : 0u;
+          const uint32_t order = lanes_under(hm), n = static_cast<uint32_t>(__popcll(hm));
+          uint32_t done = 0;
+          for (uint32_t tries = 0; done < n && tries < kHeavyParts; ++tries) {
+            unsigned long long at = 0;
+            if (lane == 0) at = atomicAdd(heavy.counter + heavy_part * kPartStride, static_cast<unsigned long long>(n - done));
+            at = read_first_lane64(at);
+            const uint32_t room = at < heavy.part ? min(n - done, heavy.part - static_cast<uint32_t>(at)) : 0u;
+            if (h && order >= done && order - done < room)
+              heavy.pairs[static_cast<uint64_t>(heavy_part) * heavy.part + at + (order - done)] =
+                  HeavyPair{c_tile(s), rank, ia, B.tile ? B.tile[pb] : pb};
+            done += room;
+            if (done < n) heavy_part = (heavy_part + 1) % kHeavyParts;
           }
           if (h) common = 0;
         }
@@ -747,6 +765,9 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
     multiply(n_queued);
     multiply(0);
     __syncthreads();
+    if constexpr (kHeavy) {
+      if (threadIdx.x < kWindow && (present >> threadIdx.x) & 1) heavy.count[c_tile(threadIdx.x)] = s_heavy[threadIdx.x];
+    }
     // Write-out: one C tile per wave at a time.
     if constexpr (kOut == kOutAppend) {
       // The window's non-empty tiles take their slots together: one counter for all of C.
@@ -800,15 +821,19 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
   }
 }
 
-// Heavy pairs to their C tile's place, and the C tiles' tasks of up to kTaskPairs pairs.
+// Heavy pairs to their C tile's place (grid: x over a part of the record, y = the part), and the C
+// tiles' tasks of up to kTaskPairs pairs.
 constexpr uint32_t kTaskPairs = 64;
-__global__ void __launch_bounds__(kBlock) heavy_scatter_kernel(const HeavyPair* __restrict__ in, uint32_t n,
-                                                               const uint32_t* __restrict__ base,
-                                                               uint32_t* __restrict__ cursor,
+__global__ void __launch_bounds__(kBlock) heavy_scatter_kernel(const HeavyPair* __restrict__ in,
+                                                               const unsigned long long* __restrict__ counter,
+                                                               uint32_t part, const uint32_t* __restrict__ base,
                                                                uint2* __restrict__ pairs) {
+  const unsigned long long taken = counter[blockIdx.y * kPartStride];
+  const uint32_t n = taken < part ? static_cast<uint32_t>(taken) : part;
+  in += static_cast<uint64_t>(blockIdx.y) * part;
   for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += static_cast<uint64_t>(gridDim.x) * kBlock) {
     const HeavyPair p = in[i];
-    pairs[base[p.c] + atomicAdd(cursor + p.c, 1u)] = uint2{p.a, p.b};
+    pairs[base[p.c] + p.rank] = uint2{p.a, p.b};
   }
 }
 
@@ -1225,28 +1250,29 @@ uint64_t run_product_dense(mg_context* ctx, const mg_tiled_matrix* a, const mg_t
     MG_HIP(hipStreamSynchronize(st));
     return 0;
   }
-  StreamBuf<HeavyPair> found(most, st);
-  StreamBuf<unsigned long long> n_found(1 + P.c.n_c, st);  // then the C tiles' counts and cursors (u32)
-  uint32_t* const count = reinterpret_cast<uint32_t*>(n_found.get() + 1);
-  uint32_t* const cursor = count + P.c.n_c;
-  clear_words_kernel<<<grid_for(n_found.size(), kBlock, 4096), kBlock, 0, st>>>(
-      reinterpret_cast<uint64_t*>(n_found.get()), n_found.size());
+  const uint32_t part = static_cast<uint32_t>((most + kHeavyParts - 1) / kHeavyParts);
+  StreamBuf<HeavyPair> found(static_cast<uint64_t>(part) * kHeavyParts, st);
+  constexpr uint32_t kCounters = kHeavyParts * kPartStride;
+  StreamBuf<unsigned long long> taken(kCounters + (P.c.n_c + 1ull) / 2, st);  // then the C tiles' counts (u32)
+  uint32_t* const count = reinterpret_cast<uint32_t*>(taken.get() + kCounters);
+  clear_words_kernel<<<grid_for(taken.size(), kBlock, 4096), kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(taken.get()),
+                                                                              taken.size());
   MG_LAUNCH_CHECK();
-  launch_product<true, kOutStruct>(ctx, P, out, HeavyRecord{found.get(), count, n_found.get(), most, min_bits});
+  launch_product<true, kOutStruct>(ctx, P, out, HeavyRecord{found.get(), count, taken.get(), part, min_bits});
   StreamBuf<uint32_t> base(P.c.n_c + 1ull, st);
   exclusive_scan_u32(ctx, count, base.get(), P.c.n_c);
-  unsigned long long n = 0;
-  read_words(ctx, {n_found.get(), &n, sizeof(n)});
+  uint32_t n = 0;
+  read_words(ctx, {base.get() + P.c.n_c, &n, sizeof(n)});
   MG_REQUIRE(n <= most, "mg_multiply_numeric_dense: more dense pairs recorded than counted");
   if (!n) return 0;
   StreamBuf<uint2> pairs(n, st);
-  const uint64_t max_tasks = std::min<uint64_t>(n, P.c.n_c + n / kTaskPairs);
+  const uint64_t max_tasks = std::min<uint64_t>(n, static_cast<uint64_t>(P.c.n_c) + n / kTaskPairs);
   StreamBuf<DenseTask> tasks(max_tasks, st);
   StreamBuf<uint32_t> n_tasks(2, st);
   clear_words_kernel<<<1, kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(n_tasks.get()), 1);
   MG_LAUNCH_CHECK();
-  heavy_scatter_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, st>>>(found.get(), static_cast<uint32_t>(n), base.get(),
-                                                                    cursor, pairs.get());
+  heavy_scatter_kernel<<<dim3(static_cast<uint32_t>(grid_for(part, kBlock, 64)), kHeavyParts), kBlock, 0, st>>>(
+      found.get(), taken.get(), part, base.get(), pairs.get());
   MG_LAUNCH_CHECK();
   heavy_tasks_kernel<<<grid_for(P.c.n_c, kBlock, 4096), kBlock, 0, st>>>(base.get(), P.c.n_c, tasks.get(), n_tasks.get());
   MG_LAUNCH_CHECK();
