@@ -821,9 +821,7 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
   }
 }
 
-// Heavy pairs to their C tile's place (grid: x over a part of the record, y = the part), and the C
-// tiles' tasks of up to kTaskPairs pairs.
-constexpr uint32_t kTaskPairs = 64;
+// Heavy pairs to their C tile's place (grid: x over a part of the record, y = the part).
 __global__ void __launch_bounds__(kBlock) heavy_scatter_kernel(const HeavyPair* __restrict__ in,
                                                                const unsigned long long* __restrict__ counter,
                                                                uint32_t part, const uint32_t* __restrict__ base,
@@ -863,11 +861,19 @@ __device__ inline mg_v8i bits_to_fp4(uint32_t x) {
   out[3] = static_cast<int>((x >> 1) & 0x44444444u);
   return out;
 }
+// From row `lane` of a tile: rows lane % 32 and 32 + lane % 32, half lane / 32 (lanes 32 to 63 of the
+// low halves change places with lanes 0 to 31 of the high ones).
+__device__ inline void split_rows(uint64_t row, uint32_t& first, uint32_t& second) {
+  const auto r = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(row), static_cast<uint32_t>(row >> 32), false, false);
+  first = r[0];
+  second = r[1];
+}
 __device__ inline mg_v16f mfma_fp4(mg_v8i a, mg_v8i b, mg_v16f c) {
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, kFp4, kFp4, 0, kOne, 0, kOne);
 }
 
 // Up to kTaskPairs of a C tile's dense pairs.
+constexpr uint32_t kTaskPairs = 64;
 struct DenseTask {
   uint32_t tile, base, n;
 };
@@ -875,10 +881,11 @@ struct DenseTask {
 // matrix cores, then one threshold; the rows are ORed into C atomically (several tasks may share a
 // C tile). The pairs are read once, one per lane, and kStep pairs' operands are loaded before the
 // step in front of them is multiplied; a last step that is not full takes the last pair twice.
-// 16.8 M pairs, 64 to a C tile: 2.4 ms (3.6e15 operations a second), 5.9 with operands in bytes,
-// whose expansion alone was 124 vector instructions a pair; now 24, and the matrix instructions
-// (0.9 ms) wait for the tiles, 1 KiB a pair from L2. Four waves a SIMD: left to itself the compiler
-// takes 204 registers, enough for two.
+// 16.8 M pairs, 64 to a C tile: 1.9 ms (4.6e15 operations a second; the matrix instructions alone 0.9),
+// 5.9 with operands in bytes, whose expansion was 124 vector instructions a pair, now 26. One 512-byte
+// load a tile and a swap of halves: 2.3 ms with two 256-byte loads of every second word. Neighbours
+// in C's order kept to one XCD: no difference. Four waves a SIMD: left to itself the compiler takes
+// 204 registers, enough for two.
 constexpr uint32_t kStep = 2;
 static_assert(kTaskPairs <= kWave);
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) dense_contract_kernel(const DenseTask* __restrict__ tasks,
@@ -888,9 +895,6 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
                                                                 const uint64_t* __restrict__ data_bt,
                                                                 uint64_t* __restrict__ data_c) {
   const uint32_t lane = lane_id();
-  const uint32_t lo = lane & 31, hi = lane >> 5;
-  const uint32_t* const half_a = reinterpret_cast<const uint32_t*>(data_a) + 2 * lo + hi;
-  const uint32_t* const half_b = reinterpret_cast<const uint32_t*>(data_bt) + 2 * lo + hi;
   const uint32_t n_tasks = *n_tasks_ptr;
   const uint32_t n_waves = gridDim.x * kWavesPerBlock;
   for (uint32_t t = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); t < n_tasks; t += n_waves) {
@@ -898,17 +902,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
     const uint32_t last = T.n - 1;
     const uint2 mine = pairs[T.base + min(lane, last)];
     mg_v16f acc00 = {}, acc01 = {}, acc10 = {}, acc11 = {};
-    uint32_t a0[kStep], a1[kStep], b0[kStep], b1[kStep];
+    uint64_t ra[kStep], rb[kStep];  // row `lane` of both tiles
     const auto fetch = [&](uint32_t first) {
 #pragma unroll
       for (uint32_t i = 0; i < kStep; ++i) {
         const int at = static_cast<int>(min(first + i, last));
-        const uint32_t* const A = half_a + static_cast<uint64_t>(lane_u32(mine.x, at)) * (2 * kTile);
-        const uint32_t* const B = half_b + static_cast<uint64_t>(lane_u32(mine.y, at)) * (2 * kTile);
-        a0[i] = A[0];
-        a1[i] = A[kTile];
-        b0[i] = B[0];
-        b1[i] = B[kTile];
+        ra[i] = data_a[static_cast<uint64_t>(lane_u32(mine.x, at)) * kTile + lane];
+        rb[i] = data_bt[static_cast<uint64_t>(lane_u32(mine.y, at)) * kTile + lane];
       }
     };
     fetch(0);
@@ -916,10 +916,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
       mg_v8i fa0[kStep], fa1[kStep], fb0[kStep], fb1[kStep];
 #pragma unroll
       for (uint32_t i = 0; i < kStep; ++i) {
-        fa0[i] = bits_to_fp4(a0[i]);
-        fa1[i] = bits_to_fp4(a1[i]);
-        fb0[i] = bits_to_fp4(b0[i]);
-        fb1[i] = bits_to_fp4(b1[i]);
+        uint32_t a0, a1, b0, b1;
+        split_rows(ra[i], a0, a1);
+        split_rows(rb[i], b0, b1);
+        fa0[i] = bits_to_fp4(a0);
+        fa1[i] = bits_to_fp4(a1);
+        fb0[i] = bits_to_fp4(b0);
+        fb1[i] = bits_to_fp4(b1);
       }
       if (p + kStep < T.n) fetch(p + kStep);
 #pragma unroll
@@ -947,15 +950,24 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
 }
 
 
+// The tasks of kBlock C tiles at a time take their places together (an addition for each wave's tiles
+// took 50 us for 262 K tiles).
 __global__ void __launch_bounds__(kBlock) heavy_tasks_kernel(const uint32_t* __restrict__ base, uint32_t n_c,
                                                              DenseTask* __restrict__ tasks,
                                                              uint32_t* __restrict__ n_tasks) {
-  for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < n_c; i += static_cast<uint64_t>(gridDim.x) * kBlock) {
-    const uint32_t p0 = base[i], p1 = base[i + 1];
-    if (p0 == p1) continue;
-    uint32_t to = atomicAdd(n_tasks, (p1 - p0 + kTaskPairs - 1) / kTaskPairs);
-    for (uint32_t p = p0; p < p1; p += kTaskPairs)
-      tasks[to++] = DenseTask{static_cast<uint32_t>(i), p, min(kTaskPairs, p1 - p)};
+  __shared__ uint32_t s_n, s_at;
+  for (uint64_t first = static_cast<uint64_t>(blockIdx.x) * kBlock; first < n_c;
+       first += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const uint64_t i = first + threadIdx.x;
+    uint32_t p = i < n_c ? base[i] : 0u;
+    const uint32_t end = i < n_c ? base[i + 1] : 0u;
+    uint32_t to = p < end ? atomicAdd(&s_n, (end - p + kTaskPairs - 1) / kTaskPairs) : 0u;
+    __syncthreads();
+    if (threadIdx.x == 0) s_at = s_n ? atomicAdd(n_tasks, s_n) : 0u;
+    __syncthreads();
+    for (to += s_at; p < end; p += kTaskPairs) tasks[to++] = DenseTask{static_cast<uint32_t>(i), p, min(kTaskPairs, end - p)};
   }
 }
 
