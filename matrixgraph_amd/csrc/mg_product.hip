@@ -1259,7 +1259,6 @@ uint64_t run_product_dense(mg_context* ctx, const mg_tiled_matrix* a, const mg_t
   if (!P.c.n_c) return 0;
   if (!most) {
     launch_product<false, kOutStruct>(ctx, P, out, HeavyRecord{});
-    MG_HIP(hipStreamSynchronize(st));
     return 0;
   }
   const uint32_t part = static_cast<uint32_t>((most + kHeavyParts - 1) / kHeavyParts);

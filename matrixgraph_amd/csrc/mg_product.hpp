@@ -120,7 +120,8 @@ struct ProductOut {
 
 void run_product(mg_context* ctx, const ProductInputs& P, int out_mode, const ProductOut& out);
 // kOutStruct with the pairs of tiles that both hold at least min_bits set bits on the matrix cores;
-// returns their number (synchronises). P needs TileHead::bits.
+// returns their number. It waits for the count; the contraction may still run when it returns. P needs
+// TileHead::bits.
 uint64_t run_product_dense(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt,
                            const ProductInputs& P, uint32_t min_bits, uint64_t* data_c);
 // Set bits of every row t of B into out[t] (P needs TileHead::bits).

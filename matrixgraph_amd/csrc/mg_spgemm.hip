@@ -1190,6 +1190,8 @@ extern "C" int mg_multiply_numeric_dense(mg_context* ctx, const mg_tiled_matrix*
     ProductInputs in;
     product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, true, true, in);
     const uint64_t recorded = run_product_dense(ctx, a, bt, in, min_bits, c->data.get());
+    // The caller may read C, or write A, from any stream once this returns.
+    MG_HIP(hipStreamSynchronize(ctx->stream));
     if (dense_products) *dense_products = recorded;
   });
 }

@@ -1,6 +1,8 @@
 """Matrix-core (int8 MFMA) tile products for dense tile pairs: bit-exact against the vector
 path and the dense oracle across densities, and the density-mixed walk computed by tile
 products (per-pair engine choice) equal to the gather walk."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -170,3 +172,21 @@ def test_contraction_of_any_number_of_pairs(ctx, pairs, full):
     got = c.download().to_dense(n)
     assert np.array_equal(got[:64, :128].astype(bool), want)
     assert not got[64:].any() and not got[:, 128:].any()
+
+
+@pytest.mark.parametrize("min_bits", [1, 4097])
+def test_dense_product_is_finished_when_the_call_returns(ctx, min_bits):
+    """256 x 256 full tiles, 16.8 M tile pairs, on the matrix cores or none of them: nothing is left
+    on the context's stream when mg_multiply_numeric_dense returns, so that the caller may read C, or
+    overwrite A, from another stream."""
+    M = mg()
+    query = M.lib().hipStreamQuery  # of the runtime that the library runs on
+    ns = 256
+    m = M.HostTiledMatrix(ns, np.arange(ns + 1, dtype=np.uint32) * ns, np.repeat(np.arange(ns, dtype=np.uint32), ns),
+                          np.tile(np.arange(ns, dtype=np.uint32), ns), np.full((ns * ns, 64), ~np.uint64(0)))
+    a = M.TiledMatrix.upload(ctx, m)
+    c, st = M.multiply_symbolic(ctx, a, a)
+    dense = M.multiply_numeric_dense(ctx, a, a, c, min_bits)
+    assert query(C.c_void_p(ctx.stream)) == 0  # hipSuccess: nothing is queued or running
+    assert dense == (st["tile_products"] if min_bits == 1 else 0)
+    assert c.popcount() == 4096 * ns * ns
