@@ -1,10 +1,7 @@
 // Context lifecycle, error reporting and host-only helpers of the C-ABI.
 #include <cstdlib>
 #include <cstring>
-#include <map>
-#include <mutex>
 #include <string>
-#include <unordered_map>
 #include <unordered_set>
 
 #include "mg_device.hpp"
@@ -19,174 +16,46 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 // --- kept device memory ------------------------------------------------------------
 namespace {
 
-struct Kept {
-  void* ptr;
-  uint64_t age;
-};
-// Blocks of one device.
-struct DeviceCache {
-  int contexts = 0;
-  size_t limit = 0;  // bytes kept at most
-  size_t bytes = 0;  // kept now
-  uint64_t next_age = 0;
-  std::multimap<size_t, Kept> kept;  // by size
-};
-struct Live {
-  size_t bytes;
-  int device;
-};
-struct Cache {
-  std::mutex mu;
-  std::unordered_map<void*, Live> live;  // blocks handed out
-  std::unordered_map<int, DeviceCache> devices;
+struct HipDriver {
+  using Status = hipError_t;
+  static constexpr hipError_t kOk = hipSuccess, kOutOfMemory = hipErrorOutOfMemory, kInvalid = hipErrorInvalidValue;
+  // Failures are the caller's to report: none is left for the next hipGetLastError.
+  static hipError_t seen(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+  }
+  static hipError_t malloc(void** p, size_t bytes) { return seen(hipMalloc(p, bytes)); }
+  static hipError_t free(void* p) { return seen(hipFree(p)); }
+  static hipError_t current_device(int* device) { return seen(hipGetDevice(device)); }
+  // hipFree of a fresh block: waits for all work on the current device under hipFree's own rules (a
+  // hipDeviceSynchronize would also break captures that hipFree leaves alone).
+  static bool wait() {
+    void* p = nullptr;
+    return malloc(&p, 256) == hipSuccess && free(p) == hipSuccess;
+  }
+  static void trim(int device) {
+    hipMemPool_t pool = nullptr;
+    if (seen(hipDeviceGetDefaultMemPool(&pool, device)) == hipSuccess) (void)seen(hipMemPoolTrimTo(pool, 0));
+  }
 };
 // Never destroyed: objects may outlive static destruction, and the driver reclaims the memory.
-Cache& cache() {
-  static Cache* const c = new Cache();
+BlockCache<HipDriver>& cache() {
+  static BlockCache<HipDriver>* const c = new BlockCache<HipDriver>();
   return *c;
-}
-
-thread_local int g_free_depth = 0;       // FreeScopes of this thread
-thread_local bool g_free_waited = false;  // the outermost scope has waited already
-
-// hipFree of a fresh block: waits for all work on the current device under hipFree's own rules (a
-// hipDeviceSynchronize would also break captures that hipFree leaves alone).
-bool wait_as_free() {
-  void* p = nullptr;
-  if (hipMalloc(&p, 256) != hipSuccess || hipFree(p) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return true;
-}
-
-void flush_device(int device) noexcept {
-  std::multimap<size_t, Kept> out;
-  {
-    std::lock_guard<std::mutex> lock(cache().mu);
-    auto it = cache().devices.find(device);
-    if (it == cache().devices.end()) return;
-    out.swap(it->second.kept);
-    it->second.bytes = 0;
-  }
-  for (auto& b : out) (void)hipFree(b.second.ptr);
 }
 
 }  // namespace
 
-FreeScope::FreeScope() {
-  if (g_free_depth++ == 0) g_free_waited = false;
-}
-FreeScope::~FreeScope() { --g_free_depth; }
-
-void cache_add_context(int device, size_t device_bytes) {
-  std::lock_guard<std::mutex> lock(cache().mu);
-  DeviceCache& d = cache().devices[device];
-  ++d.contexts;
-  d.limit = device_bytes / 64;
-}
-
-void cache_drop_context(int device) noexcept {
-  bool last = false;
-  {
-    std::lock_guard<std::mutex> lock(cache().mu);
-    last = --cache().devices[device].contexts == 0;
-  }
-  if (!last) return;
-  flush_device(device);
-  hipMemPool_t pool = nullptr;  // and the temporaries' pool (StreamBuf)
-  if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
-  (void)hipGetLastError();
-}
+void cache_add_context(int device, size_t device_bytes) { cache().add_context(device, device_bytes); }
+void cache_drop_context(int device) noexcept { cache().drop_context(device); }
 
 void* cached_alloc(size_t bytes) {
-  bytes = (bytes + 511) / 512 * 512;
-  int device = 0;
-  MG_HIP(hipGetDevice(&device));
-  {
-    std::lock_guard<std::mutex> lock(cache().mu);
-    DeviceCache& d = cache().devices[device];
-    auto it = d.kept.lower_bound(bytes);
-    if (it != d.kept.end() && it->first <= bytes + bytes / 8) {
-      void* const p = it->second.ptr;
-      cache().live[p] = Live{it->first, device};
-      d.bytes -= it->first;
-      d.kept.erase(it);
-      return p;
-    }
-  }
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    flush_device(device);
-    e = hipMalloc(&p, bytes);
-  }
-  MG_HIP(e);
-  try {
-    std::lock_guard<std::mutex> lock(cache().mu);
-    cache().live[p] = Live{bytes, device};
-  } catch (...) {
-    (void)hipFree(p);
-    throw;
-  }
+  MG_HIP(cache().alloc(bytes, &p));
   return p;
 }
 
-void cached_free(void* p) noexcept {
-  if (!p) return;
-  Live l{0, -1};
-  bool keep = false;
-  {
-    std::lock_guard<std::mutex> lock(cache().mu);
-    auto it = cache().live.find(p);
-    if (it != cache().live.end()) {
-      l = it->second;
-      cache().live.erase(it);
-      auto d = cache().devices.find(l.device);
-      keep = d != cache().devices.end() && d->second.contexts > 0 && l.bytes <= d->second.limit / 2;
-    }
-  }
-  int current = -1;
-  if (keep && (hipGetDevice(&current) != hipSuccess || current != l.device)) keep = false;
-  if (keep && !(g_free_depth > 0 && g_free_waited)) {
-    keep = wait_as_free();
-    if (keep && g_free_depth > 0) g_free_waited = true;
-  }
-  if (keep) {
-    try {
-      std::lock_guard<std::mutex> lock(cache().mu);
-      DeviceCache& d = cache().devices[l.device];
-      keep = d.contexts > 0;  // the last context may have gone since
-      if (keep) {
-        d.kept.emplace(l.bytes, Kept{p, d.next_age++});
-        d.bytes += l.bytes;
-      }
-    } catch (...) {
-      keep = false;
-    }
-  }
-  if (!keep) {
-    (void)hipFree(p);
-    return;
-  }
-  // Over the limit: the oldest blocks go back to the driver.
-  for (;;) {
-    void* old = nullptr;
-    {
-      std::lock_guard<std::mutex> lock(cache().mu);
-      DeviceCache& d = cache().devices[l.device];
-      if (d.bytes <= d.limit || d.kept.empty()) return;
-      auto oldest = d.kept.begin();
-      for (auto it = d.kept.begin(); it != d.kept.end(); ++it)
-        if (it->second.age < oldest->second.age) oldest = it;
-      old = oldest->second.ptr;
-      d.bytes -= oldest->first;
-      d.kept.erase(oldest);
-    }
-    (void)hipFree(old);
-  }
-}
+hipError_t cached_free(void* p) noexcept { return cache().free(p); }
 
 }  // namespace mgamd
 
@@ -328,7 +197,7 @@ extern "C" int mg_buffer_alloc(mg_context* ctx, size_t bytes, void** dptr) {
     hipError_t e = hipMemsetAsync(p, 0, bytes ? bytes : 1, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
-      cached_free(p);
+      (void)cached_free(p);
       MG_HIP(e);
     }
     *dptr = p;
@@ -341,7 +210,7 @@ extern "C" int mg_buffer_free(mg_context* ctx, void* dptr) {
     if (!dptr) return;
     DeviceGuard g(ctx->device);
     MG_HIP(hipStreamSynchronize(ctx->stream));
-    cached_free(dptr);
+    MG_HIP(cached_free(dptr));
   });
 }
 

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "matrixgraph_amd.h"
+#include "mg_block_cache.hpp"
 
 namespace mgamd {
 
@@ -80,13 +81,9 @@ int guarded(F&& f) {
 //    does (nothing is kept).
 // ---------------------------------------------------------------------------
 void* cached_alloc(size_t bytes);  // on the current device; throws Failure
-void cached_free(void* p) noexcept;
-struct FreeScope {
-  FreeScope();
-  ~FreeScope();
-  FreeScope(const FreeScope&) = delete;
-  FreeScope& operator=(const FreeScope&) = delete;
-};
+// The driver's answer where the block goes back to it; hipErrorInvalidValue for a block that was freed
+// before and is kept.
+hipError_t cached_free(void* p) noexcept;
 void cache_add_context(int device, size_t device_bytes);
 void cache_drop_context(int device) noexcept;
 
@@ -112,7 +109,7 @@ class DevBuf {
     n_ = n;
   }
   void release() {
-    if (p_) cached_free(p_);
+    if (p_) (void)cached_free(p_);
     p_ = nullptr;
     n_ = 0;
   }

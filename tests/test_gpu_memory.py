@@ -76,3 +76,23 @@ def test_buffers_come_back_zeroed(ctx, size):
         b = M.DeviceBuffer.from_array(ctx, np.full(size, 7, np.uint8))
         assert (b.to_array(np.uint8) == 7).all()
         b.close()
+
+
+def test_second_free_is_refused(ctx):
+    """Freeing a buffer twice is an error, whether its block is kept (1 MiB) or went back to the driver
+    (one too large to keep), and the next buffers are memory of their own."""
+    import ctypes as C
+
+    import matrixgraph_amd as M
+
+    lib = M.lib()
+    for size in (1 << 20, 4 << 30):
+        p = C.c_void_p()
+        assert lib.mg_buffer_alloc(ctx.h, size, C.byref(p)) == 0
+        assert lib.mg_buffer_free(ctx.h, p) == 0
+        assert lib.mg_buffer_free(ctx.h, p) != 0
+    a, b = (M.DeviceBuffer.from_array(ctx, np.full(1 << 20, v, np.uint8)) for v in (1, 2))
+    assert a.ptr != b.ptr
+    assert (a.to_array(np.uint8) == 1).all() and (b.to_array(np.uint8) == 2).all()
+    a.close()
+    b.close()
