@@ -219,6 +219,8 @@ struct mg_tiled_matrix {
   mgamd::DevBuf<uint32_t> row_idx;     // n_nz_tile
   mgamd::DevBuf<uint32_t> col_idx;     // n_nz_tile
   mgamd::DevBuf<uint64_t> data;        // 64 * n_nz_tile
+  // Tile pairs that meet in the product whose symbolic pass made this matrix (0: none did).
+  uint64_t product_pairs = 0;
   // Bumped by every library call that writes this matrix's tiles (the numeric passes into C).
   uint64_t version = 0;
   // mg_tiled_matrix_prepare_operand, valid while prep_version == version: payloads (16 B a tile, the

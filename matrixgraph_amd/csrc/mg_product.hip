@@ -6,6 +6,9 @@
 // on C = A*A of R-MAT 14 (25.8 K tiles, 16 edges a vertex) the 3.7 M structural pairs have 6.0 M
 // common j in all, and 47 % of them none.
 //
+// Two kernels; by_tiles chooses. tile_product_kernel: a wave per C tile, where few pairs meet in each and
+// on grids wider than kBitmapStrips. product_kernel, the rest of this comment:
+//
 // A workgroup takes a tile row x of A and a window of up to kWindow strips of C, whose tiles it
 // keeps in LDS. The pairs come straight from the lists, A(x, t) against the B(t, y) of the window,
 // nothing is searched, and each of three stages queues in LDS for the next so that every stage runs
@@ -25,6 +28,7 @@
 // of the issue slots on the second) and by the chains of ballots and LDS writes in between: filling the
 // queue of stage 3 is half of the time, the ORs themselves nothing.
 #include <algorithm>
+#include <cmath>
 #include <string>
 
 #include "mg_device.hpp"
@@ -79,37 +83,39 @@ struct HeadJob {
   TileHead* head;          // by where(i)
   TileHead* head_by_tile;  // may be null
   uint32_t* tile;          // inverse of where (may be null)
-  uint8_t* used;           // columns in use, by tile
+  uint8_t* used;           // columns in use, by tile (may be null)
+  uint32_t words0;         // first word (tile_heads_kernel without `next`)
 };
 
 // Heads and column words of the tiles of two operands (blockIdx.y). One pass over the tiles is
 // what bounds it: a wave has kHeadLoads of them in flight and transposes each (wave_transpose); a
 // workgroup takes the place of all its non-zero words in `words` with one atomic (12 ns each on one
 // address: one per wave and round would take longer than the reads). No room left, or none
-// asked for (cap 0): kNoWords.
+// asked for (cap 0): kNoWords. next null: tile i has the 64 words from job.words0 + 64 i on.
 constexpr int kHeadLoads = 8;
 constexpr int kHeadWaves = 16;
-constexpr uint32_t kHeadTiles = kHeadWaves * kHeadLoads;  // of a workgroup's round
-__global__ void __launch_bounds__(kHeadWaves* kWave) tile_heads_kernel(HeadJob job0, HeadJob job1, bool want_bits,
+template <int kLoads, int kWaves>
+__global__ void __launch_bounds__(kWaves* kWave) tile_heads_kernel(HeadJob job0, HeadJob job1, bool want_bits,
                                                                        uint64_t* __restrict__ words, uint64_t cap,
                                                                        unsigned long long* __restrict__ next) {
-  __shared__ uint32_t s_count[kHeadWaves];
+  constexpr uint32_t kTiles = kWaves * kLoads;  // of a workgroup's round
+  __shared__ uint32_t s_count[kWaves];
   __shared__ unsigned long long s_base;
   const HeadJob& job = blockIdx.y ? job1 : job0;
   const uint32_t lane = lane_id(), wave = read_first_lane(threadIdx.x / kWave), n = job.n;
-  for (uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kHeadTiles; r0 < n;
-       r0 += static_cast<uint64_t>(gridDim.x) * kHeadTiles) {
-    const uint64_t i0 = r0 + wave * kHeadLoads;
-    uint64_t word[kHeadLoads];
+  for (uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kTiles; r0 < n;
+       r0 += static_cast<uint64_t>(gridDim.x) * kTiles) {
+    const uint64_t i0 = r0 + wave * kLoads;
+    uint64_t word[kLoads];
 #pragma unroll
-    for (int q = 0; q < kHeadLoads; ++q)
+    for (int q = 0; q < kLoads; ++q)
       word[q] = i0 + q < n ? __builtin_nontemporal_load(job.data + (i0 + q) * kTile + lane) : 0ull;
-    const bool writes = lane < kHeadLoads && i0 + lane < n;  // lane q: tile i0 + q
+    const bool writes = lane < kLoads && i0 + lane < n;  // lane q: tile i0 + q
     const uint32_t at = writes ? job.where(static_cast<uint32_t>(i0) + lane) : 0u;
     uint64_t l_mask = 0;
     uint32_t l_at = 0, l_bits = 0, count = 0;
 #pragma unroll
-    for (int q = 0; q < kHeadLoads; ++q) {
+    for (int q = 0; q < kLoads; ++q) {
       word[q] = wave_transpose(word[q]);
       const uint64_t mask = ballot(word[q] != 0);
       const uint32_t bits = want_bits ? wave_sum32(static_cast<uint32_t>(__popcll(word[q]))) : 0u;
@@ -122,11 +128,15 @@ __global__ void __launch_bounds__(kHeadWaves* kWave) tile_heads_kernel(HeadJob j
     }
     bool fits = false;
     uint64_t base = 0;
-    if (cap) {
+    if (!next) {
+      fits = true;
+      base = job.words0 + i0 * kTile;
+      l_at = lane * kTile;
+    } else if (cap) {
       if (lane == 0) s_count[wave] = count;
       __syncthreads();
       uint32_t before = 0, total = 0;
-      for (uint32_t w = 0; w < kHeadWaves; ++w) {
+      for (uint32_t w = 0; w < kWaves; ++w) {
         const uint32_t c = s_count[w];
         if (w < wave) before += c;
         total += c;
@@ -140,10 +150,10 @@ __global__ void __launch_bounds__(kHeadWaves* kWave) tile_heads_kernel(HeadJob j
     if (fits) {
       uint64_t to = base;
 #pragma unroll
-      for (int q = 0; q < kHeadLoads; ++q) {
+      for (int q = 0; q < kLoads; ++q) {
         const uint64_t mask = ballot(word[q] != 0);
         if (word[q]) words[to + lanes_under(mask)] = word[q];
-        to += static_cast<uint32_t>(__popcll(mask));
+        to += next ? static_cast<uint32_t>(__popcll(mask)) : kTile;
       }
     }
     if (writes) {
@@ -152,7 +162,7 @@ __global__ void __launch_bounds__(kHeadWaves* kWave) tile_heads_kernel(HeadJob j
       job.head[at] = h;
       if (job.head_by_tile) job.head_by_tile[i] = h;
       if (job.tile) job.tile[at] = static_cast<uint32_t>(i);
-      job.used[i] = static_cast<uint8_t>(__popcll(l_mask));
+      if (job.used) job.used[i] = static_cast<uint8_t>(__popcll(l_mask));
     }
   }
 }
@@ -518,9 +528,9 @@ __device__ inline uint32_t lower_bound(const uint32_t* __restrict__ a, uint32_t 
   return lo;
 }
 
-// The outer product rows x cols into the C tile at `by_row` / `by_col`. Each lane starts at another
-// bit: neighbours' words are often alike, and equal addresses would queue up.
-__device__ inline void or_outer(unsigned long long* by_row, unsigned long long* by_col, uint64_t rows, uint64_t cols,
+// The outer product rows x cols into the C tile at `by_row` / `by_col`; true if into by_col. Each lane
+// starts at another bit: neighbours' words are often alike, and equal addresses would queue up.
+__device__ inline bool or_outer(unsigned long long* by_row, unsigned long long* by_col, uint64_t rows, uint64_t cols,
                                 uint32_t lane) {
   const bool r = __popcll(rows) <= __popcll(cols);
   unsigned long long* const acc = r ? by_row : by_col;
@@ -529,9 +539,71 @@ __device__ inline void or_outer(unsigned long long* by_row, unsigned long long* 
   uint64_t each = (word >> lane) | (word << ((64 - lane) & 63));
   if (val)
     for (; each; each &= each - 1) atomicOr(acc + ((lowest(each) + lane) & 63), val);
+  return !r && val;
 }
 
-template <bool kHeavy, int kOut, bool kBitmap>
+// Records the pairs of the lanes of `hm` (h: this lane's).
+__device__ inline void record_heavy(const HeavyRecord& heavy, uint32_t& part, bool h, uint64_t hm, const HeavyPair& pair,
+                                    uint32_t lane) {
+  const uint32_t order = lanes_under(hm), n = static_cast<uint32_t>(__popcll(hm));
+  uint32_t done = 0;
+  for (uint32_t tries = 0; done < n && tries < kHeavyParts; ++tries) {
+    unsigned long long at = 0;
+    if (lane == 0) at = atomicAdd(heavy.counter + part * kPartStride, static_cast<unsigned long long>(n - done));
+    at = read_first_lane64(at);
+    const uint32_t room = at < heavy.part ? min(n - done, heavy.part - static_cast<uint32_t>(at)) : 0u;
+    if (h && order >= done && order - done < room)
+      heavy.pairs[static_cast<uint64_t>(part) * heavy.part + at + (order - done)] = pair;
+    done += room;
+    if (done < n) part = (part + 1) % kHeavyParts;
+  }
+}
+
+// The pairs of the lanes of `wm`, which share many inner indices (or have column words that are not
+// stored), one after the other with lane = j; s: the pair's C tile in by_row / by_col. True if by_col
+// was used.
+template <int kBatch>
+__device__ inline bool or_whole_pairs(uint64_t wm, const LeftOperand& A, const RightOperand& B, const TileHead& ha,
+                                      const TileHead& hb, uint32_t ia, uint32_t pb, uint32_t s,
+                                      unsigned long long* by_row, unsigned long long* by_col, uint32_t lane) {
+  bool cols = false;
+  while (wm) {
+    uint64_t r[kBatch], c[kBatch];
+    uint32_t sp[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      r[k] = 0;
+      c[k] = 0;
+      sp[k] = 0;
+      if (wm) {
+        const int src = lowest(wm);
+        wm &= wm - 1;
+        const uint64_t ma = read_lane(ha.mask, src), mb = read_lane(hb.mask, src);
+        const uint32_t oa = lane_u32(ha.off, src), ob = lane_u32(hb.off, src);
+        sp[k] = lane_u32(s, src) * kTile;
+        const bool use = ((ma & mb) >> lane) & 1;
+        if (oa != kNoWords) {
+          if (use) r[k] = A.words[oa + lanes_under(ma)];
+        } else {
+          const uint64_t t = wave_transpose(A.data[static_cast<uint64_t>(lane_u32(ia, src)) * kTile + lane]);
+          if (use) r[k] = t;
+        }
+        if (ob != kNoWords) {
+          if (use) c[k] = B.words[ob + lanes_under(mb)];
+        } else {
+          const uint32_t p = lane_u32(pb, src);
+          const uint64_t t = wave_transpose(B.data[static_cast<uint64_t>(B.tile ? B.tile[p] : p) * kTile + lane]);
+          if (use) c[k] = t;
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) cols |= or_outer(by_row + sp[k], by_col + sp[k], r[k], c[k], lane);
+  }
+  return cols;
+}
+
+template <bool kHeavy, int kOut>
 __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTiles C, const Window* __restrict__ windows,
                                                                    const uint32_t* __restrict__ n_windows, uint32_t wpr,
                                                                    LeftOperand A, RightOperand B, ProductOut out,
@@ -617,58 +689,13 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
         const uint64_t hm = ballot(h);
         if (hm) {
           const uint32_t rank = h ? atomicAdd(&s_heavy[s], 1u) : 0u;
-          const uint32_t order = lanes_under(hm), n = static_cast<uint32_t>(__popcll(hm));
-          uint32_t done = 0;
-          for (uint32_t tries = 0; done < n && tries < kHeavyParts; ++tries) {
-            unsigned long long at = 0;
-            if (lane == 0) at = atomicAdd(heavy.counter + heavy_part * kPartStride, static_cast<unsigned long long>(n - done));
-            at = read_first_lane64(at);
-            const uint32_t room = at < heavy.part ? min(n - done, heavy.part - static_cast<uint32_t>(at)) : 0u;
-            if (h && order >= done && order - done < room)
-              heavy.pairs[static_cast<uint64_t>(heavy_part) * heavy.part + at + (order - done)] =
-                  HeavyPair{c_tile(s), rank, ia, B.tile ? B.tile[pb] : pb};
-            done += room;
-            if (done < n) heavy_part = (heavy_part + 1) % kHeavyParts;
-          }
+          record_heavy(heavy, heavy_part, h, hm, h ? HeavyPair{c_tile(s), rank, ia, B.tile ? B.tile[pb] : pb} : HeavyPair{}, lane);
           if (h) common = 0;
         }
       }
       const int n_common = __popcll(common);
       const bool whole = n_common > kFewCommon || (common && (ha.off == kNoWords || hb.off == kNoWords));
-      // Pairs with many common indices (or words that are not stored): lane = j.
-      for (uint64_t wm = ballot(whole); wm;) {
-        uint64_t r[kPairBatch], c[kPairBatch];
-        uint32_t sp[kPairBatch];
-#pragma unroll
-        for (int k = 0; k < kPairBatch; ++k) {
-          r[k] = 0;
-          c[k] = 0;
-          sp[k] = 0;
-          if (wm) {
-            const int src = lowest(wm);
-            wm &= wm - 1;
-            const uint64_t ma = read_lane(ha.mask, src), mb = read_lane(hb.mask, src);
-            const uint32_t oa = lane_u32(ha.off, src), ob = lane_u32(hb.off, src);
-            sp[k] = lane_u32(s, src) * kTile;
-            const bool use = ((ma & mb) >> lane) & 1;
-            if (oa != kNoWords) {
-              if (use) r[k] = A.words[oa + lanes_under(ma)];
-            } else {
-              const uint64_t t = wave_transpose(A.data[static_cast<uint64_t>(lane_u32(ia, src)) * kTile + lane]);
-              if (use) r[k] = t;
-            }
-            if (ob != kNoWords) {
-              if (use) c[k] = B.words[ob + lanes_under(mb)];
-            } else {
-              const uint32_t p = lane_u32(pb, src);
-              const uint64_t t = wave_transpose(B.data[static_cast<uint64_t>(B.tile ? B.tile[p] : p) * kTile + lane]);
-              if (use) c[k] = t;
-            }
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < kPairBatch; ++k) or_outer(by_row + sp[k], by_col + sp[k], r[k], c[k], lane);
-      }
+      or_whole_pairs<kPairBatch>(ballot(whole), A, B, ha, hb, ia, pb, s, by_row, by_col, lane);
       if (whole) common = 0;
       // The rest, two j per lane at a time (1.32 ms instead of 1.43: a step's ballots, branch and LDS
       // writes are one dependent chain), a 32-bit half of the masks after the other: bits of the half
@@ -700,65 +727,34 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
     };
 
     // Stage 1: the row's tiles, dealt one by one to the waves, so that short rows use them all.
-    if constexpr (kBitmap) {
-      for (uint32_t k0 = a0; k0 < a1; k0 += kWave * n_waves) {
-        const uint32_t ia = k0 + lane * n_waves + wave;
-        uint32_t bits = 0, pb = 0;  // strips of the window, and the position of the lowest
-        if (ia < a1) {
-          const uint32_t t = A.col[ia];
-          const BitmapWord w = B.bm[static_cast<uint64_t>(t) * wpr + (y0 >> 6)];
-          bits = static_cast<uint32_t>(w.bits >> (y0 & 63)) & ((1u << kWindow) - 1);
-          pb = w.at + static_cast<uint32_t>(__popcll(w.bits & ((1ull << (y0 & 63)) - 1)));
-        }
-        const uint32_t all = bits;
-        bits &= present;
-        const auto put = [&](uint32_t left, uint64_t m) {
-          if (left) {
-            const uint32_t below = (left - 1) & ~left;
-            const uint32_t to = n_pairs + lanes_under(m);
-            q.pair_a[to] = ia;
-            q.pair_b[to] = pb + static_cast<uint32_t>(__popc(all & below));
-            q.pair_s[to] = static_cast<uint8_t>(__popc(below));
-          }
-          n_pairs += static_cast<uint32_t>(__popcll(m));
-        };
-        for (uint64_t m = ballot(bits != 0); m; m = ballot(bits != 0)) {
-          const uint32_t next = bits & (bits - 1);
-          const uint64_t m_next = ballot(next != 0);
-          put(bits, m);
-          put(next, m_next);
-          bits = next & (next - 1);
-          while (n_pairs >= kWave) filter(kWave);
-        }
+    for (uint32_t k0 = a0; k0 < a1; k0 += kWave * n_waves) {
+      const uint32_t ia = k0 + lane * n_waves + wave;
+      uint32_t bits = 0, pb = 0;  // strips of the window, and the position of the lowest
+      if (ia < a1) {
+        const uint32_t t = A.col[ia];
+        const BitmapWord w = B.bm[static_cast<uint64_t>(t) * wpr + (y0 >> 6)];
+        bits = static_cast<uint32_t>(w.bits >> (y0 & 63)) & ((1u << kWindow) - 1);
+        pb = w.at + static_cast<uint32_t>(__popcll(w.bits & ((1ull << (y0 & 63)) - 1)));
       }
-    } else {
-      // Wide grid: every strip's Bt row against A's, the shorter searched in the longer.
-      for (uint32_t left = present; left; left &= left - 1) {
-        const uint32_t s = static_cast<uint32_t>(__ffs(static_cast<int>(left)) - 1);
-        const uint32_t b0 = B.bt_off[y0 + s], b1 = B.bt_off[y0 + s + 1];
-        const bool a_short = a1 - a0 <= b1 - b0;
-        const uint32_t s0 = a_short ? a0 : b0, s1 = a_short ? a1 : b1, l0 = a_short ? b0 : a0, l1 = a_short ? b1 : a1;
-        const uint32_t* const s_col = a_short ? A.col : B.bt_col;
-        const uint32_t* const l_col = a_short ? B.bt_col : A.col;
-        for (uint32_t k0 = s0; k0 < s1; k0 += kWave * n_waves) {
-          const uint32_t k = k0 + lane * n_waves + wave;
-          uint32_t at = l1;
-          bool has = k < s1;
-          if (has) {
-            const uint32_t key = s_col[k];
-            at = lower_bound(l_col, l0, l1, key);
-            has = at < l1 && l_col[at] == key;
-          }
-          const uint64_t m = ballot(has);
-          if (has) {
-            const uint32_t to = n_pairs + lanes_under(m);
-            q.pair_a[to] = a_short ? k : at;
-            q.pair_b[to] = a_short ? at : k;
-            q.pair_s[to] = static_cast<uint8_t>(s);
-          }
-          n_pairs += static_cast<uint32_t>(__popcll(m));
-          if (n_pairs >= kWave) filter(kWave);
+      const uint32_t all = bits;
+      bits &= present;
+      const auto put = [&](uint32_t left, uint64_t m) {
+        if (left) {
+          const uint32_t below = (left - 1) & ~left;
+          const uint32_t to = n_pairs + lanes_under(m);
+          q.pair_a[to] = ia;
+          q.pair_b[to] = pb + static_cast<uint32_t>(__popc(all & below));
+          q.pair_s[to] = static_cast<uint8_t>(__popc(below));
         }
+        n_pairs += static_cast<uint32_t>(__popcll(m));
+      };
+      for (uint64_t m = ballot(bits != 0); m; m = ballot(bits != 0)) {
+        const uint32_t next = bits & (bits - 1);
+        const uint64_t m_next = ballot(next != 0);
+        put(bits, m);
+        put(next, m_next);
+        bits = next & (next - 1);
+        while (n_pairs >= kWave) filter(kWave);
       }
     }
     while (n_pairs || fetched) filter(n_pairs);
@@ -818,6 +814,150 @@ __global__ void __launch_bounds__(kProductWaves* kWave) product_kernel(ProductTi
       }
     }
     __syncthreads();
+  }
+}
+
+// The product C tile by C tile, for products that by_tiles picks: a wave takes `run` neighbouring C
+// tiles, one after the other, each with 1 KiB of LDS. Lane = tile of the shorter of A's row and Bt's,
+// searched in the longer, then the same two stages as product_kernel's, without queues: few pairs meet
+// here, and what bounds it is the chain of dependent loads (rows, search, heads, words), which 32
+// waves a CU hide, not idle lanes. A window that holds a tile or two costs a workgroup, 30 KiB of LDS
+// and their clearing. Erdos-Renyi A*A with a quarter of an edge a vertex, operands prepared: 2^18
+// vertices (1.0 M C tiles) 0.255 ms, by windows 1.40; 2^20 (4.2 M) 1.21 and 7.86; 2^21 (8.3 M, too wide
+// for windows by bitmap) 2.57, by windows that search 25.9. 2^12 vertices with half an edge, 4096 C
+// tiles: 15 us and 29.
+constexpr uint32_t kTileRun = 8;
+constexpr int kTilePairBatch = 2;  // as kPairBatch; 64 registers hold no more
+template <bool kHeavy, int kOut>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) tile_product_kernel(ProductTiles C, LeftOperand A, RightOperand B,
+                                                              ProductOut out, HeavyRecord heavy, uint32_t run) {
+  __shared__ unsigned long long s_row[kWavesPerBlock][kTile], s_col[kWavesPerBlock][kTile];
+  __shared__ uint64_t s_done[kOut == kOutAppend ? kWavesPerBlock * kTileRun * kTile : 1];
+  const uint32_t lane = lane_id(), wave = read_first_lane(threadIdx.x / kWave);
+  unsigned long long* const by_row = s_row[wave];
+  unsigned long long* const by_col = s_col[wave];
+  by_row[lane] = by_col[lane] = 0;
+  wave_lds_sync();
+  const uint32_t first = blockIdx.x * kWavesPerBlock + wave;
+  uint32_t heavy_part = first % kHeavyParts;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kWavesPerBlock * run;
+  for (uint64_t i0 = static_cast<uint64_t>(first) * run; i0 < C.n_c; i0 += stride) {
+    const uint32_t n = C.n_c - i0 < run ? static_cast<uint32_t>(C.n_c - i0) : run;
+    uint32_t used = 0;  // of the run's tiles (kOutAppend)
+    // Lane q: the rows of tile i0 + q, so that a run waits for them once.
+    uint32_t ra0 = 0, ra1 = 0, rb0 = 0, rb1 = 0;
+    if (lane < n) {
+      const uint32_t x = C.row[i0 + lane], y = C.col[i0 + lane];
+      ra0 = A.off[x];
+      ra1 = A.off[x + 1];
+      rb0 = B.bt_off[y];
+      rb1 = B.bt_off[y + 1];
+    }
+    for (uint32_t q = 0; q < n; ++q) {
+      const uint32_t i = static_cast<uint32_t>(i0) + q;
+      if constexpr (kOut == kOutRest) {
+        if (!out.flag[i] || out.slot[i] < out.capacity) continue;
+      }
+      const int src = static_cast<int>(q);
+      const uint32_t a0 = lane_u32(ra0, src), a1 = lane_u32(ra1, src), b0 = lane_u32(rb0, src), b1 = lane_u32(rb1, src);
+      const bool a_short = a1 - a0 <= b1 - b0;
+      const uint32_t s0 = a_short ? a0 : b0, s1 = a_short ? a1 : b1, l0 = a_short ? b0 : a0, l1 = a_short ? b1 : a1;
+      const uint32_t* const s_idx = a_short ? A.col : B.bt_col;
+      const uint32_t* const l_idx = a_short ? B.bt_col : A.col;
+      uint32_t n_heavy = 0;
+      uint64_t some = 0;  // lanes with a common index so far
+      bool cols = false;  // this lane used by_col
+      for (uint32_t k0 = s0; k0 < s1; k0 += kWave) {
+        const uint32_t k = k0 + lane;
+        uint32_t at = l1;
+        bool has = k < s1;
+        if (has) {
+          const uint32_t key = s_idx[k];
+          at = lower_bound(l_idx, l0, l1, key);
+          has = at < l1 && l_idx[at] == key;
+        }
+        const uint32_t ia = a_short ? k : at, ib = a_short ? at : k;
+        TileHead ha{0, 0, 0}, hb{0, 0, 0};
+        if (has) {
+          ha = A.head[ia];
+          hb = B.head[ib];
+        }
+        uint64_t common = ha.mask & hb.mask;
+        if constexpr (kHeavy) {
+          const bool h = has && ha.bits >= heavy.min_bits && hb.bits >= heavy.min_bits;
+          const uint64_t hm = ballot(h);
+          if (hm) {
+            record_heavy(heavy, heavy_part, h, hm, HeavyPair{i, n_heavy + lanes_under(hm), ia, ib}, lane);
+            n_heavy += static_cast<uint32_t>(__popcll(hm));
+            if (h) common = 0;
+          }
+        }
+        some |= ballot(common != 0);
+        const bool whole = __popcll(common) > kFewCommon || (common && (ha.off == kNoWords || hb.off == kNoWords));
+        cols |= or_whole_pairs<kTilePairBatch>(ballot(whole), A, B, ha, hb, ia, ib, 0, by_row, by_col, lane);
+        if (whole) common = 0;
+        while (ballot(common != 0)) {
+          uint64_t r[2] = {0, 0}, c[2] = {0, 0};
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            if (common) {
+              const uint64_t below = (common - 1) & ~common;
+              r[u] = A.words[ha.off + static_cast<uint32_t>(__popcll(ha.mask & below))];
+              c[u] = B.words[hb.off + static_cast<uint32_t>(__popcll(hb.mask & below))];
+              common &= common - 1;
+            }
+          cols |= or_outer(by_row, by_col, r[0], c[0], lane);
+          cols |= or_outer(by_row, by_col, r[1], c[1], lane);
+        }
+      }
+      // Tiles with no common index (63 of 64 pairs of tiles with a bit each) stay out of LDS.
+      uint64_t val = 0;
+      if (some) {
+        wave_lds_sync();
+        val = by_row[lane];
+        by_row[lane] = 0;
+        if (ballot(cols)) {
+          val |= wave_transpose(by_col[lane]);
+          by_col[lane] = 0;
+        }
+        wave_lds_sync();
+      }
+      if constexpr (kHeavy) {
+        if (lane == 0) heavy.count[i] = n_heavy;
+      }
+      if constexpr (kOut == kOutStruct) {
+        if (val) atomicOr(reinterpret_cast<unsigned long long*>(out.data) + static_cast<uint64_t>(i) * kTile + lane,
+                          static_cast<unsigned long long>(val));
+      } else if constexpr (kOut == kOutAppend) {
+        s_done[(wave * kTileRun + q) * kTile + lane] = val;
+        used |= ballot(val != 0) ? 1u << q : 0u;
+      } else if constexpr (kOut == kOutRest) {
+        out.data[(out.slot[i] - out.capacity) * kTile + lane] = val;
+      } else {
+        const bool nz = ballot(val != 0) != 0;
+        if constexpr (kOut == kOutFlag) {
+          if (lane == 0) out.flag[i] = nz ? 1u : 0u;
+        } else if (nz) {
+          out.data[static_cast<uint64_t>(out.pos[i]) * kTile + lane] = val;
+        }
+      }
+    }
+    if constexpr (kOut == kOutAppend) {
+      // The run's non-empty tiles take their slots together: one counter for all of C.
+      unsigned long long slot0 = 0;
+      if (lane == 0 && used) slot0 = atomicAdd(out.counter, static_cast<unsigned long long>(__popc(used)));
+      slot0 = read_first_lane64(slot0);
+      for (uint32_t q = 0; q < n; ++q) {
+        const bool nz = (used >> q) & 1;
+        const uint64_t slot = slot0 + static_cast<uint32_t>(__popc(used & ((1u << q) - 1)));
+        if (lane == 0) {
+          out.flag[i0 + q] = nz ? 1u : 0u;
+          if (nz) out.slot[i0 + q] = static_cast<uint32_t>(slot);
+        }
+        // Each lane reads back what it wrote itself.
+        if (nz && slot < out.capacity) out.data[slot * kTile + lane] = s_done[(wave * kTileRun + q) * kTile + lane];
+      }
+    }
   }
 }
 
@@ -975,13 +1115,18 @@ template <bool kHeavy, int kOut>
 void launch_product(mg_context* ctx, const ProductInputs& P, const ProductOut& out, const HeavyRecord& heavy) {
   const ProductTiles& C = P.c;
   if (!C.n_c) return;
-  const uint32_t grid = std::min(65536u, C.n_c), wpr = (P.n_strips + 63) / 64;
-  if (P.b.bm)
-    product_kernel<kHeavy, kOut, true><<<grid, kProductWaves * kWave, 0, ctx->stream>>>(C, P.windows, P.n_windows, wpr, P.a, P.b, out,
-                                                                                    heavy);
-  else
-    product_kernel<kHeavy, kOut, false><<<grid, kProductWaves * kWave, 0, ctx->stream>>>(C, P.windows, P.n_windows, wpr, P.a, P.b, out,
-                                                                                     heavy);
+  if (P.b.bm) {
+    product_kernel<kHeavy, kOut><<<std::min(65536u, C.n_c), kProductWaves * kWave, 0, ctx->stream>>>(
+        C, P.windows, P.n_windows, (P.n_strips + 63) / 64, P.a, P.b, out, heavy);
+  } else {
+    // Runs that leave all the chip's waves work; where pairs are many they are not alike, and a run only
+    // makes the last waves longer. Appends want runs: a slot counter's atomic each.
+    const bool few = P.pairs <= (kOut == kOutAppend ? 16ull : 4ull) * C.n_c;
+    const uint32_t per_run = kOut == kOutAppend ? (few ? 4096u : 65536u) : (few ? 32768u : ~0u);
+    const uint32_t run = std::clamp(C.n_c / per_run, 1u, kTileRun);
+    tile_product_kernel<kHeavy, kOut><<<grid_for(C.n_c, kWavesPerBlock * run, 65536), kBlock, 0, ctx->stream>>>(
+        C, P.a, P.b, out, heavy, run);
+  }
   MG_LAUNCH_CHECK();
 }
 
@@ -1014,8 +1159,15 @@ void launch_heads(hipStream_t st, const HeadJob& a, const HeadJob& b, bool want_
                   unsigned long long* next) {
   const uint32_t most = std::max(a.n, b.n);
   if (!most) return;
-  tile_heads_kernel<<<dim3(grid_for(most, kHeadTiles, 4096), 2), kHeadWaves * kWave, 0, st>>>(a, b, want_bits, words, cap,
-                                                                                             next);
+  if (next) {
+    constexpr uint32_t kTiles = kHeadLoads * kHeadWaves;
+    tile_heads_kernel<kHeadLoads, kHeadWaves><<<dim3(grid_for(most, kTiles, 4096), 2), kHeadWaves * kWave, 0, st>>>(
+        a, b, want_bits, words, cap, next);
+  } else {
+    // Few tiles: a wave each, so that they spread over the chip.
+    tile_heads_kernel<1, kWavesPerBlock><<<dim3(grid_for(most, kWavesPerBlock, 8192), 2), kBlock, 0, st>>>(
+        a, b, want_bits, words, cap, nullptr);
+  }
   MG_LAUNCH_CHECK();
 }
 
@@ -1028,9 +1180,29 @@ void launch_weights(hipStream_t st, const WeightJob& a, const WeightJob& b, uint
 // Words of an operand's row weights: the rows', their total, and those of kWindow rows each.
 uint32_t weight_words(uint32_t ns) { return ns + 1 + (ns + kWindow - 1) / kWindow; }
 
+constexpr uint64_t kSpreadHeads = 65536;
 // Room for column words: every one of up to 2^20 tiles, 16 a tile beyond (and no less than that).
 uint64_t word_room(uint64_t n) {
   return std::min<uint64_t>(kNoWords - 1ull, std::min<uint64_t>(n * kTile, std::max<uint64_t>(1ull << 26, 16 * n)));
+}
+
+// Which kernel a product runs on: tile_product_kernel (true) or product_kernel by windows of C, from the
+// numbers of tiles and of the tile pairs that meet; `indexed`: B's index is there already.
+// Times in ns, fitted to products of R-MAT and Erdos-Renyi graphs of 2^8 to 2^21 vertices with 1/16 to 16
+// edges a vertex and of frontiers with them: by windows 12 us of launches (45 with B's index to build, and 3
+// passes over its bitmap) and 2.5 a window that holds a tile, by tiles 0.22 a tile, and 0.02 and
+// 0.06 a pair. Where many pairs meet in each C tile, one wave is at it for long (up to 2.6 us a pair of
+// dense tiles): windows, sooner where they cost no index.
+constexpr uint64_t kPairsPerTile = 64, kPairsPerTileIndexed = 12;
+bool by_tiles(uint32_t ns, uint64_t n_a, uint64_t n_c, uint64_t pairs, bool indexed) {
+  if (ns > kBitmapStrips) return true;
+  if (pairs > (indexed ? kPairsPerTileIndexed : kPairsPerTile) * n_c) return false;
+  const double strip_windows = static_cast<double>((ns + kWindow - 1) / kWindow);
+  const double slots = std::max(1.0, std::min<double>(ns, static_cast<double>(n_a)) * strip_windows);
+  const double windows = -slots * std::expm1(-static_cast<double>(n_c) / slots);  // tiles spread evenly
+  const double index = indexed ? 12e3 : 45e3 + 0.01 * ns * ((ns + 63) / 64);
+  return 0.22 * static_cast<double>(n_c) + 0.06 * static_cast<double>(pairs) <
+         index + 2.5 * windows + 0.02 * static_cast<double>(pairs);
 }
 
 }  // namespace
@@ -1052,7 +1224,7 @@ void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
   m->prep_weight.alloc(weight_words(ns));
   clear_u32(st, m->prep_weight.get(), weight_words(ns));
   HeadJob as_a{m->data.get(), n, {}, reinterpret_cast<TileHead*>(m->prep_head.get()), nullptr, nullptr,
-               used.get()};
+               used.get(), 0};
   HeadJob as_b{};
   if (bitmap) {
     m->prep_right_head.alloc(2ull * std::max<uint32_t>(1, n));
@@ -1083,21 +1255,24 @@ void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
 }
 
 void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const ProductTiles& c,
-                    bool want_bits, bool want_words, ProductInputs& P, const RightIndex& known) {
+                    bool want_bits, bool want_words, uint64_t pairs, ProductInputs& P, const RightIndex& known) {
   hipStream_t st = ctx->stream;
   const uint32_t ns = a->n_strips, wpr = (ns + 63) / 64;
-  const bool bitmap = ns <= kBitmapStrips;
-  const bool pa = prepared(a), pb = prepared(bt), same = a == bt && bitmap;
+  const bool pa = prepared(a), pb = prepared(bt), same = a == bt;
+  // Unknown: as many as there are where the tiles spread evenly.
+  P.pairs = pairs ? pairs : static_cast<uint64_t>(a->n_nz_tile) * bt->n_nz_tile / std::max(1u, ns);
+  const bool bitmap = !by_tiles(ns, a->n_nz_tile, c.n_c, P.pairs, pb || known.bm);
   const uint64_t na = pa ? 0 : a->n_nz_tile, nb = pb ? 0 : bt->n_nz_tile;
   const bool index_b = bitmap && !pb;
   const uint64_t bm = index_b && !known.bm ? 2ull * ns * wpr : 0;  // u64 words
-  // Cleared: counters (column words taken; windows) and the weights.
-  const uint64_t weights = pa && pb ? 0 : 2ull * weight_words(ns);
+  // Cleared: counters (column words taken; windows) and the weights. No windows or weights by tiles.
+  const uint64_t weights = !bitmap || (pa && pb) ? 0 : 2ull * weight_words(ns);
   const uint64_t clear = (2 + (weights + 1) / 2 + 1) & ~1ull;
-  const uint64_t heads_at = clear + bm, windows_at = heads_at + 2 * (na + nb), words_at = windows_at + 4ull * c.n_c;
+  const uint64_t heads_at = clear + bm, windows_at = heads_at + 2 * (na + nb), words_at = windows_at + (bitmap ? 4ull * c.n_c : 0);
   const uint64_t index32 = index_b ? 2ull * ns + 1 + nb : 0;  // row pointer, scratch, tiles by position
-  const uint64_t u32s = index32 + (na + nb + 3) / 4;          // then the tiles' columns in use (u8)
-  uint64_t room = want_words ? word_room(same && !pa ? nb : na + nb) : 0;
+  const uint64_t u32s = index32 + (bitmap ? (na + nb + 3) / 4 : 0);  // then the tiles' columns in use (u8)
+  const uint64_t n_heads = same && !pa ? nb : na + nb;
+  uint64_t room = want_words ? word_room(n_heads) : 0;
   uint64_t* base = nullptr;
   try {
     base = ctx_scratch(ctx, words_at + room + (u32s + 1) / 2);
@@ -1118,11 +1293,16 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   P.windows = reinterpret_cast<Window*>(base + windows_at);
   uint64_t* const words = base + words_at;
   uint32_t* const at32 = reinterpret_cast<uint32_t*>(words + room);
-  clear_words_kernel<<<grid_for(clear, kBlock, 4096), kBlock, 0, st>>>(base, clear);
-  MG_LAUNCH_CHECK();
+  // By tiles, few heads: 64 words a tile (32 MiB here) need no counter, so that two launches are all.
+  const bool spread = !bitmap && n_heads <= kSpreadHeads && room == n_heads * kTile;
+  if (bitmap || (n_heads && !spread)) {
+    clear_words_kernel<<<grid_for(clear, kBlock, 4096), kBlock, 0, st>>>(base, clear);
+    MG_LAUNCH_CHECK();
+  }
   uint8_t* const used = reinterpret_cast<uint8_t*>(at32 + index32);
-  HeadJob job_a{a->data.get(), static_cast<uint32_t>(na), {}, head_a, nullptr, nullptr, used};
-  HeadJob job_b{bt->data.get(), static_cast<uint32_t>(nb), {}, head_b, nullptr, nullptr, used + na};
+  HeadJob job_a{a->data.get(), static_cast<uint32_t>(na), {}, head_a, nullptr, nullptr, bitmap ? used : nullptr,
+                static_cast<uint32_t>(nb * kTile)};
+  HeadJob job_b{bt->data.get(), static_cast<uint32_t>(nb), {}, head_b, nullptr, nullptr, bitmap ? used + na : nullptr, 0};
   if (index_b) {
     P.b.bm = known.bm;
     P.b.off = known.off;
@@ -1137,11 +1317,11 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
     P.b.tile = job_b.tile;
   }
   if (same && !pa) {  // one pass makes both operands' heads
-    job_b.head_by_tile = head_a;
+    job_b.head_by_tile = bitmap ? head_a : nullptr;
     job_a.n = 0;
   }
-  launch_heads(st, job_a, job_b, want_bits, words, room, next);
-  if (c.n_c) {
+  launch_heads(st, job_a, job_b, want_bits, words, room, spread ? nullptr : next);
+  if (bitmap && c.n_c) {
     launch_weights(st, pa || same ? WeightJob{} : WeightJob{used, a->offset_row.get(), weight},
                    pb ? WeightJob{} : WeightJob{used + na, bt->offset_row.get(), weight2}, ns);
     const uint32_t* const weight_b = pb ? bt->prep_weight.get() : weight2;
@@ -1150,7 +1330,7 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
                                                                       weight_b + ns + 1, P.windows, P.n_windows);
     MG_LAUNCH_CHECK();
   }
-  P.a = {head_a, words, a->data.get(), a->offset_row.get(), a->col_idx.get()};
+  P.a = {same && !bitmap ? head_b : head_a, words, a->data.get(), a->offset_row.get(), a->col_idx.get()};
   if (pa) {
     P.a.head = reinterpret_cast<const TileHead*>(a->prep_head.get());
     P.a.words = a->prep_words.get();

@@ -31,15 +31,15 @@ struct BitmapWord {
   uint64_t bits;
   uint32_t at, pad;
 };
-// Right operand B, from Bt's tiles (y, t). Up to kBitmapStrips strips by its tile rows t: positions
-// off[t] .. off[t + 1] - 1 are the tiles B(t, y) in ascending y, found through the bitmap. Wider
-// grids: position = tile of Bt, found in Bt's own rows.
+// Right operand B, from Bt's tiles (y, t). For product_kernel by its tile rows t: positions
+// off[t] .. off[t + 1] - 1 are the tiles B(t, y) in ascending y, found through the bitmap. For
+// tile_product_kernel: position = tile of Bt, found in Bt's own rows.
 struct RightOperand {
   const TileHead* head;   // by position
   const uint64_t* words;
   const uint64_t* data;   // Bt's tiles
   const uint32_t* tile;   // position -> tile of Bt
-  const BitmapWord* bm;   // null: wide grid
+  const BitmapWord* bm;   // null: by tiles of Bt
   const uint32_t* off;
   const uint32_t* bt_off;
   const uint32_t* bt_col;
@@ -90,15 +90,17 @@ struct ProductInputs {
   ProductTiles c{};
   LeftOperand a{};
   RightOperand b{};
+  uint64_t pairs = 0;         // tile pairs that meet, or an estimate
   Window* windows = nullptr;  // *n_windows of them
   uint32_t* n_windows = nullptr;
 };
 
 // Stream-ordered, no synchronisation; no allocation if the context's scratch is large enough.
-// want_bits: TileHead::bits; want_words: false leaves the column words out (heads only). known: B's
-// index if it is made already.
+// want_bits: TileHead::bits; want_words: false leaves the column words out (heads only). pairs: the tile
+// pairs that meet, 0 if not known (only the choice of kernel depends on it). known: B's index if it is
+// made already.
 void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const ProductTiles& c,
-                    bool want_bits, bool want_words, ProductInputs& P, const RightIndex& known = {});
+                    bool want_bits, bool want_words, uint64_t pairs, ProductInputs& P, const RightIndex& known = {});
 // Operand kept with its handle (mg_tiled_matrix_prepare_operand): all but the payloads.
 bool prepared(const mg_tiled_matrix* m);
 void prepare_operand(mg_context* ctx, mg_tiled_matrix* m);

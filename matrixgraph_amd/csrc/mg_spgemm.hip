@@ -875,6 +875,7 @@ extern "C" int mg_multiply_symbolic(mg_context* ctx, const mg_tiled_matrix* a, c
     auto c = std::make_unique<mg_tiled_matrix>();
     c->device = ctx->device;
     alloc_tiled_matrix(c.get(), S.n, static_cast<uint32_t>(S.n_c));
+    c->product_pairs = S.tile_products;
     MG_HIP(hipMemcpyAsync(c->offset_row.get(), S.rows.off_c, sizeof(uint32_t) * (S.n + 1ull),
                           hipMemcpyDeviceToDevice, s));
     if (S.n_c) {
@@ -921,7 +922,7 @@ extern "C" int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, co
     ++c->version;
     if (c->n_nz_tile == 0) return;
     ProductInputs in;
-    product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, false, true, in);
+    product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, false, true, c->product_pairs, in);
     ProductOut out{};
     out.data = c->data.get();
     run_product(ctx, in, kOutStruct, out);
@@ -953,7 +954,7 @@ void pruned_prepare(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   P.slot = P.flag + n_s;
   P.pos = P.slot + n_s;
   structural_emit(ctx, a, P.S, P.row_s, P.col_s);
-  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s, P.col_s}, want_bits, true, P.in, P.S.b);
+  product_inputs(ctx, a, bt, ProductTiles{n_s, P.row_s, P.col_s}, want_bits, true, P.S.tile_products, P.in, P.S.b);
 }
 
 // Features of every C row into feat (device, n_strips x kRowFeatures).
@@ -1140,7 +1141,7 @@ extern "C" int mg_multiply_row_features(mg_context* ctx, const mg_tiled_matrix* 
     const uint32_t n = S.n;
     StreamBuf<float> feat(static_cast<uint64_t>(n) * kRowFeatures, s);
     ProductInputs in;
-    product_inputs(ctx, a, bt, ProductTiles{}, true, false, in, S.b);
+    product_inputs(ctx, a, bt, ProductTiles{}, true, false, S.tile_products, in, S.b);
     StreamBuf<unsigned long long> brow(n, s);
     row_features_into(ctx, a, bt, S, in, brow.get(), feat.get());
     if (n) {
@@ -1188,7 +1189,7 @@ extern "C" int mg_multiply_numeric_dense(mg_context* ctx, const mg_tiled_matrix*
     DeviceGuard g(ctx->device);
     ++c->version;
     ProductInputs in;
-    product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, true, true, in);
+    product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, true, true, c->product_pairs, in);
     const uint64_t recorded = run_product_dense(ctx, a, bt, in, min_bits, c->data.get());
     // The caller may read C, or write A, from any stream once this returns.
     MG_HIP(hipStreamSynchronize(ctx->stream));
