@@ -2258,16 +2258,17 @@ __global__ void __launch_bounds__(kBlock) numeric_use_kernel(const uint32_t* __r
   }
 }
 
-// Copy words [w0, w0+n_words) of every vertex, in vertex order, into a compact
-// (n_vertices x n_words) array.
-__global__ void __launch_bounds__(kBlock) frontier_slice_kernel(const uint64_t* __restrict__ x, uint64_t n_vertices,
-                                                                uint32_t W, uint32_t w0, uint32_t n_words,
+// Copy words [w0, w0+n_words) of the n_vertices vertices from `first` on, in vertex order, into a
+// compact (n_vertices x n_words) array.
+__global__ void __launch_bounds__(kBlock) frontier_slice_kernel(const uint64_t* __restrict__ x, uint64_t first,
+                                                                uint64_t n_vertices, uint32_t W, uint32_t w0,
+                                                                uint32_t n_words,
                                                                 const uint32_t* __restrict__ map,
                                                                 uint64_t* __restrict__ out) {
   const uint64_t total = n_vertices * n_words;
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride)
-    out[i] = x[engine_row(map, i / n_words) * W + w0 + (i % n_words)];
+    out[i] = x[engine_row(map, first + i / n_words) * W + w0 + (i % n_words)];
 }
 
 // Set bits of each chunk's A^T tiles (from the tile payloads): those of the chunk's panel
@@ -3710,11 +3711,18 @@ extern "C" int mg_walk_frontier_download(mg_context* ctx, const mg_walk* w, uint
     if (!map) {
       MG_HIP(hipMemcpyAsync(xt, x.get(), words * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     } else {
-      uint64_t* const tmp = ctx_scratch(ctx, words);  // X_hop in vertex order
-      frontier_slice_kernel<<<grid_for(words, kBlock * 8, 16384), kBlock, 0, ctx->stream>>>(x.get(), nv, w->e.W, 0,
-                                                                                           w->e.W, map, tmp);
-      MG_LAUNCH_CHECK();
-      MG_HIP(hipMemcpyAsync(xt, tmp, words * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+      // In vertex order, by pieces of at most 64 MiB, which is all that the context's scratch keeps of it (a
+      // whole X_hop is 2 GiB for 4096 sources on 2^22 vertices). A piece's copy to host memory takes 3 ms, the
+      // kernel in front of it 30 us.
+      const uint64_t piece = std::min<uint64_t>(nv, (1ull << 23) / w->e.W);
+      uint64_t* const tmp = ctx_scratch(ctx, piece * w->e.W);
+      for (uint64_t v = 0; v < nv; v += piece) {
+        const uint64_t n = std::min(piece, nv - v), n_words = n * w->e.W;
+        frontier_slice_kernel<<<grid_for(n_words, kBlock * 8, 16384), kBlock, 0, ctx->stream>>>(x.get(), v, n, w->e.W, 0,
+                                                                                               w->e.W, map, tmp);
+        MG_LAUNCH_CHECK();
+        MG_HIP(hipMemcpyAsync(xt + v * w->e.W, tmp, n_words * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+      }
     }
     MG_HIP(hipStreamSynchronize(ctx->stream));
   });
@@ -4114,7 +4122,7 @@ extern "C" int mg_walk_batch_query_download(mg_context* ctx, const mg_walk_batch
     const uint64_t nv = static_cast<uint64_t>(p.n_strips) * 64;
     DevBuf<uint64_t> tmp(nv * P.n_words);
     frontier_slice_kernel<<<grid_for(nv * P.n_words, kBlock * 8, 16384), kBlock, 0, ctx->stream>>>(
-        p.x[P.hops].get(), nv, b->e.W, P.w0, P.n_words, b->e.graphs[P.graph].device_map(), tmp.get());
+        p.x[P.hops].get(), 0, nv, b->e.W, P.w0, P.n_words, b->e.graphs[P.graph].device_map(), tmp.get());
     MG_LAUNCH_CHECK();
     MG_HIP(hipMemcpyAsync(out, tmp.get(), tmp.bytes(), hipMemcpyDeviceToHost, ctx->stream));
     MG_HIP(hipStreamSynchronize(ctx->stream));

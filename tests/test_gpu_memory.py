@@ -96,3 +96,36 @@ def test_second_free_is_refused(ctx):
     assert (a.to_array(np.uint8) == 1).all() and (b.to_array(np.uint8) == 2).all()
     a.close()
     b.close()
+
+
+def pool_bytes(M):
+    """Bytes of the device's default pool that are handed out (temporaries and contexts' scratch)."""
+    import ctypes as C
+
+    lib, pool, used = M.lib(), C.c_void_p(), C.c_uint64()
+    assert lib.hipDeviceGetDefaultMemPool(C.byref(pool), 0) == 0
+    assert lib.hipMemPoolGetAttribute(pool, 7, C.byref(used)) == 0  # hipMemPoolAttrUsedMemCurrent
+    return used.value
+
+
+def test_frontier_download_keeps_a_bounded_piece():
+    """A frontier of several pieces, in the engine's permuted strip order: what the context keeps after
+    the download is one piece of 64 MiB, and the frontier is the oracle's."""
+    import matrixgraph_amd as M
+
+    scale, n_src = 18, 4096
+    n = 1 << scale
+    with M.Context(0) as c:
+        el = M.EdgeList.rmat(c, scale, 16, 0.57, 0.19, 0.19, 9)
+        at = el.to_tiled_matrix(True)
+        el.close()
+        w = M.Walk(c, at, n_src, 1)
+        sources = O.sample_sources(n, n_src, 3)
+        w.run(sources, 1)
+        before = pool_bytes(M)
+        got = w.frontier(1)
+        assert pool_bytes(M) - before <= 64 << 20
+        w.close()
+        at.close()
+    s, d = O.rmat_edges(scale, 16, 0.57, 0.19, 0.19, 9)
+    assert np.array_equal(got, O.walk_frontiers(n, s, d, sources, 1, W=64)[1])
