@@ -3,8 +3,9 @@
 // its own:
 //   Status, kOk, kOutOfMemory, kInvalid;
 //   malloc(void**, bytes), free(void*), current_device(int*): Status;
-//   wait(): waits as free does, false if that failed; trim(device): the temporaries' pool gives back
-//   what it does not use.
+//   Stream, pool_malloc(void**, bytes, Stream): Status, from the temporaries' pool;
+//   wait(): waits as free does, false if that failed; settle(Stream): waits for the stream, false if it
+//   may not (a capture); trim(device): the pool gives back what it does not use.
 #pragma once
 
 #include <cstddef>
@@ -44,8 +45,7 @@ class BlockCache {
       std::lock_guard<std::mutex> lock(mu_);
       if (--devices_[device].contexts) return;
     }
-    flush(device);
-    D::trim(device);
+    give_back(device);
   }
 
   // A kept block of at least `bytes`, and at most an eighth more, or a fresh one. On the current device.
@@ -71,7 +71,8 @@ class BlockCache {
     void* p = nullptr;
     e = D::malloc(&p, bytes);
     if (e == D::kOutOfMemory) {
-      flush(device);
+      (void)D::wait();  // frees that are queued on streams
+      give_back(device);
       e = D::malloc(&p, bytes);
     }
     if (e != D::kOk) return e;
@@ -143,6 +144,23 @@ class BlockCache {
       }
       (void)D::free(old);
     }
+  }
+
+  // A temporary from the pool, on the current device.
+  Status pool_alloc(size_t bytes, typename D::Stream stream, void** out) {
+    *out = nullptr;
+    Status e = D::pool_malloc(out, bytes, stream);
+    if (e != D::kOutOfMemory) return e;
+    int device = 0;
+    if (!D::settle(stream) || D::current_device(&device) != D::kOk) return e;
+    give_back(device);
+    return D::pool_malloc(out, bytes, stream);
+  }
+
+  // What the library holds on the device without using it, back to the driver.
+  void give_back(int device) noexcept {
+    flush(device);
+    D::trim(device);
   }
 
   // Every kept block of the device back to the driver.

@@ -33,6 +33,13 @@ struct HipDriver {
     void* p = nullptr;
     return malloc(&p, 256) == hipSuccess && free(p) == hipSuccess;
   }
+  using Stream = hipStream_t;
+  static hipError_t pool_malloc(void** p, size_t bytes, hipStream_t st) { return seen(hipMallocAsync(p, bytes, st)); }
+  static bool settle(hipStream_t st) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (seen(hipStreamIsCapturing(st, &capture)) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+    return seen(hipStreamSynchronize(st)) == hipSuccess;
+  }
   static void trim(int device) {
     hipMemPool_t pool = nullptr;
     if (seen(hipDeviceGetDefaultMemPool(&pool, device)) == hipSuccess) (void)seen(hipMemPoolTrimTo(pool, 0));
@@ -56,6 +63,12 @@ void* cached_alloc(size_t bytes) {
 }
 
 hipError_t cached_free(void* p) noexcept { return cache().free(p); }
+
+void* pool_alloc(size_t bytes, hipStream_t stream) {
+  void* p = nullptr;
+  MG_HIP(cache().pool_alloc(bytes, stream, &p));
+  return p;
+}
 
 }  // namespace mgamd
 

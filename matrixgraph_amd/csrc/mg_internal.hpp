@@ -75,8 +75,9 @@ int guarded(F&& f) {
 //  - cached_free waits for all work on the device, as hipFree does, so a kept block is idle whichever
 //    streams used it. Inside a FreeScope the frees share one wait.
 //  - Kept: at most 1/64 of the device's memory, oldest blocks out first, none above half of that;
-//    all of it is given back when the device's last context is destroyed, or when an allocation
-//    fails. Without a context alive blocks go straight to hipFree.
+//    all of it is given back when the device's last context is destroyed, and, with what the
+//    temporaries' pool does not use, when an allocation here or from the pool finds no memory, which is
+//    then tried again. Without a context alive blocks go straight to hipFree.
 //  - Safe from any thread. In a stream capture that forbids hipFree, cached_free does what hipFree
 //    does (nothing is kept).
 // ---------------------------------------------------------------------------
@@ -84,6 +85,8 @@ void* cached_alloc(size_t bytes);  // on the current device; throws Failure
 // The driver's answer where the block goes back to it; hipErrorInvalidValue for a block that was freed
 // before and is kept.
 hipError_t cached_free(void* p) noexcept;
+// A temporary from the device's default pool, in stream order (hipFreeAsync gives it back); throws Failure.
+void* pool_alloc(size_t bytes, hipStream_t stream);
 void cache_add_context(int device, size_t device_bytes);
 void cache_drop_context(int device) noexcept;
 
@@ -140,7 +143,7 @@ class StreamBuf {
     release();
     s_ = s;
     if (n == 0) n = 1;
-    MG_HIP(hipMallocAsync(reinterpret_cast<void**>(&p_), n * sizeof(T), s_));
+    p_ = static_cast<T*>(pool_alloc(n * sizeof(T), s_));
     n_ = n;
   }
   void release() {

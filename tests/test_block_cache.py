@@ -33,7 +33,7 @@ struct Driver {
     std::lock_guard<std::mutex> lock(mu);
     ++mallocs;
     last_bytes = bytes;
-    if (bytes > capacity || used + idle_pool > capacity - bytes) return kOutOfMemory;
+    if (bytes > capacity || used + idle_pool + queued_pool > capacity - bytes) return kOutOfMemory;
     *p = reinterpret_cast<void*>(next);
     next += (bytes + 4096) / 4096 * 4096;
     blocks[*p] = bytes;
@@ -51,6 +51,19 @@ struct Driver {
   }
   static int current_device(int* d) { *d = device; return kOk; }
   static bool wait() { ++waits; return true; }
+  using Stream = int;  // kCapturing: one that must not be waited for
+  static constexpr int kCapturing = 7;
+  static inline size_t queued_pool = 0;  // freed, but work in front of the free has not finished
+  static int pool_malloc(void** p, size_t bytes, Stream) {
+    if (bytes <= idle_pool) idle_pool -= bytes;
+    return malloc(p, bytes);
+  }
+  static bool settle(Stream s) {
+    if (s == kCapturing) return false;
+    idle_pool += queued_pool;
+    queued_pool = 0;
+    return true;
+  }
   static void trim(int) { idle_pool = 0; }
 };
 using Cache = BlockCache<Driver>;
@@ -188,14 +201,44 @@ static int threads() {
   return 0;
 }
 
+// A device that is full but for kept blocks and the pool's idle memory: an object and a temporary both
+// get memory once these are given back, and fail as before where that is not enough.
+static int out_of_memory() {
+  Cache c;
+  c.add_context(0, 64 * 40 * kMB);
+  Driver::capacity = 100 * kMB;
+  void* p = nullptr;
+  auto fill = [&] {  // 20 MB of kept blocks, 30 MB idle in the pool, 10 MB on their way there
+    void *a = take(c, 10 * kMB), *b = take(c, 10 * kMB);
+    c.free(a);
+    c.free(b);
+    Driver::idle_pool = 30 * kMB;
+    Driver::queued_pool = 10 * kMB;
+  };
+  fill();
+  CHECK(c.alloc(70 * kMB, &p) == Driver::kOk && Driver::used == 70 * kMB && Driver::idle_pool == 0);
+  c.free(p);
+  Driver::queued_pool = 0;
+  fill();
+  CHECK(c.pool_alloc(90 * kMB, 0, &p) == Driver::kOk && Driver::used == 90 * kMB);
+  Driver::free(p);
+  fill();
+  CHECK(c.pool_alloc(101 * kMB, 0, &p) == Driver::kOutOfMemory && !p);
+  CHECK(c.alloc(101 * kMB, &p) == Driver::kOutOfMemory && !p);
+  fill();
+  CHECK(c.pool_alloc(90 * kMB, Driver::kCapturing, &p) == Driver::kOutOfMemory);
+  CHECK(Driver::idle_pool == 30 * kMB && Driver::used == 20 * kMB);  // nothing was touched
+  return 0;
+}
+
 int main(int, char** argv) {
 #define RUN(f) if (!std::strcmp(argv[1], #f)) return f();
-  RUN(freed_twice) RUN(foreign) RUN(sizes) RUN(limit) RUN(last_context) RUN(devices) RUN(waits) RUN(threads)
+  RUN(freed_twice) RUN(foreign) RUN(sizes) RUN(limit) RUN(last_context) RUN(devices) RUN(waits) RUN(threads) RUN(out_of_memory)
   std::printf("no check %s\n", argv[1]);
   return 2;
 }
 """
-CHECKS = ("freed_twice", "foreign", "sizes", "limit", "last_context", "devices", "waits", "threads")
+CHECKS = ("freed_twice", "foreign", "sizes", "limit", "last_context", "devices", "waits", "threads", "out_of_memory")
 
 
 @pytest.fixture(scope="module")
