@@ -106,6 +106,7 @@ extern "C" int mg_context_create(int device, mg_context** out) {
     auto* ctx = new mg_context();
     ctx->device = device;
     ctx->n_cu = prop.multiProcessorCount;
+    ctx->scratch_limit = prop.totalGlobalMem / 64;
     hipError_t e = hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
       delete ctx;

@@ -463,6 +463,7 @@ extern "C" int mg_edges_rmat(mg_context* ctx, uint32_t scale, uint32_t edge_fact
     const uint64_t n_draws = static_cast<uint64_t>(edge_factor) << scale;
     MG_REQUIRE(n_draws < (1ull << 31), "mg_edges_rmat: more than 2^31 draws");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     StreamBuf<uint64_t> keys(n_draws, ctx->stream);
     if (n_draws) {
       rmat_kernel<<<grid_for(n_draws, 256, 65536), 256, 0, ctx->stream>>>(
@@ -483,6 +484,7 @@ extern "C" int mg_edges_er(mg_context* ctx, uint32_t log2_n, uint64_t p_num, uin
     MG_REQUIRE(p_log2_den >= 1 && p_log2_den <= 63 && p_num < (1ull << p_log2_den),
                "mg_edges_er: p must be p_num / 2^m with 1 <= m <= 63 and p_num < 2^m");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     BernoulliSpec s{};
     s.n_vertices = 1u << log2_n;
     s.n_blocks = (s.n_vertices + 63) / 64;
@@ -509,6 +511,7 @@ extern "C" int mg_edges_communities(mg_context* ctx, uint32_t n_vertices, uint32
                "mg_edges_communities: p must be p_num / 2^m with 1 <= m <= 63 and p_num < 2^m");
     MG_REQUIRE(static_cast<uint64_t>(n_comm) * comm_size < (1ull << 32), "mg_edges_communities: too many rows");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     BernoulliSpec s{};
     s.n_vertices = n_vertices;
     s.n_blocks = (n_vertices + 63) / 64;
@@ -528,6 +531,7 @@ extern "C" int mg_edges_union(mg_context* ctx, const mg_edge_list* a, const mg_e
     *out = nullptr;
     MG_REQUIRE(a->n_vertices == b->n_vertices, "mg_edges_union: vertex counts differ");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     const uint64_t n = a->n_edges + b->n_edges;
     StreamBuf<uint64_t> keys(n, ctx->stream);
     if (a->n_edges)
@@ -876,6 +880,7 @@ extern "C" int mg_edges_upload(mg_context* ctx, uint32_t n_vertices, uint64_t n_
     MG_REQUIRE(n_edges == 0 || (src && dst), "mg_edges_upload: NULL edge arrays");
     MG_REQUIRE(n_vertices >= 1, "mg_edges_upload: n_vertices == 0");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     hipStream_t st = ctx->stream;
     const SortScratch w = sort_scratch(ctx, n_edges, 0, edge_bits(n_vertices, false), true);
     unsigned long long* const bad = ctx->counters.get();
@@ -945,6 +950,7 @@ extern "C" int mg_edges_to_tiled_matrix(mg_context* ctx, const mg_edge_list* el,
     MG_REQUIRE(ctx && el && out, "mg_edges_to_tiled_matrix: NULL argument");
     *out = nullptr;
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     hipStream_t st = ctx->stream;
     const uint32_t n_strips = (el->n_vertices + 63) / 64;
     MG_REQUIRE(n_strips < (1u << 26), "mg_edges_to_tiled_matrix: n_strips >= 2^26");

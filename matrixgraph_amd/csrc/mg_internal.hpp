@@ -208,8 +208,11 @@ struct mg_context {
   mgamd::DevBuf<unsigned long long> counters;  // small scratch for reductions (host-synchronised calls)
   hipEvent_t timer[2] = {nullptr, nullptr};    // mg_context_timer_start / _stop
   // Per-call device temporaries of asynchronous calls on `stream` (calls on one context run
-  // in stream order, so the next call may reuse them); grown by ctx_scratch, stream-ordered.
+  // in stream order, so the next call may reuse them); grown by ctx_scratch, stream-ordered. At most
+  // scratch_limit bytes stay from one call to the next (ScratchScope).
   mgamd::StreamBuf<uint64_t> scratch;
+  size_t scratch_limit = 0;  // 1/64 of the device's memory, as for kept blocks
+  int scratch_users = 0;     // ScratchScopes
   mgamd::PinnedBuf<uint32_t> mail;  // read_words
 };
 
@@ -255,6 +258,24 @@ inline uint64_t* ctx_scratch(mg_context* ctx, size_t n) {
   if (ctx->scratch.size() < n) ctx->scratch.alloc(n, ctx->stream);
   return ctx->scratch.get();
 }
+
+// Around an entry point that uses ctx_scratch: once the outermost is left, a scratch above the limit is
+// freed, in stream order. Not inside a capture, whose graph goes on using it.
+struct ScratchScope {
+  mg_context* ctx;
+  explicit ScratchScope(mg_context* c) : ctx(c) { ++ctx->scratch_users; }
+  ~ScratchScope() {
+    if (--ctx->scratch_users || ctx->scratch.bytes() <= ctx->scratch_limit) return;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    if (capture == hipStreamCaptureStatusNone) ctx->scratch.release();
+  }
+  ScratchScope(const ScratchScope&) = delete;
+  ScratchScope& operator=(const ScratchScope&) = delete;
+};
 
 // Static payload scratch of mg_multiply_numeric_noalloc (mg_spgemm.hip): 32 MiB per device,
 // 16 bytes per tile of both operands plus 16 (kNoAllocMaxTiles tiles in A and Bt together).

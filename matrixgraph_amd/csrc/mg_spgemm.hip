@@ -919,6 +919,7 @@ extern "C" int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, co
     MG_REQUIRE(a->n_strips == bt->n_strips && c->n_strips == a->n_strips,
                "mg_multiply_numeric: operands differ in n_strips");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     ++c->version;
     if (c->n_nz_tile == 0) return;
     ProductInputs in;
@@ -1072,6 +1073,7 @@ extern "C" int mg_multiply_pruned(mg_context* ctx, const mg_tiled_matrix* a, con
     MG_REQUIRE(ctx && a && bt && c_out, "mg_multiply_pruned: NULL argument");
     *c_out = nullptr;
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     PrunedPlan P;
     pruned_prepare(ctx, a, bt, P, false, "mg_multiply_pruned");
     auto c = std::make_unique<mg_tiled_matrix>();
@@ -1095,6 +1097,7 @@ extern "C" int mg_multiply_pruned_model(mg_context* ctx, const mg_tiled_matrix* 
     MG_REQUIRE(n_in == kRowFeatures && n_out >= 1,
                "mg_multiply_pruned_model: the model must take MG_ROW_FEATURES inputs");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     hipStream_t s = ctx->stream;
     PrunedPlan P;
     pruned_prepare(ctx, a, bt, P, true, "mg_multiply_pruned_model");
@@ -1135,6 +1138,7 @@ extern "C" int mg_multiply_row_features(mg_context* ctx, const mg_tiled_matrix* 
   return guarded([&] {
     MG_REQUIRE(ctx && a && bt && features, "mg_multiply_row_features: NULL argument");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     hipStream_t s = ctx->stream;
     Structural S;
     structural_pass(ctx, a, bt, S, "mg_multiply_row_features");
@@ -1187,6 +1191,7 @@ extern "C" int mg_multiply_numeric_dense(mg_context* ctx, const mg_tiled_matrix*
     MG_REQUIRE(a->n_strips == bt->n_strips && c->n_strips == a->n_strips,
                "mg_multiply_numeric_dense: operands differ in n_strips");
     DeviceGuard g(ctx->device);
+    ScratchScope scratch(ctx);
     ++c->version;
     ProductInputs in;
     product_inputs(ctx, a, bt, ProductTiles{c->n_nz_tile, c->row_idx.get(), c->col_idx.get()}, true, true, c->product_pairs, in);

@@ -129,3 +129,26 @@ def test_frontier_download_keeps_a_bounded_piece():
         at.close()
     s, d = O.rmat_edges(scale, 16, 0.57, 0.19, 0.19, 9)
     assert np.array_equal(got, O.walk_frontiers(n, s, d, sources, 1, W=64)[1])
+
+
+def test_scratch_above_the_limit_is_given_back():
+    """300 M uploaded edges (all the same) sort in 4.8 GB of scratch, more than the 1/64 of the card that a
+    context keeps: none of it stays. A small upload's scratch does."""
+    import ctypes as C
+
+    import matrixgraph_amd as M
+
+    free, total = C.c_size_t(), C.c_size_t()
+    with M.Context(0) as c:
+        assert M.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        n = total.value // 64 // 16 + (1 << 20)
+        ids = np.zeros(n, np.uint32)
+        before = pool_bytes(M)
+        el = M.EdgeList.upload(c, 7, ids, ids)
+        assert el.info() == (7, 1)
+        el.close()
+        assert pool_bytes(M) == before
+        el = M.EdgeList.upload(c, 7, ids[:1 << 20], ids[:1 << 20])
+        assert el.info() == (7, 1)
+        el.close()
+        assert (16 << 20) <= pool_bytes(M) - before <= total.value // 64
