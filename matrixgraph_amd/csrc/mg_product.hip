@@ -1209,14 +1209,13 @@ bool by_tiles(uint32_t ns, uint64_t n_a, uint64_t n_c, uint64_t pairs, bool inde
 
 bool prepared(const mg_tiled_matrix* m) { return m->prep_version == m->version && m->prep_head.get(); }
 
-void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
+void prepare_operand(mg_context* ctx, mg_tiled_matrix* m, uint64_t used_columns) {
   hipStream_t st = ctx->stream;
   const uint32_t n = m->n_nz_tile, ns = m->n_strips;
   const bool bitmap = ns <= kBitmapStrips;
   const uint32_t wpr = (ns + 63) / 64;
   const uint64_t bm = bitmap ? 2ull * ns * wpr : 0;  // u64 words
   m->prep_head.alloc(2ull * std::max<uint32_t>(1, n));
-  m->prep_words.alloc(1);
   StreamBuf<unsigned long long> next(1, st);
   clear_words_kernel<<<1, kBlock, 0, st>>>(reinterpret_cast<uint64_t*>(next.get()), 1);
   MG_LAUNCH_CHECK();
@@ -1240,18 +1239,18 @@ void prepare_operand(mg_context* ctx, mg_tiled_matrix* m) {
     as_b.tile = m->prep_index.get() + ns + 1;
     as_a.n = 0;
   }
-  const uint64_t room = word_room(n);
-  StreamBuf<uint64_t> words(room, st);
-  launch_heads(st, as_a, as_b, true, words.get(), room, next.get());
-  launch_weights(st, WeightJob{used.get(), m->offset_row.get(), m->prep_weight.get()}, WeightJob{}, ns);
-  unsigned long long taken = 0;
-  MG_HIP(hipMemcpyAsync(&taken, next.get(), sizeof(taken), hipMemcpyDeviceToHost, st));
-  MG_HIP(hipStreamSynchronize(st));
-  taken = std::min<unsigned long long>(taken, room);
-  if (taken) {
-    m->prep_words.alloc(taken);
-    MG_HIP(hipMemcpyAsync(m->prep_words.get(), words.get(), taken * sizeof(uint64_t), hipMemcpyDeviceToDevice, st));
+  // Last, as many column words as the tiles have, or, without memory for them (or 32-bit places), none:
+  // the products then make them from the tiles.
+  uint64_t room = used_columns < kNoWords ? used_columns : 0;
+  try {
+    m->prep_words.alloc(std::max<uint64_t>(1, room));
+  } catch (const Failure& e) {
+    if (e.code != MG_ERR_OOM || !room) throw;
+    room = 0;
+    m->prep_words.alloc(1);
   }
+  launch_heads(st, as_a, as_b, true, m->prep_words.get(), room, next.get());
+  launch_weights(st, WeightJob{used.get(), m->offset_row.get(), m->prep_weight.get()}, WeightJob{}, ns);
 }
 
 void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt, const ProductTiles& c,

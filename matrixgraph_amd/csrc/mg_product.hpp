@@ -103,7 +103,8 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
                     bool want_bits, bool want_words, uint64_t pairs, ProductInputs& P, const RightIndex& known = {});
 // Operand kept with its handle (mg_tiled_matrix_prepare_operand): all but the payloads.
 bool prepared(const mg_tiled_matrix* m);
-void prepare_operand(mg_context* ctx, mg_tiled_matrix* m);
+// used_columns: columns in use of all tiles, which is the number of column words.
+void prepare_operand(mg_context* ctx, mg_tiled_matrix* m, uint64_t used_columns);
 
 // Where a finished C tile goes: ORed into data at its index (kOutStruct), or, for a pruned product,
 // only if it is non-zero: into the next slot of data, whether and which in flag and slot

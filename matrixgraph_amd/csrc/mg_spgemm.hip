@@ -139,10 +139,16 @@ __device__ inline uint32_t wide_entry(WidePayload p, uint32_t i) {
 }
 
 // Wide payload of every tile of both operands, one wave per tile (lane r holds row r): tiles
-// [0, n_a) of data_a, then the n_bt tiles of data_bt, at the same positions of `payload`.
+// [0, n_a) of data_a, then the n_bt tiles of data_bt, at the same positions of `payload`. used (may be
+// null) gets the tiles' columns in use added up.
 __global__ void __launch_bounds__(kBlock) payload_kernel(const uint64_t* __restrict__ data_a, uint32_t n_a,
                                                          const uint64_t* __restrict__ data_bt, uint32_t n_bt,
-                                                         WidePayload* __restrict__ payload) {
+                                                         WidePayload* __restrict__ payload,
+                                                         unsigned long long* __restrict__ used) {
+  __shared__ unsigned long long s_used;
+  if (threadIdx.x == 0) s_used = 0;
+  __syncthreads();
+  uint64_t n_used = 0;
   const uint32_t n_waves = gridDim.x * kWavesPerBlock;
   const uint64_t n_tiles = static_cast<uint64_t>(n_a) + n_bt;
   for (uint64_t i = read_first_lane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave); i < n_tiles; i += n_waves) {
@@ -150,6 +156,7 @@ __global__ void __launch_bounds__(kBlock) payload_kernel(const uint64_t* __restr
     const uint64_t total = wave_sum(__popcll(word));
     WidePayload pl = {0, static_cast<uint64_t>(kWideDense) << 60};
     const uint64_t cols = wave_or(word);
+    n_used += static_cast<uint32_t>(__popcll(cols));
     if (total > kWideMax) pl.x = cols;
     if (total <= kWideMax) {
       uint64_t w[2] = {0, 0};
@@ -167,6 +174,10 @@ __global__ void __launch_bounds__(kBlock) payload_kernel(const uint64_t* __restr
     }
     if (lane_id() == 0) payload[i] = pl;
   }
+  if (!used) return;
+  if (lane_id() == 0 && n_used) atomicAdd(&s_used, static_cast<unsigned long long>(n_used));
+  __syncthreads();
+  if (threadIdx.x == 0 && s_used) atomicAdd(used, s_used);
 }
 
 // Payloads alone of A's tiles at pl[0, n_a) and of Bt's at pl[n_a, n_a + n_bt) (the allocation-free
@@ -179,7 +190,7 @@ void launch_payloads(hipStream_t st, const mg_tiled_matrix* a, const mg_tiled_ma
   const uint32_t ma = pa ? 0 : na, mb = pb ? 0 : nb;
   if (ma + mb == 0) return;
   payload_kernel<<<grid_for(static_cast<uint64_t>(ma) + mb, kWavesPerBlock, 65536), kBlock, 0, st>>>(
-      a->data.get(), ma, bt->data.get(), mb, pa ? pl + na : pl);
+      a->data.get(), ma, bt->data.get(), mb, pa ? pl + na : pl, nullptr);
   MG_LAUNCH_CHECK();
 }
 
@@ -901,12 +912,16 @@ extern "C" int mg_tiled_matrix_prepare_operand(mg_context* ctx, mg_tiled_matrix*
     hipStream_t st = ctx->stream;
     const uint32_t n = m->n_nz_tile;
     m->prep_payload.alloc(2ull * std::max<uint32_t>(1, n));
+    unsigned long long used = 0;
     if (n) {
-      payload_kernel<<<grid_for(n, kWavesPerBlock, 65536), kBlock, 0, st>>>(
-          m->data.get(), n, nullptr, 0, reinterpret_cast<WidePayload*>(m->prep_payload.get()));
+      unsigned long long* const sum = ctx->counters.get();
+      MG_HIP(hipMemsetAsync(sum, 0, sizeof(*sum), st));
+      payload_kernel<<<grid_for(n, kWavesPerBlock, 16384), kBlock, 0, st>>>(
+          m->data.get(), n, nullptr, 0, reinterpret_cast<WidePayload*>(m->prep_payload.get()), sum);
       MG_LAUNCH_CHECK();
+      read_words(ctx, {sum, &used, sizeof(used)});
     }
-    prepare_operand(ctx, m);
+    prepare_operand(ctx, m, used);
     MG_HIP(hipStreamSynchronize(st));
     m->prep_version = m->version;
   });

@@ -152,3 +152,49 @@ def test_scratch_above_the_limit_is_given_back():
         assert el.info() == (7, 1)
         el.close()
         assert (16 << 20) <= pool_bytes(M) - before <= total.value // 64
+
+
+def test_prepare_without_memory_for_column_words():
+    """2.25 M full tiles, whose column words (1.2 GB) do not fit beside what else is on the device: the
+    operand is prepared without them, and its products are the same."""
+    import ctypes as C
+
+    import matrixgraph_amd as M
+
+    lib, ns = M.lib(), 1500
+    free, total = C.c_size_t(), C.c_size_t()
+    filled = []
+    with M.Context(0) as c:
+        bt = M.TiledMatrix.upload(c, M.HostTiledMatrix(
+            ns, np.arange(ns + 1, dtype=np.uint32) * ns, np.repeat(np.arange(ns, dtype=np.uint32), ns),
+            np.tile(np.arange(ns, dtype=np.uint32), ns), np.full((ns * ns, 64), ~np.uint64(0))))
+        off = np.full(ns + 1, 3, np.uint32)
+        off[0] = 0
+        data = np.zeros((3, 64), np.uint64)
+        data[:, 5] = np.uint64(1) << np.uint64(9)
+        a = M.TiledMatrix.upload(c, M.HostTiledMatrix(ns, off, np.zeros(3, np.uint32), np.array([0, 7, 1499], np.uint32), data))
+        want, _ = M.multiply(c, a, bt)
+        M.multiply_numeric(c, a, bt, want)
+        try:
+            while True:
+                assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+                if free.value < 1 << 30:
+                    break
+                p = C.c_void_p()
+                assert lib.hipMalloc(C.byref(p), C.c_size_t(min(free.value - (800 << 20), 64 << 30))) == 0
+                filled.append(p)
+            bt.prepare_operand()
+            assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+            assert free.value > 256 << 20  # the words are not there
+        finally:
+            for p in filled:
+                assert lib.hipFree(p) == 0
+        got, _ = M.multiply(c, a, bt)
+        got, want = got.download(), want.download()
+        assert np.array_equal(got.data, want.data) and len(got.data) == ns
+        assert (got.data[:, 5] == ~np.uint64(0)).all() and not np.delete(got.data, 5, axis=1).any()
+        dense, _ = M.multiply_symbolic(c, a, bt)
+        assert M.multiply_numeric_dense(c, a, bt, dense, 1) == 3 * ns
+        assert np.array_equal(dense.download().data, want.data)
+        for m in (a, bt, dense):
+            m.close()

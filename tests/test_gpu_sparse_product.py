@@ -33,9 +33,10 @@ def want_product(a, bt):
     return c_row, c_col, O.tile_numeric(a[0], a[1:], bt[1:], c_row, c_col), tp
 
 
-# Pairs per C tile from 1 to 13 (12: the last by tiles); 153 K C tiles: runs of several.
+# Pairs per C tile from 1 to 13 (12: the last by tiles); 153 K C tiles: runs of several; the widest grid
+# with bitmaps and the first without.
 @pytest.mark.parametrize("ns,occupied", [(1, 1.0), (2, 1.0), (12, 1.0), (13, 1.0), (17, 0.1), (63, 0.2), (65, 0.45),
-                                         (300, 0.02), (4096, 0.0015)])
+                                         (300, 0.02), (4096, 0.0015), (16384, 2e-5), (16385, 2e-5)])
 @pytest.mark.parametrize("prepare", [False, True])
 def test_both_kernels_match_oracle(ctx, ns, occupied, prepare):
     import matrixgraph_amd as M
