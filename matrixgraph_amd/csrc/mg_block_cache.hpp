@@ -51,6 +51,7 @@ class BlockCache {
   // A kept block of at least `bytes`, and at most an eighth more, or a fresh one. On the current device.
   Status alloc(size_t bytes, void** out) {
     *out = nullptr;
+    if (bytes > SIZE_MAX - 511) return D::kOutOfMemory;  // rounding up would wrap to nothing
     bytes = (bytes + 511) / 512 * 512;
     int device = 0;
     Status e = D::current_device(&device);

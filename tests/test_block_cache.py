@@ -231,14 +231,26 @@ static int out_of_memory() {
   return 0;
 }
 
+// Sizes that rounding up would wrap.
+static int size_wraps() {
+  Cache c;
+  c.add_context(0, 64 * 100 * kMB);
+  void* p = &c;
+  for (size_t bytes : {SIZE_MAX, SIZE_MAX - 1, SIZE_MAX - 510}) {
+    CHECK(c.alloc(bytes, &p) == Driver::kOutOfMemory && !p && Driver::mallocs == 0);
+  }
+  CHECK(c.alloc(SIZE_MAX - 511, &p) == Driver::kOutOfMemory && Driver::last_bytes == SIZE_MAX - 511);
+  return 0;
+}
+
 int main(int, char** argv) {
 #define RUN(f) if (!std::strcmp(argv[1], #f)) return f();
-  RUN(freed_twice) RUN(foreign) RUN(sizes) RUN(limit) RUN(last_context) RUN(devices) RUN(waits) RUN(threads) RUN(out_of_memory)
+  RUN(freed_twice) RUN(foreign) RUN(sizes) RUN(limit) RUN(last_context) RUN(devices) RUN(waits) RUN(threads) RUN(out_of_memory) RUN(size_wraps)
   std::printf("no check %s\n", argv[1]);
   return 2;
 }
 """
-CHECKS = ("freed_twice", "foreign", "sizes", "limit", "last_context", "devices", "waits", "threads", "out_of_memory")
+CHECKS = ("freed_twice", "foreign", "sizes", "limit", "last_context", "devices", "waits", "threads", "out_of_memory", "size_wraps")
 
 
 @pytest.fixture(scope="module")

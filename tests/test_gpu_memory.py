@@ -198,3 +198,14 @@ def test_prepare_without_memory_for_column_words():
         assert np.array_equal(dense.download().data, want.data)
         for m in (a, bt, dense):
             m.close()
+
+
+@pytest.mark.parametrize("size", [(1 << 64) - 1, (1 << 64) - 600, 1 << 50])
+def test_impossible_sizes_are_out_of_memory(ctx, size):
+    import ctypes as C
+
+    import matrixgraph_amd as M
+
+    p = C.c_void_p(1)
+    assert M.lib().mg_buffer_alloc(ctx.h, C.c_size_t(size), C.byref(p)) == 3  # MG_ERR_OOM
+    assert not p.value
