@@ -388,10 +388,12 @@ enum {
                                    (results, digests, downloads and exports are the same) */
 };
 enum {
-  MG_HOP_SWEEP = 0u, /* the hop took every strip of A^T in vertex-row words: by its tiles, or by its
-                        job list (walks of at most 2048 sources; a first hop that is not pushed) */
+  MG_HOP_SWEEP = 0u, /* the hop swept every strip of A^T: by its tiles (4096-source walks with 0 segments,
+                        and their first hop, if it is not pushed, with 2, 4 or 8), or the one kernel of
+                        walks of at most 2048 sources */
   MG_HOP_PUSH = 1u,  /* first hop pushed from the source strips' A^T columns */
-  MG_HOP_JOBS = 2u   /* the hop read A^T's job list by row segments (mg_walk_set_hop_kernel) */
+  MG_HOP_JOBS = 2u   /* a hop of a 4096-source walk read A^T's job list by row segments
+                        (mg_walk_set_hop_kernel); with 1 segment also a first hop that is not pushed */
 };
 
 typedef struct mg_hop_stats {
@@ -424,7 +426,8 @@ typedef struct mg_hop_stats {
  * most half of its tiles; results and statistics are the same either way. */
 int mg_walk_create(mg_context* ctx, const mg_tiled_matrix* at, uint32_t max_sources,
                    uint32_t max_hops, uint32_t flags, mg_walk** out);
-/* Hop kernel of the 4096-source (64-word) levels from hop 2 on. segments = 0: the
+/* Hop kernel of the 4096-source (64-word) levels from hop 2 on (segments = 1: from hop 1 on, where that is
+ * not pushed). segments = 0: the
  * tile-decoding sweep (every hop decodes the A^T tiles' payloads into gathers of whole
  * 512-byte source rows); 1, 2, 4 or 8: the job-list kernel, which reads a list of at's set
  * bits built once (4 bytes per set bit plus 4 per tile and per strip, on first use) and

@@ -2900,6 +2900,8 @@ struct Engine {
   // G = 1 also takes the first hop where it is swept (4096 sources on R-MAT 14: 694 us a walk before, 278).
   uint32_t seg = 0;
   uint32_t seg_from = 1;
+  // Row segments of level k's job-list kernel; 0: another kernel runs it (unless its hop is pushed).
+  uint32_t segments_of(uint32_t k) const { return W == 64 && !logging && (k >= seg_from || seg == 1) ? seg : 0; }
   // One-graph walks of fewer than 64 words: the hops run walk_narrow_kernel; used_words: words of
   // X that hold sources in the current run.
   bool narrow = false;
@@ -3244,7 +3246,7 @@ void launch_level_w(hipStream_t st, Engine* e, uint32_t k, hipEvent_t ev[4]) {
   if (ev) MG_HIP(hipEventRecord(ev[0], st));
   if (ev) MG_HIP(hipEventRecord(ev[1], st));
   if (ev) MG_HIP(hipEventRecord(ev[2], st));
-  const uint32_t G = (W == 64 && e->seg && !e->logging && (k >= e->seg_from || e->seg == 1)) ? e->seg : 0;
+  const uint32_t G = W == 64 ? e->segments_of(k) : 0;
   if (e->n_chunks[k]) {
     ChunkLog* const log = e->logging ? e->logs[k].get() : nullptr;
     if constexpr (W == 64) {
@@ -3651,7 +3653,7 @@ extern "C" int mg_walk_hop_stats(mg_context* ctx, mg_walk* w, uint32_t hop, mg_h
     }
     if (hop == 1 && w->last_push) {
       out->kernel = MG_HOP_PUSH;
-    } else if (w->e.W == 64 && w->e.seg && hop - 1 >= w->e.seg_from) {
+    } else if (w->e.segments_of(hop - 1)) {
       out->kernel = MG_HOP_JOBS;
       out->segments = w->e.seg;
     } else {

@@ -514,3 +514,22 @@ def test_pieces_of_heavy_strips(ctx, n_sources, sweep):
             assert np.array_equal(got[:n], xs[k]) and not got[n:].any(), k
             assert w.hop_stats(k)["popcount"] == np.bitwise_count(xs[k]).sum()
     w.close()
+
+
+def test_swept_first_hop_names_its_kernel(ctx):
+    """A 4096-source walk whose first hop is never pushed: with one segment it is read from the job list
+    like the others, with more or none it is swept by tiles, and the statistics say which."""
+    M = mg()
+    n = 1 << 12
+    el, at, s, d = setup_graph(ctx, 12, 6)
+    w = M.Walk(ctx, at, 4096, 2, flags=M.WALK_SWEEP_FIRST_HOP)
+    sources = O.sample_sources(n, 4000, 3)
+    xs = O.walk_frontiers(n, s, d, sources, 2, W=64)
+    for segments in (1, 0, 4, 1):
+        assert w.set_hop_kernel(segments) == segments
+        w.run(sources, 2)
+        first, second = w.hop_stats(1), w.hop_stats(2)
+        assert (first["kernel"], first["segments"]) == ((M.HOP_JOBS, 1) if segments == 1 else (M.HOP_SWEEP, 0))
+        assert (second["kernel"], second["segments"]) == ((M.HOP_JOBS, segments) if segments else (M.HOP_SWEEP, 0))
+        for k in (1, 2):
+            assert np.array_equal(w.frontier(k), xs[k])
