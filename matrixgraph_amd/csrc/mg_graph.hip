@@ -905,14 +905,30 @@ extern "C" int mg_edges_info(const mg_edge_list* el, uint32_t* n_vertices, uint6
   });
 }
 
+namespace {
+constexpr uint64_t kSplitOnHost = 1ull << 16;  // edges
+}
+
 extern "C" int mg_edges_download(mg_context* ctx, const mg_edge_list* el, uint32_t* src, uint32_t* dst) {
   return guarded([&] {
     MG_REQUIRE(ctx && el, "mg_edges_download: NULL argument");
     if (el->n_edges == 0) return;
     MG_REQUIRE(src && dst, "mg_edges_download: NULL output arrays");
     DeviceGuard g(ctx->device);
-    // Split on the device, a piece at a time, straight into the caller's arrays.
     hipStream_t st = ctx->stream;
+    // A copy to host memory takes about 0.13 ms whatever it copies: a short list takes one and is split here
+    // (16 K edges 0.13 ms, by two copies 0.26; as long from 0.2 M edges on).
+    if (el->n_edges <= kSplitOnHost) {
+      std::vector<uint64_t> h(el->n_edges);
+      MG_HIP(hipMemcpyAsync(h.data(), el->keys.get(), 8 * el->n_edges, hipMemcpyDeviceToHost, st));
+      MG_HIP(hipStreamSynchronize(st));
+      for (uint64_t i = 0; i < el->n_edges; ++i) {
+        src[i] = static_cast<uint32_t>(h[i] >> 32);
+        dst[i] = static_cast<uint32_t>(h[i]);
+      }
+      return;
+    }
+    // Split on the device, a piece at a time, straight into the caller's arrays.
     const uint64_t piece = std::min<uint64_t>(el->n_edges, 1ull << 23);
     StreamBuf<uint32_t> ids(2 * piece, st);
     for (uint64_t i = 0; i < el->n_edges; i += piece) {

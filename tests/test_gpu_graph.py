@@ -279,3 +279,16 @@ def test_upload_sorts_and_tiles_any_list(ctx, n, edges):
             M.EdgeList.upload(ctx, n, bad, d)
     for m in (el, un):
         m.close()
+
+
+@pytest.mark.parametrize("n_edges", [1, (1 << 16) - 1, 1 << 16, (1 << 16) + 1, 300000])
+def test_edge_download_of_any_length(ctx, n_edges):
+    """Short lists are split into sources and destinations on the host, longer ones on the device."""
+    import matrixgraph_amd as M
+
+    ids = np.random.default_rng(n_edges).permutation(1 << 20)[:n_edges].astype(np.uint32)
+    src, dst = ids, (ids * np.uint32(2654435761)) >> np.uint32(12)
+    el = M.EdgeList.upload(ctx, 1 << 20, src, dst)
+    s, d = el.download()
+    order = np.argsort(src)
+    assert np.array_equal(s, src[order]) and np.array_equal(d, dst[order])
