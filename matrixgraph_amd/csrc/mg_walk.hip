@@ -1539,7 +1539,11 @@ __device__ inline void few_gather(std::integer_sequence<int, K...>, uint32_t job
 // (few_gather). kLeanMixed: some have. Kernels of their own because the others fit in 64 VGPRs only
 // without few_gather: kLeanMixed spills ten more, which costs its wider panels 3-6 %, but two launches
 // one after the other cost more (a batch of 16 queries on three graphs: 2.04 ms mixed, 2.35 in two
-// launches, 2.67 without few_gather).
+// launches, 2.67 without few_gather). A level is mixed where the panels with few live words have at least
+// 1 / kMixedShare of its jobs, else kLeanPartial. Batches of uneven queries on eight graphs, mixed at
+// every level and at none: 16 queries (shares 0.83 to 1) 4.79 and 6.12 ms, 64 (0.12 to 0.98) 9.50 and
+// 10.96, 32 (0.15 to 0.5) 10.03 and 10.28, 192 (0.01 to 0.2) 26.9 and 26.3, 512 (0.02 to 0.15) 78.0 and 76.1.
+constexpr uint64_t kMixedShare = 8;
 enum : int { kLeanWhole = 0, kLeanPartial = 1, kLeanFew = 2, kLeanMixed = 3 };
 template <int kMode>
 __global__ void __launch_bounds__(kLeanBlock) __attribute__((amdgpu_waves_per_eu(kLeanWaves, kLeanWaves)))
@@ -3139,15 +3143,20 @@ void build_engine(Engine* e, hipStream_t st) {
     e->lv[k].alloc(P);
     MG_HIP(hipMemcpyAsync(e->lv[k].get(), lv.data(), sizeof(PanelLevel) * P, hipMemcpyHostToDevice, st));
     e->host_lv.push_back(lv);
-    bool some_dead = false, some_few = false, some_many = false;
-    for (const auto& L : lv) {
+    bool some_dead = false;
+    uint64_t few = 0, all = 0;  // jobs of the panels with few live words, and of all
+    for (uint32_t pi = 0; pi < lv.size(); ++pi) {
+      const PanelLevel& L = lv[pi];
       if (!L.x_in) continue;
-      const bool is_few = __builtin_popcountll(L.alive_in) <= kFewWords;
+      const uint64_t jobs = std::max<uint64_t>(1, e->graphs[e->panels[pi].graph].total_bits);
       some_dead |= L.alive_in != ~0ull;
-      some_few |= is_few;
-      some_many |= !is_few;
+      all += jobs;
+      if (__builtin_popcountll(L.alive_in) <= kFewWords) few += jobs;
     }
-    e->partial.push_back(some_few ? (some_many ? kLeanMixed : kLeanFew) : some_dead ? kLeanPartial : kLeanWhole);
+    e->partial.push_back(!some_dead                  ? kLeanWhole
+                         : few == all               ? kLeanFew
+                         : kMixedShare * few >= all ? kLeanMixed
+                                                    : kLeanPartial);
     e->n_chunks[k] = static_cast<uint32_t>(ch.size());
     e->host_chunks[k] = ch;
     e->chunks[k].alloc(std::max<size_t>(1, ch.size()));

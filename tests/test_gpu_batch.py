@@ -151,3 +151,27 @@ def test_batch_of_few_live_words(ctx, sizes):
             assert b.query_digest(i) == w.frontier_digest(q.hops), i
             w.close()
     b.close()
+
+
+@pytest.mark.parametrize("few_on", [0, 1])
+def test_batch_with_few_live_words_in_a_small_or_large_share(ctx, few_on):
+    """Two graphs, one with sixteen times the edges of the other: the panel with at most 16 live words holds
+    nearly none of a level's jobs, or nearly all, beside one with 40; each query is its own walk's."""
+    M = mg()
+    graphs, queries = [], []
+    for g, (n, m) in enumerate(((3000, 6000), (9000, 96000))):
+        rng = np.random.default_rng(g)
+        s, d = (rng.integers(0, n, m).astype(np.uint32) for _ in range(2))
+        d[: m // 4] = 70
+        graphs.append(M.EdgeList.upload(ctx, n, s, d).to_tiled_matrix(transpose=True))
+        sources = rng.permutation(n)[:900 if g == few_on else 2500].astype(np.uint32)
+        queries.append(M.workloads.QuerySpec(g, sources, 4))
+    b = M.WalkBatch(ctx, graphs, queries)
+    for _ in range(2):
+        b.run()
+        for i, q in enumerate(queries):
+            w = M.Walk(ctx, graphs[q.graph], len(q.sources), q.hops)
+            w.run(q.sources, q.hops)
+            assert b.query_digest(i) == w.frontier_digest(q.hops), i
+            w.close()
+    b.close()
