@@ -2966,7 +2966,7 @@ namespace {
 void sort_by_cost(const Engine& e, std::vector<Chunk>& ch, const std::vector<uint64_t>& cost) {
   std::vector<uint32_t> idx(ch.size());
   std::iota(idx.begin(), idx.end(), 0u);
-  std::sort(idx.begin(), idx.end(), [&](uint32_t i, uint32_t j) {
+  const auto before = [&](uint32_t i, uint32_t j) {
     const Chunk &a = ch[i], &b = ch[j];
     if (cost[i] != cost[j]) return cost[i] > cost[j];
     const uint32_t ga = e.panels[a.panel].graph, gb = e.panels[b.panel].graph;
@@ -2974,7 +2974,12 @@ void sort_by_cost(const Engine& e, std::vector<Chunk>& ch, const std::vector<uin
     if (a.strip_begin != b.strip_begin) return a.strip_begin < b.strip_begin;
     if (a.tile_begin != b.tile_begin) return a.tile_begin < b.tile_begin;
     return a.panel < b.panel;
-  });
+  };
+  // The pieces of chunks in this order are in it already, but for those of cut chunks, which come last:
+  // only they are sorted (a level of a large batch has 0.3 M chunks).
+  const auto tail = std::is_sorted_until(idx.begin(), idx.end(), before);
+  std::sort(tail, idx.end(), before);
+  std::inplace_merge(idx.begin(), tail, idx.end(), before);
   std::vector<Chunk> sorted(ch.size());
   for (size_t i = 0; i < idx.size(); ++i) sorted[i] = ch[idx[i]];
   ch.swap(sorted);
@@ -2983,20 +2988,23 @@ void sort_by_cost(const Engine& e, std::vector<Chunk>& ch, const std::vector<uin
 // The pieces of a level's chunks: heaviest first, or in the chunks' launch order (one that the caller
 // has set).
 std::vector<Chunk> level_pieces(const Engine& e, uint32_t k, bool by_cost) {
-  std::vector<Chunk> out;
-  std::vector<uint64_t> cost;
+  std::vector<Chunk> out, cut;
+  std::vector<uint64_t> cost, cut_cost;
   for (const Chunk& c : e.host_chunks[k]) {
     const GraphPlan& g = e.graphs[e.panels[c.panel].graph];
     const auto it = std::lower_bound(g.chunks.begin(), g.chunks.end(), c, [](const Chunk& a, const Chunk& b) {
       return a.strip_begin != b.strip_begin ? a.strip_begin < b.strip_begin : a.tile_begin < b.tile_begin;
     });
     const size_t i = static_cast<size_t>(it - g.chunks.begin());
+    const bool later = by_cost && g.piece_off[i + 1] - g.piece_off[i] > 1;
     for (uint32_t p = g.piece_off[i]; p < g.piece_off[i + 1]; ++p) {
-      out.push_back(g.pieces[p]);
-      out.back().panel = c.panel;
-      cost.push_back(g.piece_cost[p]);
+      (later ? cut : out).push_back(g.pieces[p]);
+      (later ? cut : out).back().panel = c.panel;
+      (later ? cut_cost : cost).push_back(g.piece_cost[p]);
     }
   }
+  out.insert(out.end(), cut.begin(), cut.end());
+  cost.insert(cost.end(), cut_cost.begin(), cut_cost.end());
   if (by_cost) sort_by_cost(e, out, cost);
   return out;
 }
