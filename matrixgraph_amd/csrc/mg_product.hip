@@ -1028,6 +1028,9 @@ struct DenseTask {
 // 204 registers, enough for two.
 constexpr uint32_t kStep = 2;
 static_assert(kTaskPairs <= kWave);
+// Every operand value is 0, 1 or 2 and every product 0, 1 or 4, so the FP32 sums are integers below 2^24
+// in any order of the additions: no bit of a count is lost and sums > 0 is exactly counts > 0.
+static_assert(kTaskPairs * kTile * 4 <= 1u << 24, "FP32 sums of a task are exact");
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) dense_contract_kernel(const DenseTask* __restrict__ tasks,
                                                                 const uint32_t* __restrict__ n_tasks_ptr,
                                                                 const uint2* __restrict__ pairs,
