@@ -1195,11 +1195,12 @@ uint64_t word_room(uint64_t n) {
 // edges a vertex and of frontiers with them: by windows 12 us of launches (45 with B's index to build, and 3
 // passes over its bitmap) and 2.5 a window that holds a tile, by tiles 0.22 a tile, and 0.02 and
 // 0.06 a pair. Where many pairs meet in each C tile, one wave is at it for long (up to 2.6 us a pair of
-// dense tiles): windows, sooner where they cost no index.
-constexpr uint64_t kPairsPerTile = 64, kPairsPerTileIndexed = 12;
-bool by_tiles(uint32_t ns, uint64_t n_a, uint64_t n_c, uint64_t pairs, bool indexed) {
+// dense tiles): windows, sooner where they cost no index, and for callers that ask for set bits, whose
+// tiles are dense (64 pairs a C tile, all of them recorded: 0.18 ms by windows, 0.38 by tiles).
+constexpr uint64_t kPairsPerTile = 64, kFewPairsPerTile = 12;
+bool by_tiles(uint32_t ns, uint64_t n_a, uint64_t n_c, uint64_t pairs, bool indexed, bool want_bits) {
   if (ns > kBitmapStrips) return true;
-  if (pairs > (indexed ? kPairsPerTileIndexed : kPairsPerTile) * n_c) return false;
+  if (pairs > (indexed || want_bits ? kFewPairsPerTile : kPairsPerTile) * n_c) return false;
   const double strip_windows = static_cast<double>((ns + kWindow - 1) / kWindow);
   const double slots = std::max(1.0, std::min<double>(ns, static_cast<double>(n_a)) * strip_windows);
   const double windows = -slots * std::expm1(-static_cast<double>(n_c) / slots);  // tiles spread evenly
@@ -1263,7 +1264,7 @@ void product_inputs(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_ma
   const bool pa = prepared(a), pb = prepared(bt), same = a == bt;
   // Unknown: as many as there are where the tiles spread evenly.
   P.pairs = pairs ? pairs : static_cast<uint64_t>(a->n_nz_tile) * bt->n_nz_tile / std::max(1u, ns);
-  const bool bitmap = !by_tiles(ns, a->n_nz_tile, c.n_c, P.pairs, pb || known.bm);
+  const bool bitmap = !by_tiles(ns, a->n_nz_tile, c.n_c, P.pairs, pb || known.bm, want_bits);
   const uint64_t na = pa ? 0 : a->n_nz_tile, nb = pb ? 0 : bt->n_nz_tile;
   const bool index_b = bitmap && !pb;
   const uint64_t bm = index_b && !known.bm ? 2ull * ns * wpr : 0;  // u64 words
