@@ -1193,10 +1193,12 @@ uint64_t word_room(uint64_t n) {
 // numbers of tiles and of the tile pairs that meet; `indexed`: B's index is there already.
 // Times in ns, fitted to products of R-MAT and Erdos-Renyi graphs of 2^8 to 2^21 vertices with 1/16 to 16
 // edges a vertex and of frontiers with them: by windows 12 us of launches (45 with B's index to build, and 3
-// passes over its bitmap) and 2.5 a window that holds a tile, by tiles 0.22 a tile, and 0.02 and
-// 0.06 a pair. Where many pairs meet in each C tile, one wave is at it for long (up to 2.6 us a pair of
-// dense tiles): windows, sooner where they cost no index, and for callers that ask for set bits, whose
-// tiles are dense (64 pairs a C tile, all of them recorded: 0.18 ms by windows, 0.38 by tiles).
+// passes over its bitmap), 2.5 a window that holds a tile and 0.02 a pair; by tiles 0.22 a tile, 0.06 a pair
+// and twice that for pairs beyond kFewPairsPerTile in each C tile, which come from denser tiles (R-MAT 13, 46
+// pairs: 108 us by windows, 122 by tiles; Erdos-Renyi 2^12 vertices, 62 pairs: 60 and 20). Where many meet, one wave
+// is at it for long (up to 2.6 us a pair of dense tiles): windows, sooner where they cost no index, and
+// for callers that ask for set bits, whose tiles are dense (64 pairs a C tile, all of them recorded: 0.18 ms
+// by windows, 0.38 by tiles).
 constexpr uint64_t kPairsPerTile = 64, kFewPairsPerTile = 12;
 bool by_tiles(uint32_t ns, uint64_t n_a, uint64_t n_c, uint64_t pairs, bool indexed, bool want_bits) {
   if (ns > kBitmapStrips) return true;
@@ -1205,8 +1207,8 @@ bool by_tiles(uint32_t ns, uint64_t n_a, uint64_t n_c, uint64_t pairs, bool inde
   const double slots = std::max(1.0, std::min<double>(ns, static_cast<double>(n_a)) * strip_windows);
   const double windows = -slots * std::expm1(-static_cast<double>(n_c) / slots);  // tiles spread evenly
   const double index = indexed ? 12e3 : 45e3 + 0.01 * ns * ((ns + 63) / 64);
-  return 0.22 * static_cast<double>(n_c) + 0.06 * static_cast<double>(pairs) <
-         index + 2.5 * windows + 0.02 * static_cast<double>(pairs);
+  const double few = static_cast<double>(std::min(pairs, kFewPairsPerTile * n_c)), all = static_cast<double>(pairs);
+  return 0.22 * static_cast<double>(n_c) + 0.06 * few + 0.12 * (all - few) < index + 2.5 * windows + 0.02 * all;
 }
 
 }  // namespace
