@@ -244,18 +244,21 @@ int mg_multiply_symbolic(mg_context* ctx, const mg_tiled_matrix* a, const mg_til
  * X_{k+1} = X_k * A, takes A^T at every hop. Per tile 16 bytes of payload, twice 16 bytes of head,
  * 4 bytes of index and 8 bytes per column in use; up to 16384 strips a bitmap of 16 bytes per 64 tiles
  * of the n_strips x n_strips grid. No counterpart in the reference (its products re-read every
- * tile). The kept copy is dropped by the next library call that writes m's tiles (a numeric pass
+ * tile). Without memory for the column words it keeps the rest, and the products make the words from
+ * the tiles. The kept copy is dropped by the next library call that writes m's tiles (a numeric pass
  * into m); after writing m's arrays through the pointers of mg_tiled_matrix_device_arrays, call it
  * again. A call while the kept copy is current does nothing; otherwise it synchronises the
  * context's stream. */
 int mg_tiled_matrix_prepare_operand(mg_context* ctx, mg_tiled_matrix* m);
 /* Numeric pass into a C produced by mg_multiply_symbolic (OR-accumulates).
  * Replaces PPRQuery::FillTilesUnifiedMemory (ppr_query.cu:459-780). Asynchronous on the
- * context's stream; keeps 32 bytes per C tile and, of operands that are not prepared, 16 bytes of
- * head per tile, 8 per column in use of a tile and B's index in the context's scratch, which grows
+ * context's stream. In the context's scratch: 16 bytes of head per tile of operands that are not
+ * prepared and room for their column words, 8 bytes a column in use of a tile; where the product goes
+ * by windows of C (see mg_product.hip) also 32 bytes per C tile and B's index. The scratch grows
  * in stream order (hipMallocAsync/hipFreeAsync on that stream: queued work that reads the old
- * buffer finishes before its memory is reused). Without memory for the column words it makes them
- * from the tiles. */
+ * buffer finishes before its memory is reused); above 1/64 of the card's memory it is given back in
+ * stream order when the call returns. Without memory for the column words it makes them from the
+ * tiles. */
 int mg_multiply_numeric(mg_context* ctx, const mg_tiled_matrix* a, const mg_tiled_matrix* bt,
                         mg_tiled_matrix* c);
 /* The numeric pass with a per-tile-pair choice of engine: a pair whose two tiles both have
@@ -418,10 +421,9 @@ typedef struct mg_hop_stats {
 } mg_hop_stats;
 
 /* Allocates X_0..X_max_hops (W = ceil(max_sources/64) rounded up to a power of two,
- * max_sources <= 4096) plus the strip scheduler, the per-tile row-occupancy masks of at
- * a job list of at (4 bytes per set bit, tile and strip) and (unless MG_WALK_SWEEP_FIRST_HOP) a
- * column index of it (16 bytes per tile). at must
- * outlive w and keep its contents (the masks are taken here).
+ * max_sources <= 4096) plus the strip scheduler and, of at, per-tile row-occupancy masks, a job list
+ * (4 bytes per set bit, tile and strip) and (unless MG_WALK_SWEEP_FIRST_HOP) a column index
+ * (16 bytes per tile). at must outlive w and keep its contents (the masks are taken here).
  * The first hop of a run is pushed from the source strips when their columns of at hold at
  * most half of its tiles; results and statistics are the same either way. */
 int mg_walk_create(mg_context* ctx, const mg_tiled_matrix* at, uint32_t max_sources,

@@ -64,7 +64,7 @@ Dims make_dims(uint32_t n_in, uint32_t n_out) {
 // (unit_of(t, v, 0), unit_of(t, v, 32)) with no data moved between lanes; the weights (A operands)
 // are loaded once per wave in that order. A wave that streamed samples with lane = unit needed a
 // broadcast per multiply and 256 samples in series: 200 K rows forward took 104 us, the gradient of
-// 4096 rows 370 us; now 33 (the matrix instructions alone 12) and 15. Relative error against 64
+// 4096 rows 370 us; now 36 (the matrix instructions alone 12) and 14. Relative error against 64
 // bits, 100 to 40 K rows: outputs 1.36e-7 (1.60e-7 before), gradients 0.81e-7 (1.25e-7).
 typedef float mg_v16f __attribute__((ext_vector_type(16)));
 constexpr uint32_t kTileRows = 32;

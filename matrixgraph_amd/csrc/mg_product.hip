@@ -24,9 +24,9 @@
 // Measured (both operands prepared), against one wave per C tile that searches the shorter tile list
 // in the longer one and multiplies payloads of 16 bytes: A*A of R-MAT 14 119 us, before 518; of
 // R-MAT 16 with 16 planted communities (191 K tiles, 70 M pairs) 1.28 ms, before 4.63; a frontier of
-// 1000 rows x R-MAT 18 (7.3 K tiles, 6.8 M pairs) 140 us, before 482. Bound by the vector ALUs (75 %
-// of the issue slots on the second) and by the chains of ballots and LDS writes in between: filling the
-// queue of stage 3 is half of the time, the ORs themselves nothing.
+// 1000 rows x R-MAT 18 (7.3 K tiles, 6.8 M pairs) 140 us, before 482. Bound by the chains of ballots
+// and LDS writes between the stages and by the vector ALUs (58 % of the issue slots on the second): filling
+// the queue of stage 3 is half of the time, the ORs themselves nothing.
 #include <algorithm>
 #include <cmath>
 #include <string>
